@@ -248,3 +248,46 @@ def tolerance(case):
     # 50000 values, exponentials, tanh) were within 1.2e-7 and 3.5e-7.
     dtype = case.get("dtype", "bfloat16" if kind == "matmul_int8" else "float32")
     return {"bfloat16": {"rel": 7e-3, "max": 1.6e-2}, "float16": {"rel": 9e-4, "max": 2e-3}, "float32": {"rel": 1e-6, "max": 4e-6}}[dtype]
+
+
+def exact(case, seed):
+    """The outputs of `run` for these inputs by plain torch in float64; None for integers made by rounding."""
+    c, kind = case, case["kind"]
+    generator = torch.Generator(device="cuda")
+    generator.manual_seed(seed)
+    inputs = _inputs(c, generator)
+
+    def const(value):   # constants of a description are float32
+        return torch.tensor(value, dtype=torch.float32, device="cuda").double()
+
+    if kind == "segment_sum":
+        data, ids = inputs
+        return [torch.zeros(c["segments"], c["width"], dtype=torch.float64, device="cuda").index_add_(0, ids.long(), data.double())]
+    d = [t.double() for t in inputs]
+    del inputs
+    if kind == "elementwise":
+        return [torch.tanh((d[0] + d[1]) * d[2])]
+    if kind == "masked_softmax":
+        return [torch.softmax((1 - d[0]) * -10000.0 + 0.125 * d[1], -1)]
+    if kind == "attention":
+        return [torch.softmax(torch.bmm(d[0], d[1].transpose(1, 2).contiguous()) * const(c["k"] ** -0.5) + d[2], -1)]
+    if kind == "quant":
+        return [None, (d[0] + d[1]).abs().amax(1) / 127]
+    if kind == "bias_grad":
+        return [(d[0] * d[1]).sum(0), d[0].sum(0)]
+    if kind == "layernorm" or kind == "batchnorm":
+        axes = (1,) if kind == "layernorm" else (0, 2, 3)
+        mean = d[0].mean(axes, keepdim=True)
+        centred = d[0] - mean
+        variance = (centred * centred).mean(axes, keepdim=True)
+        y = centred * torch.rsqrt(variance + const(1e-5)) * d[1] + d[2]
+        return [y + d[3]] if kind == "layernorm" else [y, mean, variance]
+    if kind == "matmul":
+        y = d[0] @ (d[1].t() if c["tb"] else d[1]) + d[2]
+        if c["act"] == "relu":
+            return [y.clamp_(min=0)]
+    else:
+        y = d[0] @ (d[2].t() if c["tb"] else d[2]) * d[1] * d[3] + d[4]
+    if kind == "matmul_int8" or c["act"] == "gelu":
+        y = y * (torch.tanh((y + y * y * y * const(0.044715)) * const(0.7978845608028654)) + 1) * 0.5
+    return [y]
