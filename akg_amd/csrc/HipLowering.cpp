@@ -18,6 +18,7 @@ const char *kernelFamilyName(KernelFamily f) {
     case KernelFamily::ColumnReduce: return "column_reduce";
     case KernelFamily::Indexed: return "indexed";
     case KernelFamily::SegmentSum: return "segment_sum";
+    case KernelFamily::GemmRows: return "gemm_rows";
     case KernelFamily::Staged: return "staged";
   }
   return "?";
@@ -607,7 +608,18 @@ LoweredKernel lowerToHip(const OpGraph &described, const LoweringOptions &option
     if (op.kind == OpKind::SegmentSum) return lowerSegmentSumToHip(graph, options);
   }
   if (wantsIndexedKernel(graph)) return lowerIndexedToHip(graph, options);
-  if (hasMatMul) return lowerGemmToHip(graph, options);
+  if (hasMatMul) {
+    bool reduces = false;
+    for (const OpNode &op : graph.ops) reduces = reduces || lowering::isReduceKind(op.kind);
+    if (reduces && !options.extentAsArgument && !(options.variant & 16)) {
+      try {
+        return lowerGemmRowsToHip(graph);
+      } catch (const LoweringError &) {
+        // several kernels then: the contraction's refusal below is what cuts the description behind it
+      }
+    }
+    return lowerGemmToHip(graph, options);
+  }
   if (wantsStreamReduce(graph)) {
     // A reduction result that meets the unreduced tensor again is not for the streaming kernels, which keep nothing of
     // what they read: the column kernel keeps the run in registers, if it fits. Failing both, the first reason stands.

@@ -31,7 +31,7 @@ class LoweringError : public std::runtime_error {
   explicit LoweringError(const std::string &msg) : std::runtime_error(msg) {}
 };
 
-enum class KernelFamily { Elementwise, RowReduce, GemmEpilogue, StreamReduce, Indexed, SegmentSum, Staged, ColumnReduce };
+enum class KernelFamily { Elementwise, RowReduce, GemmEpilogue, StreamReduce, Indexed, SegmentSum, Staged, ColumnReduce, GemmRows };
 const char *kernelFamilyName(KernelFamily f);
 
 // Tuning knobs; 0 means "let the heuristic decide". They can be set through the environment
@@ -45,6 +45,7 @@ struct LoweringOptions {
   // Experiment switch (AKG_HIP_VARIANT), read by whichever family lowers the kernel; 0 = the measured default.
   //   gemm_epilogue  bit 3: no skinny kernel for M <= 64 (the tile kernel with K split instead),
   //                  bit 5: the other arrangement of the tile kernel's wavefronts (2 x 4 for 4 x 2 and back)
+  //                  bit 4: a contraction and the row reductions behind it as two kernels (no gemm_rows)
   //   row_reduce     1: keep the row in registers, 2: walk the row (no packing), 4: walk it, packed if possible
   //   stream_reduce  7: no column kernel (several kernels instead)
   //   column_reduce  5: one strip per workgroup (no second set of resident registers)
@@ -101,6 +102,8 @@ LoweredKernel lowerToHip(const OpGraph &graph, const LoweringOptions &options);
 
 // Family-specific entries used by lowerToHip (HipLoweringGemm.cpp, HipLoweringReduce.cpp, HipLoweringIndexed.cpp).
 LoweredKernel lowerGemmToHip(const OpGraph &graph, const LoweringOptions &options);
+// A contraction with reductions over the rows of its result (HipLoweringGemmRows.cpp).
+LoweredKernel lowerGemmRowsToHip(const OpGraph &graph);
 LoweredKernel lowerStreamReduceToHip(const OpGraph &graph, const LoweringOptions &options);
 // One reduced axis that is not the innermost one, reduction results used against the unreduced tensor (HipLoweringColumn.cpp).
 LoweredKernel lowerColumnToHip(const OpGraph &graph, const LoweringOptions &options);

@@ -1,0 +1,359 @@
+/**
+ * Lowering of a contraction whose result meets reductions over its last axis: attention probabilities (scores, scale,
+ * mask, softmax) in one kernel. The scores of sixteen rows stay in the registers of the workgroup that computed them
+ * (kernels/akg_gemm_rows.hpp), so the float32 [batch,M,N] tensor between the contraction and the row kernel never
+ * exists in memory. What this kernel does not take runs as a contraction followed by a row kernel.
+ *
+ * The reference lowers the two parts as separate loop nests over the materialised scores
+ * (akg-mlir/lib/Conversion/MindSporeToLinalg/MindSporeToLinalg.cpp:791-901,1511-1546).
+ */
+#include <algorithm>
+#include <sstream>
+
+#include "HipLowering.h"
+
+namespace akg {
+namespace {
+
+using lowering::computeTypeName;
+using lowering::dtypeTag;
+
+enum class Rank { None, Const, Row, Full };   // Row: one value per row of C (or one value); Full: a value per element
+
+class GemmRowsEmitter {
+ public:
+  explicit GemmRowsEmitter(const OpGraph &g) : g_(g) {}
+
+  LoweredKernel run() {
+    analyse();
+    pickSchedule();
+    emitBody();
+    LoweredKernel k;
+    k.kernelName = g_.name + "_kernel";
+    k.source = assemble();
+    k.family = KernelFamily::GemmRows;
+    k.grid[0] = static_cast<unsigned>(perXcd() * 8);
+    k.block[0] = static_cast<unsigned>(64 * wavesC_ * wavesR_);
+    k.algorithmicBytes = lowering::countAlgorithmicBytes(g_);
+    k.algorithmicOps = 2ull * static_cast<uint64_t>(batch_ * m_) * static_cast<uint64_t>(n_ * k_);
+    k.shapeArgs = lowering::buildShapeArgs(g_);
+    std::ostringstream note;
+    note << "gemm_rows batch=" << batch_ << " M=" << m_ << " N=" << n_ << " K=" << k_ << " rows per workgroup=" << groupRows()
+         << " wavefronts per row=" << wavesC_ << " units of 32 columns per wavefront=" << chunks_ << " grid=" << k.grid[0];
+    k.scheduleNote = note.str();
+    return k;
+  }
+
+ private:
+  struct Val {
+    Rank rank = Rank::None;
+    std::string ident;
+  };
+
+  const OpGraph &g_;
+  std::ostringstream src_;
+  std::vector<Val> vals_;
+  std::vector<bool> relaxed_;
+  int matmulOp_ = -1, aId_ = -1, bId_ = -1, accId_ = -1;
+  int64_t batch_ = 1, m_ = 0, n_ = 0, k_ = 0;
+  int wavesC_ = 1, wavesR_ = 1, rowTiles_ = 1, chunks_ = 1, reductions_ = 0;
+
+  int64_t groupRows() const { return 16L * rowTiles_ * wavesR_; }
+  int64_t rowGroups() const { return (m_ + groupRows() - 1) / groupRows(); }
+  int64_t perXcd() const { return (batch_ * rowGroups() + 7) / 8; }
+  const char *mma() const { return g_.tensor(aId_).dtype == DType::BF16 ? "akg::MmaBF16" : "akg::MmaF16"; }
+
+  void analyse() {
+    bool reduces = false;
+    for (size_t i = 0; i < g_.ops.size(); ++i) {
+      const OpNode &op = g_.ops[i];
+      if (op.outputs.size() != 1) throw LoweringError("op " + op.name + ": multiple results are not supported");
+      if (op.kind == OpKind::MatMul) {
+        if (matmulOp_ >= 0) throw LoweringError("only one MatMul per kernel is supported");
+        matmulOp_ = static_cast<int>(i);
+      } else if (lowering::isReduceKind(op.kind)) {
+        reduces = true;
+      } else if (!lowering::isElementwiseKind(op.kind) || op.kind == OpKind::Assign || op.kind == OpKind::Iota) {
+        throw LoweringError("op " + op.name + " cannot follow a MatMul in one kernel with its row reductions");
+      }
+    }
+    if (matmulOp_ < 0 || !reduces) throw LoweringError("no MatMul with reductions behind it");
+    const OpNode &mm = g_.ops[static_cast<size_t>(matmulOp_)];
+    aId_ = mm.inputs[0];
+    bId_ = mm.inputs[1];
+    accId_ = mm.outputs[0];
+    const TensorValue &a = g_.tensor(aId_), &b = g_.tensor(bId_), &c = g_.tensor(accId_);
+    const size_t rank = a.shape.size();
+    if (mm.transposeA || !mm.transposeB || a.inputIndex < 0 || b.inputIndex < 0 || a.dtype != b.dtype ||
+        (a.dtype != DType::BF16 && a.dtype != DType::F16) || c.dtype != DType::F32 || (rank != 2 && rank != 3) ||
+        b.shape.size() != rank || c.shape.size() != rank) {
+      throw LoweringError("MatMul: row reductions follow 16-bit operands [M,K] x [N,K] with a float32 result");
+    }
+    batch_ = rank == 3 ? a.shape[0] : 1;
+    m_ = a.shape[rank - 2];
+    k_ = a.shape[rank - 1];
+    n_ = b.shape[rank - 2];
+    if ((rank == 3 && (b.shape[0] != batch_ || c.shape[0] != batch_)) || b.shape[rank - 1] != k_ || c.shape[rank - 2] != m_ ||
+        c.shape[rank - 1] != n_ || batch_ < 1 || m_ < 1) {
+      throw LoweringError("MatMul: inconsistent shapes");
+    }
+    // Where the line lies (bf16 or f16, GPU time of one kernel against a contraction and a row kernel):
+    //   [192,512,64]x512 77 us for 149, [384,256,64]x256 43 for 142, [24,2048,64]x2048 174 for 238, [380,77,64]x80 8.7 for 48;
+    //   every row group reads all of B from the L2, which costs more than the scores' way through memory once B is large
+    //   ([20,1200,128]x2048, 512 KiB of B: 136 us for 126; [384,37,128]x1000, 250 KiB: 61 for 85), and a single query uses one of its sixteen rows ([300,1,64]x2048:
+    //   24 us for 17, four rows 31 for 32);
+    //   few row groups leave the chip idle ([1,256,64]x1024, 16 groups: 9.1 us for 7.9; [3,512,128]x512, 96: 7.8 for 10.1);
+    //   scores below 1 MiB stay in the caches, and both forms take the time of their launches.
+    if (k_ % 32 != 0 || n_ % 8 != 0 || n_ > 2048 || n_ * k_ > (1LL << 17)) throw LoweringError("MatMul: operands of this shape have no row kernel");
+    if (m_ < 4 || batch_ * m_ * n_ * 4 < (1LL << 20)) throw LoweringError("MatMul: too few rows or scores for the row kernel");
+    for (const OpNode &op : g_.ops) {
+      if (op.kind == OpKind::MatMul) continue;
+      for (int in : op.inputs) {
+        if (in == aId_ || in == bId_) throw LoweringError("MatMul operands cannot also feed the ops behind it");
+      }
+    }
+    for (const TensorValue &t : g_.tensors) {
+      if (!t.isConst && (t.inputIndex >= 0 || t.outputIndex >= 0) && t.numel() * static_cast<int64_t>(dtypeSize(t.dtype)) >= (1LL << 31)) {
+        throw LoweringError("tensor " + t.name + ": the row kernel addresses less than 2 GiB per tensor");
+      }
+    }
+  }
+
+  // Wavefronts that share a row: at most four units of 32 columns each (32 values a lane) up to 2048 columns; short rows
+  // fill the workgroup with row groups instead. Two row tiles per wavefront where 512 workgroups are left: every
+  // fragment of B is then read for 32 rows ([192,512,64] x 512: 77 us, one row tile 95, four 76; with 48 workgroups
+  // instead of 96 [3,512,128] x 512 takes 9.9 us instead of 7.8).
+  void pickSchedule() {
+    const int64_t units = (n_ + 31) / 32;
+    wavesC_ = 1;
+    while (wavesC_ < 16 && units > 4 * wavesC_) wavesC_ *= 2;
+    chunks_ = static_cast<int>((units + wavesC_ - 1) / wavesC_);
+    auto shape = [&](int rowTiles) {
+      rowTiles_ = rowTiles;
+      wavesR_ = 1;
+      while (wavesC_ * wavesR_ < 4 && m_ > 16L * rowTiles_ * wavesR_) wavesR_ *= 2;
+      return batch_ * rowGroups();
+    };
+    if (m_ <= 16 || shape(2) < 512) shape(1);
+    if (batch_ * rowGroups() < 64) throw LoweringError("MatMul: too few row groups for the row kernel");
+  }
+
+  std::string ctOf(int id) const { return computeTypeName(g_.tensor(id).dtype); }
+  std::string tagOf(int id) const { return dtypeTag(g_.tensor(id).dtype); }
+  std::string operand(int id) const {
+    const Val &v = vals_[static_cast<size_t>(id)];
+    return v.rank == Rank::Full ? v.ident + "[j][e]" : v.ident;
+  }
+
+  // extents of a tensor against [batch, M, N]: every one is 1 or the full extent
+  std::vector<int64_t> spread(const TensorValue &t) const {
+    std::vector<int64_t> s = t.shape;
+    while (s.size() > 3 && s.front() == 1) s.erase(s.begin());
+    if (s.size() > 3) throw LoweringError("tensor " + t.name + " does not broadcast to the MatMul result");
+    while (s.size() < 3) s.insert(s.begin(), 1);
+    const int64_t full[3] = {batch_, m_, n_};
+    for (int d = 0; d < 3; ++d) {
+      if (s[static_cast<size_t>(d)] != 1 && s[static_cast<size_t>(d)] != full[d]) {
+        throw LoweringError("tensor " + t.name + " does not broadcast to the MatMul result");
+      }
+    }
+    return s;
+  }
+
+  // row of the tensor (in rows of its last extent) that belongs to row akg_mc of batch akg_b
+  std::string rowOf(const std::vector<int64_t> &s) const {
+    const bool b = s[0] != 1, m = s[1] != 1;
+    if (b && m) return "(akg_b * M + akg_mc)";
+    if (b) return "akg_b";
+    return m ? "akg_mc" : "0L";
+  }
+
+  void loops(const std::string &indent) {
+    src_ << "#pragma unroll\n" << indent << "for (int j = 0; j < NCHUNK; ++j) {\n#pragma unroll\n" << indent << "  for (int e = 0; e < 8; ++e) ";
+  }
+
+  void emitInput(size_t i) {
+    const int id = g_.inputs[i];
+    const TensorValue &t = g_.tensor(id);
+    if (id == aId_ || id == bId_ || !t.used) return;
+    const std::vector<int64_t> s = spread(t);
+    Val &v = vals_[static_cast<size_t>(id)];
+    const std::string tag = tagOf(id), ct = ctOf(id);
+    if (s[2] == 1) {
+      v.rank = Rank::Row;
+      v.ident = "r_in" + std::to_string(i);
+      src_ << "    const " << ct << " " << v.ident << " = " << tag << "::load(in" << i << "[" << rowOf(s) << "]);\n";
+      return;
+    }
+    v.rank = Rank::Full;
+    v.ident = "t_in" + std::to_string(i);
+    src_ << "    " << ct << " " << v.ident << "[NCHUNK][8];\n#pragma unroll\n    for (int j = 0; j < NCHUNK; ++j) akg::load_chunk_if<" << tag
+         << ", 8, false>(b_in" << i << ", akg_ok[j], " << rowOf(s) << " * N + akg_cols[j], " << v.ident << "[j]);\n";
+  }
+
+  void emitReduction(const OpNode &op) {
+    const int in = op.inputs[0], out = op.outputs[0];
+    const TensorValue &it = g_.tensor(in), &ot = g_.tensor(out);
+    if (vals_[static_cast<size_t>(in)].rank != Rank::Full || it.numel() != batch_ * m_ * n_ || op.axes.size() != 1 ||
+        op.axes[0] + 1 != static_cast<int64_t>(it.shape.size()) || it.shape.back() != n_) {
+      throw LoweringError("op " + op.name + ": only reductions of the whole scores over their last axis");
+    }
+    const lowering::ReduceSpec spec = lowering::reduceSpec(op, ot.dtype);
+    if (spec.ordered || spec.roundEachStep || ctOf(in) != ctOf(out) || (ctOf(out) != "float" && ctOf(out) != "int")) {
+      throw LoweringError("op " + op.name + ": the row kernel reduces 32-bit values");
+    }
+    if (!op.keepDims) {
+      for (const OpNode &user : g_.ops) {
+        for (int u : user.inputs) {
+          if (u == out) throw LoweringError("op " + op.name + ": a result without keep_dims is only written");
+        }
+      }
+    }
+    const std::string ct = ctOf(out), acc = "acc" + std::to_string(out), u = "u" + std::to_string(out);
+    const std::string value = vals_[static_cast<size_t>(in)].ident;
+    src_ << "    " << ct << " " << acc << " = " << spec.init << ";  // " << op.name << " -> " << ot.name << "\n"
+         << "#pragma unroll\n    for (int j = 0; j < NCHUNK; ++j) {\n"
+         << "      " << ct << " akg_part = " << value << "[j][0];\n#pragma unroll\n"
+         << "      for (int e = 1; e < 8; ++e) akg_part = " << spec.combiner << "::apply(akg_part, " << value << "[j][e]);\n"
+         << "      " << acc << " = akg_ok[j] ? " << spec.combiner << "::apply(" << acc << ", akg_part) : " << acc << ";\n    }\n"
+         << "    const " << ct << " " << u << " = akg::row_scores_reduce<" << spec.combiner << ", WC>(" << acc
+         << ", reinterpret_cast<" << ct << " (*)[16]>(akg_slots[" << reductions_ << "][rt][wr]), wc, lane);\n";
+    ++reductions_;
+    vals_[static_cast<size_t>(out)].rank = Rank::Row;
+    vals_[static_cast<size_t>(out)].ident = u;
+  }
+
+  void emitElementwise(const OpNode &op) {
+    const int out = op.outputs[0];
+    const TensorValue &ot = g_.tensor(out);
+    const std::vector<int64_t> shape = spread(ot);
+    Rank rank = Rank::Row;
+    std::vector<std::string> operands;
+    for (int in : op.inputs) {
+      const Val &v = vals_[static_cast<size_t>(in)];
+      if (v.rank == Rank::None) throw LoweringError("op " + op.name + ": operand " + g_.tensor(in).name + " is undefined");
+      if (!g_.tensor(in).isConst) spread(g_.tensor(in));
+      if (v.rank == Rank::Full) rank = Rank::Full;
+      operands.push_back(operand(in));
+    }
+    if ((rank == Rank::Full) != (shape[2] == n_)) throw LoweringError("op " + op.name + ": result shape does not match its operands");
+    const bool relaxed = relaxed_[static_cast<size_t>(out)];
+    const std::string ct = ctOf(out), id = std::to_string(out);
+    std::string expr;
+    // a float32 division by a per-row value: the reciprocal (or the divisor's parts) once per row, as in the row kernel
+    const bool uniformDivisor = op.kind == OpKind::Div && rank == Rank::Full && op.inputs.size() == 2 &&
+                                vals_[static_cast<size_t>(op.inputs[1])].rank != Rank::Full && ct == "float" &&
+                                ctOf(op.inputs[0]) == "float" && ctOf(op.inputs[1]) == "float";
+    if (uniformDivisor) {
+      if (relaxed) {
+        src_ << "    const float d" << id << " = akg::fast_rcp(" << operands[1] << ");\n";
+        expr = "(" + operands[0] + " * d" + id + ")";
+      } else {
+        src_ << "    const akg::UniformDivisor d" << id << " = akg::make_divisor(" << operands[1] << ");\n";
+        expr = "akg::div_uniform(" + operands[0] + ", d" + id + ")";
+      }
+      if (ot.dtype == DType::F16 || ot.dtype == DType::BF16) expr = tagOf(out) + "::rnd(" + expr + ")";
+    } else {
+      expr = lowering::elementwiseExpr(g_, op, operands, relaxed);
+    }
+    Val &v = vals_[static_cast<size_t>(out)];
+    v.rank = rank;
+    if (rank == Rank::Full) {
+      v.ident = "t" + id;
+      src_ << "    " << ct << " " << v.ident << "[NCHUNK][8];  // " << op.name << " -> " << ot.name << "\n";
+      loops("    ");
+      src_ << v.ident << "[j][e] = " << expr << ";\n    }\n";
+    } else {
+      v.ident = "u" + id;
+      src_ << "    const " << ct << " " << v.ident << " = " << expr << ";  // " << op.name << " -> " << ot.name << "\n";
+    }
+  }
+
+  void emitBody() {
+    vals_.assign(g_.tensors.size(), Val());
+    relaxed_ = lowering::relaxedPrecisionTensors(g_);
+    for (size_t t = 0; t < g_.tensors.size(); ++t) {
+      if (!g_.tensors[t].isConst) continue;
+      vals_[t].rank = Rank::Const;
+      vals_[t].ident = lowering::literalFor(g_.tensors[t].dtype, g_.tensors[t].constValue);
+    }
+    vals_[static_cast<size_t>(accId_)].rank = Rank::Full;
+    vals_[static_cast<size_t>(accId_)].ident = "akg_s[rt]";
+    for (size_t i = 0; i < g_.inputs.size(); ++i) emitInput(i);
+    for (const OpNode &op : g_.ops) {
+      if (op.kind == OpKind::MatMul) continue;
+      if (lowering::isReduceKind(op.kind)) {
+        emitReduction(op);
+      } else {
+        emitElementwise(op);
+      }
+    }
+    for (size_t i = 0; i < g_.outputs.size(); ++i) {
+      const int id = g_.outputs[i];
+      const TensorValue &t = g_.tensor(id);
+      const Val &v = vals_[static_cast<size_t>(id)];
+      if (v.rank == Rank::Full && t.numel() == batch_ * m_ * n_) {
+        src_ << "#pragma unroll\n    for (int j = 0; j < NCHUNK; ++j) akg::store_chunk_if<" << tagOf(id) << ", 8, false>(b_out" << i
+             << ", akg_ok[j] && akg_row_ok, (akg_b * M + akg_m) * N + akg_cols[j], " << v.ident << "[j]);\n";
+      } else if (v.rank == Rank::Row && t.numel() == batch_ * m_ && t.inputIndex < 0) {
+        src_ << "    if (akg_row_ok && wc == 0 && lane < 16) out" << i << "[akg_b * M + akg_m] = " << tagOf(id) << "::store(" << v.ident << ");\n";
+      } else {
+        throw LoweringError("output " + t.name + ": shape is neither the scores' nor one value per row");
+      }
+    }
+  }
+
+  std::string assemble() const {
+    std::ostringstream o;
+    o << "// Generated by the akg HIP lowering for gfx950. Op description: " << g_.name << "\n"
+      << "// family: gemm_rows, fusion class: " << operatorTemplateName(g_.operatorTemplate) << "\n"
+      << "#include \"akg_rt.hpp\"\n#include \"akg_gemm_mfma.hpp\"\n#include \"akg_gemm_rows.hpp\"\n\n"
+      << "extern \"C\" __global__ __launch_bounds__(" << 64 * wavesC_ * wavesR_ << ") void " << g_.name << "_kernel(";
+    size_t argc = 0;
+    for (size_t i = 0; i < g_.inputs.size(); ++i, ++argc) {
+      o << (argc ? ", " : "") << "const " << tagOf(g_.inputs[i]) << "::storage *__restrict__ in" << i;
+    }
+    for (size_t i = 0; i < g_.outputs.size(); ++i, ++argc) {
+      o << (argc ? ", " : "") << tagOf(g_.outputs[i]) << "::storage *__restrict__ out" << i;
+    }
+    o << ") {\n  constexpr long M = " << m_ << "L, N = " << n_ << "L, GROUPS = " << rowGroups() << "L;\n"
+      << "  constexpr int RT = " << rowTiles_ << ", NCHUNK = " << chunks_ << ", WC = " << wavesC_ << ", WR = " << wavesR_ << ";\n"
+      << "  __shared__ float akg_slots[" << std::max(1, reductions_) << "][RT][WR][WC][16];\n"
+      << "  // consecutive workgroups go round-robin to the 8 XCDs: regrouped, so that the workgroups of a batch share an L2\n"
+      << "  const long akg_linear = static_cast<long>(blockIdx.x % 8u) * " << perXcd() << "L + static_cast<long>(blockIdx.x / 8u);\n"
+      << "  if (akg_linear >= " << batch_ * rowGroups() << "L) return;\n"
+      << "  const long akg_b = akg_linear / GROUPS;\n"
+      << "  const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;\n"
+      << "  const int wc = wave % WC, wr = wave / WC;\n"
+      << "  const long akg_row0 = (akg_linear % GROUPS) * " << groupRows() << "L + wr * (16 * RT);\n";
+    for (size_t i = 0; i < g_.inputs.size(); ++i) {
+      const TensorValue &t = g_.tensor(g_.inputs[i]);
+      if (g_.inputs[i] == aId_ || g_.inputs[i] == bId_ || !t.used) continue;
+      o << "  const akg::Buffer b_in" << i << " = akg::make_buffer(in" << i << ", " << t.numel() * static_cast<int64_t>(dtypeSize(t.dtype)) << "L);\n";
+    }
+    for (size_t i = 0; i < g_.outputs.size(); ++i) {
+      const TensorValue &t = g_.tensor(g_.outputs[i]);
+      o << "  const akg::Buffer b_out" << i << " = akg::make_buffer(out" << i << ", " << t.numel() * static_cast<int64_t>(dtypeSize(t.dtype)) << "L);\n";
+    }
+    o << "  long akg_cols[NCHUNK];\n  bool akg_ok[NCHUNK];\n#pragma unroll\n  for (int j = 0; j < NCHUNK; ++j) {\n"
+      << "    akg_cols[j] = 32L * akg::row_unit<NCHUNK, WC>(j, wc) + 8 * (lane >> 4);\n    akg_ok[j] = "
+      << (n_ % (32L * wavesC_) == 0 ? "true" : "akg_cols[j] < N") << ";\n  }\n"
+      << "  float akg_s[RT][NCHUNK][8];\n" 
+      << "  akg::row_scores<" << mma() << ", M, N, " << k_ * 2 << "L, RT, NCHUNK, WC>(in" << g_.tensor(aId_).inputIndex << " + akg_b * "
+      << m_ * k_ << "L, in" << g_.tensor(bId_).inputIndex << " + akg_b * " << n_ * k_ << "L, akg_row0, wc, lane, akg_s);\n"
+      << "#pragma unroll\n  for (int rt = 0; rt < RT; ++rt) {\n"
+      << "    const long akg_m = akg_row0 + 16 * rt + (lane & 15);\n    const bool akg_row_ok = akg_m < M;\n"
+      << "    const long akg_mc = akg_row_ok ? akg_m : M - 1;\n    (void)akg_mc;\n"
+      << src_.str() << "  }\n}\n";
+    return o.str();
+  }
+};
+
+}  // namespace
+
+LoweredKernel lowerGemmRowsToHip(const OpGraph &graph) {
+  GemmRowsEmitter emitter(graph);
+  return emitter.run();
+}
+
+}  // namespace akg

@@ -1,0 +1,99 @@
+/**
+ * Scores of a contraction kept in registers for the row reductions behind them (attention probabilities: Q K^T, scale,
+ * mask, softmax): C[M,N] = A[M,K] * B[N,K]^T, sixteen rows of A against all N columns in one workgroup, so that a row
+ * of results is never written before its reductions are done.
+ *
+ * A unit is 16 rows x 32 columns: two 16 x 16 MFMAs per 64 bytes of K with the operands EXCHANGED (the columns of C, rows
+ * of B, are the rows of the MFMA): lane (c = lane % 16, g = lane / 16) then owns row c of the tile, and with column
+ * 8 (r / 4) + 4 h + r % 4 of the unit in row r of MFMA h it owns the EIGHT ADJACENT columns 8 g .. 8 g + 7: a mask or a
+ * result is read and written 16 bytes a lane, whole lines over the four lanes of a row, and a row reduction ends with
+ * two exchanges between lanes (distances 16 and 32) and one LDS step between the wavefronts of a row.
+ * The wavefronts of a row take its units in pairs (row_unit). No LDS holds operands: B is read once per workgroup, straight into MFMA
+ * fragments, from the L2 (the launch keeps the workgroups of a batch on one XCD).
+ * What bounds it: memory (mask in, probabilities out) and the fragments of B from the L2 about equally: bf16
+ * [192,512,64] x 512 with its mask takes 77 us, 4.2 TB/s of what has to move; as a contraction and a row kernel 149 us,
+ * the float32 scores written and read in between. Measured and left out: the mask requested in front of the MFMAs (77 us
+ * either way, more registers: 2048 columns 201 us for 174), non-temporal loads of it (86 us), non-temporal stores (79 us).
+ */
+#pragma once
+
+namespace akg {
+
+// Unit j of wavefront wc: neighbouring units in pairs where their number is even, so that the 16-bit results of a pair
+// fill a whole cache line from one wavefront.
+template <int NCHUNK, int WC>
+AKG_DEV constexpr int row_unit(int j, int wc) {
+  return NCHUNK % 2 == 0 ? ((j / 2) * WC + wc) * 2 + j % 2 : j * WC + wc;
+}
+
+// s[rt][j] = the eight columns of unit j * WC + wc (columns beyond N hold copies of column N - 1) in row
+// row0 + 16 rt + lane % 16 (rows beyond M hold copies of row M - 1). KB: bytes of K per row, a multiple of 64.
+template <typename Mma, long M, long N, long KB, int RT, int NCHUNK, int WC>
+AKG_DEV void row_scores(const void *__restrict__ A, const void *__restrict__ B, long row0, int wc, int lane,
+                        float (&s)[RT][NCHUNK][8]) {
+  static_assert(KB % 64 == 0 && M * KB < (1L << 31) && N * KB < (1L << 31), "operand shapes of the fragments");
+  constexpr int kSlabs = static_cast<int>(KB / 64);
+  const int c = lane & 15, g = lane >> 4;
+  const char *a = static_cast<const char *>(A);
+  const char *b = static_cast<const char *>(B);
+  v4i qf[RT][kSlabs];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const long row = row0 + 16 * rt + c;
+    const u32 off = static_cast<u32>((row < M ? row : M - 1) * KB) + 16u * static_cast<u32>(g);
+#pragma unroll
+    for (int i = 0; i < kSlabs; ++i) qf[rt][i] = *reinterpret_cast<const v4i *>(a + off + 64 * i);
+  }
+  // The fragments of kBatch units are requested together, in front of their MFMAs (left alone, the compiler keeps two
+  // loads in flight and the wavefront waits out the L2 once per MFMA).
+  constexpr int kBatch = kSlabs >= 8 ? 1 : 8 / kSlabs;
+#pragma unroll
+  for (int j0 = 0; j0 < NCHUNK; j0 += kBatch) {
+    v4i kf[kBatch][2][kSlabs];
+#pragma unroll
+    for (int j = j0; j < j0 + kBatch && j < NCHUNK; ++j) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        long col = 32L * row_unit<NCHUNK, WC>(j, wc) + 8 * (c >> 2) + 4 * h + (c & 3);
+        if constexpr (N % (32L * WC) != 0) col = col < N ? col : N - 1;
+        const u32 off = static_cast<u32>(col * KB) + 16u * static_cast<u32>(g);
+#pragma unroll
+        for (int i = 0; i < kSlabs; ++i) kf[j - j0][h][i] = *reinterpret_cast<const v4i *>(b + off + 64 * i);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = j0; j < j0 + kBatch && j < NCHUNK; ++j) {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          typename Mma::acc4_v acc = {0, 0, 0, 0};
+#pragma unroll
+          for (int i = 0; i < kSlabs; ++i) acc = Mma::mma16(kf[j - j0][h][i], qf[rt][i], acc);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) s[rt][j][4 * h + v] = acc[v];
+        }
+      }
+    }
+  }
+}
+
+// One value per row from the lanes' partial values: the four lanes of a row, then its WC wavefronts through `slots`
+// (every reduction of a kernel has slots of its own, so one barrier each is enough).
+template <typename Red, int WC, typename T>
+AKG_DEV T row_scores_reduce(T v, T (*slots)[16], int wc, int lane) {
+  v = Red::apply(v, lane_partner<16>(v));
+  v = Red::apply(v, lane_partner<32>(v));
+  if constexpr (WC > 1) {
+    if (lane < 16) slots[wc][lane] = v;
+    __syncthreads();
+    T r = slots[0][lane & 15];
+#pragma unroll
+    for (int w = 1; w < WC; ++w) r = Red::apply(r, slots[w][lane & 15]);
+    return r;
+  }
+  return v;
+}
+
+}  // namespace akg
