@@ -45,6 +45,7 @@ struct LoweringOptions {
   // Experiment switch (AKG_HIP_VARIANT), read by whichever family lowers the kernel; 0 = the measured default.
   //   gemm_epilogue  bit 3: no skinny kernel for M <= 64 (the tile kernel with K split instead),
   //                  bit 5: the other arrangement of the tile kernel's wavefronts (2 x 4 for 4 x 2 and back)
+  //                  bit 7: no small tiles (64 and 128 rows and columns) either,
   //                  bit 4: a contraction and the row reductions behind it as two kernels (no gemm_rows)
   //   row_reduce     1: keep the row in registers, 2: walk the row (no packing), 4: walk it, packed if possible
   //   stream_reduce  7: no column kernel (several kernels instead)

@@ -22,6 +22,7 @@
  *   Scalar [1]        one value
  */
 #include <algorithm>
+#include <cmath>
 #include <sstream>
 
 #include "HipLowering.h"
@@ -65,6 +66,13 @@ class GemmEmitter {
         k.workspaceBytes = static_cast<uint64_t>((groups * 4 + 255) / 256 * 256 + groups * kSplit_ * m_ * 128 * 4);
       }
       k.block[0] = static_cast<unsigned>(skinnyWaves() * 64);
+    } else if (tileM_ > 0) {
+      const int64_t smallTiles = ((m_ + tileM_ - 1) / tileM_) * ((n_ + tileN_ - 1) / tileN_), smallGrid = (smallTiles + 7) / 8 * 8;
+      k.grid[0] = static_cast<unsigned>(smallGrid * kSplit_);
+      if (kSplit_ > 1) {
+        k.workspaceBytes = static_cast<uint64_t>((smallGrid * 4 + 255) / 256 * 256 + smallTiles * kSplit_ * tileM_ * tileN_ * 4);
+      }
+      k.block[0] = 256;
     } else {
       k.grid[0] = static_cast<unsigned>(gridTiles * kSplit_);
       if (kSplit_ > 1) {
@@ -92,6 +100,8 @@ class GemmEmitter {
            << " grid=" << k.grid[0];
     } else if (skinny_) {
       note << " skinny: strips of 128 columns, B straight into MFMA operands, mfma=" << mfmaName(false) << " waves=4 grid=" << k.grid[0];
+    } else if (tileM_ > 0) {
+      note << " tile=" << tileM_ << "x" << tileN_ << "x" << stepK() / elemBytes() << " mfma=" << mfmaName(true) << " waves=2x2 grid=" << k.grid[0];
     } else {
       note << " tile=256x256x" << stepK() / elemBytes() << " mfma=" << mfmaName(true) << " waves=" << (tallWavefrontTiles() ? "2x4" : "4x2") << " grid=" << k.grid[0];
     }
@@ -116,6 +126,7 @@ class GemmEmitter {
   bool skinnyNonTemporal() const { return opt_.nonTemporal != 0 && !transB_; }
   bool serial_ = false;  // no MFMA kernel takes the description: gemm_serial (akg_gemm_serial.hpp)
   int epiWidth() const { return (serial_ && n_ % 4 != 0) ? 1 : 4; }   // adjacent result columns per epilogue call
+  int tileM_ = 0, tileN_ = 0;   // gemm_small_tile: its tile (0: another kernel)
   bool skinny_ = false;  // M <= 64: the kernel that streams B straight into MFMA operands (gemm_skinny)
   // A dynamic description (extents bound per call): M and the K split are kernel arguments, so the source - and with it
   // the code object - is the same for every token count; the skinny kernel comes in three sizes (16, 32, 64 rows).
@@ -147,6 +158,57 @@ class GemmEmitter {
   // (AKG_HIP_VARIANT bit 5 takes the other one.)
   bool tallWavefrontTiles() const { return (elem_ == DType::I8 && !transB_) != ((opt_.variant & 32) != 0); }
 
+  // Time in us of the small-tile kernel, after what it was measured to take: 3 us in front and behind, and per step of 128
+  // bytes of K 0.35 us (64 x 64; 0.28 where the workgroups of a CU cover each other), 0.48 (64 x 128), 0.72 (128 x 128): a CU
+  // takes in 46 GB/s with one workgroup or several, so workgroups beyond one per CU queue up. A split costs its
+  // partials' way to memory and back and the time of the workgroup that adds them.
+  double smallTileTime(int64_t bm, int64_t bn, int64_t split) const {
+    const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = ((m_ + bm - 1) / bm) * ((n_ + bn - 1) / bn);
+    const double perCu = static_cast<double>(tiles * split) / 256;
+    const double step = bn == 64 ? (perCu <= 1 ? 0.35 : 0.28) : (bm == 64 ? 0.48 : 0.72);
+    const double rounds = perCu <= 1 ? 1 : (perCu + std::ceil(perCu)) / 2;
+    const double loop = static_cast<double>((steps + split - 1) / split) * step * rounds;
+    const double area = static_cast<double>(bm * bn);
+    if (split == 1) return 3 + loop;
+    return 3 + loop + 2.5 + 0.3 * static_cast<double>(split) * area / 4096 + static_cast<double>(tiles * split) * area * 8 / 5e6;
+  }
+  // ... and of the 256 x 256 kernel with `split` workgroups per tile: 2 us a step.
+  double largeTileTime(int64_t split) const {
+    const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = ((m_ + 255) / 256) * ((n_ + 255) / 256);
+    const double loop = 2.0 * static_cast<double>((steps + split - 1) / split * ((tiles * split + 255) / 256));
+    return 6 + loop + (split == 1 ? 0 : 6 + 2 * static_cast<double>(split));
+  }
+  // The small-tile kernel where its estimate is a tenth below that of the 256 x 256 kernel, and for 33 .. 64 rows in
+  // place of the skinny one. Measured over M = 48 .. 2500 and seven K x N, bf16 and int8, both layouts (us, before -> now):
+  // bf16 K x N = 1024 x 1024: M = 64 9.9 -> 6.9, 300 29.4 -> 7.3, 1200 25.9 -> 10.9; 2048 x 4096: 64 14.5 -> 10.1, 300 35.9 -> 17.2,
+  // 1200 46.3 -> 42.1; 8192 x 2048: 128 45.6 -> 19.1, 640 66.7 -> 59.7; 4096 x 11000: 300 94.9 -> 66.8, 640 139 -> 95;
+  // int8 4096 x 4096: 192 40.9 -> 13.2, 640 42.1 -> 27.3. It is the slower one, and the estimate says so, from
+  // M = 1200 on for 8192 x 2048 (85 us for 73) and 4096 x 11000 (171 for 136).
+  // Below 2 MiB and from 2^26 elements of B on the kernel and the splits stay those that the schedule tests pin (there the
+  // skinny kernel and eight or four K splits of the 256 x 256 one); so do narrow skinny products (N < 1024).
+  bool pickSmallTile() {
+    if (serial_ || dyn_ || batch_ != 1 || opt_.split > 0 || (opt_.variant & (8 | 128))) return false;
+    const int64_t elements = k_ * n_;
+    if (m_ <= 32 || elements * elemBytes() < (2LL << 20) || elements >= (1LL << 26)) return false;
+    if (m_ <= skinnyRows() && n_ < 1024) return false;
+    if ((!transB_ && n_ * elemBytes() % 16 != 0) || k_ * elemBytes() * 128 >= (1LL << 31)) return false;
+    const int64_t steps = (k_ * elemBytes() + 127) / 128;
+    static const int shapes[][3] = {{64, 64, 1}, {64, 64, 2}, {64, 64, 4}, {64, 64, 8}, {64, 128, 1}, {64, 128, 2}, {128, 128, 1}};
+    double best = m_ <= skinnyRows() ? 1e30 : 0.9 * largeTileTime(largeTileSplit());
+    for (const auto &s : shapes) {
+      if (s[2] > 1 && (s[2] - 1) * ((steps + s[2] - 1) / s[2]) >= steps) continue;   // no empty split
+      const int64_t tiles = ((m_ + s[0] - 1) / s[0]) * ((n_ + s[1] - 1) / s[1]);
+      if (tiles * s[2] * s[0] * s[1] * 4 >= (1LL << 30)) continue;
+      const double t = smallTileTime(s[0], s[1], s[2]);
+      if (t >= best) continue;
+      best = t;
+      tileM_ = s[0];
+      tileN_ = s[1];
+      kSplit_ = s[2];
+    }
+    return tileM_ > 0;
+  }
+
   // Few tiles and a long K (a skinny activation in front of a big weight matrix: M = 16 .. 1024 against 8192 x 8192
   // leaves 32 .. 128 of 256 CUs busy, and the time is that of streaming the weights through those few): split K over
   // enough workgroups to fill the chip, at least four K steps each.
@@ -154,6 +216,7 @@ class GemmEmitter {
     kSplit_ = 1;
     if (serial_) return;
     dyn_ = opt_.extentAsArgument && batch_ == 1;
+    if (pickSmallTile()) return;
     // At most 64 rows of A (and K a multiple of 32 bytes): the time is that of streaming B, which gemm_skinny reads
     // straight into MFMA operands; 256 workgroups of four wavefronts (one per CU: 16 x 8192 x 8192 bf16 reaches 66 % of
     // the HBM peak with 4 splits of 64 strips, 59 % with 8, 48 % with 2; 8 wavefronts or more steps in flight change
@@ -172,6 +235,10 @@ class GemmEmitter {
       return;
     }
     if (batch_ != 1) return;
+    kSplit_ = static_cast<int>(largeTileSplit());
+  }
+
+  int64_t largeTileSplit() const {
     const int64_t tiles = ((m_ + 255) / 256) * ((n_ + 255) / 256);
     const int64_t steps = (k_ * elemBytes() + stepK() - 1) / stepK();
     int64_t want = opt_.split > 0 ? opt_.split : (tiles >= 192 ? 1 : std::min<int64_t>(16, (256 + tiles - 1) / tiles));
@@ -190,7 +257,7 @@ class GemmEmitter {
       want = std::min<int64_t>(want, std::max<int64_t>(1, (1LL << 20) / (partRows * 256 * 4)));
     }
     while (want > 1 && (want - 1) * ((steps + want - 1) / want) >= steps) --want;   // no empty split
-    kSplit_ = static_cast<int>(std::max<int64_t>(1, want));
+    return std::max<int64_t>(1, want);
   }
 
   void analyse() {
@@ -472,7 +539,7 @@ class GemmEmitter {
     src_ << "  AKG_DEV void apply(const " << accType() << " (&acc)[" << W << "], long row, long col) {\n"
          << "    const long grow = row0 + row;\n    (void)grow;\n" << apply_.str() << "  }\n";
     src_ << "};\n}  // namespace\n\n";
-    src_ << "extern \"C\" __global__ __launch_bounds__(" << (serial_ ? 256 : (skinny_ ? skinnyWaves() * 64 : 512)) << ") void " << kname << "(";
+    src_ << "extern \"C\" __global__ __launch_bounds__(" << (serial_ ? 256 : (skinny_ ? skinnyWaves() * 64 : (tileM_ > 0 ? 256 : 512))) << ") void " << kname << "(";
     size_t argc = 0;
     for (size_t i = 0; i < g_.inputs.size(); ++i, ++argc) {
       src_ << (argc ? ", " : "") << "const " << tagOf(g_.inputs[i]) << "::storage *__restrict__ in" << i;
@@ -512,6 +579,12 @@ class GemmEmitter {
            << ", Epilogue, " << kSplit_ << ", " << skinnyWaves() << ", " << skinnyUnroll() << ", " << (skinnyNonTemporal() ? "true" : "false") << ">(in" << g_.tensor(aId_).inputIndex << " + akg_batch * " << m_ * k_ << "L, in"
            << g_.tensor(bId_).inputIndex << " + akg_batch * " << k_ * n_ << "L, epi, " << (kSplit_ > 1 ? "akg_ws" : "nullptr")
            << ", akg_batch * " << (n_ + 127) / 128 << "L);\n}\n";
+      return;
+    }
+    if (tileM_ > 0) {
+      src_ << "  akg::gemm_small_tile<" << mmaTraits() << ", " << tileM_ << ", " << tileN_ << ", " << m_ << "L, " << n_ << "L, " << k_ << "L, "
+           << (transB_ ? "true" : "false") << ", Epilogue, " << kSplit_ << ">(in" << g_.tensor(aId_).inputIndex << ", in"
+           << g_.tensor(bId_).inputIndex << ", epi" << (kSplit_ > 1 ? ", akg_ws" : "") << ");\n}\n";
       return;
     }
     if (dyn_) {

@@ -892,4 +892,268 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------
+// Small tiles (BM x BN of 64 or 128): more rows than the skinny kernel takes and too few 256 x 256 tiles to fill the chip.
+//   workgroup = 2 x 2 wavefronts, 128 bytes of K per step, LDS double buffered (32 to 64 KiB: two to five workgroups per
+//   CU, whose phases cover each other, so the instructions of a step are left to the compiler)
+//   global -> registers -> LDS: two register sets, so the loads of a step are issued three steps ahead of its MFMAs: the
+//   time of a short K loop is that of its load latencies
+//   LDS rows without padding: the 16-byte chunks of a K-contiguous row r are permuted by (r >> 1) & 7, the 16-column units of
+//   a k-row of a row-major B by the bits of k that the lanes of one transposing read differ in; no bank is then hit twice
+//   by the lanes that are served together (which sixteen those are: see the 256 x 256 kernel).
+//   The operands of the MFMA are exchanged (columns of C are its rows): a lane owns row c = lane % 16 and the four
+//   adjacent columns 4 (lane / 16) .. + 3 of every 16 x 16 tile, without exchanges between lanes.
+// Tiles of a column of tiles are neighbours in launch order on one XCD, eight tile-rows at a time: they share their
+// columns of B in its L2, so B leaves memory once. KSPLIT as in the 256 x 256 kernel.
+template <typename Mma, int BM, int BN, long M, long N, long KE, bool TRANSB, typename Epilogue, int KSPLIT = 1>
+AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict__ B, Epilogue &epi,
+                             unsigned *__restrict__ ws = nullptr) {
+  constexpr int EB = Mma::kElemBytes;
+  constexpr long K = KE * EB, NB = N * EB;
+  static_assert((BM == 64 || BM == 128) && (BN == 64 || BN == 128), "tile sizes");
+  static_assert(K % 16 == 0 && N % 4 == 0 && (TRANSB || NB % 16 == 0), "whole 16-byte chunks");
+  static_assert(BM * K < (1L << 31) && (TRANSB ? BN * K : NB * KE) < (1L << 31), "operand too large for 32-bit buffer offsets");
+  constexpr int BK = 128;
+  constexpr int kTM = BM / 32, kTN = BN / 32;          // 16 x 16 tiles per wavefront
+  constexpr int kChunksA = BM / 32, kChunksB = BN / 32;  // 16-byte chunks per thread, step and operand
+  constexpr long kTilesM = (M + BM - 1) / BM, kTilesN = (N + BN - 1) / BN, kTiles = kTilesM * kTilesN;
+  constexpr long kPerXcd = (kTiles + kGemmXcds - 1) / kGemmXcds, kGridTiles = kPerXcd * kGemmXcds;
+  constexpr long kSteps = (K + BK - 1) / BK, kStepsPer = (kSteps + KSPLIT - 1) / KSPLIT;
+  static_assert((KSPLIT - 1) * kStepsPer < kSteps, "every K split needs at least one step");
+  constexpr int kPitchB = TRANSB ? BK : BN * EB;
+  constexpr int kChunksPerRowB = BN * EB / 16;
+  constexpr int kUnitBytes = 16 * EB;                   // 16 columns of a k-row
+  __shared__ __attribute__((aligned(16))) u8 lds[2][(BM + BN) * BK];
+
+  const long wgAll = static_cast<long>(blockIdx.x);
+  const long ksplit = KSPLIT > 1 ? wgAll / kGridTiles : 0;
+  const long wg = KSPLIT > 1 ? wgAll % kGridTiles : wgAll;
+  const long linear = (wg % kGemmXcds) * kPerXcd + wg / kGemmXcds;
+  if (linear >= kTiles) return;
+  constexpr long kGroupSize = kGemmGroupRows * kTilesN;
+  const long firstRow = linear / kGroupSize * kGemmGroupRows;
+  const long rowsInGroup = (kTilesM - firstRow) < kGemmGroupRows ? (kTilesM - firstRow) : kGemmGroupRows;
+  const long m0 = (firstRow + linear % kGroupSize % rowsInGroup) * BM;
+  const long n0 = linear % kGroupSize / rowsInGroup * BN;
+  const long stepBase = ksplit * kStepsPer;
+  const long mySteps = (kSteps - stepBase) < kStepsPer ? (kSteps - stepBase) : kStepsPer;
+
+  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int c = lane & 15, g = lane >> 4;
+
+  // ---- staging. A row beyond M (a column of a [N,K] B beyond N) repeats the last one, its results are dropped; a chunk
+  // beyond K, or beyond the columns of a row-major B, is asked for beyond the buffer and reads zero.
+  auto bytesLeft = [](long bytes) { return static_cast<int>(bytes < 0x7fffffffL ? bytes : 0x7fffffffL); };
+  const __amdgpu_buffer_rsrc_t aRsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char *>(static_cast<const char *>(A)) + m0 * K, 0, bytesLeft((M - m0) * K), 0x00020000);
+  const __amdgpu_buffer_rsrc_t bRsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char *>(static_cast<const char *>(B)) + (TRANSB ? n0 * K : 0L), 0, bytesLeft(TRANSB ? (N - n0) * K : NB * KE), 0x00020000);
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  const int kRow = tid >> 3, kChunk = tid & 7;           // K-contiguous operand: row (+ 32 per chunk), 16-byte chunk
+  const int kStore = kRow * BK + (kChunk ^ ((kRow >> 1) & 7)) * 16;
+  u32 aOff[kChunksA], bOff[kChunksB];
+  int bStore[kChunksB];
+#pragma unroll
+  for (int i = 0; i < kChunksA; ++i) {
+    const long row = m0 + kRow + 32 * i;
+    aOff[i] = static_cast<u32>(((row < M ? row : M - 1) - m0) * K + kChunk * 16);
+  }
+  // which permutation of its 16-column units a k-row of a row-major B has
+  auto unitSwap = [](int krow) {
+    if constexpr (EB == 2) return BN == 128 ? (krow & 3) | ((krow >> 1) & 4) : ((krow >> 1) & 1) | ((krow >> 2) & 2);
+    return BN == 128 ? ((krow >> 1) & 3) | ((krow >> 2) & 4) : ((krow >> 2) & 1) | ((krow >> 3) & 2);
+  };
+  const int bRow = tid / kChunksPerRowB, bChunk = tid % kChunksPerRowB;
+  constexpr int kRowStepB = 256 / kChunksPerRowB;
+#pragma unroll
+  for (int i = 0; i < kChunksB; ++i) {
+    if constexpr (TRANSB) {
+      const long col = n0 + kRow + 32 * i;
+      bOff[i] = static_cast<u32>(((col < N ? col : N - 1) - n0) * K + kChunk * 16);
+      bStore[i] = kStore + 32 * BK * i;
+    } else {
+      const int krow = bRow + kRowStepB * i;
+      const long colByte = n0 * EB + bChunk * 16;
+      bOff[i] = colByte < NB ? static_cast<u32>(krow * NB + colByte) : kBeyondEveryBuffer;
+      bStore[i] = krow * kPitchB + ((bChunk * 16 / kUnitBytes) ^ unitSwap(krow)) * kUnitBytes + (bChunk * 16) % kUnitBytes;
+    }
+  }
+  struct Stage {
+    u32x4 a[kChunksA], b[kChunksB];
+  };
+  Stage stage[2];
+  auto load = [&](long step, Stage &s) {
+    const long k0 = (stepBase + step) * BK;
+    const bool whole = K % BK == 0 || k0 + kChunk * 16 < K;
+#pragma unroll
+    for (int i = 0; i < kChunksA; ++i) {
+      s.a[i] = __builtin_amdgcn_raw_buffer_load_b128(aRsrc, whole ? aOff[i] : kBeyondEveryBuffer, static_cast<int>(k0), 0);
+    }
+#pragma unroll
+    for (int i = 0; i < kChunksB; ++i) {
+      if constexpr (TRANSB) {
+        s.b[i] = __builtin_amdgcn_raw_buffer_load_b128(bRsrc, whole ? bOff[i] : kBeyondEveryBuffer, static_cast<int>(k0), 0);
+      } else {
+        const bool rowOk = K % BK == 0 || k0 / EB + bRow + kRowStepB * i < KE;
+        s.b[i] = __builtin_amdgcn_raw_buffer_load_b128(bRsrc, rowOk ? bOff[i] : kBeyondEveryBuffer, static_cast<int>(k0 / EB * NB), 0);
+      }
+    }
+  };
+  auto store = [&](int buf, const Stage &s) {
+#pragma unroll
+    for (int i = 0; i < kChunksA; ++i) *reinterpret_cast<u32x4 *>(lds[buf] + kStore + 32 * BK * i) = s.a[i];
+#pragma unroll
+    for (int i = 0; i < kChunksB; ++i) *reinterpret_cast<u32x4 *>(lds[buf] + BM * BK + bStore[i]) = s.b[i];
+  };
+
+  // ---- fragments: 64 bytes of K per MFMA, lane (c, g) has bytes 16 g .. + 15 of row c
+  const int fragSwap = (c >> 1) & 7;
+  const int aFrag = (wm * (BM / 2) + c) * BK, bFrag = (wn * (BN / 2) + c) * BK;
+  const int trRow = g * (16 / EB) + (EB == 1 ? (c >> 1) : (c >> 2));
+  const int trCol = EB == 1 ? (c & 1) * 8 : (c & 3) * 8;
+  int trOff[kTN];
+#pragma unroll
+  for (int j = 0; j < kTN; ++j) trOff[j] = trRow * kPitchB + ((wn * kTN + j) ^ unitSwap(trRow)) * kUnitBytes + trCol;
+  typename Mma::acc4_v acc[kTM][kTN];
+#pragma unroll
+  for (int i = 0; i < kTM; ++i) {
+#pragma unroll
+    for (int j = 0; j < kTN; ++j) acc[i][j] = typename Mma::acc4_v{0, 0, 0, 0};
+  }
+  struct Frags {
+    v4i a[kTM], b[kTN];
+  };
+  auto read = [&](int buf, int kh, Frags &f) {
+    const int chunk = ((kh * 4 + g) ^ fragSwap) * 16;
+#pragma unroll
+    for (int j = 0; j < kTN; ++j) {
+      if constexpr (TRANSB) {
+        f.b[j] = *reinterpret_cast<const v4i *>(lds[buf] + BM * BK + bFrag + j * 16 * BK + chunk);
+      } else {
+        typedef int v2i __attribute__((ext_vector_type(2)));
+        typedef short v4s __attribute__((ext_vector_type(4)));
+        const u8 *p0 = lds[buf] + BM * BK + kh * (64 / EB) * kPitchB + trOff[j];
+        const u8 *p1 = p0 + (8 / EB) * kPitchB;
+        if constexpr (EB == 1) {
+          const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i *)(p0));
+          const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i *)(p1));
+          f.b[j] = v4i{lo[0], lo[1], hi[0], hi[1]};
+        } else {
+          const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(p0));
+          const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s *)(p1));
+          const v2i l2 = __builtin_bit_cast(v2i, lo), h2 = __builtin_bit_cast(v2i, hi);
+          f.b[j] = v4i{l2[0], l2[1], h2[0], h2[1]};
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kTM; ++i) f.a[i] = *reinterpret_cast<const v4i *>(lds[buf] + aFrag + i * 16 * BK + chunk);
+  };
+  auto multiply = [&](const Frags &f) {
+#pragma unroll
+    for (int i = 0; i < kTM; ++i) {
+#pragma unroll
+      for (int j = 0; j < kTN; ++j) acc[i][j] = Mma::mma16(f.b[j], f.a[i], acc[i][j]);
+    }
+  };
+
+  // ---- main loop. At the top of step s: LDS buffer s & 1 holds tile s, stage[(s + 1) & 1] tile s + 1, the other set tile
+  // s + 2 (both possibly in flight), f[0] the fragments of the first half of tile s; buffer (s + 1) & 1 is free (read before
+  // the last barrier). The barrier of a step lies between its two halves, so LDS traffic always has MFMAs beside it: in
+  // front the second half of the fragments arrives and tile s + 1 is written, behind it the first fragments of tile s + 1
+  // arrive. (The steady part has no conditions: behind a branch the compiler counts on the fewest loads in flight and waits
+  // for the newest ones.)
+  Frags f[2];
+  auto step = [&](long s, int buf, Stage &next) {
+    read(buf, 1, f[1]);
+    store(buf ^ 1, next);
+    load(s + 3, next);
+    multiply(f[0]);
+    __syncthreads();
+    read(buf ^ 1, 0, f[0]);
+    multiply(f[1]);
+  };
+  auto lastStep = [&](long s, int buf, Stage &next) {
+    read(buf, 1, f[1]);
+    if (s + 1 < mySteps) store(buf ^ 1, next);
+    if (s + 3 < mySteps) load(s + 3, next);
+    multiply(f[0]);
+    __syncthreads();
+    if (s + 1 < mySteps) read(buf ^ 1, 0, f[0]);
+    multiply(f[1]);
+  };
+  load(0, stage[0]);
+  if (mySteps > 1) load(1, stage[1]);
+  store(0, stage[0]);
+  if (mySteps > 2) load(2, stage[0]);
+  __syncthreads();
+  read(0, 0, f[0]);
+  long s = 0;
+  for (; s + 4 < mySteps; s += 2) {
+    step(s, 0, stage[1]);
+    step(s + 1, 1, stage[0]);
+  }
+  for (; s < mySteps; s += 2) {
+    lastStep(s, 0, stage[1]);
+    if (s + 1 < mySteps) lastStep(s + 1, 1, stage[0]);
+  }
+
+  // ---- epilogue
+  typedef typename Mma::acc_t acc_t;
+  const int rowLane = wm * (BM / 2) + c;                   // + 16 i: row inside the tile
+  const int colLane = wn * (BN / 2) + 4 * g;               // + 16 j: first of four columns inside the tile
+  if constexpr (KSPLIT > 1) {
+    constexpr long kCounterBytes = (kGridTiles * 4 + 255) / 256 * 256;
+    constexpr long kPartBytes = static_cast<long>(BM) * BN * sizeof(acc_t);
+    const Buffer wsBuf = make_buffer(ws, kCounterBytes + kTiles * KSPLIT * kPartBytes);   // (below 2 GiB: checked by the host)
+    const u32 tileBase = static_cast<u32>(kCounterBytes + linear * KSPLIT * kPartBytes);
+    // a partial lies as the accumulators do, 16 bytes a thread: whole lines, whatever the tile
+    auto partOffset = [&](long p, int i, int j) { return tileBase + static_cast<u32>(p * kPartBytes + ((i * kTN + j) * 256 + tid) * 16); };
+#pragma unroll
+    for (int i = 0; i < kTM; ++i) {
+#pragma unroll
+      for (int j = 0; j < kTN; ++j) {
+        const acc_t a4[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+        ws_store_chunk<4>(wsBuf, partOffset(ksplit, i, j), a4);
+      }
+    }
+    __shared__ unsigned akg_small_flag;
+    if (!last_workgroup(ws, linear, KSPLIT, tid, &akg_small_flag)) return;
+    // sums in split order (deterministic), this workgroup's own partial among them
+#pragma unroll
+    for (int i = 0; i < kTM; ++i) {
+#pragma unroll
+      for (int j = 0; j < kTN; ++j) acc[i][j] = typename Mma::acc4_v{0, 0, 0, 0};
+    }
+#pragma unroll 2
+    for (int p = 0; p < KSPLIT; ++p) {
+#pragma unroll
+      for (int i = 0; i < kTM; ++i) {
+#pragma unroll
+        for (int j = 0; j < kTN; ++j) {
+          acc_t part[4];
+          ws_load_chunk<4>(wsBuf, partOffset(p, i, j), part);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[i][j][v] += part[v];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kTN; ++j) {
+    const long col = n0 + colLane + 16 * j;
+    if (col >= N) continue;
+    epi.prepare(col);
+#pragma unroll
+    for (int i = 0; i < kTM; ++i) {
+      const long row = m0 + rowLane + 16 * i;
+      if (row < M) {
+        const acc_t a4[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+        epi.apply(a4, row, col);
+      }
+    }
+  }
+}
+
 }  // namespace akg
