@@ -42,17 +42,24 @@ class _KernelInfo(ctypes.Structure):
 
 
 _lib = None
+_launch = None          # the extension module of the launch path (csrc/launch_module.cpp)
+_current_device = None  # torch's current device and the raw handle of its current stream, without a Stream object
+_raw_stream = None
 
 
 def load_library():
     """Load libakg_hip.so from the package directory. There is no fallback: without the native library nothing runs."""
-    global _lib
+    global _lib, _launch, _current_device, _raw_stream
     if _lib is not None:
         return _lib
     # torch wheels bundle their own HIP runtime. Two HIP runtimes in one process cannot both own the GPU, so when
     # torch is installed it is imported first and libakg_hip.so then binds to the runtime torch already loaded.
     try:
         import torch  # noqa: F401  pylint: disable=unused-import,import-outside-toplevel
+        _current_device = torch.cuda.current_device
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # pylint: disable=protected-access
+        if _raw_stream is None:
+            _raw_stream = lambda device: torch.cuda.current_stream(device).cuda_stream   # noqa: E731
     except ImportError:
         pass
     if not os.path.exists(LIB_PATH):
@@ -85,6 +92,8 @@ def load_library():
                                                   ctypes.POINTER(vp)]
     lib.akg_hip_dynamic_destroy.argtypes = [vp]
     lib.akg_hip_dynamic_destroy.restype = None
+    from . import _launch as launch_module  # pylint: disable=import-outside-toplevel
+    _launch = launch_module
     _lib = lib
     return lib
 
@@ -138,6 +147,13 @@ class HipDynamicKernel:
         """The reference's dynamic calling form (LLVMParameterPacking.cpp:91-194): `device_ptrs` for inputs then outputs,
         `shapes` their concrete shapes; packs [0, sizes, strides] per tensor like transform_data_to_ctypes
         (mlir_driver.py:186-252) and returns the HipKernel that ran."""
+        if self._handle:
+            packed = _launch.launch_packed(self._handle.value, device_ptrs, shapes, stream or 0)
+            if packed is not None:
+                rc, key = packed
+                if rc:
+                    _check(rc)
+                return self._by_handle.get(key) or self._borrowed(key)
         n = len(device_ptrs)
         width = 1 + 2 * max([len(s) for s in shapes] + [1])
         lists = []
@@ -152,12 +168,13 @@ class HipDynamicKernel:
         used = ctypes.c_void_p()
         _check(self._lib.akg_hip_dynamic_launch_packed(self._handle, ptrs, lptrs, n, ctypes.c_void_p(stream or 0),
                                                        ctypes.byref(used)))
-        key = used.value
-        if key not in self._by_handle:
-            k = HipKernel(None, _borrowed=used)
-            k._keepalive = self
-            self._by_handle[key] = k
-        return self._by_handle[key]
+        return self._by_handle.get(used.value) or self._borrowed(used.value)
+
+    def _borrowed(self, key):
+        k = HipKernel(None, _borrowed=ctypes.c_void_p(key))
+        k._keepalive = self
+        self._by_handle[key] = k
+        return k
 
     def __del__(self):
         h = getattr(self, "_handle", None)
@@ -202,6 +219,7 @@ class HipKernel:
             raw_desc = _TensorDesc()
             _check(self._lib.akg_hip_kernel_tensor(self._handle, i, ctypes.byref(raw_desc)))
             self.tensors.append(TensorDesc(raw_desc))
+        self._nbytes = tuple(t.nbytes for t in self.tensors)
         info = _KernelInfo()
         _check(self._lib.akg_hip_kernel_get_info(self._handle, ctypes.byref(info)))
         self.kernel_name = info.kernel_name.decode("utf-8")
@@ -264,6 +282,12 @@ class HipKernel:
 
     def launch(self, tensors, stream=None):
         """Launch on torch device tensors (inputs then outputs), on `stream` (a torch stream) or the current one."""
+        if self._handle:
+            rc = _launch.launch(self._handle.value, self._nbytes, tensors, stream, _current_device, _raw_stream)
+            if rc == 0:
+                return
+            if rc is not None:
+                _check(rc)
         import torch
         for t, d in zip(tensors, self.tensors):
             if not t.is_cuda or not t.is_contiguous():
