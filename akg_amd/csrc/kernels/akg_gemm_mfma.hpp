@@ -655,13 +655,13 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
 
 // ---------------------------------------------------------------------------------------------------------
 // Skinny A (M <= 64 rows: a decoding step, a GEMV): the time is that of streaming B once, so B goes from global memory
-// straight into MFMA operands, without LDS and without barriers in the main loop.
+// into MFMA operands without barriers in the main loop.
 //   workgroup = 4 wavefronts, one strip of 128 columns, one range of K (KSPLIT ranges per strip)
 //   wavefront w takes the MFMA steps (32 bytes of K each) w, w + 4, ... of that range, two steps' loads in flight
 //   lane (n = lane % 32, g = lane / 32) owns the 4 ADJACENT columns 4n .. 4n+3 of the strip and the 16 bytes
 //   [32 t + 16 g, +16) of K: for a row-major B it loads a (16 bytes of K) x (4 columns) block (8 rows x 8 bytes or
-//   16 rows x 4 bytes) and transposes it in registers into four operands, for [N,K] it loads the four operands as they
-//   are; one MFMA per column of the four, all against the same one or two A operands (32 rows each; rows beyond M repeat row M-1 and are dropped)
+//   16 rows x 4 bytes) and transposes it in registers into four operands; a [N,K] weight comes in whole cache lines
+//   through LDS of the wavefront's own (a short K: the operands as they are); one MFMA per column of the four, all against the same one or two A operands (32 rows each; rows beyond M repeat row M-1 and are dropped)
 // The four wavefronts add their accumulators through LDS (only the M real rows), the KSPLIT workgroups of a strip
 // through the workspace in split order (counter per strip, then M x 128 partials per strip and split), and the thread
 // that owns (row, 4 columns) runs the epilogue on the sums. Deterministic; B is read exactly once.
@@ -690,7 +690,16 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
   const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
   const long strip = static_cast<long>(blockIdx.x) % kStrips;   // neighbours in launch order read neighbouring columns
   const int ksplit = static_cast<int>(static_cast<long>(blockIdx.x) / kStrips);
-  const long t0 = kSteps * ksplit / kSplits, t1 = kSteps * (ksplit + 1) / kSplits;
+  constexpr int kLine = 128;   // bytes of K that a wavefront takes at a time from every column of a [N,K] weight
+  // Below 512 bytes of K not every wavefront would get a line: the fragments are then loaded as they are.
+  constexpr bool kLines = TRANSB && K >= kWaves * kLine;
+  // Whole lines need no second look, so a weight larger than what the caches hold is read past them: bf16 16 x 8192 x 8192
+  // 28.4 us without the hint, 26.4 with it; 11008 x 4096 20.6 and 20.5; 2048 x 2048, which stays cached, 7.8 and 8.5; int8
+  // 8192 x 8192 17.0 and 17.1.
+  constexpr bool kLinesNonTemporal = K % kLine == 0 && N * K >= (96L << 20);
+  constexpr long kUnit = kLines ? kLine / 32 : 1, kUnits = (kSteps + kUnit - 1) / kUnit;   // a range of K ends on a whole line
+  const long t0 = kUnits * ksplit / kSplits * kUnit, tEnd = kUnits * (ksplit + 1) / kSplits * kUnit;
+  const long t1 = tEnd < kSteps ? tEnd : kSteps;
   const int n32 = lane & 31, kg = lane >> 5;
   const long myCol = strip * 128 + 4 * n32;
   const long ldCol = myCol + 3 < N ? myCol : 0;   // columns beyond N: load something valid, the results are dropped
@@ -779,24 +788,92 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
       for (int c = 0; c < 4; ++c) acc[rt][c] = Mma::mma(r.a[rt], b[c], acc[rt][c]);
     }
   };
-  // (For a [N,K] weight, whose columns are contiguous along K, giving a wavefront a run of adjacent steps instead of
-  // every fourth changes nothing: 36.9 us either way on bf16 16 x 8192 x 8192; the L1 merges the pieces of a line.)
-  for (long t = t0 + wave; t < t1; t += kWaves * U) {   // (uniform per wavefront)
-    Raw r[U];
+  constexpr int kHalfRows = MS < 16 ? static_cast<int>(MS) : 16;
+  constexpr int kSumBytes = kWaves * kHalfRows * 128 * 4;
+  constexpr int kLdsBytes = kLines && kWaves * 128 * kLine > kSumBytes ? kWaves * 128 * kLine : kSumBytes;
+  __shared__ __attribute__((aligned(16))) u8 akg_skinny_lds[kLdsBytes];
+  if constexpr (kLines) {
+    // A wavefront loads the line of eight columns per instruction and turns the 128 columns into operands through LDS of its
+    // own (chunks permuted by the column: every bank once among the lanes served together), the next lines in flight
+    // beside the MFMAs. Loading the operands as they are touches 32 lines by 32 bytes per instruction, and a line is evicted
+    // from the L1 before its fourth piece is read. bf16, before -> lines in order -> lines rotated (us): 16 x 8192 x 8192
+    // 38.8 -> 33.2 -> 26.4, 16 x 4096 x 11008 32.7 -> 23.2 -> 20.5, 64 x 8192 x 8192 46.3 -> 39.0 -> 34.8, 16 x 8192 x 1024 11.6 ->
+    // 9.8 -> 9.9; int8 16 x 8192 x 8192 20.6 -> 17.3 -> 17.0. Rotation or adjacent pieces alone, without whole lines: 37 .. 42.
+    constexpr int kSub = kLine / 32;   // MFMA steps per line
+    const long lines = (t1 - t0 + kSub - 1) / kSub;
+    u8 *__restrict__ tile = akg_skinny_lds + wave * (128 * kLine);
+    const int lc = lane >> 3, chunk = lane & 7;
+    v4i raw[16], ra[kRowTiles][kSub];
+    // Strips begin at different lines of their range: the same line of all strips lies a multiple of the row pitch apart, on
+    // few memory channels if that is a power of two.
+    const long rot = lines > 0 ? strip % lines : 0;
+    auto stepOf = [&](long i) { return t0 + (i + rot >= lines ? i + rot - lines : i + rot) * kSub; };
+    auto loadLine = [&](long i) {
+      const long t = stepOf(i);
+      const long tc = t + (chunk >> 1) < t1 ? t + (chunk >> 1) : t1 - 1;
+      const char *from = B + tc * 32 + (chunk & 1) * 16;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (t + u * kWaves < t1) load(t + u * kWaves, r[u]);
+      for (int j = 0; j < 16; ++j) {
+        long bc = strip * 128 + 8 * j + lc;
+        if constexpr (N % 128 != 0) bc = bc < N ? bc : 0;
+        const v4i *bp = reinterpret_cast<const v4i *>(from + bc * K);
+        raw[j] = kLinesNonTemporal ? __builtin_nontemporal_load(bp) : *bp;
+      }
+#pragma unroll
+      for (int u = 0; u < kSub; ++u) {
+#pragma unroll
+        for (int rt = 0; rt < kRowTiles; ++rt) ra[rt][u] = *reinterpret_cast<const v4i *>(A[rt] + (t + u < t1 ? t + u : t1 - 1) * 32);
+      }
+    };
+    if (wave < lines) loadLine(wave);
+    for (long i = wave; i < lines; i += kWaves) {   // (uniform per wavefront)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int bc = 8 * j + lc;
+        *reinterpret_cast<v4i *>(tile + bc * kLine + (chunk ^ ((bc >> 2) & 7)) * 16) = raw[j];
+      }
+      v4i a[kRowTiles][kSub];
+#pragma unroll
+      for (int u = 0; u < kSub; ++u) {
+#pragma unroll
+        for (int rt = 0; rt < kRowTiles; ++rt) a[rt][u] = ra[rt][u];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      loadLine(i + kWaves < lines ? i + kWaves : i);
+      const long t = stepOf(i);
+#pragma unroll
+      for (int u = 0; u < kSub; ++u) {
+        if (t + u < t1) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const v4i b = *reinterpret_cast<const v4i *>(tile + (4 * n32 + c) * kLine + ((2 * u + kg) ^ (n32 & 7)) * 16);
+#pragma unroll
+            for (int rt = 0; rt < kRowTiles; ++rt) acc[rt][c] = Mma::mma(a[rt][u], b, acc[rt][c]);
+          }
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
     }
+    __syncthreads();   // the sums below lie where the lines did
+  } else {
+    for (long t = t0 + wave; t < t1; t += kWaves * U) {   // (uniform per wavefront)
+      Raw r[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (t + u * kWaves < t1) mfma(r[u]);
+      for (int u = 0; u < U; ++u) {
+        if (t + u * kWaves < t1) load(t + u * kWaves, r[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (t + u * kWaves < t1) mfma(r[u]);
+      }
     }
   }
 
   // ---- the four wavefronts' sums, rows below M only, 16 rows at a time: accumulator v of a lane is row
   // 8 (v / 4) + 4 g + v % 4; thread (c4, r0) then owns 4 columns of the strip and the rows r0, r0 + 8, ...
-  constexpr int kHalfRows = MS < 16 ? static_cast<int>(MS) : 16;
-  __shared__ acc_t akg_skinny_sum[kWaves][kHalfRows][128];
+  acc_t (*akg_skinny_sum)[kHalfRows][128] = reinterpret_cast<acc_t (*)[kHalfRows][128]>(akg_skinny_lds);
   const int c4 = tid & 31, r0 = (tid >> 5) & 7;
   const long col = strip * 128 + 4 * c4;
   const bool colOk = col < N && tid < 256;   // (of 8 wavefronts the first four finish the sums)

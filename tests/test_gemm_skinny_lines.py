@@ -1,0 +1,51 @@
+"""The skinny kernel on a [N,K] weight: whole lines of K through LDS, their tails, ragged columns and split ranges."""
+import pytest
+
+from akg_amd import driver, op_desc
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,n,dtype", [
+    (16, 240, 136, "bfloat16"),     # below one line per wavefront: the operands as they are
+    (16, 256, 128, "bfloat16"),     # one line each, one strip
+    (3, 272, 132, "float16"),       # a quarter of a line behind the last one, four columns beyond a strip
+    (1, 1024, 1000, "bfloat16"),    # one row, ragged last strip, split ranges
+    (32, 4144, 520, "bfloat16"),    # splits that end on whole lines, a tail of three quarters
+    (33, 2048, 516, "float16"),     # two row tiles
+    (64, 8192, 264, "bfloat16"),    # the most rows and splits
+    (7, 11008, 1040, "bfloat16"),   # more strips than a range has lines: the rotation wraps
+    (16, 8192, 6400, "bfloat16"),   # read past the caches
+    (32, 8256, 272, "int8"), (5, 544, 140, "int8"),
+])
+def test_lines_of_a_transposed_weight_against_float64(m, k, n, dtype):
+    """float32 sums of k products differ from the exact sum by at most k * 2^-24 of the sum of the products' magnitudes, in
+    whatever order, and a result by one half unit of its type; 8-bit sums are exact. Twice: the counters of the split are left ready."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    dev = "cuda"
+    if dtype == "int8":
+        text = op_desc.gemm_int8_dequant_bias_gelu(m, k, n, transpose_b=True)
+        a, w = (torch.randint(-127, 128, s, generator=g, device=dev).to(torch.int8) for s in ((m, k), (n, k)))
+        scale, scale_n = torch.full((m, 1), 2.0 ** -6, device=dev), torch.full((n,), 2.0 ** -10, device=dev)
+        bias = torch.randn(n, generator=g, device=dev).bfloat16()
+        y = a.double() @ w.double().t().contiguous() * 2.0 ** -16 + bias.double()
+        y = y * (torch.tanh((y + y ** 3 * 0.044715) * 0.7978845608028654) + 1) * 0.5
+        # the factors are powers of two; float32 GELU: 2^-20 of the argument's magnitude, and the rounding to bfloat16
+        inputs, td, bound = [a, scale, w, scale_n, bias], torch.bfloat16, y.abs() * (2.0 ** -8 + 2.0 ** -19) + 2.0 ** -16
+    else:
+        td = getattr(torch, dtype)
+        text = op_desc.gemm_bias_act(m, k, n, dtype, "none", transpose_b=True)
+        a, w, bias = (torch.randn(s, generator=g, device=dev).to(td) for s in ((m, k), (n, k), (n,)))
+        y = a.double() @ w.double().t().contiguous() + bias.double()
+        sums = a.double().abs() @ w.double().abs().t().contiguous()
+        unit = 2.0 ** -8 if dtype == "bfloat16" else 2.0 ** -11
+        inputs, bound = [a, w, bias], sums * (k * 2.0 ** -24) + y.abs() * (unit + 2.0 ** -23) + 2.0 ** -24
+    kernel = driver.HipKernel(text, out_dir=None)
+    assert "gemm_skinny<" in kernel.source
+    print("case", m, k, n, dtype, kernel.grid, flush=True)
+    for _ in range(2):
+        out = torch.full((m, n), float("nan"), device=dev, dtype=td)
+        kernel.launch(inputs + [out])
+        torch.cuda.synchronize()
+        gap = (out.double() - y).abs()
+        assert bool((gap <= bound).all()), float((gap / bound).max())
