@@ -106,6 +106,22 @@ class GemmRowsEmitter {
     //   scores below 1 MiB stay in the caches, and both forms take the time of their launches.
     if (k_ % 32 != 0 || n_ % 8 != 0 || n_ > 2048 || n_ * k_ > (1LL << 17)) throw LoweringError("MatMul: operands of this shape have no row kernel");
     if (m_ < 4 || batch_ * m_ * n_ * 4 < (1LL << 20)) throw LoweringError("MatMul: too few rows or scores for the row kernel");
+    // With a longer K a row group reads more of B from the L2, and the contraction kernel gains where its 256 x 256 tiles are
+    // full. bf16 with softmax behind it, one kernel for two (us). K = 160 .. 224: 46 of 47 shapes faster, [12510,192]x312 20.1
+    // for 19.3. Batches of fewer than 1000 rows: 164 x [343,256]x240 50 for 105, 271 x [487,384]x320 195 for 237, 64 x
+    // [512,512]x256 50 for 62, but 64 x [46,512]x224 18.2 for 15.7; longer ones: 20 x [1378,256]x176 30 for 24, 4 x [3575,256]x400 34
+    // for 26, few columns 107 x [2032,256]x56 50 for 70. One batch: [6024,256]x312 13.9 for 15.5, [9674,256]x328 20.5 for 19.2,
+    // [93571,256]x256 64 for 56; at most 64 columns: [28955,256]x40 9.9 for 12.8, [16384,512]x64 12.3 for 18.5, [36288,256]x48 15.0 for
+    // 13.4, [65536,512]x64 28 for 23; at most 24: [16384,1024]x16 11.1 for 20.0, [32768,4096]x8 61 for 80, [65536,7168]x16 172 for
+    // 165. ([16384,2048]x64 38 for 28, [8192,4096]x32 44 for 33.)
+    const bool batches = batch_ > 1 && m_ < 1000;
+    int64_t longest = n_ <= 24 ? 4096 : 224;
+    if (batches || batch_ * m_ <= 8192 || (batch_ > 1 && n_ <= 64)) longest = std::max<int64_t>(longest, 384);
+    if ((batches && m_ >= 64) || (n_ <= 64 && batch_ * m_ <= 32768)) longest = std::max<int64_t>(longest, 512);
+    if (k_ > longest) throw LoweringError("MatMul: K is too long for the row kernel");
+    // Scores that are an output are written either way: bf16 [28,2048,64]x1024 with the probabilities in both types 174 us
+    // for 144, [14,2048,64]x2048 118 for 100; up to 256 columns one kernel is faster ([400,300,64]x256 57 for 135).
+    if (g_.tensor(accId_).outputIndex >= 0 && n_ > 256) throw LoweringError("MatMul: scores of this size that are written leave nothing to save");
     for (const OpNode &op : g_.ops) {
       if (op.kind == OpKind::MatMul) continue;
       for (int in : op.inputs) {
@@ -135,7 +151,30 @@ class GemmRowsEmitter {
       return batch_ * rowGroups();
     };
     if (m_ <= 16 || shape(2) < 512) shape(1);
+    // Every tensor of the scores' columns takes eight registers per unit, and a workgroup of sixteen wavefronts leaves 128 a
+    // lane: beyond half as many again the spills cost more than the scores' way through memory. [*,*,64] x 2048 by the number
+    // wideTensors() (us for two kernels): 3 (a float32 result and a mask) 122 .. 135 for 120 .. 136, 4 115 .. 179 for 139 .. 194,
+    // 5 244 for 224, 6 145 .. 268 for 146 .. 215, 7 198 .. 359 for 140 .. 240; eight wavefronts, 6 121 for 138, 8 147 for 128.
+    const int registers = wavesC_ >= 16 ? 192 : (wavesC_ == 8 ? 256 : 512);
+    if (8 * chunks_ * (rowTiles_ + wideTensors()) > registers) throw LoweringError("MatMul: too many tensors of the scores' size for the row kernel's registers");
     if (batch_ * rowGroups() < 64) throw LoweringError("MatMul: too few row groups for the row kernel");
+  }
+
+  // Tensors of the scores' columns besides the scores, in 32-bit values per element: what is read and what is written (a
+  // float32 result is computed by the longer forms of the functions in front of it: one more).
+  int wideTensors() const {
+    int words = 0;
+    auto add = [&](int id, bool result) {
+      const TensorValue &t = g_.tensor(id);
+      if (t.shape.empty() || t.shape.back() != n_) return;
+      const bool whole = dtypeSize(t.dtype) >= 4;
+      words += (dtypeSize(t.dtype) + 3) / 4 + (result && whole ? 1 : 0);
+    };
+    for (int id : g_.inputs) {
+      if (id != aId_ && id != bId_ && g_.tensor(id).used) add(id, false);
+    }
+    for (int id : g_.outputs) add(id, true);
+    return words;
   }
 
   std::string ctOf(int id) const { return computeTypeName(g_.tensor(id).dtype); }

@@ -26,55 +26,96 @@ AKG_DEV constexpr int row_unit(int j, int wc) {
   return NCHUNK % 2 == 0 ? ((j / 2) * WC + wc) * 2 + j % 2 : j * WC + wc;
 }
 
-// s[rt][j] = the eight columns of unit j * WC + wc (columns beyond N hold copies of column N - 1) in row
+// A number of 64-byte slabs of K as a type.
+template <int N>
+struct SlabCount {
+  static constexpr int value = N;
+};
+
+// s[rt][j] = the eight columns of unit row_unit(j, wc) (columns beyond N hold copies of column N - 1) in row
 // row0 + 16 rt + lane % 16 (rows beyond M hold copies of row M - 1). KB: bytes of K per row, a multiple of 64.
+// Up to seven slabs of 64 bytes the rows of A stay in registers; a longer K is taken in blocks of four with the
+// accumulators live, so the registers do not grow with K (bf16, 512 x 256 with softmax: 180 a lane at K = 512, 332 with all of K
+// held, where K = 1024 and more spilled; K = 512 50 us either way, and the next block's rows requested beside the MFMAs of a block
+// gave nothing).
 template <typename Mma, long M, long N, long KB, int RT, int NCHUNK, int WC>
 AKG_DEV void row_scores(const void *__restrict__ A, const void *__restrict__ B, long row0, int wc, int lane,
                         float (&s)[RT][NCHUNK][8]) {
   static_assert(KB % 64 == 0 && M * KB < (1L << 31) && N * KB < (1L << 31), "operand shapes of the fragments");
   constexpr int kSlabs = static_cast<int>(KB / 64);
+  constexpr int kBlock = kSlabs <= 7 ? kSlabs : 4, kBlocks = kSlabs / kBlock, kRest = kSlabs % kBlock;
   const int c = lane & 15, g = lane >> 4;
   const char *a = static_cast<const char *>(A);
   const char *b = static_cast<const char *>(B);
-  v4i qf[RT][kSlabs];
+  u32 aOff[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const long row = row0 + 16 * rt + c;
-    const u32 off = static_cast<u32>((row < M ? row : M - 1) * KB) + 16u * static_cast<u32>(g);
-#pragma unroll
-    for (int i = 0; i < kSlabs; ++i) qf[rt][i] = *reinterpret_cast<const v4i *>(a + off + 64 * i);
+    aOff[rt] = static_cast<u32>((row < M ? row : M - 1) * KB) + 16u * static_cast<u32>(g);
   }
+  typename Mma::acc4_v acc[RT][NCHUNK][2];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+    for (int j = 0; j < NCHUNK; ++j) acc[rt][j][0] = acc[rt][j][1] = typename Mma::acc4_v{0, 0, 0, 0};
+  }
+  v4i qf[RT][kBlock];
+  auto loadRows = [&](auto slabs, u32 at) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+      for (int i = 0; i < slabs.value; ++i) qf[rt][i] = *reinterpret_cast<const v4i *>(a + aOff[rt] + at + 64 * i);
+    }
+  };
   // The fragments of kBatch units are requested together, in front of their MFMAs (left alone, the compiler keeps two
   // loads in flight and the wavefront waits out the L2 once per MFMA).
-  constexpr int kBatch = kSlabs >= 8 ? 1 : 8 / kSlabs;
+  auto multiply = [&](auto slabs, u32 at) {
+    constexpr int kCount = slabs.value, kBatch = kCount >= 8 ? 1 : 8 / kCount;
 #pragma unroll
-  for (int j0 = 0; j0 < NCHUNK; j0 += kBatch) {
-    v4i kf[kBatch][2][kSlabs];
+    for (int j0 = 0; j0 < NCHUNK; j0 += kBatch) {
+      v4i kf[kBatch][2][kCount];
 #pragma unroll
-    for (int j = j0; j < j0 + kBatch && j < NCHUNK; ++j) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        long col = 32L * row_unit<NCHUNK, WC>(j, wc) + 8 * (c >> 2) + 4 * h + (c & 3);
-        if constexpr (N % (32L * WC) != 0) col = col < N ? col : N - 1;
-        const u32 off = static_cast<u32>(col * KB) + 16u * static_cast<u32>(g);
-#pragma unroll
-        for (int i = 0; i < kSlabs; ++i) kf[j - j0][h][i] = *reinterpret_cast<const v4i *>(b + off + 64 * i);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = j0; j < j0 + kBatch && j < NCHUNK; ++j) {
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
+      for (int j = j0; j < j0 + kBatch && j < NCHUNK; ++j) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          typename Mma::acc4_v acc = {0, 0, 0, 0};
+          long col = 32L * row_unit<NCHUNK, WC>(j, wc) + 8 * (c >> 2) + 4 * h + (c & 3);
+          if constexpr (N % (32L * WC) != 0) col = col < N ? col : N - 1;
+          const u32 off = static_cast<u32>(col * KB) + 16u * static_cast<u32>(g) + at;
 #pragma unroll
-          for (int i = 0; i < kSlabs; ++i) acc = Mma::mma16(kf[j - j0][h][i], qf[rt][i], acc);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) s[rt][j][4 * h + v] = acc[v];
+          for (int i = 0; i < kCount; ++i) kf[j - j0][h][i] = *reinterpret_cast<const v4i *>(b + off + 64 * i);
         }
       }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = j0; j < j0 + kBatch && j < NCHUNK; ++j) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i < kCount; ++i) acc[rt][j][h] = Mma::mma16(kf[j - j0][h][i], qf[rt][i], acc[rt][j][h]);
+          }
+        }
+      }
+    }
+  };
+  loadRows(SlabCount<kBlock>(), 0);
+#pragma unroll 1
+  for (int t = 0; t < kBlocks; ++t) {
+    const u32 at = static_cast<u32>(t) * (64 * kBlock);
+    multiply(SlabCount<kBlock>(), at);
+    if (t + 1 < kBlocks) loadRows(SlabCount<kBlock>(), at + 64 * kBlock);
+  }
+  if constexpr (kRest > 0) {
+    loadRows(SlabCount<kRest>(), 64 * kBlock * kBlocks);
+    multiply(SlabCount<kRest>(), 64 * kBlock * kBlocks);
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+    for (int j = 0; j < NCHUNK; ++j) {
+#pragma unroll
+      for (int v = 0; v < 8; ++v) s[rt][j][v] = acc[rt][j][v >> 2][v & 3];
     }
   }
 }

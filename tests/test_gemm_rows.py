@@ -83,3 +83,94 @@ def test_scores_and_their_row_reductions(batch, m, k, n, dtype, mask, outputs):
             floor = 2.0 ** -25 if d.dtype == "float16" else 2.0 ** -126   # half a subnormal unit; results that underflow
             bad = (got - want).abs() > rel * want.abs() + (1e-4 if name == "max" else floor)
             assert not bool(bad.any()), "%s: %d of %d, first %d" % (name, int(bad.sum()), bad.numel(), int(bad.nonzero()[0]))
+
+
+def _scratch_bytes(directory):
+    """Private bytes per lane of the code objects under `directory` (the kernel descriptor's note, a MessagePack map)."""
+    import glob
+    import os
+    sizes = []
+    for path in glob.glob(os.path.join(str(directory), "**", "*.hsaco"), recursive=True):
+        data = open(path, "rb").read()
+        key = b".private_segment_fixed_size"
+        at = data.index(key) + len(key)
+        width = {0xcc: 1, 0xcd: 2, 0xce: 4}.get(data[at], 0)
+        sizes.append(int.from_bytes(data[at + 1:at + 1 + width], "big") if width else data[at])
+    return sizes
+
+
+@pytest.mark.parametrize("batch,m,k,n,family", [
+    (0, 16384, 224, 320, "gemm_rows"), (0, 16384, 256, 320, "staged"),      # one batch of many rows
+    (0, 8192, 384, 320, "gemm_rows"), (0, 8192, 416, 312, "staged"),        # ... of fewer
+    (0, 32768, 512, 64, "gemm_rows"), (0, 32768, 544, 64, "staged"), (0, 33024, 256, 64, "staged"),   # few columns
+    (0, 65536, 4096, 24, "gemm_rows"), (0, 65536, 4128, 24, "staged"), (0, 65536, 7168, 16, "staged"),
+    (0, 16384, 2048, 64, "staged"), (0, 16384, 1024, 128, "staged"),        # routers whose rows the registers did not hold
+    (64, 512, 512, 256, "gemm_rows"), (64, 512, 1024, 128, "staged"), (64, 46, 512, 224, "staged"), (64, 46, 384, 224, "gemm_rows"),
+    (20, 1378, 256, 176, "staged"), (107, 2032, 384, 56, "gemm_rows"),
+])
+def test_a_long_k_takes_the_row_kernel_where_it_is_the_faster_one_and_needs_no_scratch(batch, m, k, n, family, tmp_path):
+    kernel = driver.HipKernel(_scores(batch, m, k, n, "bfloat16", None, ["p"]), out_dir=str(tmp_path))
+    assert kernel.family == family
+    if family == "gemm_rows":
+        sizes = _scratch_bytes(tmp_path)
+        assert sizes and not any(sizes), sizes
+
+
+def test_wide_descriptions_run_as_two_kernels():
+    def family(n, masks, outputs, batch=64):
+        b = op_desc.DescBuilder("wide_%d_%d_%s" % (n, masks, outputs.replace("+", "_")))
+        q, kk = b.input([batch, 512, 64], "bfloat16"), b.input([batch, n, 64], "bfloat16")
+        attrs = [{"data_type": "bool", "name": "transpose_a", "value": False}, {"data_type": "bool", "name": "transpose_b", "value": True}]
+        raw = b.op("BatchMatMul", [q, kk], [batch, 512, n], "float32", attrs=attrs)
+        s = raw
+        for _ in range(masks):
+            s = b.add(s, b.input([batch, 512, n], "float32"))
+        e = b.unary("Exp", b.sub(s, b.reduce("ReduceMax", s, [2], True)))
+        p = b.div(e, b.reduce("ReduceSum", e, [2], True))
+        made = {"raw": lambda: raw, "masked": lambda: s, "p": lambda: p, "half": lambda: b.cast(p, "bfloat16")}
+        return driver.HipKernel(b.dumps([made[o]() for o in outputs.split("+")]), out_dir=None).family
+    assert family(2048, 3, "half", 32) == "gemm_rows" and family(2048, 4, "half", 32) == "staged"     # two row tiles: 4 and 5 beside the scores
+    assert family(2048, 4, "half", 16) == "gemm_rows" and family(2048, 5, "half", 16) == "staged"     # one: 5 and 6
+    assert family(2048, 2, "p", 32) == "gemm_rows" and family(2048, 1, "masked+p", 32) == "staged"
+    assert family(1024, 5, "half", 32) == "gemm_rows" and family(1024, 6, "half", 32) == "staged"
+    assert family(512, 8, "half") == "gemm_rows"
+    # scores that are written anyway
+    assert family(264, 1, "raw+half") == "staged" and family(256, 1, "raw+half") == "gemm_rows"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,m,k,n,dtype", [
+    (64, 70, 160, 72, "bfloat16"),      # five slabs of K held whole
+    (40, 130, 224, 104, "float16"),     # seven
+    (40, 130, 256, 200, "bfloat16"),    # two blocks
+    (33, 65, 288, 136, "bfloat16"),     # a block of one slab behind two
+    (0, 6100, 352, 264, "float16"),     # ... of three; three units of columns, one beyond N in part
+    (64, 70, 512, 248, "bfloat16"),
+    (0, 20000, 1056, 24, "bfloat16"),   # 33 slabs; fewer columns than a unit
+    (0, 33000, 4096, 8, "float16"),
+])
+def test_blocks_of_a_long_k(batch, m, k, n, dtype):
+    """Against float64. A score's float32 sum of k products is off by at most k * 2^-24 of the sum of the products'
+    magnitudes, a probability by twice the largest such error of its row (relative), beside 2^-14 for the exponential and
+    the row sum and half a unit of the result's type."""
+    import torch
+    kernel = driver.HipKernel(_scores(batch, m, k, n, dtype, None, ["p", "max"]), out_dir=None)
+    assert kernel.family == "gemm_rows"
+    print("case", batch, m, k, n, dtype, kernel.grid, kernel.block, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(k + n)
+    td = {"bfloat16": torch.bfloat16, "float16": torch.float16}[dtype]
+    q = torch.randn([max(batch, 1), m, k], generator=g, device="cuda").to(td)
+    kk = torch.randn([max(batch, 1), n, k], generator=g, device="cuda").to(td)
+    outs = [torch.full([d.nbytes], 255, dtype=torch.uint8, device="cuda") for d in kernel.outputs]
+    scale = float(np.float32(k ** -0.5))
+    s = torch.matmul(q.double(), kk.double().transpose(1, 2).contiguous()) * scale
+    off = torch.matmul(q.double().abs(), kk.double().abs().transpose(1, 2).contiguous()).amax(2, keepdim=True) * (scale * k * 2.0 ** -24)
+    for launch in range(2):
+        kernel.launch([q, kk] + outs)
+        torch.cuda.synchronize()
+        p, top = outs[0].view(td).double().reshape(s.shape), outs[1].view(torch.float32).double().reshape(off.shape)
+        want = torch.softmax(s, 2)
+        unit = 2.0 ** -8 if dtype == "bfloat16" else 2.0 ** -11
+        bad = (p - want).abs() > (2 * off + 2.0 ** -14 + unit) * want + 2.0 ** -25
+        assert not bool(bad.any()), "%d of %d, first %s" % (int(bad.sum()), bad.numel(), bad.nonzero()[0].tolist())
+        assert bool(((top - s.amax(2, keepdim=True)).abs() <= off + top.abs() * 2.0 ** -23).all())
