@@ -689,7 +689,7 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
   typedef typename Mma::acc_v acc_v;
   const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
   const long strip = static_cast<long>(blockIdx.x) % kStrips;   // neighbours in launch order read neighbouring columns
-  const int ksplit = static_cast<int>(static_cast<long>(blockIdx.x) / kStrips);
+  const int ksplit = kSplitPossible ? static_cast<int>(static_cast<long>(blockIdx.x) / kStrips) : 0;
   constexpr int kLine = 128;   // bytes of K that a wavefront takes at a time from every column of a [N,K] weight
   // Below 512 bytes of K not every wavefront would get a line: the fragments are then loaded as they are.
   constexpr bool kLines = TRANSB && K >= kWaves * kLine;
@@ -796,9 +796,10 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
     // A wavefront loads the line of eight columns per instruction and turns the 128 columns into operands through LDS of its
     // own (chunks permuted by the column: every bank once among the lanes served together), the next lines in flight
     // beside the MFMAs. Loading the operands as they are touches 32 lines by 32 bytes per instruction, and a line is evicted
-    // from the L1 before its fourth piece is read. bf16, before -> lines in order -> lines rotated (us): 16 x 8192 x 8192
-    // 38.8 -> 33.2 -> 26.4, 16 x 4096 x 11008 32.7 -> 23.2 -> 20.5, 64 x 8192 x 8192 46.3 -> 39.0 -> 34.8, 16 x 8192 x 1024 11.6 ->
-    // 9.8 -> 9.9; int8 16 x 8192 x 8192 20.6 -> 17.3 -> 17.0. Rotation or adjacent pieces alone, without whole lines: 37 .. 42.
+    // from the L1 before its fourth piece is read. bf16 (us): 16 x 8192 x 8192 38.8 with the operands as they are, 33.2 by whole
+    // lines, 28.4 with the strips rotated, 26.4 past the caches, 25.1 without a last request that nobody reads; 16 x 4096 x 11008
+    // 32.7 -> 20.3, 64 x 8192 x 8192 46.3 -> 32.0, 16 x 8192 x 1024 11.6 -> 9.6; int8 16 x 8192 x 8192 20.6 -> 16.6. Rotation or adjacent
+    // pieces alone, without whole lines: 37 .. 42.
     constexpr int kSub = kLine / 32;   // MFMA steps per line
     const long lines = (t1 - t0 + kSub - 1) / kSub;
     u8 *__restrict__ tile = akg_skinny_lds + wave * (128 * kLine);
@@ -825,8 +826,8 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
         for (int rt = 0; rt < kRowTiles; ++rt) ra[rt][u] = *reinterpret_cast<const v4i *>(A[rt] + (t + u < t1 ? t + u : t1 - 1) * 32);
       }
     };
-    if (wave < lines) loadLine(wave);
-    for (long i = wave; i < lines; i += kWaves) {   // (uniform per wavefront)
+    // one line per trip; the next one is requested behind its store (`more`: there is one)
+    auto trip = [&](long i, bool more) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int bc = 8 * j + lc;
@@ -840,7 +841,7 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      loadLine(i + kWaves < lines ? i + kWaves : i);
+      if (more) loadLine(i + kWaves);
       const long t = stepOf(i);
 #pragma unroll
       for (int u = 0; u < kSub; ++u) {
@@ -855,6 +856,12 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
+    };
+    if (wave < lines) {   // (uniform per wavefront)
+      long i = wave;
+      loadLine(i);
+      for (; i + kWaves < lines; i += kWaves) trip(i, true);
+      trip(i, false);
     }
     __syncthreads();   // the sums below lie where the lines did
   } else {

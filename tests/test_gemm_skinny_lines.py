@@ -49,3 +49,16 @@ def test_lines_of_a_transposed_weight_against_float64(m, k, n, dtype):
         torch.cuda.synchronize()
         gap = (out.double() - y).abs()
         assert bool((gap <= bound).all()), float((gap / bound).max())
+
+
+def test_every_line_of_the_weight_is_requested_once(tmp_path):
+    """512 bytes of K and one strip: each of the four wavefronts has one line of 128 columns, 16 loads of 16 bytes a lane, and
+    four of its row of A. A request for a line beyond the last one would be further loads in the code."""
+    import glob
+    import os
+    import subprocess
+    driver.HipKernel(op_desc.gemm_bias_act(16, 256, 128, "bfloat16", "none", transpose_b=True), out_dir=str(tmp_path))
+    path = glob.glob(os.path.join(str(tmp_path), "**", "*.hsaco"), recursive=True)[0]
+    objdump = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
+    code = subprocess.run([objdump, "-d", path], check=True, capture_output=True, text=True).stdout
+    assert code.count("global_load_dwordx4") == 16 + 4
