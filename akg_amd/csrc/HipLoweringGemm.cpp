@@ -179,14 +179,36 @@ class GemmEmitter {
     const double loop = 2.0 * static_cast<double>((steps + split - 1) / split * ((tiles * split + 255) / 256));
     return 6 + loop + (split == 1 ? 0 : 6 + 2 * static_cast<double>(split));
   }
-  // The small-tile kernel where its estimate is a tenth below that of the 256 x 256 kernel, and for 33 .. 64 rows in
-  // place of the skinny one. Measured over M = 48 .. 2500 and seven K x N, bf16 and int8, both layouts (us, before -> now):
-  // bf16 K x N = 1024 x 1024: M = 64 9.9 -> 6.9, 300 29.4 -> 7.3, 1200 25.9 -> 10.9; 2048 x 4096: 64 14.5 -> 10.1, 300 35.9 -> 17.2,
-  // 1200 46.3 -> 42.1; 8192 x 2048: 128 45.6 -> 19.1, 640 66.7 -> 59.7; 4096 x 11000: 300 94.9 -> 66.8, 640 139 -> 95;
-  // int8 4096 x 4096: 192 40.9 -> 13.2, 640 42.1 -> 27.3. It is the slower one, and the estimate says so, from
-  // M = 1200 on for 8192 x 2048 (85 us for 73) and 4096 x 11000 (171 for 136).
-  // Below 2 MiB and from 2^26 elements of B on the kernel and the splits stay those that the schedule tests pin (there the
-  // skinny kernel and eight or four K splits of the 256 x 256 one); so do narrow skinny products (N < 1024).
+  // 33 .. 64 rows: time in us of the skinny kernel and of 64 x 64 tiles, fitted to 1256 measured products (both layouts, 8 and
+  // 16 bits, K 512 .. 14336, N 1024 .. 16384; the first within 11 %, the second within a quarter; standard deviations 3 and 6 %).
+  double skinnyTime(int64_t split) const {
+    const double mb = static_cast<double>(k_ * n_ * elemBytes()) * 1e-6, rows = static_cast<double>(m_);
+    const double groups = static_cast<double>((n_ + 127) / 128 * split);
+    const bool wide = elemBytes() == 2;
+    const double start = transB_ ? (wide ? 9.1 : 7.8) : (wide ? 7.0 : 5.9), rate = transB_ ? (wide ? 0.155 : 0.175) : (wide ? 0.179 : 0.224);
+    const double perRow = (transB_ ? (wide ? 0.035 : 0.047) : 0.068) / 32, idle = transB_ ? 0.105 : (wide ? 0.16 : 0.136);
+    const double pitch = !transB_ && n_ * elemBytes() % 128 != 0 ? 0.04 : 0;   // rows of B begin inside a cache line
+    return start + mb * (rate + perRow * (rows - 33) + idle * std::max(0.0, 224 / groups - 1) + pitch) + 0.4 * static_cast<double>(split) * rows / 64;
+  }
+  double smallTileRowsTime(int64_t split) const {
+    const int64_t steps = (k_ * elemBytes() + 127) / 128;
+    const double perCu = static_cast<double>((n_ + 63) / 64 * split) / 256, mb = static_cast<double>(k_ * n_ * elemBytes()) * 1e-6;
+    const bool transposing8 = elemBytes() == 1 && !transB_;
+    const double step = perCu <= 1 ? (transposing8 ? 0.35 : 0.23) : (transposing8 ? 0.6 : 0.41), rate = transposing8 ? 0.17 : 0.113;
+    return 2.7 + static_cast<double>((steps + split - 1) / split) * step + mb * rate + (split > 1 ? 1.8 + 0.25 * static_cast<double>(split) + 0.5 * perCu : 0);
+  }
+  // The small-tile kernel where its estimate is a tenth below that of the 256 x 256 kernel, and for 33 .. 64 rows where the
+  // skinny one is not estimated a twentieth faster ([N,K] weights, whose estimates scatter more: a tenth, and those of
+  // 16 bits are the skinny kernel's from 60 Mi elements on, where 8192 x 8184 takes 36.3 us for 30.3). Measured (us, the other
+  // kernel -> small tiles): bf16 K x N = 1024 x 1024: M = 64 10.3 -> 6.7, 300 29.4 -> 7.3, 1200 25.9 -> 10.9; 2048 x 4096: 64 16.8 -> 10.0, 300 35.9 -> 17.2, 1200 46.3 -> 42.1; 8192 x 2048:
+  // 128 45.6 -> 19.1, 640 66.7 -> 59.7; 4096 x 11000: 300 94.9 -> 53, 640 139 -> 95; int8 4096 x 4096: 192 40.9 -> 13.2, 640 42.1 ->
+  // 27.3. It is the slower one, and the estimates say so, from M = 1200 on for 8192 x 2048 (85 us for 73) and 4096 x 11000 (171 for
+  // 136), and at 33 rows for [K,N] weights of bf16 8192 x 6144 (30.9 for 26.1), int8 4096 x 6144 (14.8 for 13.4) and 6144 x 9216
+  // (27.9 for 20.0), for [N,K] of bf16 11008 x 5120 (34.1 for 28.1).
+  // Below 2 MiB and from 2^26 elements of B on the kernels and splits of the other two stand. From 65 rows on that is not where the
+  // small tiles stop being the faster ones: bf16 512 x 768 with 256 rows takes 21.4 us for their 4.8, 8192 x 8192 with 96
+  // rows 50.7 for 41.5, with 256 rows 72.5 for 71.3, 14336 x 8192 with 256 rows 109 for 128. Narrow products of at most 64 rows (N <
+  // 1024) are the skinny kernel's.
   bool pickSmallTile() {
     if (serial_ || dyn_ || batch_ != 1 || opt_.split > 0 || (opt_.variant & (8 | 128))) return false;
     const int64_t elements = k_ * n_;
@@ -207,7 +229,23 @@ class GemmEmitter {
       tileN_ = s[1];
       kSplit_ = s[2];
     }
+    const bool large = transB_ && elemBytes() == 2 && elements >= (60LL << 20);
+    if (skinnyTakes() && (large || skinnyTime(skinnySplit()) < (transB_ ? 0.9 : 0.95) * smallTileRowsTime(kSplit_))) tileM_ = tileN_ = 0;
     return tileM_ > 0;
+  }
+
+  bool skinnyTakes() const {
+    return m_ <= skinnyRows() && (k_ * elemBytes()) % 32 == 0 && (transB_ || n_ % 4 == 0) && !(opt_.variant & 8);
+  }
+  int64_t skinnySplit() const {
+    const int64_t strips = (n_ + 127) / 128, steps = k_ * elemBytes() / 32;
+    int64_t want = opt_.split > 0 ? opt_.split : std::max<int64_t>(1, 256 / (strips * batch_));
+    want = std::min<int64_t>(want, std::max<int64_t>(1, opt_.split > 0 ? steps : steps / 16));
+    // (the last workgroup of a strip adds the partials of all its splits: 16 x 8192 x 1024 takes 10.1 us with 16
+    // splits, 12.9 with the 32 that would fill the chip)
+    want = std::min<int64_t>(want, 16);
+    while (want > 1 && strips * batch_ * want * m_ * 128 * 4 >= (1LL << 30)) --want;
+    return want;
   }
 
   // Few tiles and a long K (a skinny activation in front of a big weight matrix: M = 16 .. 1024 against 8192 x 8192
@@ -218,21 +256,15 @@ class GemmEmitter {
     if (serial_) return;
     dyn_ = opt_.extentAsArgument && batch_ == 1;
     if (pickSmallTile()) return;
+    kSplit_ = 1;
     // At most 64 rows of A (and K a multiple of 32 bytes): the time is that of streaming B, which gemm_skinny reads
     // straight into MFMA operands; 256 workgroups of four wavefronts (one per CU: 16 x 8192 x 8192 bf16 reaches 66 % of
     // the HBM peak with 4 splits of 64 strips, 59 % with 8, 48 % with 2; 8 wavefronts or more steps in flight change
     // nothing), each wavefront with at least 4 MFMA steps.
     // AKG_HIP_VARIANT bit 3 keeps the 256 x 256 tile kernel.
-    skinny_ = m_ <= skinnyRows() && (k_ * elemBytes()) % 32 == 0 && (transB_ || n_ % 4 == 0) && !(opt_.variant & 8);
+    skinny_ = skinnyTakes();
     if (skinny_) {
-      const int64_t strips = (n_ + 127) / 128, steps = k_ * elemBytes() / 32;
-      int64_t want = opt_.split > 0 ? opt_.split : std::max<int64_t>(1, 256 / (strips * batch_));
-      want = std::min<int64_t>(want, std::max<int64_t>(1, opt_.split > 0 ? steps : steps / 16));
-      // (the last workgroup of a strip adds the partials of all its splits: 16 x 8192 x 1024 takes 10.1 us with 16
-      // splits, 12.9 with the 32 that would fill the chip)
-      want = std::min<int64_t>(want, 16);
-      while (want > 1 && strips * batch_ * want * m_ * 128 * 4 >= (1LL << 30)) --want;
-      kSplit_ = static_cast<int>(want);
+      kSplit_ = static_cast<int>(skinnySplit());
       return;
     }
     if (batch_ != 1) return;

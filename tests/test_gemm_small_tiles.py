@@ -85,3 +85,18 @@ def test_small_tiles_against_float64(m, k, n, dtype, tb, tile, tmp_path):
         torch.cuda.synchronize()
         bad = (out.double() - exact).abs() > slack
         assert not bool(bad.any()), "launch %d: %d wrong, first %s" % (launch, int(bad.sum()), bad.nonzero()[0].tolist())
+
+
+@pytest.mark.parametrize("m,k,n,dtype,tb,kernel", [
+    # [K,N] weights: the skinny kernel is the faster one where the tiles leave CUs with two workgroups
+    (33, 8192, 6144, "bfloat16", False, "skinny"), (33, 8192, 2048, "bfloat16", False, "tile"), (64, 4096, 4096, "bfloat16", False, "tile"),
+    (33, 14336, 4096, "bfloat16", False, "skinny"), (33, 8192, 8184, "bfloat16", False, "tile"),   # (rows of B inside cache lines)
+    (33, 4096, 6144, "int8", False, "skinny"), (48, 6144, 9216, "int8", False, "skinny"), (64, 4096, 4096, "int8", False, "tile"),
+    (33, 2048, 4096, "int8", False, "tile"),
+    # [N,K] weights
+    (33, 11008, 5120, "bfloat16", True, "skinny"), (64, 11008, 5120, "bfloat16", True, "skinny"), (33, 4096, 4096, "bfloat16", True, "tile"),
+    (33, 8192, 4096, "bfloat16", True, "tile"), (33, 8192, 8184, "bfloat16", True, "skinny"), (33, 4096, 11008, "int8", True, "tile"), (33, 8192, 6144, "int8", True, "tile"),
+])
+def test_33_to_64_rows_take_the_faster_of_skinny_and_small_tiles(m, k, n, dtype, tb, kernel, tmp_path):
+    note = _schedule(_product(m, k, n, dtype, tb, "rows_%s_%d_%d_%d_%d" % (dtype, m, k, n, tb)), tmp_path)
+    assert (" skinny" in note) == (kernel == "skinny") and ("tile=64x64" in note) == (kernel == "tile"), note
