@@ -39,7 +39,7 @@ const char *kernelFamilyName(KernelFamily f);
 struct LoweringOptions {
   int vec = 0;          // elements per chunk
   int threadsPerRow = 0;
-  int chunks = 0;       // chunks per thread
+  int chunks = 0;       // chunks per thread (skinny contractions: steps in flight; whole lines of a [N,K] weight are always one)
   int block = 0;        // threads per workgroup
   int split = 0;        // streaming reductions: workgroups sharing one group of outputs (AKG_HIP_SPLIT)
   // Experiment switch (AKG_HIP_VARIANT), read by whichever family lowers the kernel; 0 = the measured default.

@@ -99,7 +99,8 @@ class GemmEmitter {
       note << " serial: the reference's k-ordered sum in the declared type on the vector ALUs, tile=64x" << 16 * epiWidth()
            << " grid=" << k.grid[0];
     } else if (skinny_) {
-      note << " skinny: strips of 128 columns, B straight into MFMA operands, mfma=" << mfmaName(false) << " waves=4 grid=" << k.grid[0];
+      note << " skinny: strips of 128 columns, B " << (skinnyLines() ? (streamsLines() ? "by whole lines past the caches" : "by whole lines") : "straight into MFMA operands")
+           << ", mfma=" << mfmaName(false) << " waves=" << skinnyWaves() << " grid=" << k.grid[0];
     } else if (tileM_ > 0) {
       note << " tile=" << tileM_ << "x" << tileN_ << "x" << stepK() / elemBytes() << " mfma=" << mfmaName(true) << " waves=2x2 grid=" << k.grid[0];
     } else {
@@ -122,13 +123,22 @@ class GemmEmitter {
   int skinnyWaves() const { return opt_.block == 512 ? 8 : 4; }
   int skinnyUnroll() const { return opt_.chunks > 0 ? opt_.chunks : 2; }
   // A [N,K] weight with a short K is read in 32-byte pieces, four per cache line, by instructions that follow each other:
-  // with the non-temporal hint the line is not kept for the next piece. (For a longer K the kernel reads whole lines and
-  // decides by the size of the weight.)
+  // with the non-temporal hint the line is not kept for the next piece. (For a longer K the kernel reads whole lines.)
   bool skinnyNonTemporal() const { return opt_.nonTemporal != 0 && !transB_; }
+  bool skinnyLines() const { return transB_ && k_ * elemBytes() >= 128 * skinnyWaves(); }   // (kLines of gemm_skinny)
+  // Whole lines of a [N,K] weight are read once, so from 16 MiB on (all batches together) they are read past the caches. Weights
+  // not used for 600 MB of traffic, with the hint and without (us): bf16 16 x 2048 x 2048 (8 MiB) 7.3 and 7.0, 16 x 4096 x 2048 (16 MiB)
+  // 10.2 and 10.5, 16 x 4096 x 4096 11.2 and 11.7, 16 x 8192 x 8192 25.0 and 27.6, 64 x 8192 x 8192 31.8 and 34.4, int8 16 x 4096 x 2048 (8 MiB)
+  // 7.5 and 7.2, 16 x 4096 x 4096 (16 MiB) 9.2 and 9.8, 64 batches of 16 x 512 x 2048 26.2 and 28.4. The same weight in call after call:
+  // 9.1 either way for 4096 x 4096, 23.0 and 22.6 for 8192 x 8192, 16 batches of 16 x 2048 x 2048 28.5 and 22.6. A line that does not end
+  // with the column belongs to two of them and needs its second look.
+  bool streamsLines() const {
+    return opt_.nonTemporal != 0 && skinnyLines() && k_ * elemBytes() % 128 == 0 && batch_ * n_ * k_ * elemBytes() >= (16LL << 20);
+  }
   bool serial_ = false;  // no MFMA kernel takes the description: gemm_serial (akg_gemm_serial.hpp)
   int epiWidth() const { return (serial_ && n_ % 4 != 0) ? 1 : 4; }   // adjacent result columns per epilogue call
   int tileM_ = 0, tileN_ = 0;   // gemm_small_tile: its tile (0: another kernel)
-  bool skinny_ = false;  // M <= 64: the kernel that streams B straight into MFMA operands (gemm_skinny)
+  bool skinny_ = false;  // M <= 64: the kernel that streams B, without barriers (gemm_skinny)
   // A dynamic description (extents bound per call): M and the K split are kernel arguments, so the source - and with it
   // the code object - is the same for every token count; the skinny kernel comes in three sizes (16, 32, 64 rows).
   bool dyn_ = false;
@@ -605,13 +615,13 @@ class GemmEmitter {
       if (dyn_) {
         src_ << "  akg::gemm_skinny<" << mmaTraits() << ", " << skinnyBucket() << "L, " << n_ << "L, " << k_ << "L, " << (transB_ ? "true" : "false")
              << ", Epilogue, 1, " << skinnyWaves() << ", " << skinnyUnroll() << ", " << (skinnyNonTemporal() ? "true" : "false") << ", true>(in"
-             << g_.tensor(aId_).inputIndex << ", in" << g_.tensor(bId_).inputIndex << ", epi, akg_ws, 0L, akg_m, static_cast<int>(akg_ksplit));\n}\n";
+             << g_.tensor(aId_).inputIndex << ", in" << g_.tensor(bId_).inputIndex << ", epi, akg_ws, 0L, akg_m, static_cast<int>(akg_ksplit)" << (streamsLines() ? ", akg::StreamedLines()" : "") << ");\n}\n";
         return;
       }
       src_ << "  akg::gemm_skinny<" << mmaTraits() << ", " << m_ << "L, " << n_ << "L, " << k_ << "L, " << (transB_ ? "true" : "false")
            << ", Epilogue, " << kSplit_ << ", " << skinnyWaves() << ", " << skinnyUnroll() << ", " << (skinnyNonTemporal() ? "true" : "false") << ">(in" << g_.tensor(aId_).inputIndex << " + akg_batch * " << m_ * k_ << "L, in"
            << g_.tensor(bId_).inputIndex << " + akg_batch * " << k_ * n_ << "L, epi, " << (kSplit_ > 1 ? "akg_ws" : "nullptr")
-           << ", akg_batch * " << (n_ + 127) / 128 << "L);\n}\n";
+           << ", akg_batch * " << (n_ + 127) / 128 << "L" << (streamsLines() ? ", 0L, 1, akg::StreamedLines()" : "") << ");\n}\n";
       return;
     }
     if (tileM_ > 0) {

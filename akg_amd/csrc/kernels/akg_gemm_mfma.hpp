@@ -667,9 +667,17 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
 // that owns (row, 4 columns) runs the epilogue on the sums. Deterministic; B is read exactly once.
 // DYN: MS is the most rows the code object takes (16, 32 or 64), the actual row count and the number of K splits are
 // kernel arguments (`mDyn` <= MS, `ksDyn`); `ws` is always a valid pointer.
-template <typename Mma, long MS, long N, long KE, bool TRANSB, typename Epilogue, int KSPLIT, int WAVES = 4, int UNROLL = 2, bool NT = false, bool DYN = false>
+// UNROLL and NT are those of the operands loaded as they are; whole lines of a [N,K] weight are one in flight, past the
+// caches with StreamedLines.
+struct CachedLines {
+  static constexpr bool kPastCaches = false;
+};
+struct StreamedLines {
+  static constexpr bool kPastCaches = true;
+};
+template <typename Mma, long MS, long N, long KE, bool TRANSB, typename Epilogue, int KSPLIT, int WAVES = 4, int UNROLL = 2, bool NT = false, bool DYN = false, typename Lines = CachedLines>
 AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ Bv, Epilogue &epi,
-                         unsigned *__restrict__ ws, long group0, long mDyn = 0, int ksDyn = 1) {
+                         unsigned *__restrict__ ws, long group0, long mDyn = 0, int ksDyn = 1, Lines = Lines()) {
   const long M = DYN ? mDyn : MS;
   const int kSplits = DYN ? ksDyn : KSPLIT;
   constexpr bool kSplitPossible = DYN || KSPLIT > 1;
@@ -693,10 +701,7 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
   constexpr int kLine = 128;   // bytes of K that a wavefront takes at a time from every column of a [N,K] weight
   // Below 512 bytes of K not every wavefront would get a line: the fragments are then loaded as they are.
   constexpr bool kLines = TRANSB && K >= kWaves * kLine;
-  // Whole lines need no second look, so a weight larger than what the caches hold is read past them: bf16 16 x 8192 x 8192
-  // 28.4 us without the hint, 26.4 with it; 11008 x 4096 20.6 and 20.5; 2048 x 2048, which stays cached, 7.8 and 8.5; int8
-  // 8192 x 8192 17.0 and 17.1.
-  constexpr bool kLinesNonTemporal = K % kLine == 0 && N * K >= (96L << 20);
+  static_assert(!Lines::kPastCaches || K % kLine == 0, "a line at the end of a column is read for two columns");
   constexpr long kUnit = kLines ? kLine / 32 : 1, kUnits = (kSteps + kUnit - 1) / kUnit;   // a range of K ends on a whole line
   const long t0 = kUnits * ksplit / kSplits * kUnit, tEnd = kUnits * (ksplit + 1) / kSplits * kUnit;
   const long t1 = tEnd < kSteps ? tEnd : kSteps;
@@ -818,7 +823,7 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
         long bc = strip * 128 + 8 * j + lc;
         if constexpr (N % 128 != 0) bc = bc < N ? bc : 0;
         const v4i *bp = reinterpret_cast<const v4i *>(from + bc * K);
-        raw[j] = kLinesNonTemporal ? __builtin_nontemporal_load(bp) : *bp;
+        raw[j] = Lines::kPastCaches ? __builtin_nontemporal_load(bp) : *bp;
       }
 #pragma unroll
       for (int u = 0; u < kSub; ++u) {

@@ -832,7 +832,7 @@ def test_streaming_schedules_follow_what_was_measured():
     assert "k_splits=8" in _meta_schedule(k)
     k = driver.HipKernel(op_desc.gemm_bias_act(16, 8192, 1024, "bfloat16", "gelu", False, "float32", "sched_split_skinny"))
     assert "k_splits=16" in _meta_schedule(k)
-    # a [N,K] weight is loaded without the non-temporal hint, a row-major one with it
+    # the operands of a [N,K] weight loaded as they are carry no non-temporal hint (its whole lines have a rule of their own)
     k = driver.HipKernel(op_desc.gemm_bias_act(16, 8192, 8192, "bfloat16", "gelu", True, "float32", "sched_skinny_nk"), out_dir=None)
     assert "true, Epilogue, 4, 4, 2, false>" in k.source
 
