@@ -42,7 +42,7 @@ class _KernelInfo(ctypes.Structure):
 
 
 _lib = None
-_launch = None          # the extension module of the launch path (csrc/launch_module.cpp)
+_launch = None          # the extension module of the launch path (csrc/launch_module.cpp), where there is one
 _current_device = None  # torch's current device and the raw handle of its current stream, without a Stream object
 _raw_stream = None
 
@@ -92,8 +92,11 @@ def load_library():
                                                   ctypes.POINTER(vp)]
     lib.akg_hip_dynamic_destroy.argtypes = [vp]
     lib.akg_hip_dynamic_destroy.restype = None
-    from . import _launch as launch_module  # pylint: disable=import-outside-toplevel
-    _launch = launch_module
+    try:
+        from . import _launch as launch_module  # pylint: disable=import-outside-toplevel
+        _launch = launch_module
+    except ImportError:
+        _launch = None   # not built for this interpreter: launches go through ctypes
     _lib = lib
     return lib
 
@@ -147,7 +150,7 @@ class HipDynamicKernel:
         """The reference's dynamic calling form (LLVMParameterPacking.cpp:91-194): `device_ptrs` for inputs then outputs,
         `shapes` their concrete shapes; packs [0, sizes, strides] per tensor like transform_data_to_ctypes
         (mlir_driver.py:186-252) and returns the HipKernel that ran."""
-        if self._handle:
+        if self._handle and _launch is not None:
             packed = _launch.launch_packed(self._handle.value, device_ptrs, shapes, stream or 0)
             if packed is not None:
                 rc, key = packed
@@ -282,7 +285,7 @@ class HipKernel:
 
     def launch(self, tensors, stream=None):
         """Launch on torch device tensors (inputs then outputs), on `stream` (a torch stream) or the current one."""
-        if self._handle:
+        if self._handle and _launch is not None:
             rc = _launch.launch(self._handle.value, self._nbytes, tensors, stream, _current_device, _raw_stream)
             if rc == 0:
                 return

@@ -35,6 +35,44 @@ def test_arguments_that_the_native_path_leaves_to_python():
         d.launch_packed([1], [[5, 64]])
 
 
+def test_without_the_module_launches_go_through_ctypes():
+    """An interpreter that no module was built for imports the driver all the same, and what is refused is refused alike."""
+    import os
+    import subprocess
+    import sys
+    import sysconfig
+    assert os.path.basename(driver._launch.__file__) == "_launch" + sysconfig.get_config_var("EXT_SUFFIX")   # (no other one loads it)
+    code = """
+import sys
+class Absent:
+    def find_spec(self, name, path=None, target=None):
+        if name == "akg_amd._launch":
+            raise ImportError("built for another interpreter")
+sys.meta_path.insert(0, Absent())
+import torch
+from akg_amd import driver, op_desc
+k = driver.HipKernel(op_desc.elementwise_tanh_add_mul(7, 33), out_dir=None)
+assert driver._launch is None
+try:
+    k.launch([torch.zeros(7, 33) for _ in range(4)])
+except ValueError as e:
+    assert "contiguous device tensor" in str(e)
+else:
+    raise AssertionError("a host tensor was launched on")
+b = op_desc.DescBuilder("launch_module_absent")
+x = b.input([-1, 64], "float32")
+d = driver.HipDynamicKernel(b.dumps([b.op("Tanh", [x], [-1, 64], "float32")]), out_dir=None)
+try:
+    d.launch_packed([1, 2], [[5, 64], [6, 64]])
+except driver.AkgHipError as e:
+    assert "does not follow from the input shapes" in str(e)
+else:
+    raise AssertionError("inconsistent shapes were launched")
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=root, env=dict(os.environ, PYTHONPATH=root))
+
+
 @pytest.mark.gpu
 def test_launches_on_the_current_and_on_a_given_stream():
     k = driver.HipKernel(op_desc.elementwise_tanh_add_mul(37, 130), out_dir=None)
@@ -64,3 +102,20 @@ def test_launches_on_the_current_and_on_a_given_stream():
         used = d.launch_packed([x.data_ptr(), y.data_ptr()], [x.shape, list(y.shape)], torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
         assert torch.allclose(y, torch.tanh(x), rtol=1e-5, atol=1e-6) and used is d.launch_packed([x.data_ptr(), y.data_ptr()], [x.shape, y.shape])
+
+
+@pytest.mark.gpu
+def test_without_the_module_the_results_are_the_same(monkeypatch):
+    k = driver.HipKernel(op_desc.elementwise_tanh_add_mul(37, 130), out_dir=None)
+    d = driver.HipDynamicKernel(_dynamic())
+    a, b, c = (torch.randn(37, 130, device="cuda") for _ in range(3))
+    x = torch.randn(5, 64, device="cuda")
+    results = []
+    for module in (driver._launch, None):
+        monkeypatch.setattr(driver, "_launch", module)
+        out, y = torch.zeros(37, 130, device="cuda"), torch.zeros(5, 64, device="cuda")
+        k.launch([a, b, c, out])
+        d.launch_packed([x.data_ptr(), y.data_ptr()], [x.shape, y.shape], torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        results.append((out, y))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
