@@ -128,6 +128,9 @@ class GemmRowsEmitter {
         if (in == aId_ || in == bId_) throw LoweringError("MatMul operands cannot also feed the ops behind it");
       }
     }
+    for (size_t i = 0; i < g_.outputs.size(); ++i) {
+      if (std::count(g_.outputs.begin(), g_.outputs.end(), g_.outputs[i]) > 1) throw LoweringError("an output is listed twice");
+    }
     for (const TensorValue &t : g_.tensors) {
       if (!t.isConst && (t.inputIndex >= 0 || t.outputIndex >= 0) && t.numel() * static_cast<int64_t>(dtypeSize(t.dtype)) >= (1LL << 31)) {
         throw LoweringError("tensor " + t.name + ": the row kernel addresses less than 2 GiB per tensor");

@@ -138,6 +138,21 @@ def test_wide_descriptions_run_as_two_kernels():
     assert family(264, 1, "raw+half") == "staged" and family(256, 1, "raw+half") == "gemm_rows"
 
 
+def test_what_two_kernels_refuse_is_refused(monkeypatch):
+    """An output that is listed twice: refused by the plan of several kernels, whichever kernel is asked first."""
+    text = _scores(64, 256, 64, 256, "bfloat16", None, ["p32", "p32"])
+    b = op_desc.DescBuilder("scores_twice")
+    q, kk = b.input([64, 256, 64], "bfloat16"), b.input([64, 256, 64], "bfloat16")
+    attrs = [{"data_type": "bool", "name": "transpose_a", "value": False}, {"data_type": "bool", "name": "transpose_b", "value": True}]
+    s = b.op("BatchMatMul", [q, kk], [64, 256, 256], "float32", attrs=attrs)
+    p = b.sub(s, b.reduce("ReduceMax", s, [2], True))
+    assert driver.HipKernel(text, out_dir=None).family == "gemm_rows"    # (two results that happen to be equal)
+    for variant in ("0", "16"):
+        monkeypatch.setenv("AKG_HIP_VARIANT", variant)
+        with pytest.raises(driver.AkgHipError):
+            driver.HipKernel(b.dumps([p, p]), out_dir=None)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,m,k,n,dtype", [
     (64, 70, 160, 72, "bfloat16"),      # five slabs of K held whole
