@@ -189,3 +189,88 @@ def test_blocks_of_a_long_k(batch, m, k, n, dtype):
         bad = (p - want).abs() > (2 * off + 2.0 ** -14 + unit) * want + 2.0 ** -25
         assert not bool(bad.any()), "%d of %d, first %s" % (int(bad.sum()), bad.numel(), bad.nonzero()[0].tolist())
         assert bool(((top - s.amax(2, keepdim=True)).abs() <= off + top.abs() * 2.0 ** -23).all())
+
+
+def _typed(mask_type, n, batch=48, m=250):
+    """Scores with a mask of `mask_type` and results of several types, among them whole numbers and truth values."""
+    b = op_desc.DescBuilder("typed_%s_%d" % (mask_type, n))
+    q, kk = b.input([batch, m, 64], "bfloat16"), b.input([batch, n, 64], "bfloat16")
+    x = b.input([batch, m, n], mask_type)
+    attrs = [{"data_type": "bool", "name": "transpose_a", "value": False}, {"data_type": "bool", "name": "transpose_b", "value": True}]
+    s = b.mul(b.op("BatchMatMul", [q, kk], [batch, m, n], "float32", attrs=attrs), b.const(0.125, "float32"))
+    if mask_type == "bool":
+        s = b.op("Select", [x, s, b.const(-10000.0, "float32")], [batch, m, n], "float32")
+    else:
+        s = b.add(s, x if mask_type == "float32" else b.cast(x, "float32"))
+    top = b.reduce("ReduceMax", s, [2], True)
+    e = b.unary("Exp", b.sub(s, top))
+    p = b.div(e, b.reduce("ReduceSum", e, [2], True))
+    if mask_type == "float32":
+        return b.dumps([b.cast(p, "float16"), top])
+    if mask_type == "bool":
+        return b.dumps([b.op("Greater", [p, b.const(0.01, "float32")], [batch, m, n], "bool")])
+    if mask_type == "int8":
+        return b.dumps([b.cast(b.mul(p, b.const(127.0, "float32")), "int8"), b.reduce("ReduceMax", b.cast(s, "int32"), [2], True)])
+    if mask_type == "int64":
+        return b.dumps([b.cast(p, "bfloat16"), b.reduce("ReduceMin", s, [2], False)])
+    return b.dumps([b.cast(p, "float64")])
+
+
+@pytest.mark.parametrize("mask_type", ["float32", "bool", "int8", "int64", "float64"])
+def test_types_that_take_the_row_kernel(mask_type):
+    assert driver.HipKernel(_typed(mask_type, 200), out_dir=None).family == "gemm_rows"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [200, 1032])
+@pytest.mark.parametrize("mask_type", ["float32", "bool", "int8", "int64", "float64"])
+def test_types_masks_and_values_at_the_ends_against_two_kernels(mask_type, n, monkeypatch):
+    """The one-kernel form against a contraction and a row kernel, which work on the same float32 scores. Scores that are
+    masked throughout, by a large number, the lowest one or -inf, and NaN and infinity in an operand: where the two forms
+    have NaN or infinity has to be the same. Finite results: a score differs by the order of 64 products of bfloat16 (2 * 64 * 2^-24
+    of the sum of their magnitudes, below 2^-10 here: |q k| < 300), a probability by twice that, 2^-13 for the exponential
+    and the row sums, and a unit of its type; a whole number by one and a truth value only next to the line."""
+    import torch
+    text = _typed(mask_type, n)
+    one = driver.HipKernel(text, out_dir=None)
+    monkeypatch.setenv("AKG_HIP_VARIANT", "16")
+    two = driver.HipKernel(text, out_dir=None)
+    assert one.family == "gemm_rows" and two.family == "staged"
+    print("case", mask_type, n, one.grid, one.block, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    q = torch.randn([48, 250, 64], generator=g, device="cuda").bfloat16()
+    kk = torch.randn([48, n, 64], generator=g, device="cuda").bfloat16()
+    x = torch.randn([48, 250, n], generator=g, device="cuda")
+    if mask_type == "bool":
+        x = x > -0.5
+        x[0, 0] = False
+        x[5, 249, n - 1] = False
+    elif mask_type in ("int8", "int64"):
+        x = (x * 3).to(getattr(torch, mask_type))
+        x[0, 0] = -128
+    else:
+        low = float(np.finfo(np.float32).min)
+        x = torch.where(torch.rand(x.shape, generator=g, device="cuda") < 0.3, torch.full_like(x, -10000.0), x).to(getattr(torch, mask_type))
+        x[0, 0], x[0, 1], x[0, 2, : n // 2], x[47, 249, 1:] = float("-inf"), low, float("-inf"), low
+        x[1, 7, n - 1] = float("nan")
+    q[2, 3, 5] = float("nan")
+    kk[3, n - 1, 0] = float("nan")
+    q[4, 249, 63] = float("inf")
+    results = []
+    for kernel in (one, two):
+        outs = [torch.full([d.nbytes], 255, dtype=torch.uint8, device="cuda") for d in kernel.outputs]
+        kernel.launch([q, kk, x] + outs)
+        torch.cuda.synchronize()
+        results.append([o.view(getattr(torch, d.dtype)).double() for o, d in zip(outs, kernel.outputs)])
+    unit = {"bfloat16": 2.0 ** -7, "float16": 2.0 ** -10, "float32": 2.0 ** -22, "float64": 2.0 ** -22}
+    for d, a, b in zip(one.outputs, *results):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()), d.dtype
+        finite = a.isfinite()
+        a, b = a[finite], b[finite]
+        if d.dtype == "bool":
+            assert int((a != b).sum()) <= a.numel() // 1000       # (|p - 0.01| < 0.01 * 2^-8 for fewer than one in a thousand)
+        elif d.dtype in ("int8", "int32"):
+            assert bool(((a - b).abs() <= 1).all()) and int((a != b).sum()) <= a.numel() // 100
+        else:
+            bound = b.abs() * (2.0 ** -9 + 2.0 ** -13 + unit[d.dtype]) + (2.0 ** -9 if a.numel() <= 48 * 250 else 2.0 ** -24)
+            assert bool(((a - b).abs() <= bound).all()), (d.dtype, float(((a - b).abs() / bound).max()))

@@ -119,3 +119,40 @@ def test_without_the_module_the_results_are_the_same(monkeypatch):
         torch.cuda.synchronize()
         results.append((out, y))
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
+@pytest.mark.gpu
+def test_two_threads_launch_through_the_module():
+    """One static and one dynamic handle, launched by two threads on streams of their own: each gets its own results and its
+    own errors (a refused launch in one thread says nothing in the other)."""
+    import threading
+    k = driver.HipKernel(op_desc.elementwise_tanh_add_mul(37, 130), out_dir=None)
+    k.prepare()
+    d = driver.HipDynamicKernel(_dynamic())
+    failures = []
+
+    def work(seed):
+        try:
+            g = torch.Generator(device="cuda").manual_seed(seed)
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                a, b, c = (torch.randn(37, 130, generator=g, device="cuda") for _ in range(3))
+                x = torch.randn(5 + seed, 64, generator=g, device="cuda")
+                for step in range(50):
+                    out, y = torch.zeros(37, 130, device="cuda"), torch.zeros(5 + seed, 64, device="cuda")
+                    k.launch([a, b, c, out])
+                    d.launch_packed([x.data_ptr(), y.data_ptr()], [x.shape, y.shape], stream.cuda_stream)
+                    with pytest.raises(driver.AkgHipError, match="does not follow"):
+                        d.launch_packed([x.data_ptr(), y.data_ptr()], [x.shape, (4 + seed, 64)], stream.cuda_stream)
+                    stream.synchronize()
+                    assert torch.allclose(out, torch.tanh((a + b) * c), rtol=1e-5, atol=1e-6), step
+                    assert torch.allclose(y, torch.tanh(x), rtol=1e-5, atol=1e-6), step
+        except BaseException as e:   # pylint: disable=broad-except
+            failures.append((seed, e))
+
+    threads = [threading.Thread(target=work, args=(seed,)) for seed in (1, 2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
