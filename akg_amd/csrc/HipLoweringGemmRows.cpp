@@ -97,6 +97,7 @@ class GemmRowsEmitter {
         c.shape[rank - 1] != n_ || batch_ < 1 || m_ < 1) {
       throw LoweringError("MatMul: inconsistent shapes");
     }
+    if (batch_ > 65535) throw LoweringError("MatMul: batch extent out of range");   // (the contraction kernel's limit)
     // Where the line lies (bf16 or f16, GPU time of one kernel against a contraction and a row kernel):
     //   [192,512,64]x512 77 us for 149, [384,256,64]x256 43 for 142, [24,2048,64]x2048 174 for 238, [380,77,64]x80 8.7 for 48;
     //   every row group reads all of B from the L2, which costs more than the scores' way through memory once B is large

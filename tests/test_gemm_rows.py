@@ -139,7 +139,7 @@ def test_wide_descriptions_run_as_two_kernels():
 
 
 def test_what_two_kernels_refuse_is_refused(monkeypatch):
-    """An output that is listed twice: refused by the plan of several kernels, whichever kernel is asked first."""
+    """An output that is listed twice, more batches than the contraction kernel takes: refused whichever kernel is asked first."""
     text = _scores(64, 256, 64, 256, "bfloat16", None, ["p32", "p32"])
     b = op_desc.DescBuilder("scores_twice")
     q, kk = b.input([64, 256, 64], "bfloat16"), b.input([64, 256, 64], "bfloat16")
@@ -151,6 +151,9 @@ def test_what_two_kernels_refuse_is_refused(monkeypatch):
         monkeypatch.setenv("AKG_HIP_VARIANT", variant)
         with pytest.raises(driver.AkgHipError):
             driver.HipKernel(b.dumps([p, p]), out_dir=None)
+        assert driver.HipKernel(_scores(65535, 8, 32, 8, "bfloat16", None, ["p"]), out_dir=None).family == ("gemm_rows" if variant == "0" else "staged")
+        with pytest.raises(driver.AkgHipError):
+            driver.HipKernel(_scores(65536, 8, 32, 8, "bfloat16", None, ["p"]), out_dir=None)
 
 
 @pytest.mark.gpu

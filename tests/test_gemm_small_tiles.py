@@ -100,3 +100,20 @@ def test_small_tiles_against_float64(m, k, n, dtype, tb, tile, tmp_path):
 def test_33_to_64_rows_take_the_faster_of_skinny_and_small_tiles(m, k, n, dtype, tb, kernel, tmp_path):
     note = _schedule(_product(m, k, n, dtype, tb, "rows_%s_%d_%d_%d_%d" % (dtype, m, k, n, tb)), tmp_path)
     assert (" skinny" in note) == (kernel == "skinny") and ("tile=64x64" in note) == (kernel == "tile"), note
+
+
+@pytest.mark.parametrize("m,k,n,dtype,tb", [
+    (800, 11008, 1536, "bfloat16", False), (1600, 11008, 768, "bfloat16", True), (1200, 11008, 1024, "float16", True),   # more than 16 MiB
+    (1000, 11008, 1536, "bfloat16", True), (2048, 11008, 768, "bfloat16", False), (3000, 8192, 512, "int8", False),      # at most, for more
+    (1000, 8192, 768, "bfloat16", True), (256, 8192, 4096, "bfloat16", False),
+])
+def test_split_small_tiles_stay_within_the_static_scratch_where_the_large_ones_do(m, k, n, dtype, tb, tmp_path, monkeypatch):
+    """16 MiB is what a launch without allocations has. (The largest workspaces among 5500 products that take small tiles, M 33 ..
+    4096, K 512 .. 11008, N 512 .. 12288, reach 20 MiB; none of those products had less than 16 MiB on the 256 x 256 kernel.)"""
+    text = _product(m, k, n, dtype, tb, "scratch_%s_%d_%d_%d_%d" % (dtype, m, k, n, tb))
+    small = driver.HipKernel(text, out_dir=None)
+    assert "gemm_small_tile<" in small.source
+    monkeypatch.setenv("AKG_HIP_VARIANT", "128")
+    large = driver.HipKernel(text, out_dir=None)
+    assert "gemm_small_tile<" not in large.source
+    assert small.workspace_bytes <= 16 << 20 or large.workspace_bytes > 16 << 20
