@@ -171,7 +171,7 @@ class GemmEmitter {
 
   // Time in us of the small-tile kernel, after what it was measured to take: 3 us in front and behind, and per step of 128
   // bytes of K 0.35 us (64 x 64; 0.28 where the workgroups of a CU cover each other), 0.48 (64 x 128), 0.72 (128 x 128): a CU
-  // takes in 46 GB/s with one workgroup or several, so workgroups beyond one per CU queue up. A split costs its
+  // takes in 46 .. 53 GB/s of operands with one workgroup or several, so workgroups beyond one per CU queue up. A split costs its
   // partials' way to memory and back and the time of the workgroup that adds them.
   double smallTileTime(int64_t bm, int64_t bn, int64_t split) const {
     const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = ((m_ + bm - 1) / bm) * ((n_ + bn - 1) / bn);

@@ -799,12 +799,12 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
   __shared__ __attribute__((aligned(16))) u8 akg_skinny_lds[kLdsBytes];
   if constexpr (kLines) {
     // A wavefront loads the line of eight columns per instruction and turns the 128 columns into operands through LDS of its
-    // own (chunks permuted by the column: every bank once among the lanes served together), the next lines in flight
-    // beside the MFMAs. Loading the operands as they are touches 32 lines by 32 bytes per instruction, and a line is evicted
-    // from the L1 before its fourth piece is read. bf16 (us): 16 x 8192 x 8192 38.8 with the operands as they are, 33.2 by whole
-    // lines, 28.4 with the strips rotated, 26.4 past the caches, 25.1 without a last request that nobody reads; 16 x 4096 x 11008
-    // 32.7 -> 20.3, 64 x 8192 x 8192 46.3 -> 32.0, 16 x 8192 x 1024 11.6 -> 9.6; int8 16 x 8192 x 8192 20.6 -> 16.6. Rotation or adjacent
-    // pieces alone, without whole lines: 37 .. 42.
+    // own (chunks permuted by the column: the writes touch every bank once, the reads half of the banks twice, with the LDS
+    // pipe 16 % busy), the next lines in flight beside the MFMAs. Loading the operands as they are touches 32 lines by 32 bytes
+    // per instruction: the L1 then asks the L2 2.5 times for a line, now once. bf16 (us): 16 x 8192 x 8192 38.8 with the operands
+    // as they are, 33.2 by whole lines, 28.4 with the strips rotated, 26.4 past the caches, 25.1 without a last request that
+    // nobody reads; 16 x 4096 x 11008 32.7 -> 19.3, 64 x 8192 x 8192 46.3 -> 32.0, 16 x 8192 x 1024 11.6 -> 9.6; int8 16 x 8192 x
+    // 8192 20.6 -> 15.5. Rotation or adjacent pieces alone, without whole lines: 37 .. 42.
     constexpr int kSub = kLine / 32;   // MFMA steps per line
     const long lines = (t1 - t0 + kSub - 1) / kSub;
     u8 *__restrict__ tile = akg_skinny_lds + wave * (128 * kLine);

@@ -10,8 +10,8 @@
  * two exchanges between lanes (distances 16 and 32) and one LDS step between the wavefronts of a row.
  * The wavefronts of a row take its units in pairs (row_unit). No LDS holds operands: B is read once per workgroup, straight into MFMA
  * fragments, from the L2 (the launch keeps the workgroups of a batch on one XCD).
- * What bounds it: memory (mask in, probabilities out) and the fragments of B from the L2 about equally: bf16
- * [192,512,64] x 512 with its mask takes 77 us, 4.2 TB/s of what has to move; as a contraction and a row kernel 149 us,
+ * What bounds it: memory (mask in, probabilities out) and the fragments of B, of which the L1s ask the L2s for as many lines
+ * (1.57 million each): bf16 [192,512,64] x 512 with its mask takes 74 us, 4.4 TB/s of what has to move; as a contraction and a row kernel 149 us,
  * the float32 scores written and read in between. Measured and left out: the mask requested in front of the MFMAs (77 us
  * either way, more registers: 2048 columns 201 us for 174), non-temporal loads of it (86 us), non-temporal stores (79 us).
  */
@@ -26,7 +26,7 @@ AKG_DEV constexpr int row_unit(int j, int wc) {
   return NCHUNK % 2 == 0 ? ((j / 2) * WC + wc) * 2 + j % 2 : j * WC + wc;
 }
 
-// A number of 64-byte slabs of K as a type.
+// A number (of 64-byte slabs of K) as a type.
 template <int N>
 struct SlabCount {
   static constexpr int value = N;
@@ -35,7 +35,7 @@ struct SlabCount {
 // s[rt][j] = the eight columns of unit row_unit(j, wc) (columns beyond N hold copies of column N - 1) in row
 // row0 + 16 rt + lane % 16 (rows beyond M hold copies of row M - 1). KB: bytes of K per row, a multiple of 64.
 // Up to seven slabs of 64 bytes the rows of A stay in registers; a longer K is taken in blocks of four with the
-// accumulators live, so the registers do not grow with K (bf16, 512 x 256 with softmax: 180 a lane at K = 512, 332 with all of K
+// accumulators live, so the registers do not grow with K (bf16, 512 x 256 with softmax: 200 a lane at K = 512, 332 with all of K
 // held, where K = 1024 and more spilled; K = 512 50 us either way, and the next block's rows requested beside the MFMAs of a block
 // gave nothing).
 template <typename Mma, long M, long N, long KB, int RT, int NCHUNK, int WC>
@@ -53,12 +53,6 @@ AKG_DEV void row_scores(const void *__restrict__ A, const void *__restrict__ B, 
     const long row = row0 + 16 * rt + c;
     aOff[rt] = static_cast<u32>((row < M ? row : M - 1) * KB) + 16u * static_cast<u32>(g);
   }
-  typename Mma::acc4_v acc[RT][NCHUNK][2];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-    for (int j = 0; j < NCHUNK; ++j) acc[rt][j][0] = acc[rt][j][1] = typename Mma::acc4_v{0, 0, 0, 0};
-  }
   v4i qf[RT][kBlock];
   auto loadRows = [&](auto slabs, u32 at) {
 #pragma unroll
@@ -69,7 +63,7 @@ AKG_DEV void row_scores(const void *__restrict__ A, const void *__restrict__ B, 
   };
   // The fragments of kBatch units are requested together, in front of their MFMAs (left alone, the compiler keeps two
   // loads in flight and the wavefront waits out the L2 once per MFMA).
-  auto multiply = [&](auto slabs, u32 at) {
+  auto multiply = [&](auto slabs, u32 at, auto first) {   // (into s, which the first block starts)
     constexpr int kCount = slabs.value, kBatch = kCount >= 8 ? 1 : 8 / kCount;
 #pragma unroll
     for (int j0 = 0; j0 < NCHUNK; j0 += kBatch) {
@@ -92,31 +86,29 @@ AKG_DEV void row_scores(const void *__restrict__ A, const void *__restrict__ B, 
         for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
+            typename Mma::acc4_v acc = {0, 0, 0, 0};
+            const float *sum = s[rt][j] + 4 * h;
+            if constexpr (first.value == 0) acc = typename Mma::acc4_v{sum[0], sum[1], sum[2], sum[3]};
 #pragma unroll
-            for (int i = 0; i < kCount; ++i) acc[rt][j][h] = Mma::mma16(kf[j - j0][h][i], qf[rt][i], acc[rt][j][h]);
+            for (int i = 0; i < kCount; ++i) acc = Mma::mma16(kf[j - j0][h][i], qf[rt][i], acc);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) s[rt][j][4 * h + v] = acc[v];
           }
         }
       }
     }
   };
   loadRows(SlabCount<kBlock>(), 0);
+  multiply(SlabCount<kBlock>(), 0, SlabCount<1>());
 #pragma unroll 1
-  for (int t = 0; t < kBlocks; ++t) {
+  for (int t = 1; t < kBlocks; ++t) {
     const u32 at = static_cast<u32>(t) * (64 * kBlock);
-    multiply(SlabCount<kBlock>(), at);
-    if (t + 1 < kBlocks) loadRows(SlabCount<kBlock>(), at + 64 * kBlock);
+    loadRows(SlabCount<kBlock>(), at);
+    multiply(SlabCount<kBlock>(), at, SlabCount<0>());
   }
   if constexpr (kRest > 0) {
     loadRows(SlabCount<kRest>(), 64 * kBlock * kBlocks);
-    multiply(SlabCount<kRest>(), 64 * kBlock * kBlocks);
-  }
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-    for (int j = 0; j < NCHUNK; ++j) {
-#pragma unroll
-      for (int v = 0; v < 8; ++v) s[rt][j][v] = acc[rt][j][v >> 2][v & 3];
-    }
+    multiply(SlabCount<kRest>(), 64 * kBlock * kBlocks, SlabCount<0>());
   }
 }
 
