@@ -210,10 +210,12 @@ class GemmEmitter {
   // The small-tile kernel where its estimate is a tenth below that of the 256 x 256 kernel, and for 33 .. 64 rows where the
   // skinny one is not estimated a twentieth faster ([N,K] weights, whose estimates scatter more: a tenth, and those of
   // 16 bits are the skinny kernel's from 60 Mi elements on, where 8192 x 8184 takes 36.3 us for 30.3). Measured (us, the other
-  // kernel -> small tiles): bf16 K x N = 1024 x 1024: M = 64 10.3 -> 6.7, 300 29.4 -> 7.3, 1200 25.9 -> 10.9; 2048 x 4096: 64 16.8 -> 10.0, 300 35.9 -> 17.2, 1200 46.3 -> 42.1; 8192 x 2048:
-  // 128 45.6 -> 19.1, 640 66.7 -> 59.7; 4096 x 11000: 300 94.9 -> 53, 640 139 -> 95; int8 4096 x 4096: 192 40.9 -> 13.2, 640 42.1 ->
-  // 27.3. It is the slower one, and the estimates say so, from M = 1200 on for 8192 x 2048 (85 us for 73) and 4096 x 11000 (171 for
-  // 136), and at 33 rows for [K,N] weights of bf16 8192 x 6144 (30.9 for 26.1), int8 4096 x 6144 (14.8 for 13.4) and 6144 x 9216
+  // kernel -> small tiles): bf16 K x N = 1024 x 1024: M = 64 10.3 -> 6.7, 300 30.4 -> 6.0, 1200 28.4 -> 9.0; 2048 x 4096: 64 16.8 ->
+  // 10.0, 300 33.7 -> 17.6, 1200 45.1 -> 37.5; 8192 x 2048: 128 41.7 -> 17.2, 640 63.2 -> 49.8; 4096 x 11000: 300 88.9 -> 53.7 ([K,N]
+  // 95.2 -> 59.2), 640 129 -> 75.8; int8 4096 x 4096: 192 32.3 -> 13.8, 640 39.7 -> 25.9; 512 x 7768: 1494 21.4 -> 16.9. It is the slower
+  // one, and the estimates say so, from M = 1200 on for 8192 x 2048 (82 us for 67) and 4096 x 11000 (147 for 118); of 376 products that
+  // the estimates give it two are slower than on 256 x 256 tiles (bf16 1600 x 2048 x 5120 55.3 for 51.7).
+  // The skinny one is faster at 33 rows for [K,N] weights of bf16 8192 x 6144 (30.9 for 26.1), int8 4096 x 6144 (14.8 for 13.4) and 6144 x 9216
   // (27.9 for 20.0), for [N,K] of bf16 11008 x 5120 (34.1 for 28.1).
   // Below 2 MiB and from 2^26 elements of B on the kernels and splits of the other two stand. From 65 rows on that is not where the
   // small tiles stop being the faster ones: bf16 512 x 768 with 256 rows takes 21.4 us for their 4.8, 8192 x 8192 with 96
