@@ -126,14 +126,14 @@ class GemmEmitter {
   // with the non-temporal hint the line is not kept for the next piece. (For a longer K the kernel reads whole lines.)
   bool skinnyNonTemporal() const { return opt_.nonTemporal != 0 && !transB_; }
   bool skinnyLines() const { return transB_ && k_ * elemBytes() >= 128 * skinnyWaves(); }   // (kLines of gemm_skinny)
-  // Whole lines of a [N,K] weight are read once, so from 16 MiB on (all batches together) they are read past the caches. Weights
-  // not used for 600 MB of traffic, with the hint and without (us): bf16 16 x 2048 x 2048 (8 MiB) 7.3 and 7.0, 16 x 4096 x 2048 (16 MiB)
-  // 10.2 and 10.5, 16 x 4096 x 4096 11.2 and 11.7, 16 x 8192 x 8192 25.0 and 27.6, 64 x 8192 x 8192 31.8 and 34.4, int8 16 x 4096 x 2048 (8 MiB)
-  // 7.5 and 7.2, 16 x 4096 x 4096 (16 MiB) 9.2 and 9.8, 64 batches of 16 x 512 x 2048 26.2 and 28.4. The same weight in call after call:
-  // 9.1 either way for 4096 x 4096, 23.0 and 22.6 for 8192 x 8192, 16 batches of 16 x 2048 x 2048 28.5 and 22.6. A line that does not end
-  // with the column belongs to two of them and needs its second look.
+  // Whole lines of a [N,K] weight are read once, so from 96 MiB on (all batches together) they are read past the caches. Below, the
+  // last-level cache (256 MiB) may hold the weight beside others, and the hint costs more than it gives where it does not. With the
+  // hint and without, three such weights in turn / not used for 640 MB (us): bf16 2 x 2048 x 8192 (32 MiB) 10.5 and 10.2 / 10.8 and
+  // 11.9, 16 x 3648 x 8704 (61 MiB) 15.8 and 14.3 / 16.3 and 17.5, 16 x 8192 x 4096 (64 MiB) 15.7 and 14.4 / 15.9 and 17.2,
+  // 16 x 8192 x 5120 (80 MiB) 18.7 and 16.9 / 18.8 and 20.1; 16 x 8192 x 8704 (136 MiB) 27.3 and 30.1 / 26.4 and 29.0, int8 16 x 16384 x
+  // 8704 27.7 and 30.4 / 26.6 and 29.4. A line that does not end with the column belongs to two of them and needs its second look.
   bool streamsLines() const {
-    return opt_.nonTemporal != 0 && skinnyLines() && k_ * elemBytes() % 128 == 0 && batch_ * n_ * k_ * elemBytes() >= (16LL << 20);
+    return opt_.nonTemporal != 0 && skinnyLines() && k_ * elemBytes() % 128 == 0 && batch_ * n_ * k_ * elemBytes() >= (96LL << 20);
   }
   bool serial_ = false;  // no MFMA kernel takes the description: gemm_serial (akg_gemm_serial.hpp)
   int epiWidth() const { return (serial_ && n_ % 4 != 0) ? 1 : 4; }   // adjacent result columns per epilogue call

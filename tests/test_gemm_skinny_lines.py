@@ -64,18 +64,18 @@ def test_every_line_of_the_weight_is_requested_once(tmp_path):
     assert code.count("global_load_dwordx4") == 16 + 4
 
 
-def test_lines_are_read_past_the_caches_from_16_mib_of_all_batches_on(monkeypatch):
+def test_lines_are_read_past_the_caches_from_96_mib_of_all_batches_on(monkeypatch):
     def streamed(text):
         kernel = driver.HipKernel(text, out_dir=None)
         assert "gemm_skinny<" in kernel.source
         return "akg::StreamedLines()" in kernel.source
-    assert streamed(op_desc.gemm_bias_act(16, 4096, 2048, "bfloat16", "none", transpose_b=True))
-    assert not streamed(op_desc.gemm_bias_act(16, 4096, 2044, "bfloat16", "none", transpose_b=True))
-    assert not streamed(op_desc.gemm_int8_dequant_bias_gelu(16, 4096, 2048, transpose_b=True))
-    assert not streamed(op_desc.gemm_bias_act(16, 4112, 4096, "bfloat16", "none", transpose_b=True))   # columns end inside a line
-    assert not streamed(op_desc.gemm_bias_act(16, 128, 131072, "bfloat16", "none", transpose_b=True))  # operands as they are
+    assert streamed(op_desc.gemm_bias_act(16, 8192, 6144, "bfloat16", "none", transpose_b=True))
+    assert not streamed(op_desc.gemm_bias_act(16, 8192, 6140, "bfloat16", "none", transpose_b=True))
+    assert not streamed(op_desc.gemm_int8_dequant_bias_gelu(16, 8192, 8192, transpose_b=True))
+    assert not streamed(op_desc.gemm_bias_act(16, 4112, 12288, "bfloat16", "none", transpose_b=True))   # columns end inside a line
+    assert not streamed(op_desc.gemm_bias_act(16, 128, 524288, "bfloat16", "none", transpose_b=True))   # operands as they are
     assert not streamed(op_desc.gemm_bias_act(16, 8192, 8192, "bfloat16", "none", transpose_b=False))
-    assert streamed(op_desc.batch_matmul_scale_mask(32, 16, 512, 512, "bfloat16", True, "lines_batch"))
-    assert not streamed(op_desc.batch_matmul_scale_mask(31, 16, 512, 512, "bfloat16", True, "lines_batch"))
+    assert streamed(op_desc.batch_matmul_scale_mask(192, 16, 512, 512, "bfloat16", True, "lines_batch"))
+    assert not streamed(op_desc.batch_matmul_scale_mask(191, 16, 512, 512, "bfloat16", True, "lines_batch"))
     monkeypatch.setenv("AKG_HIP_NT", "0")
     assert not streamed(op_desc.gemm_bias_act(16, 8192, 8192, "bfloat16", "none", transpose_b=True))
