@@ -123,17 +123,31 @@ class GemmEmitter {
   int skinnyWaves() const { return opt_.block == 512 ? 8 : 4; }
   int skinnyUnroll() const { return opt_.chunks > 0 ? opt_.chunks : 2; }
   // A [N,K] weight with a short K is read in 32-byte pieces, four per cache line, by instructions that follow each other:
-  // with the non-temporal hint the line is not kept for the next piece. (For a longer K the kernel reads whole lines.)
+  // with the non-temporal hint the line is not kept for the next piece. (skinnyLines() reads whole lines.)
   bool skinnyNonTemporal() const { return opt_.nonTemporal != 0 && !transB_; }
-  bool skinnyLines() const { return transB_ && k_ * elemBytes() >= 128 * skinnyWaves(); }   // (kLines of gemm_skinny)
+  // Where columns end inside a line, a piece of 128 bytes lies in two lines, and a short K gives the wavefronts uneven shares: a
+  // weight of less than 4 MiB (all batches together) is then loaded as it is. Operands as they are and whole lines,
+  // three such weights in turn / not used for 640 MB of traffic (us), of 207 sizes from 0.3 to 103 MiB: bf16 2 x 544 x 1024
+  // (1.1 MiB) 5.0 and 5.6 / 5.6 and 5.9, 16 x 1184 x 1024 (2.3 MiB) 5.9 and 6.2 / 6.5 and 6.6, 39 x 3120 x 512 (3 MiB) 9.7 and 10.3 / 10.4
+  // and 10.8, int8 16 x 1632 x 2048 (3.2 MiB) 6.3 and 6.7 / 6.8 and 7.2; above, bf16 16 x 2080 x 1024 (4.1 MiB) 6.4 and 6.5 / 7.4 and 7.1,
+  // int8 16 x 3136 x 2048 (6.1 MiB) 7.1 and 6.8 / 8.5 and 7.9, bf16 16 x 4128 x 4096 12.3 and 11.9 / 14.5 and 12.9.
+  int64_t weightBytes() const { return batch_ * n_ * k_ * elemBytes(); }
+  bool skinnyLines() const {
+    return transB_ && k_ * elemBytes() >= 128 * skinnyWaves() && (k_ * elemBytes() % 128 == 0 || weightBytes() >= (4LL << 20));
+  }
   // Whole lines of a [N,K] weight are read once, so from 96 MiB on (all batches together) they are read past the caches. Below, the
-  // last-level cache (256 MiB) may hold the weight beside others, and the hint costs more than it gives where it does not. With the
+  // last-level cache (256 MiB) may hold the weight beside others: the hint then costs what it gives otherwise. With the
   // hint and without, three such weights in turn / not used for 640 MB (us): bf16 2 x 2048 x 8192 (32 MiB) 10.5 and 10.2 / 10.8 and
   // 11.9, 16 x 3648 x 8704 (61 MiB) 15.8 and 14.3 / 16.3 and 17.5, 16 x 8192 x 4096 (64 MiB) 15.7 and 14.4 / 15.9 and 17.2,
   // 16 x 8192 x 5120 (80 MiB) 18.7 and 16.9 / 18.8 and 20.1; 16 x 8192 x 8704 (136 MiB) 27.3 and 30.1 / 26.4 and 29.0, int8 16 x 16384 x
   // 8704 27.7 and 30.4 / 26.6 and 29.4. A line that does not end with the column belongs to two of them and needs its second look.
   bool streamsLines() const {
-    return opt_.nonTemporal != 0 && skinnyLines() && k_ * elemBytes() % 128 == 0 && batch_ * n_ * k_ * elemBytes() >= (96LL << 20);
+    return opt_.nonTemporal != 0 && skinnyLines() && k_ * elemBytes() % 128 == 0 && weightBytes() >= (96LL << 20);
+  }
+  // ... as the kernel's last argument, behind the other ones that have defaults
+  std::string linesArgument(const std::string &before) const {
+    if (!transB_) return "";
+    return streamsLines() ? before + ", akg::StreamedLines()" : (skinnyLines() ? "" : before + ", akg::NoLines()");
   }
   bool serial_ = false;  // no MFMA kernel takes the description: gemm_serial (akg_gemm_serial.hpp)
   int epiWidth() const { return (serial_ && n_ % 4 != 0) ? 1 : 4; }   // adjacent result columns per epilogue call
@@ -617,13 +631,13 @@ class GemmEmitter {
       if (dyn_) {
         src_ << "  akg::gemm_skinny<" << mmaTraits() << ", " << skinnyBucket() << "L, " << n_ << "L, " << k_ << "L, " << (transB_ ? "true" : "false")
              << ", Epilogue, 1, " << skinnyWaves() << ", " << skinnyUnroll() << ", " << (skinnyNonTemporal() ? "true" : "false") << ", true>(in"
-             << g_.tensor(aId_).inputIndex << ", in" << g_.tensor(bId_).inputIndex << ", epi, akg_ws, 0L, akg_m, static_cast<int>(akg_ksplit)" << (streamsLines() ? ", akg::StreamedLines()" : "") << ");\n}\n";
+             << g_.tensor(aId_).inputIndex << ", in" << g_.tensor(bId_).inputIndex << ", epi, akg_ws, 0L, akg_m, static_cast<int>(akg_ksplit)" << linesArgument("") << ");\n}\n";
         return;
       }
       src_ << "  akg::gemm_skinny<" << mmaTraits() << ", " << m_ << "L, " << n_ << "L, " << k_ << "L, " << (transB_ ? "true" : "false")
            << ", Epilogue, " << kSplit_ << ", " << skinnyWaves() << ", " << skinnyUnroll() << ", " << (skinnyNonTemporal() ? "true" : "false") << ">(in" << g_.tensor(aId_).inputIndex << " + akg_batch * " << m_ * k_ << "L, in"
            << g_.tensor(bId_).inputIndex << " + akg_batch * " << k_ * n_ << "L, epi, " << (kSplit_ > 1 ? "akg_ws" : "nullptr")
-           << ", akg_batch * " << (n_ + 127) / 128 << "L" << (streamsLines() ? ", 0L, 1, akg::StreamedLines()" : "") << ");\n}\n";
+           << ", akg_batch * " << (n_ + 127) / 128 << "L" << linesArgument(", 0L, 1") << ");\n}\n";
       return;
     }
     if (tileM_ > 0) {

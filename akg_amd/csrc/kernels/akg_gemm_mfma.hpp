@@ -668,12 +668,15 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
 // DYN: MS is the most rows the code object takes (16, 32 or 64), the actual row count and the number of K splits are
 // kernel arguments (`mDyn` <= MS, `ksDyn`); `ws` is always a valid pointer.
 // UNROLL and NT are those of the operands loaded as they are; whole lines of a [N,K] weight are one in flight, past the
-// caches with StreamedLines.
+// caches with StreamedLines. With NoLines the operands are loaded as they are whatever the length of K.
 struct CachedLines {
-  static constexpr bool kPastCaches = false;
+  static constexpr bool kWhole = true, kPastCaches = false;
 };
 struct StreamedLines {
-  static constexpr bool kPastCaches = true;
+  static constexpr bool kWhole = true, kPastCaches = true;
+};
+struct NoLines {
+  static constexpr bool kWhole = false, kPastCaches = false;
 };
 template <typename Mma, long MS, long N, long KE, bool TRANSB, typename Epilogue, int KSPLIT, int WAVES = 4, int UNROLL = 2, bool NT = false, bool DYN = false, typename Lines = CachedLines>
 AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ Bv, Epilogue &epi,
@@ -700,7 +703,7 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
   const int ksplit = kSplitPossible ? static_cast<int>(static_cast<long>(blockIdx.x) / kStrips) : 0;
   constexpr int kLine = 128;   // bytes of K that a wavefront takes at a time from every column of a [N,K] weight
   // Below 512 bytes of K not every wavefront would get a line: the fragments are then loaded as they are.
-  constexpr bool kLines = TRANSB && K >= kWaves * kLine;
+  constexpr bool kLines = TRANSB && Lines::kWhole && K >= kWaves * kLine;
   static_assert(!Lines::kPastCaches || K % kLine == 0, "a line at the end of a column is read for two columns");
   constexpr long kUnit = kLines ? kLine / 32 : 1, kUnits = (kSteps + kUnit - 1) / kUnit;   // a range of K ends on a whole line
   const long t0 = kUnits * ksplit / kSplits * kUnit, tEnd = kUnits * (ksplit + 1) / kSplits * kUnit;

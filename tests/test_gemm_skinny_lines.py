@@ -16,6 +16,9 @@ from akg_amd import driver, op_desc
     (7, 11008, 1040, "bfloat16"),   # more strips than a range has lines: the rotation wraps
     (16, 8192, 6400, "bfloat16"),   # read past the caches
     (32, 8256, 272, "int8"), (5, 544, 140, "int8"),
+    # columns that end inside a line: whole lines from 4 MiB of weight on, tails of a quarter, a half and three quarters
+    (3, 272, 7720, "float16"), (5, 8256, 520, "int8"), (40, 2096, 1012, "bfloat16"),
+    (39, 528, 516, "bfloat16"), (64, 1088, 904, "int8"),   # ... and below: as they are, two row tiles, ragged strips
 ])
 def test_lines_of_a_transposed_weight_against_float64(m, k, n, dtype):
     """float32 sums of k products differ from the exact sum by at most k * 2^-24 of the sum of the products' magnitudes, in
@@ -79,3 +82,18 @@ def test_lines_are_read_past_the_caches_from_96_mib_of_all_batches_on(monkeypatc
     assert not streamed(op_desc.batch_matmul_scale_mask(191, 16, 512, 512, "bfloat16", True, "lines_batch"))
     monkeypatch.setenv("AKG_HIP_NT", "0")
     assert not streamed(op_desc.gemm_bias_act(16, 8192, 8192, "bfloat16", "none", transpose_b=True))
+
+
+def test_lines_of_columns_that_end_inside_one_are_whole_from_4_mib_of_all_batches_on():
+    def whole(text):
+        kernel = driver.HipKernel(text, out_dir=None)
+        assert "gemm_skinny<" in kernel.source
+        return "akg::NoLines()" not in kernel.source
+    assert whole(op_desc.gemm_bias_act(16, 1040, 2020, "bfloat16", "none", transpose_b=True))
+    assert not whole(op_desc.gemm_bias_act(16, 1040, 2016, "bfloat16", "none", transpose_b=True))
+    assert whole(op_desc.gemm_int8_dequant_bias_gelu(2, 1056, 3972, transpose_b=True))
+    assert not whole(op_desc.gemm_int8_dequant_bias_gelu(2, 1056, 3968, transpose_b=True))
+    assert whole(op_desc.gemm_bias_act(16, 256, 128, "bfloat16", "none", transpose_b=True))       # columns of whole lines
+    assert not whole(op_desc.gemm_bias_act(16, 240, 16384, "bfloat16", "none", transpose_b=True))  # not a line per wavefront
+    assert whole(op_desc.batch_matmul_scale_mask(8, 16, 528, 512, "bfloat16", True, "lines_seam"))
+    assert not whole(op_desc.batch_matmul_scale_mask(7, 16, 528, 512, "bfloat16", True, "lines_seam"))
