@@ -284,9 +284,10 @@ class GemmEmitter {
     if (pickSmallTile()) return;
     kSplit_ = 1;
     // At most 64 rows of A (and K a multiple of 32 bytes): the time is that of streaming B, which gemm_skinny reads
-    // straight into MFMA operands; 256 workgroups of four wavefronts (one per CU: 16 x 8192 x 8192 bf16 reaches 66 % of
-    // the HBM peak with 4 splits of 64 strips, 59 % with 8, 48 % with 2; 8 wavefronts or more steps in flight change
-    // nothing), each wavefront with at least 4 MFMA steps.
+    // straight into MFMA operands, or a [N,K] one by whole lines through LDS of each wavefront (skinnyLines()); 256
+    // workgroups of four wavefronts (one per CU: 16 x 8192 x 8192 bf16 with a [K,N] weight reaches 66 % of the HBM peak
+    // with 4 splits of 64 strips, 59 % with 8, 48 % with 2; 8 wavefronts or more steps in flight change nothing), each
+    // wavefront with at least 4 MFMA steps.
     // AKG_HIP_VARIANT bit 3 keeps the 256 x 256 tile kernel.
     skinny_ = skinnyTakes();
     if (skinny_) {
