@@ -16,6 +16,7 @@ const char *kernelFamilyName(KernelFamily f) {
     case KernelFamily::GemmEpilogue: return "gemm_epilogue";
     case KernelFamily::StreamReduce: return "stream_reduce";
     case KernelFamily::ColumnReduce: return "column_reduce";
+    case KernelFamily::PlaneReduce: return "plane_reduce";
     case KernelFamily::Indexed: return "indexed";
     case KernelFamily::SegmentSum: return "segment_sum";
     case KernelFamily::GemmRows: return "gemm_rows";
@@ -629,6 +630,11 @@ LoweredKernel lowerToHip(const OpGraph &described, const LoweringOptions &option
       if (options.variant == 7) throw;
       try {
         return lowerColumnToHip(graph, options);
+      } catch (const LoweringError &) {
+        // reduced on both sides of the kept axes?
+      }
+      try {
+        return lowerPlaneToHip(graph, options);
       } catch (const LoweringError &) {
         throw streaming;
       }

@@ -31,7 +31,7 @@ class LoweringError : public std::runtime_error {
   explicit LoweringError(const std::string &msg) : std::runtime_error(msg) {}
 };
 
-enum class KernelFamily { Elementwise, RowReduce, GemmEpilogue, StreamReduce, Indexed, SegmentSum, Staged, ColumnReduce, GemmRows };
+enum class KernelFamily { Elementwise, RowReduce, GemmEpilogue, StreamReduce, Indexed, SegmentSum, Staged, ColumnReduce, GemmRows, PlaneReduce };
 const char *kernelFamilyName(KernelFamily f);
 
 // Tuning knobs; 0 means "let the heuristic decide". They can be set through the environment
@@ -41,14 +41,14 @@ struct LoweringOptions {
   int threadsPerRow = 0;
   int chunks = 0;       // chunks per thread (skinny contractions: steps in flight; whole lines of a [N,K] weight are always one)
   int block = 0;        // threads per workgroup
-  int split = 0;        // streaming reductions: workgroups sharing one group of outputs (AKG_HIP_SPLIT)
+  int split = 0;        // streaming reductions: workgroups sharing one group of outputs (AKG_HIP_SPLIT); plane kernel: per channel
   // Experiment switch (AKG_HIP_VARIANT), read by whichever family lowers the kernel; 0 = the measured default.
   //   gemm_epilogue  bit 3: no skinny kernel for M <= 64 (the tile kernel with K split instead),
   //                  bit 5: the other arrangement of the tile kernel's wavefronts (2 x 4 for 4 x 2 and back)
   //                  bit 7: no small tiles (64 and 128 rows and columns) either,
   //                  bit 4: a contraction and the row reductions behind it as two kernels (no gemm_rows)
   //   row_reduce     1: keep the row in registers, 2: walk the row (no packing), 4: walk it, packed if possible
-  //   stream_reduce  7: no column kernel (several kernels instead)
+  //   stream_reduce  7: no column or plane kernel (several kernels instead)
   //   column_reduce  5: one strip per workgroup (no second set of resident registers)
   //   segment_sum    1: every workgroup scans all ids, 2: positions grouped by segment first (whatever the size),
   //                  3: grouped by bucket of segments first (whatever the number of buckets)
@@ -108,6 +108,8 @@ LoweredKernel lowerGemmRowsToHip(const OpGraph &graph);
 LoweredKernel lowerStreamReduceToHip(const OpGraph &graph, const LoweringOptions &options);
 // One reduced axis that is not the innermost one, reduction results used against the unreduced tensor (HipLoweringColumn.cpp).
 LoweredKernel lowerColumnToHip(const OpGraph &graph, const LoweringOptions &options);
+// Reduced axes on both sides of the kept ones, reduction results used against the unreduced tensor (HipLoweringPlane.cpp).
+LoweredKernel lowerPlaneToHip(const OpGraph &graph, const LoweringOptions &options);
 LoweredKernel lowerTileToHip(const OpGraph &graph, const LoweringOptions &options);      // elementwise, row_reduce
 LoweredKernel lowerIndexedToHip(const OpGraph &graph, const LoweringOptions &options);
 LoweredKernel lowerSegmentSumToHip(const OpGraph &graph, const LoweringOptions &options);

@@ -1,0 +1,122 @@
+"""Reductions on both sides of the kept axes whose results meet the tensor again (family plane_reduce): which descriptions
+take it, and its results against the oracle's evaluation in float64."""
+import json
+
+import numpy as np
+import pytest
+
+from akg_amd import driver, harness, op_desc
+
+
+def _bn(n, c, h, w, dtype):
+    return op_desc.batchnorm_train_forward(n, c, h, w, dtype)
+
+
+def _backward(n, c, h, w):
+    """Batch-norm backward: two full-sized inputs, statistics per channel, two sums, three outputs (one without the reduced axes)."""
+    b = op_desc.DescBuilder("bn_backward_%dx%dx%dx%d" % (n, c, h, w))
+    x, dy = b.input([n, c, h, w], "bfloat16"), b.input([n, c, h, w], "float32")
+    gamma, mean = b.input([1, c, 1, 1], "float32"), b.input([1, c, 1, 1], "float32")
+    xc = b.sub(b.cast(x, "float32"), mean)
+    dgamma = b.reduce("ReduceSum", b.mul(dy, xc), [0, 2, 3], True)
+    dbeta = b.reduce("ReduceSum", dy, [0, 2, 3], False)
+    inv = b.const(1.0 / (n * h * w), "float32")
+    part = b.mul(b.add(b.reshape(dbeta, [1, c, 1, 1]), b.mul(xc, dgamma)), inv)
+    return b.dumps([b.mul(b.sub(dy, part), gamma), dgamma, dbeta])
+
+
+def _range(shape, axes, dtype):
+    """(x - min) beside max - min: extrema, two reductions of one level, no rounding at all."""
+    b = op_desc.DescBuilder("range_%s_%s" % (dtype, "x".join(map(str, shape))))
+    x = b.input(shape, dtype)
+    low, high = b.reduce("ReduceMin", x, axes, True), b.reduce("ReduceMax", x, axes, True)
+    return b.dumps([b.sub(x, low), b.sub(high, low)])
+
+
+def _statistics(n, c, h, w):
+    """Mean and variance alone: the last launch of the form with several workgroups per channel has values per channel only."""
+    b = op_desc.DescBuilder("bn_mean_var_%dx%dx%dx%d" % (n, c, h, w))
+    x = b.input([n, c, h, w], "float32")
+    inv = b.const(1.0 / (n * h * w), "float32")
+    mean = b.mul(b.reduce("ReduceSum", x, [0, 2, 3], True), inv)
+    xc = b.sub(x, mean)
+    return b.dumps([mean, b.mul(b.reduce("ReduceSum", b.mul(xc, xc), [0, 2, 3], True), inv)])
+
+
+def test_descriptions_that_take_the_plane_kernel_and_those_that_do_not():
+    def family(text):
+        return driver.HipKernel(text, out_dir=None).family
+    assert family(_bn(4, 16, 8, 8, "bfloat16")) == family(_range([8, 40, 5, 7], [0, 2, 3], "int32")) == "plane_reduce"
+    assert family(_bn(4, 15, 8, 8, "bfloat16")) == "staged"       # few channels
+    assert family(_bn(2, 16, 8, 8, "bfloat16")) == "staged"       # channels of less than half a wavefront
+    b = op_desc.DescBuilder("kept_on_both_sides")
+    x = b.input([8, 32, 40, 24], "float32")
+    assert family(b.dumps([b.sub(x, b.reduce("ReduceMax", x, [0, 2], True))])) == "staged"
+    b = op_desc.DescBuilder("sums_that_round")
+    x = b.input([8, 32, 40, 24], "float16")
+    assert family(b.dumps([b.sub(x, b.reduce("ReduceSum", x, [0, 2, 3], True))])) == "staged"
+    b = op_desc.DescBuilder("dropped_axes_meet_the_last_one")
+    x = b.input([8, 32, 40, 32], "float32")
+    assert family(b.dumps([b.sub(x, b.reduce("ReduceMax", x, [0, 2, 3], False))])) == "staged"
+    b = op_desc.DescBuilder("weight_per_column")
+    x, w = b.input([8, 32, 40, 24], "float32"), b.input([24], "float32")
+    y = b.mul(x, w)
+    assert family(b.dumps([b.sub(y, b.reduce("ReduceMax", y, [0, 2, 3], True))])) == "staged"
+
+
+CASES = [
+    (_bn(64, 16, 7, 7, "bfloat16"), "1"),            # a chunk shared by two slots of a run of 49
+    (_bn(33, 17, 28, 28, "bfloat16"), "1"),          # whole chunks, the last ones of a thread beyond the channel
+    (_bn(40, 16, 3, 1, "float32"), "1"),             # runs of three elements: narrow chunks
+    (_bn(127, 16, 31, 33, "float16"), "1"),          # nearly the registers of a workgroup
+    (_bn(6, 300, 9, 9, "float16"), "1"),             # many channels of one short workgroup
+    (_bn(64, 16, 7, 7, "bfloat16"), "3"),            # several workgroups per channel
+    (_bn(9, 19, 33, 35, "float32"), "11"),
+    (_bn(5, 16, 200, 210, "float32"), "0"),          # beyond a workgroup's registers
+    (_bn(3, 16, 100, 100, "bfloat16"), "60/64"),     # sixty short workgroups per channel
+    (_bn(2, 16, 120, 150, "float32"), "150/64"),     # more workgroups per channel than threads in one
+    (_backward(12, 20, 14, 14), "1"), (_backward(12, 20, 14, 14), "4"),
+    (_range([8, 40, 5, 7], [0, 2, 3], "int32"), "1"), (_range([3, 4, 2, 9, 1, 70], [0, 1, 4, 5], "float16"), "2"),
+    (_statistics(8, 24, 30, 30), "1"), (_statistics(8, 24, 30, 30), "5"),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("index", range(len(CASES)))
+def test_results_against_the_oracle(index, monkeypatch):
+    """Sums against float64 with the bound of a reassociated float32 sum of their terms; extrema and their differences bit
+    for bit. Three launches of one handle give the same bits."""
+    import torch
+    from oracle import np_ref
+    text, schedule = CASES[index]
+    split, _, block = schedule.partition("/")
+    if split != "0":
+        monkeypatch.setenv("AKG_HIP_SPLIT", split)
+    if block:
+        monkeypatch.setenv("AKG_HIP_BLOCK", block)
+    desc = json.loads(text)
+    kernel = driver.HipKernel(text, out_dir=None)
+    print("case %s split %s: grid %d block %d" % (desc["op"], schedule, kernel.grid[0], kernel.block[0]), flush=True)
+    assert kernel.family == "plane_reduce" and (kernel.workspace_bytes > 0) == (split != "1")
+    inputs = harness.make_inputs(desc, seed=harness.BASE_SEED + 811 + index)
+    wide = [a.astype(np.float64) if a.dtype == np.float32 else a for a in inputs]
+    exact = np_ref.evaluate(harness.widen_to_float64(desc), wide)
+    sums = any(o["name"] == "ReduceSum" for o in desc["op_desc"])
+    terms = int(np.prod(desc["input_desc"][0][0]["shape"]))
+    on_device = [torch.from_numpy(np.ascontiguousarray(a).view(np.int16) if a.dtype == np.uint16 else np.ascontiguousarray(a)).cuda() for a in inputs]
+    first = None
+    for _ in range(3):
+        outs = [torch.full(d.shape, 77, dtype={"bfloat16": torch.int16, "float16": torch.float16, "float32": torch.float32, "int32": torch.int32}[d.dtype],
+                           device="cuda") for d in kernel.outputs]
+        kernel.launch(on_device + outs)
+        torch.cuda.synchronize()
+        got = [o.cpu().numpy() for o in outs]
+        first = first or got
+        for d, g, f, x in zip(kernel.outputs, got, first, exact):
+            assert np.array_equal(g.view(np.uint8), f.view(np.uint8)), d.name
+            g = g.view(np.uint16) if d.dtype == "bfloat16" else g
+            if d.dtype == "float32" and sums:
+                ok, msg = harness.compare_reassociated(g, x, d.dtype, terms)
+            else:
+                ok, msg = harness.compare(g, x, d.dtype)
+            assert ok, "%s output %s: %s" % (desc["op"], d.name, msg)
