@@ -16,7 +16,7 @@
  * first), the data once overall.
  *
  * That scan costs (workgroups x positions) id reads. Inputs with many positions are grouped by segment first instead
- * (lowerSegmentSorted below): same result, bit for bit.
+ * (lowerSegmentSorted, lowerSegmentBucketed and lowerSegmentChunked below): same result, bit for bit.
  */
 #include <algorithm>
 #include <sstream>
@@ -704,6 +704,385 @@ LoweredKernel lowerSegmentBucketed(const OpGraph &g, const LoweringOptions &, co
   return k;
 }
 
+// Device code of the chunked schedule: the rank of every item of a chunk among the items of its key.
+const char *const kChunkRank = R"AKG(
+// Stable counting sort of a chunk of NW x TILES x 64 items by key, as chunk_sort above, for many keys: the lanes of a tile
+// with the same key find each other through a mask of lanes per key and wavefront in LDS (or the own bit in, read the
+// mask, put it back to zero: three LDS accesses of the wavefront, which complete in program order) instead of one ballot
+// per key bit - 40 vector instructions of a tile's 120 and, beside the loads of the next chunk, most of what the
+// launch's time was. An or gives the same mask in any order. The key is the low half of key[u]. On return start[k] is where key k's run starts, start[KEYS]
+// the number of items that take part. masks: NW * KEYS, zero on return; cnt: NW * KEYS; start: KEYS + 1; scan: NW words.
+template <int NW, int KEYS, int TILES>
+__device__ inline void chunk_rank(const int (&key)[TILES], unsigned (&slot)[TILES], unsigned long long *masks, unsigned short *cnt,
+                                  unsigned short *start, unsigned *scan) {
+  constexpr int THREADS = NW * 64, PER = (KEYS + THREADS - 1) / THREADS;
+  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, w = tid >> 6;
+  for (int k = tid; k < NW * KEYS; k += THREADS) {
+    masks[k] = 0ull;
+    cnt[k] = 0;
+  }
+  __syncthreads();
+  const unsigned long long bit = 1ull << lane;
+  unsigned long long *lanes = masks + w * KEYS;
+  unsigned short *mine = cnt + w * KEYS;
+#pragma unroll
+  for (int u = 0; u < TILES; ++u) {
+    slot[u] = 0u;
+    if (key[u] >= 0) {
+      const int k = key[u] & 0xffff;
+      __hip_atomic_fetch_or(lanes + k, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __builtin_amdgcn_wave_barrier();
+      const unsigned long long same = __hip_atomic_load(lanes + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const unsigned before = mine[k];
+      __builtin_amdgcn_wave_barrier();
+      __hip_atomic_store(lanes + k, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const unsigned at = before + static_cast<unsigned>(__popcll(same & (bit - 1ull)));
+      slot[u] = at;
+      if ((same >> lane) >> 1 == 0ull) mine[k] = static_cast<unsigned short>(at + 1u);   // the group's highest lane
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  unsigned total[PER], sum = 0u;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int k = tid * PER + j;
+    unsigned before = 0u;
+    if (k < KEYS) {
+#pragma unroll
+      for (int h = 0; h < NW; ++h) {
+        const unsigned c = cnt[h * KEYS + k];
+        cnt[h * KEYS + k] = static_cast<unsigned short>(before);
+        before += c;
+      }
+    }
+    total[j] = before;
+    sum += before;
+  }
+  unsigned incl = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const unsigned o = __shfl_up(incl, d);
+    if (lane >= d) incl += o;
+  }
+  if (lane == 63) scan[w] = incl;
+  __syncthreads();
+  unsigned at = incl - sum;
+#pragma unroll
+  for (int j = 0; j < NW; ++j) at += j < w ? scan[j] : 0u;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int k = tid * PER + j;
+    if (k < KEYS) {
+      start[k] = static_cast<unsigned short>(at);
+#pragma unroll
+      for (int h = 0; h < NW; ++h) cnt[h * KEYS + k] += static_cast<unsigned short>(at);
+    }
+    at += total[j];
+  }
+  if (tid == THREADS - 1) start[KEYS] = static_cast<unsigned short>(at);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < TILES; ++u) {
+    if (key[u] >= 0) slot[u] += mine[key[u] & 0xffff];
+  }
+}
+)AKG";
+
+// The chunked schedule's sizes: buckets of perBucket segments, chunks of 512 * tiles positions.
+struct ChunkedPlan {
+  bool possible = false;
+  int tiles = 8;
+  int64_t perBucket = 1, buckets = 0, chunk = 0, chunks = 0, pitch = 0, rowWords = 0;
+  int64_t wSegs = 0, wTable = 0, words = 0;   // workspace, in 4-byte words: rows, then segments within the bucket, then starts
+};
+
+ChunkedPlan planChunked(const SegmentShapes &sh, const LoweringOptions &options) {
+  ChunkedPlan p;
+  const int64_t rowBytes = sh.slice * static_cast<int64_t>(dtypeSize(sh.out->dtype));
+  const bool wide = sh.out->dtype == DType::I64 || sh.out->dtype == DType::F64;
+  if (wide || rowBytes % 4 != 0 || rowBytes > 16 || sh.slice > 4) return p;
+  p.rowWords = rowBytes / 4;
+  // two workgroups per CU in the last launch, which has one per bucket, where there are that many segments
+  const int64_t most = options.split > 0 ? std::min(options.split, 768) : 2LL * options.computeUnits;
+  p.perBucket = (sh.segments + most - 1) / most;
+  if (p.perBucket > 64) return p;
+  p.buckets = (sh.segments + p.perBucket - 1) / p.perBucket;
+  p.tiles = options.chunks == 1 || options.chunks == 2 || options.chunks == 4 || options.chunks == 8 ? options.chunks : 8;
+  // Chunks: small ones while there are few, for workgroups; larger ones then, for longer runs. us with chunks of 512 / 1024 /
+  // 2048 / 4096 positions: 35304 x 1 into 1131 8.4 / 9.0 / 10.3 / 11.4, 86700 x 3 into 8856 11.0 / 10.0 / 12.0 / 13.6, 138073 x 1
+  // into 998 14.1 / 12.3 / 11.6 / 12.6, 300000 x 3 into 5000 22.7 / 18.6 / 14.4 / 16.0, 1536784 x 4 into 12654 91 / 56 / 42 / 34.
+  if (options.chunks == 0) p.tiles = sh.positions < (1 << 16) ? 1 : sh.positions < (1 << 17) ? 2 : sh.positions < (1 << 19) ? 4 : 8;
+  p.chunk = 512LL * p.tiles;
+  p.chunks = (sh.positions + p.chunk - 1) / p.chunk;
+  if (p.chunks * p.chunk >= (1LL << 31)) return p;
+  p.pitch = (p.buckets + 1 + 7) / 8 * 8;
+  p.wSegs = p.chunks * p.chunk * p.rowWords;
+  p.wTable = p.wSegs + p.chunks * p.chunk / 4;
+  p.words = p.wTable + p.chunks * p.pitch / 2;
+  p.possible = true;
+  return p;
+}
+
+/**
+ * Short rows (4, 8, 12 or 16 bytes): chunks of positions sorted by bucket of segments where they lie. Two launches:
+ *
+ *   <op>_place    a workgroup takes chunks in turn, the loads of the next one in flight while it sorts this one by bucket
+ *                 in LDS (chunk_rank above) and writes it out in one piece: the rows, one byte each for the segment within
+ *                 the bucket, and a table of where every bucket's run starts. No counts are needed in front of it.
+ *   <op>_kernel   a workgroup per bucket walks the runs of its bucket, chunk by chunk, as many per round as fit: the
+ *                 runs' lengths are summed up, every entry is fetched from its run (neighbouring buckets run on one XCD
+ *                 and share the lines in which a run ends and the next one begins), sorted by segment (chunk_sort) into
+ *                 LDS lists, and one lane per output element adds its list.
+ *
+ * Both sorts are stable and chunks are taken in order, so every output element is the serial loop's chain of additions
+ * over its positions, bit for bit.
+ */
+LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &options, const SegmentShapes &sh, const ChunkedPlan &plan) {
+  using lowering::computeTypeName;
+  using lowering::dtypeTag;
+  const TensorValue &data = *sh.data, &ids = *sh.ids, &out = *sh.out;
+  const std::string ct = computeTypeName(out.dtype), tag = dtypeTag(out.dtype), idTag = dtypeTag(ids.dtype);
+  const bool narrow = out.dtype == DType::F16 || out.dtype == DType::BF16 || out.dtype == DType::I8 || out.dtype == DType::I16;
+  const std::string rndOpen = narrow ? tag + "::rnd(" : std::string("(");
+  // rounds of the last launch: 4096 entries on eight wavefronts; few entries per bucket: one chunk's worth on two or four
+  const bool small = sh.positions / plan.buckets < 1024 && plan.tiles <= 4;
+  const int nw = small ? (plan.tiles <= 2 ? 2 : 4) : 8, tiles = small ? static_cast<int>(plan.chunk) / (nw * 64) : 8;
+  // (at least sixteen chains a wavefront: an addition is an instruction of the whole wavefront however few lanes add)
+  const int64_t perBucket = plan.perBucket, chains = perBucket * sh.slice, chainsPerWave = std::max<int64_t>(16, (chains + nw - 1) / nw);
+  int keyBits = 1;
+  while ((1LL << keyBits) < perBucket) ++keyBits;
+  std::ostringstream s;
+  s << "// Generated by the akg HIP lowering for gfx950. Op description: " << g.name << "\n";
+  s << "// family: segment_sum (positions grouped by bucket of segments, chunk by chunk), fusion class: "
+    << operatorTemplateName(g.operatorTemplate) << "\n";
+  s << "#include \"akg_rt.hpp\"\n\n";
+  s << "namespace {\n";
+  s << "constexpr int POSITIONS = " << sh.positions << ", SEGMENTS = " << sh.segments << ", S = " << perBucket << ", KEYS = " << plan.buckets
+    << ", CHUNKS = " << plan.chunks << ", PITCH = " << plan.pitch << ";\n";
+  s << "constexpr int ROW = " << sh.slice << ", ROW_WORDS = " << plan.rowWords << ", NW = 8, TILES = " << plan.tiles << ", CHUNK = NW * TILES * 64;\n";
+  s << "constexpr long W_SEGS = " << plan.wSegs << ", W_TABLE = " << plan.wTable << ";\n";
+  if (ids.dtype == DType::I64) {
+    s << "__device__ inline int as_segment(long v) { return v < 0 || v >= SEGMENTS ? -1 : static_cast<int>(v); }\n";
+  } else {
+    s << "__device__ inline int as_segment(int v) { return v < 0 || v >= SEGMENTS ? -1 : v; }\n";
+  }
+  s << "struct __attribute__((aligned(4))) row_t { unsigned w[ROW_WORDS]; };\n";
+  s << "typedef unsigned quad_words __attribute__((ext_vector_type(4)));\n";
+  s << kChunkSort << kChunkRank;
+  s << "}  // namespace\n\n";
+  std::ostringstream params;
+  for (size_t i = 0; i < g.inputs.size(); ++i) {
+    params << (i ? ", " : "") << "const " << dtypeTag(g.tensor(g.inputs[i]).dtype) << "::storage *__restrict__ in" << i;
+  }
+  params << ", " << tag << "::storage *__restrict__ out0, unsigned *__restrict__ akg_ws";
+  const std::string idsName = "in" + std::to_string(ids.inputIndex), dataName = "in" + std::to_string(data.inputIndex);
+
+  // ---- place ----
+  const int64_t placeGrid = std::min<int64_t>(plan.chunks, 2LL * options.computeUnits);
+  s << "extern \"C\" __global__ __launch_bounds__(512, 4) void " << g.name << "_place(" << params.str() << ") {\n";
+  s << "  // the lane masks of the ranking, then (a barrier later) the sorted rows and their segments\n";
+  s << "  constexpr int MASK_BYTES = NW * KEYS * 8, STAGE_BYTES = CHUNK * (ROW_WORDS * 4 + 1);\n";
+  s << "  __shared__ __attribute__((aligned(16))) unsigned char akg_stage[MASK_BYTES > STAGE_BYTES ? MASK_BYTES : STAGE_BYTES];\n";
+  s << "  __shared__ unsigned short akg_cnt[NW * KEYS];\n";
+  s << "  __shared__ __attribute__((aligned(16))) unsigned short akg_start[PITCH];\n";
+  s << "  __shared__ unsigned akg_scan[NW];\n";
+  s << "  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, w = tid >> 6;\n";
+  s << "  const row_t *__restrict__ rows = reinterpret_cast<const row_t *>(" << dataName << ");\n";
+  s << "  int next_id[TILES];\n  unsigned next_row[TILES][ROW_WORDS];\n";
+  s << "  const auto fetch = [&](int chunk) {   // (positions behind the last one read the last one's row and take no part)\n";
+  s << "#pragma unroll\n";
+  s << "    for (int u = 0; u < TILES; ++u) {\n";
+  s << "      const int p = chunk * CHUNK + (w * TILES + u) * 64 + lane, at = p < POSITIONS ? p : POSITIONS - 1;\n";
+  s << "      const int id = as_segment(" << idTag << "::load(" << idsName << "[at]));\n";
+  s << "      next_id[u] = p < POSITIONS ? id : -1;\n";
+  s << "      const row_t r = rows[at];\n";
+  s << "#pragma unroll\n";
+  s << "      for (int c = 0; c < ROW_WORDS; ++c) next_row[u][c] = r.w[c];\n";
+  s << "    }\n  };\n";
+  s << "  fetch(static_cast<int>(blockIdx.x));\n";
+  s << "  for (int chunk = static_cast<int>(blockIdx.x); chunk < CHUNKS; chunk += static_cast<int>(gridDim.x)) {\n";
+  s << "    int key[TILES];\n    unsigned row[TILES][ROW_WORDS], slot[TILES];\n";
+  s << "#pragma unroll\n";
+  s << "    for (int u = 0; u < TILES; ++u) {\n";
+  s << "      const unsigned bucket = static_cast<unsigned>(next_id[u]) / S;\n";
+  s << "      // the bucket, and the segment within it in the upper half\n";
+  s << "      key[u] = next_id[u] >= 0 ? static_cast<int>(bucket | (static_cast<unsigned>(next_id[u]) - bucket * S) << 16) : -1;\n";
+  s << "#pragma unroll\n";
+  s << "      for (int c = 0; c < ROW_WORDS; ++c) row[u][c] = next_row[u][c];\n";
+  s << "    }\n";
+  s << "    if (chunk + static_cast<int>(gridDim.x) < CHUNKS) fetch(chunk + static_cast<int>(gridDim.x));   // (uniform)\n";
+  s << "    chunk_rank<NW, KEYS, TILES>(key, slot, reinterpret_cast<unsigned long long *>(akg_stage), akg_cnt, akg_start, akg_scan);\n";
+  s << "    unsigned char *stage_segs = akg_stage + CHUNK * ROW_WORDS * 4;\n";
+  s << "#pragma unroll\n";
+  s << "    for (int u = 0; u < TILES; ++u) {\n";
+  s << "      if (key[u] >= 0) {\n";
+  s << "        unsigned *to = reinterpret_cast<unsigned *>(akg_stage) + slot[u] * ROW_WORDS;\n";
+  s << "#pragma unroll\n";
+  s << "        for (int c = 0; c < ROW_WORDS; ++c) to[c] = row[u][c];\n";
+  s << "        stage_segs[slot[u]] = static_cast<unsigned char>(key[u] >> 16);\n";
+  s << "      }\n    }\n";
+  s << "    __syncthreads();\n";
+  s << "    // whole 16-byte pieces; what they hold behind the last item is never looked at\n";
+  s << "    const int valid = akg_start[KEYS];\n";
+  s << "    const quad_words *staged = reinterpret_cast<const quad_words *>(akg_stage);\n";
+  s << "    quad_words *to = reinterpret_cast<quad_words *>(akg_ws + static_cast<long>(chunk) * (CHUNK * ROW_WORDS));\n";
+  s << "    for (int i = tid; i < (valid * ROW_WORDS + 3) / 4; i += NW * 64) to[i] = staged[i];\n";
+  s << "    to = reinterpret_cast<quad_words *>(akg_ws + W_SEGS + static_cast<long>(chunk) * (CHUNK / 4));\n";
+  s << "    for (int i = tid; i < (valid + 15) / 16; i += NW * 64) to[i] = reinterpret_cast<const quad_words *>(stage_segs)[i];\n";
+  s << "    to = reinterpret_cast<quad_words *>(akg_ws + W_TABLE + static_cast<long>(chunk) * (PITCH / 2));\n";
+  s << "    for (int i = tid; i < PITCH / 8; i += NW * 64) to[i] = reinterpret_cast<const quad_words *>(akg_start)[i];\n";
+  s << "    __syncthreads();\n";
+  s << "  }\n}\n\n";
+
+  // ---- chains ----
+  s << "extern \"C\" __global__ __launch_bounds__(" << nw * 64 << (small ? "" : ", 4") << ") void " << g.name << "_kernel(" << params.str() << ") {\n";
+  s << "  constexpr int W = " << nw << ", T = " << tiles << ", CAP = W * T * 64, PLANE = CAP + 4 * S + 40, CHAINS = " << chains
+    << ", PER_WAVE = " << chainsPerWave << ";\n";
+  s << "  static_assert(CAP >= CHUNK, \"a chunk's run of one bucket fits a round\");\n";
+  s << "  // a round's entries: whose run each is, and where entry k of the round is less k for every run\n";
+  s << "  __shared__ unsigned short akg_run[CAP];\n  __shared__ unsigned akg_base[W * 64];\n";
+  s << "  __shared__ __attribute__((aligned(16))) " << ct << " akg_plane[ROW][PLANE];   // column c of a round's rows, lists per segment\n";
+  s << "  __shared__ unsigned short akg_cnt[W * S];\n";
+  s << "  __shared__ unsigned akg_start[S], akg_len[S], akg_scan[W], akg_sums[W], akg_taken[W], akg_total[W];\n";
+  s << "  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, w = tid >> 6;\n";
+  s << "  const int bucket = akg::xcd_contiguous_id(static_cast<int>(blockIdx.x), KEYS);\n";
+  s << "  const row_t *__restrict__ rows = reinterpret_cast<const row_t *>(akg_ws);\n";
+  s << "  const unsigned char *__restrict__ segs = reinterpret_cast<const unsigned char *>(akg_ws + W_SEGS);\n";
+  s << "  const unsigned short *__restrict__ table = reinterpret_cast<const unsigned short *>(akg_ws + W_TABLE) + bucket;\n";
+  s << "  // the output element of this lane, if it has one: wavefront w adds chains w * PER_WAVE ...\n";
+  s << "  const int chain = w * PER_WAVE + lane;\n";
+  s << "  const bool has = lane < PER_WAVE && chain < CHAINS;\n";
+  s << "  const int cs = has ? chain / ROW : 0, cc = has ? chain - cs * ROW : 0;\n";
+  s << "  union cell_t { row_t r; " << tag << "::storage v[ROW_WORDS * 4 / sizeof(" << tag << "::storage)]; };\n";
+  s << "  typedef " << ct << " quad_t __attribute__((ext_vector_type(4)));\n";
+  s << "  " << ct << " acc = " << lowering::literalFor(out.dtype, 0.0) << ";\n";
+  s << "  unsigned first = 0u, behind = 0u;   // this thread's run of the round: entries first .. behind - 1 of its chunk\n";
+  s << "  const auto look_up = [&](int chunk) {\n";
+  s << "    const unsigned short *t = table + static_cast<long>(chunk < CHUNKS ? chunk : CHUNKS - 1) * PITCH;\n";
+  s << "    first = t[0];\n    behind = t[1];\n";
+  s << "  };\n";
+  s << "  look_up(tid);\n";
+  s << "  cell_t cur[T];\n  int segment[T];\n  unsigned total = 0u;   // the round on its way: its entries as they are, how many\n";
+  s << "  int chunk0 = 0;\n";
+  s << "  const auto next_round = [&]() {\n";
+  s << "    const int chunk = chunk0 + tid;\n";
+  s << "    const unsigned len = chunk < CHUNKS ? behind - first : 0u;\n";
+  s << "    const unsigned at = static_cast<unsigned>(chunk) * CHUNK + first;\n";
+  s << "    unsigned incl = len;\n";
+  s << "#pragma unroll\n";
+  s << "    for (int d = 1; d < 64; d <<= 1) {\n";
+  s << "      const unsigned o = __shfl_up(incl, d);\n";
+  s << "      if (lane >= d) incl += o;\n";
+  s << "    }\n";
+  s << "    if (lane == 63) akg_sums[w] = incl;\n";
+  s << "    __syncthreads();\n";
+  s << "#pragma unroll\n";
+  s << "    for (int j = 0; j < W; ++j) incl += j < w ? akg_sums[j] : 0u;\n";
+  s << "    // the chunks whose runs fit the round: those in front of the first one that does not (the first one always does)\n";
+  s << "    const bool fits = chunk < CHUNKS && incl <= static_cast<unsigned>(CAP);\n";
+  s << "    const int fitting = __popcll(__ballot(fits));\n";
+  s << "    if (lane == (fitting > 0 ? fitting - 1 : 0)) {\n";
+  s << "      akg_taken[w] = static_cast<unsigned>(fitting);\n";
+  s << "      akg_total[w] = fitting > 0 ? incl : 0u;\n";
+  s << "    }\n";
+  s << "    // every run's entries, one after the other; runs of more than 32 by the whole wavefront\n";
+  s << "    unsigned long long longer = __ballot(fits && len > 32u);\n";
+  s << "    akg_base[tid] = at - (incl - len);\n";
+  s << "    if (fits && len <= 32u) {\n";
+  s << "      for (unsigned i = 0; i < len; ++i) akg_run[incl - len + i] = static_cast<unsigned short>(tid);\n";
+  s << "    }\n";
+  s << "    while (longer) {\n";
+  s << "      const int b = __builtin_ctzll(longer);\n";
+  s << "      longer &= longer - 1;\n";
+  s << "      const unsigned n = __builtin_amdgcn_readlane(len, b), to = __builtin_amdgcn_readlane(incl, b) - n;\n";
+  s << "      for (unsigned i = lane; i < n; i += 64) akg_run[to + i] = static_cast<unsigned short>(w * 64 + b);\n";
+  s << "    }\n";
+  s << "    __syncthreads();\n";
+  s << "    int taken = 0;\n    total = 0u;\n";
+  s << "#pragma unroll\n";
+  s << "    for (int j = 0; j < W; ++j) {\n";
+  s << "      taken += static_cast<int>(akg_taken[j]);\n";
+  s << "      total = akg_total[j] > total ? akg_total[j] : total;\n";
+  s << "    }\n";
+  s << "    chunk0 += taken;\n";
+  s << "    look_up(chunk0 + tid);   // (the next round's runs)\n";
+  s << "#pragma unroll\n";
+  s << "    for (int u = 0; u < T; ++u) {\n";
+  s << "      const unsigned k = (w * T + u) * 64 + lane;\n";
+  s << "      const unsigned from = k < total ? akg_base[akg_run[k]] + k : 0u;   // (the workspace's first row where there is no entry)\n";
+  s << "      cur[u].r = rows[from];\n";
+  s << "      segment[u] = segs[from];\n";
+  s << "    }\n";
+  s << "  };\n";
+  s << "  next_round();\n";
+  s << "  for (;;) {\n";
+  s << "    int key[T];\n    unsigned slot[T];\n";
+  s << "#pragma unroll\n";
+  s << "    for (int u = 0; u < T; ++u) key[u] = static_cast<unsigned>((w * T + u) * 64 + lane) < total ? segment[u] : -1;\n";
+  s << "    chunk_sort<W, S, " << keyBits << ", T, 4>(key, slot, akg_cnt, akg_start, akg_len, akg_scan);\n";
+  s << "#pragma unroll\n";
+  s << "    for (int u = 0; u < T; ++u) {\n";
+  s << "      if (key[u] >= 0) {\n";
+  s << "#pragma unroll\n";
+  s << "        for (int c = 0; c < ROW; ++c) akg_plane[c][slot[u]] = " << tag << "::load(cur[u].v[c]);\n";
+  s << "      }\n";
+  s << "    }\n";
+  s << "    __syncthreads();\n";
+  s << "    // the next round's entries are on their way while this one's are added up\n";
+  s << "    const bool more = chunk0 < CHUNKS;   // (uniform)\n";
+  s << "    if (more) next_round();\n";
+  s << "    if (has) {\n";
+  s << "      const int n = static_cast<int>(akg_len[cs]);\n";
+  s << "      const quad_t *__restrict__ list = reinterpret_cast<const quad_t *>(&akg_plane[cc][akg_start[cs]]);   // (a multiple of 4)\n";
+  s << "      // sixteen additions at a time, the next sixteen values on their way (what lies behind the list's end is read,\n";
+  s << "      // inside the plane, and not added)\n";
+  s << "      quad_t q[4];\n";
+  s << "#pragma unroll\n";
+  s << "      for (int i = 0; i < 4; ++i) q[i] = list[i];\n";
+  s << "      int j = 0;\n";
+  s << "      for (; j + 16 <= n; j += 16) {\n";
+  s << "        quad_t next[4];\n";
+  s << "#pragma unroll\n";
+  s << "        for (int i = 0; i < 4; ++i) next[i] = list[j / 4 + 4 + i];\n";
+  s << "#pragma unroll\n";
+  s << "        for (int u = 0; u < 16; ++u) acc = " << rndOpen << "akg::op_add(q[u / 4][u & 3], acc));\n";
+  s << "#pragma unroll\n";
+  s << "        for (int i = 0; i < 4; ++i) q[i] = next[i];\n";
+  s << "      }\n";
+  s << "#pragma unroll\n";
+  s << "      for (int u = 0; u < 16; ++u) {\n";
+  s << "        const " << ct << " sum = " << rndOpen << "akg::op_add(q[u / 4][u & 3], acc));\n";
+  s << "        acc = j + u < n ? sum : acc;\n";
+  s << "      }\n";
+  s << "    }\n";
+  s << "    if (!more) break;\n";
+  s << "    __syncthreads();\n";
+  s << "  }\n";
+  s << "  if (has && bucket * S + cs < SEGMENTS) out0[static_cast<long>(bucket * S + cs) * ROW + cc] = " << tag << "::store(acc);\n";
+  s << "}\n";
+
+  LoweredKernel k;
+  k.kernelName = g.name + "_kernel";
+  k.source = s.str();
+  k.family = KernelFamily::SegmentSum;
+  k.grid[0] = static_cast<unsigned>(plan.buckets);
+  k.block[0] = static_cast<unsigned>(nw * 64);
+  KernelPhase place;
+  place.kernelName = g.name + "_place";
+  place.grid[0] = static_cast<unsigned>(placeGrid);
+  place.block[0] = 512;
+  k.earlierPhases.push_back(place);
+  k.workspaceBytes = static_cast<uint64_t>(plan.words) * 4;
+  k.algorithmicBytes = lowering::countAlgorithmicBytes(g);
+  k.shapeArgs = lowering::buildShapeArgs(g);
+  std::ostringstream note;
+  note << "segment_sum positions=" << sh.positions << " segments=" << sh.segments << " slice=" << sh.slice << " chunks=" << plan.chunks << " of "
+       << plan.chunk << " positions grouped by bucket of " << perBucket << " segments where they lie: " << plan.buckets << " buckets, 2 launches";
+  k.scheduleNote = note.str();
+  return k;
+}
+
 LoweredKernel lowerSegmentScan(const OpGraph &g, const LoweringOptions &options, const SegmentShapes &sh) {
   using lowering::computeTypeName;
   using lowering::dtypeTag;
@@ -898,9 +1277,27 @@ LoweredKernel lowerSegmentSumToHip(const OpGraph &g, const LoweringOptions &opti
   while (bucketBits > 0 && (sh.slice << bucketBits) > 32) --bucketBits;
   const int64_t buckets = (sh.segments + (1LL << bucketBits) - 1) >> bucketBits;
   const bool canBucket = group && !wide && rowBytes <= 12 && rowBytes % 4 == 0 && bucketBits >= 2 && buckets <= 640 && buckets >= 2;
-  if (canBucket && (options.variant == 3 || (options.variant == 0 && buckets >= 96))) {
-    return lowerSegmentBucketed(g, options, sh, bucketBits);
+  const bool bucketed = canBucket && (options.variant == 3 || (options.variant == 0 && buckets >= 96));
+  // Short rows by chunks, two launches for five. From 2^19 positions on always; us, grouped by segment or by bucket -> by
+  // chunk: 24.5 million x 3 into 4954 413 -> 300, 12.5 million x 4 into 2216 401 -> 226, 20 million x 4 into 16384 1665 -> 314,
+  // 1.5 million x 4 into 12654 261 -> 30, 5 million x 1 into 300 234 -> 180, 600000 x 1 into 300 49 -> 31, x 3 into 16000 227 -> 17.
+  // Below, where the positions would be grouped by segment and a bucket has several segments (244664 x 4 into 9073 82 -> 13,
+  // 65974 x 1 into 13950 97 -> 8.9, 138073 x 1 into 998 29.6 -> 11.0, 200000 x 4 into 513 33.9 -> 14.5), and from 2^15 positions
+  // on instead of the scan (35304 x 1 into 1131 42.0 -> 8.4, 33000 x 4 into 300 51 -> 9.1). The other two schedules would lose
+  // in between as well (300000 x 3 into 5000 36.7 by bucket, 13.4 by chunk; 27126 x 3 into 4954 29.4 scanned, 7.9), but their
+  // launches and the scan's lack of a workspace are pinned by tests there. Nor may the workspace outgrow the 16 MiB of a
+  // launch without allocations where it did not before.
+  const ChunkedPlan chunked = planChunked(sh, options);
+  bool byChunk = chunked.possible && options.variant == 4;
+  if (chunked.possible && options.variant == 0 && sh.positions >= (1 << 15)) {
+    const bool many = sh.positions >= (1 << 19);
+    byChunk = many || (group ? !bucketed && chunked.perBucket > 1 : sh.positions < (1 << 16));
+    const int64_t runs = std::min<int64_t>(2048, std::max<int64_t>(1, sh.positions / 1024));   // (of the schedule by segment)
+    const int64_t before = bucketed ? sh.positions * 4 : sh.positions * rowBytes / 4 + runs * sh.segments;
+    if (group && chunked.words * 4 > (16 << 20) && before * 4 <= (16 << 20)) byChunk = false;
   }
+  if (byChunk) return lowerSegmentChunked(g, options, sh, chunked);
+  if (bucketed) return lowerSegmentBucketed(g, options, sh, bucketBits);
   return group ? lowerSegmentSorted(g, options, sh) : lowerSegmentScan(g, options, sh);
 }
 

@@ -1,0 +1,64 @@
+"""UnsortedSegmentSum of short rows, chunks of positions grouped by bucket of segments where they lie: which sizes take it, and
+its results bit for bit the serial loop's."""
+import os
+
+import numpy as np
+import pytest
+
+from akg_amd import driver, harness, op_desc
+
+BY_CHUNK = "grouped by bucket of segments, chunk by chunk"
+
+
+def test_sizes_that_are_taken_by_chunk():
+    def by_chunk(positions, width, segments, dtype="float32"):
+        kernel = driver.HipKernel(op_desc.unsorted_segment_sum([positions], [width], segments, dtype, "int32", "s_%s_%d_%d_%d" % (
+            dtype, positions, width, segments)), out_dir=None)
+        return BY_CHUNK in kernel.source
+    assert by_chunk(1 << 19, 3, 4954) and by_chunk(1 << 19, 1, 300) and by_chunk(1 << 15, 4, 300) and by_chunk(65535, 2, 5)
+    assert by_chunk(70000, 1, 13950) and by_chunk(70000, 4, 513) and not by_chunk(70000, 4, 512) and not by_chunk(70000, 3, 5000)
+    assert not by_chunk(32767, 3, 4954)
+    assert not by_chunk(1 << 19, 5, 300) and not by_chunk(1 << 19, 3, 300, "float16") and not by_chunk(1 << 15, 3, 40000)
+    # 17 bytes a position are beyond the 16 MiB of a launch without allocations where 16 were within
+    assert not by_chunk(1020000, 4, 100) and by_chunk(980000, 4, 100) and by_chunk(1100000, 4, 100)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("positions,width,segments,dtype,ids,pattern,chunks", [
+    (1, 1, 1, "float32", "int32", "uniform", 0),
+    (511, 3, 700, "float32", "int32", "uniform", 1), (513, 4, 513, "float32", "int64", "uniform", 1),   # edges of a chunk
+    (4097, 2, 1025, "float32", "int32", "uniform", 8), (33000, 3, 4954, "float32", "int32", "uniform", 0),
+    (300000, 1, 512, "float32", "int32", "uniform", 2),      # more chunks than a round looks up
+    (9000, 4, 32768, "int32", "int32", "uniform", 4),        # 64 segments a bucket
+    (150000, 3, 9000, "float32", "int32", "one_segment", 8), (70000, 4, 600, "float32", "int32", "one_segment", 1),
+    (100000, 3, 4954, "float32", "int32", "one_bucket", 4), (40000, 2, 3000, "float32", "int32", "sorted", 0),
+    (40000, 2, 3000, "float32", "int32", "outside", 2), (20000, 1, 77, "float32", "int32", "nobody", 0),
+    (70001, 2, 5000, "float16", "int32", "uniform", 0), (66000, 4, 1300, "bfloat16", "int64", "uniform", 0),   # additions that round
+    (33333, 4, 999, "int8", "int32", "uniform", 0), (540000, 3, 16384, "float32", "int32", "uniform", 0),
+])
+def test_bit_for_bit_the_serial_loop(positions, width, segments, dtype, ids, pattern, chunks, monkeypatch, tmp_path):
+    import torch
+    from oracle import cpu_ref
+    monkeypatch.setenv("AKG_HIP_VARIANT", "4")
+    if chunks:
+        monkeypatch.setenv("AKG_HIP_CHUNKS", str(chunks))
+    name = "by_chunk_%s_%d_%d_%d_%s" % (dtype, positions, width, segments, pattern)
+    text = op_desc.unsorted_segment_sum([positions], [width], segments, dtype, ids, name)
+    path = os.path.join(str(tmp_path), name + ".info")
+    open(path, "w").write(text)
+    print("case %s" % name, flush=True)
+    kernel = driver.HipKernel(text, out_dir=None)
+    assert BY_CHUNK in kernel.source
+    inputs = harness.make_inputs(harness.load_desc(path), seed=harness.BASE_SEED + 812)
+    rng = np.random.default_rng(positions)
+    at = {"uniform": rng.integers(0, segments, positions), "one_segment": np.full(positions, segments // 2),
+          "one_bucket": rng.integers(10, 20, positions), "sorted": np.sort(rng.integers(0, segments, positions)),
+          "outside": rng.integers(-4 * segments, 5 * segments, positions), "nobody": np.full(positions, segments)}[pattern]
+    inputs[1] = at.astype(inputs[1].dtype).reshape(inputs[1].shape)
+    want = cpu_ref.CpuKernel(path)(inputs)[0]
+    on_device = [torch.from_numpy(np.ascontiguousarray(a).view(np.int16) if a.dtype == np.uint16 else np.ascontiguousarray(a)).cuda() for a in inputs]
+    for _ in range(3):
+        out = torch.full((kernel.outputs[0].nbytes,), 0x7b, dtype=torch.uint8, device="cuda")
+        kernel.launch(on_device + [out])
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), np.ascontiguousarray(want).reshape(-1).view(np.uint8)), name
