@@ -107,6 +107,7 @@ class StreamReduceEmitter {
   // extent is walked in chunk slots, runChunks_ per run of runLength_ elements, the last one starting at
   // runLength_ - V; the elements it shares with its neighbour are left out of the reductions.
   bool xcdContiguous_ = false;
+  bool sharedLines_ = false;   // direction Y: neighbouring strips share the lines at their edges
   // The streaming loop takes `unroll_` chunks per trip: their loads first (conditions as operands, so that they issue
   // together whatever the trip holds), then the work on each. An unroll pragma on a one-chunk body left the loads of
   // the bf16 kernels one behind the other, each waited for by itself (a [16384,4096] bf16 sum of squares: 25 % of the
@@ -633,6 +634,17 @@ class StreamReduceEmitter {
     // image): the lines are shared with the neighbouring outputs' runs.
     xcdContiguous_ = !dirY_ && scatteredR && grid_ >= 64 &&
                      (fastExtent * static_cast<int64_t>(widest)) % 128 != 0 && fastExtent * static_cast<int64_t>(widest) < 2048;
+    // Column strips of rows that are not whole lines: a strip's piece of a row begins and ends inside lines that its
+    // neighbours read as well. The strips of the same rows then run on one XCD and the lines stay in its L2 (no hint); in
+    // launch order and past the caches every such line came from memory twice. Two column sums of bf16 [4100,3000]
+    // 14.9 -> 12.0 us, [16400,3000] 45.9 -> 34.8, [16400,1111] 21.0 -> 15.8; rows of whole lines keep the hint ([16400,3072]
+    // 32.9, 34.5 this way).
+    sharedLines_ = false;
+    for (int id : g_.inputs) {
+      const TensorValue &t = g_.tensor(id);
+      if (dirY_ && t.used && t.numel() == O_ * R_ * I_) sharedLines_ = sharedLines_ || (I_ * static_cast<int64_t>(dtypeSize(t.dtype))) % 128 != 0;
+    }
+    if (dirY_) xcdContiguous_ = sharedLines_ && strips_ > 1;
     // workspace: one arrival counter per group, then the partials of every reduction
     workspaceBytes_ = 0;
     partialOffset_.assign(reduces_.size(), 0);
@@ -771,7 +783,7 @@ class StreamReduceEmitter {
     const bool fastVarGiven = !(fastGroup == 2 ? iv : rv).empty();
     if (batch) {
       if (fastVarGiven && chunkContiguous(t, fastGroup)) {
-        const bool streamed = opt_.nonTemporal != 0 && t.numel() == O_ * R_ * I_;
+        const bool streamed = opt_.nonTemporal != 0 && !sharedLines_ && t.numel() == O_ * R_ * I_;
         src_ << indent << "akg::load_chunk_if<" << tag << ", V, " << (streamed ? "true" : "false") << ">(b_" << arg
              << ", akg_in, " << off << ", " << name << ");\n";
       } else {
@@ -788,7 +800,7 @@ class StreamReduceEmitter {
         src_ << indent << "const " << ct << " " << name << " = " << tag << "::load(" << arg << "[" << off << "]);\n";
       }
     } else if (fastVarGiven && chunkContiguous(t, fastGroup)) {
-      const bool streamed = opt_.nonTemporal != 0 && t.numel() == O_ * R_ * I_;
+      const bool streamed = opt_.nonTemporal != 0 && !sharedLines_ && t.numel() == O_ * R_ * I_;
       src_ << indent << ct << " " << name << "[V];\n";
       src_ << indent << "akg::load_chunk<" << tag << ", V, " << (streamed ? "true" : "false") << ">(" << memRef(arg, off)
            << ", " << name << ");\n";
@@ -940,8 +952,8 @@ class StreamReduceEmitter {
     }
     line("  (void)O; (void)I; (void)STRIPS;");
     line("  const int tid = static_cast<int>(threadIdx.x);");
-    if (!dirY_ && xcdContiguous_) {
-      // neighbouring outputs read neighbouring runs that share cache lines: keep them on one XCD (one L2)
+    if (xcdContiguous_) {
+      // neighbouring outputs read neighbouring runs (or strips of a row) that share cache lines: keep them on one XCD (one L2)
       src_ << "  const long akg_wg = akg::xcd_contiguous_id(static_cast<int>(blockIdx.x), "
            << (dynR_ ? std::string("static_cast<int>(gridDim.x)") : std::to_string(grid_)) << ");\n";
     } else {
@@ -1113,12 +1125,12 @@ class StreamReduceEmitter {
       if (phase_[static_cast<size_t>(id)] != Phase::Pre) continue;
       const std::string off = offsetExpr(g_.tensor(id), "akg_o", "r", dirY_ ? "akg_i" : "");
       if (batched_) {
-        src_ << in4 << "akg::store_chunk_if<" << tagOf(id) << ", V, " << (opt_.nonTemporal != 0 ? "true" : "false") << ">(b_out" << i
+        src_ << in4 << "akg::store_chunk_if<" << tagOf(id) << ", V, " << (opt_.nonTemporal != 0 && !sharedLines_ ? "true" : "false") << ">(b_out" << i
              << ", akg_in" << (dirY_ ? " && col_ok" : "") << ", " << off << ", " << ident_[static_cast<size_t>(id)] << ");\n";
         continue;
       }
       src_ << in4 << (dirY_ ? "if (col_ok) " : (ordered_ ? "if (akg_in) " : "")) << "akg::store_chunk<" << tagOf(id) << ", V, "
-           << (opt_.nonTemporal != 0 ? "true" : "false") << ">(" << memRef("out" + std::to_string(i), off) << ", "
+           << (opt_.nonTemporal != 0 && !sharedLines_ ? "true" : "false") << ">(" << memRef("out" + std::to_string(i), off) << ", "
            << ident_[static_cast<size_t>(id)] << ");\n";
     }
     if (batched_) line("    }");
