@@ -115,6 +115,11 @@ class TileEmitter {
   // the heads): the leading extents of the folded iteration space are kernel arguments too, and the operand's row
   // offset is computed from them, so the source does not carry them as numbers.
   bool dimsArg_ = false;
+  // The row length is an argument and a thread holds several chunks: chunk j of a short row of the bucket lies beyond the
+  // row for every lane of the wavefront. The elementwise ops and reduction steps between two row-wide results are then
+  // emitted chunk by chunk, and a wavefront leaves out the chunks none of its lanes has.
+  bool chunkwise_ = false;
+  std::ostringstream pending_;   // ... the steps of one chunk, until the next row-wide result
   int64_t bucketLow_ = 0, bucketHigh_ = 0;
   std::vector<InputAccess> access_;  // per graph input
   std::vector<ValInfo> vals_;        // per tensor
@@ -432,6 +437,12 @@ class TileEmitter {
           if (ceilDiv(rowChunks, t) <= 8) break;
         }
       }
+      // Rows of any length in the bucket that a wavefront of two chunks a lane holds: two rows a wavefront with four chunks
+      // a lane instead, of which the wavefront leaves out those beyond the row (chunkwise_). Bound by its vector
+      // instructions, and the second chunk of 64 lanes costs a row of 257 elements as much as one of 512: float32 softmax
+      // with a shared mask, us, 64 x 2 -> 32 x 4: [32,12,333,333] 71 -> 67, [32,12,512,257] 95 -> 88, 300 wide 99 -> 93, 509 wide
+      // 78.4 -> 77.7; rows of whole 64-byte pieces stay (400 wide 105 -> 112).
+      if (colsArg_ && !colsWhole_ && !ordered_ && tpr == 64 && ceilDiv(rowChunks, tpr) == 2) tpr = 32;
       tpr_ = tpr;
       int64_t perThread = ceilDiv(schedCols, static_cast<int64_t>(tpr_) * vec_);
       // More than 64 values per thread of one row-sized input, or 96 over all of them, do not stay in registers: walk the row in groups of
@@ -498,6 +509,7 @@ class TileEmitter {
       rowsPerBlock_ = block_ / tpr_;
       grid_ = ceilDiv(rows_, rowsPerBlock_);
       raggedCols_ = colsArg_ || (groups_ * chunks_ * tpr_ != rowChunks);
+      chunkwise_ = colsArg_ && !ordered_ && chunks_ > 1;
       raggedRows_ = (rows_ % rowsPerBlock_) != 0 || extentArg_;
     } else {
       block_ = opt_.block > 0 ? opt_.block : 256;
@@ -819,6 +831,7 @@ class TileEmitter {
         emitElementwise(op, clampCast_[k]);
       }
     }
+    flushChunks();
     // stores: the outputs, then the destinations of Assign ops (every thread has read its part of a destination
     // into registers above, and writes exactly the positions it read)
     for (size_t i = 0; i < g_.outputs.size(); ++i) emitOutputStore(i);
@@ -885,6 +898,22 @@ class TileEmitter {
       line("    if (akg_tail[j]) akg_cols[j] = COLS - V;");
     }
     line("  }");
+    if (chunkwise_) {
+      line("  bool akg_some[NCHUNK];   // some lane of the wavefront has this chunk");
+      line("#pragma unroll");
+      line("  for (int j = 0; j < NCHUNK; ++j) akg_some[j] = __ballot(akg_ok[j]) != 0ull;");
+    }
+  }
+
+  void flushChunks() {
+    if (!chunkwise_ || pending_.str().empty()) return;
+    line("#pragma unroll");
+    line("  for (int j = 0; j < NCHUNK; ++j) {");
+    line("    if (akg_some[j]) {");
+    src_ << pending_.str();
+    line("    }");
+    line("  }");
+    pending_.str("");
   }
 
   // Two reductions of which one waits for the other, and some per-column operand (an input that spans the row but not
@@ -1190,7 +1219,7 @@ class TileEmitter {
     std::vector<std::string> operands;
     for (int in : op.inputs) operands.push_back(operandExpr(in));
     const bool relaxed = relaxed_[static_cast<size_t>(outId)];
-    std::string expr;
+    std::string expr, chunkDivision;
     // float32 division of a tile by a per-row (or constant) divisor: hoist the reciprocal out of the element loop
     const bool uniformDivisor = op.kind == OpKind::Div && rank == ValRank::Tile && op.inputs.size() == 2 &&
                                 vals_[static_cast<size_t>(op.inputs[1])].rank != ValRank::Tile &&
@@ -1211,6 +1240,9 @@ class TileEmitter {
       } else {
         src_ << "  const akg::UniformDivisor " << hoisted << " = akg::make_divisor(" << operands[1] << ");\n";
         q = "akg::div_uniform(" + operands[0] + ", " + hoisted + ")";
+        const ValInfo &dividend = vals_[static_cast<size_t>(op.inputs[0])];
+        // (chunks of four: with eight the checks of a chunk hold its quotients back, int8 quantisation of bf16 rows 215 -> 222 us)
+        if (outT.dtype == DType::F32 && dividend.rank == ValRank::Tile && vec_ <= 4) chunkDivision = "akg::div_uniform(" + dividend.ident + "[j], " + hoisted + ", ";
       }
       const DType od = outT.dtype;
       expr = (od == DType::F16 || od == DType::BF16) ? std::string(dtypeTag(od)) + "::rnd(" + q + ")" : q;
@@ -1226,13 +1258,16 @@ class TileEmitter {
       nm << "t" << outId;
       v.ident = nm.str();
       src_ << "  " << ctOf(outId) << " " << v.ident << "[NCHUNK][V];  // " << op.name << " -> " << outT.name << "\n";
-      line("#pragma unroll");
-      line("  for (int j = 0; j < NCHUNK; ++j) {");
-      line("#pragma unroll");
-      line("    for (int e = 0; e < V; ++e) {");
-      src_ << "      " << v.ident << "[j][e] = " << expr << ";\n";
-      line("    }");
-      line("  }");
+      std::string step = "#pragma unroll\n    for (int e = 0; e < V; ++e) {\n      " + v.ident + "[j][e] = " + expr + ";\n    }\n";
+      if (!chunkDivision.empty()) step = "    " + chunkDivision + v.ident + "[j]);\n";
+      if (chunkwise_) {
+        pending_ << step;
+      } else {
+        line("#pragma unroll");
+        line("  for (int j = 0; j < NCHUNK; ++j) {");
+        src_ << step;
+        line("  }");
+      }
     } else {
       nm << "u" << outId;
       v.ident = nm.str();
@@ -1264,7 +1299,7 @@ class TileEmitter {
       throw LoweringError("op " + op.name + ": the reduced operand must span the innermost axis");
     }
     const DType od = g_.tensor(outId).dtype;
-    const std::string tag = dtypeTag(od);
+    const std::string tag = dtypeTag(od), ct = computeTypeName(od);
     const lowering::ReduceSpec spec = lowering::reduceSpec(op, od);
     const std::string acc = "acc" + std::to_string(outId);
     if (spec.ordered) {
@@ -1297,35 +1332,65 @@ class TileEmitter {
       // A maximum or minimum does not depend on the order of its steps nor on an element taken twice (the elements a
       // tail chunk shares with its neighbour): the chunk is folded by itself and joins the accumulator under the one
       // condition of the chunk, instead of every element under its own.
+      std::ostringstream fold;
+      const std::string part = "akg_part" + std::to_string(outId);
+      fold << "    " << computeTypeName(od) << " " << part << " = " << in.ident << "[j][0];\n";
+      fold << "#pragma unroll\n";
+      fold << "    for (int e = 1; e < V; ++e) " << part << " = " << spec.combiner << "::apply(" << part << ", " << in.ident << "[j][e]);\n";
+      fold << "    if (akg_ok[j]) " << acc << " = " << spec.combiner << "::apply(" << acc << ", " << part << ");\n";
+      if (chunkwise_) {
+        pending_ << fold.str();
+        return;
+      }
       line("#pragma unroll");
       line("  for (int j = 0; j < NCHUNK; ++j) {");
-      src_ << "    " << computeTypeName(od) << " akg_part = " << in.ident << "[j][0];\n";
-      line("#pragma unroll");
-      src_ << "    for (int e = 1; e < V; ++e) akg_part = " << spec.combiner << "::apply(akg_part, " << in.ident << "[j][e]);\n";
-      src_ << "    if (akg_ok[j]) " << acc << " = " << spec.combiner << "::apply(" << acc << ", akg_part);\n";
+      src_ << fold.str();
       line("  }");
+      return;
+    }
+    std::ostringstream fold;
+    if (chunkwise_ && spec.combiner == "akg::RedSum" && ct == "float" && !spec.roundEachStep) {
+      // the chunk's sum as a tree (no more roundings in a row than a thread of two chunks had), elements of its neighbour as zeros
+      const std::string part = "akg_part" + std::to_string(outId);
+      fold << "    float " << part << "[V];\n";
+      fold << "#pragma unroll\n";
+      fold << "    for (int e = 0; e < V; ++e) " << part << "[e] = akg_ok[j]" << (colsWhole_ ? "" : " && (!akg_tail[j] || e >= akg_overlap)") << " ? "
+           << in.ident << "[j][e] : 0.0f;\n";
+      fold << "#pragma unroll\n";
+      fold << "    for (int d = 1; d < V; d *= 2) {\n";
+      fold << "#pragma unroll\n";
+      fold << "      for (int e = 0; e + d < V; e += 2 * d) " << part << "[e] = akg::RedSum::apply(" << part << "[e], " << part << "[e + d]);\n";
+      fold << "    }\n";
+      fold << "    " << acc << " = akg::RedSum::apply(" << acc << ", " << part << "[0]);\n";
+      pending_ << fold.str();
+      return;
+    }
+    fold << "#pragma unroll\n";
+    fold << "    for (int e = 0; e < V; ++e) {\n";
+    std::string step = spec.combiner + "::apply(" + acc + ", " + in.ident + "[j][e])";
+    if (spec.roundEachStep) step = tag + "::rnd(" + step + ")";
+    if (colsArg_ && !colsWhole_) {
+      fold << "      if (akg_ok[j] && (!akg_tail[j] || e >= akg_overlap)) " << acc << " = " << step << ";\n";
+    } else if (overlap_ > 0) {
+      fold << "      if (akg_ok[j] && (!akg_tail[j] || e >= " << overlap_ << ")) " << acc << " = " << step << ";\n";
+    } else if (raggedCols_) {
+      fold << "      if (akg_ok[j]) " << acc << " = " << step << ";\n";
+    } else {
+      fold << "      " << acc << " = " << step << ";\n";
+    }
+    fold << "    }\n";
+    if (chunkwise_) {
+      pending_ << fold.str();
       return;
     }
     line("#pragma unroll");
     line("  for (int j = 0; j < NCHUNK; ++j) {");
-    line("#pragma unroll");
-    line("    for (int e = 0; e < V; ++e) {");
-    std::string step = spec.combiner + "::apply(" + acc + ", " + in.ident + "[j][e])";
-    if (spec.roundEachStep) step = tag + "::rnd(" + step + ")";
-    if (colsArg_ && !colsWhole_) {
-      src_ << "      if (akg_ok[j] && (!akg_tail[j] || e >= akg_overlap)) " << acc << " = " << step << ";\n";
-    } else if (overlap_ > 0) {
-      src_ << "      if (akg_ok[j] && (!akg_tail[j] || e >= " << overlap_ << ")) " << acc << " = " << step << ";\n";
-    } else if (raggedCols_) {
-      src_ << "      if (akg_ok[j]) " << acc << " = " << step << ";\n";
-    } else {
-      src_ << "      " << acc << " = " << step << ";\n";
-    }
-    line("    }");
+    src_ << fold.str();
     line("  }");
   }
 
   void emitReduceFinish(const OpNode &op) {
+    flushChunks();
     const int outId = op.outputs[0];
     const DType od = g_.tensor(outId).dtype;
     const std::string ct = computeTypeName(od);

@@ -1,0 +1,97 @@
+"""Float32 arithmetic of the row kernels: the exponential over its whole range, division by a per-row value bit for bit the
+IEEE quotient, and rows of any length whose wavefronts leave out chunks."""
+import json
+
+import numpy as np
+import pytest
+
+from akg_amd import driver, op_desc
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(kernel, arrays):
+    import torch
+    outs = [torch.full(d.shape, float("nan"), device="cuda") for d in kernel.outputs]
+    kernel.launch([torch.from_numpy(a).cuda() for a in arrays] + outs)
+    torch.cuda.synchronize()
+    return [o.cpu().numpy() for o in outs]
+
+
+def test_the_exponential_over_its_whole_range():
+    """One unit in the last place at most where the result is normal, one step of 2^-149 where it is subnormal (the hardware's
+    2^f is good to one unit, f to 2^-26); 0, infinity and NaN where they belong."""
+    b = op_desc.DescBuilder("exp_range")
+    n = 1 << 21
+    kernel = driver.HipKernel(b.dumps([b.unary("Exp", b.input([n], "float32"))]), out_dir=None)
+    rng = np.random.default_rng(11)
+    for low, high in ((-104.0, 88.722), (-1.0, 1.0), (-1e-5, 1e-5)):
+        x = rng.uniform(low, high, n).astype(np.float32)
+        special = np.float32([np.inf, -np.inf, np.nan, 88.72283, 88.72284, 100.5, 3e38, -104.0, -120.5, -3e38, 0.0, -0.0, 1e-45, -87.33655, -103.2])
+        x[:special.size] = special
+        got = _run(kernel, [x])[0]
+        with np.errstate(over="ignore", under="ignore"):
+            want = np.exp(x.astype(np.float64))
+            rounded = want.astype(np.float32)
+        finite = np.isfinite(rounded)
+        assert np.array_equal(got[~finite], rounded[~finite], equal_nan=True)
+        unit = np.maximum(np.spacing(np.abs(rounded[finite])).astype(np.float64), 2.0 ** -149)
+        assert (np.abs(got[finite].astype(np.float64) - want[finite]) / unit).max() <= 1.0
+
+
+def test_division_by_a_row_value_is_the_ieee_quotient():
+    """Zeros of both signs, subnormal and tiny dividends, infinities and NaN over positive, negative, tiny and huge divisors."""
+    rng = np.random.default_rng(12)
+    special = np.float32([0.0, -0.0, 1e-45, -1e-40, 1e-30, 2.0 ** -60, 2.0 ** -61, 2.0 ** 60, 2.0 ** 61, np.inf, -np.inf, np.nan, 3e38])
+    for divisors in (np.float32([3.0, -7.0, 1.0, 1e-3, 2.0 ** -60, 2.0 ** 60]), np.float32([1e-25, 1e30, np.inf, 0.0, -0.0, np.nan])):
+        x = (rng.standard_normal((6, 1030)) * 10.0 ** rng.uniform(-5, 5, (6, 1030))).astype(np.float32)
+        x[:, 5:5 + special.size] = special
+        x[:, 600:900] = 0.0
+        b = op_desc.DescBuilder("row_division")
+        t, d = b.input(list(x.shape), "float32"), b.input([6, 1], "float32")
+        kernel = driver.HipKernel(b.dumps([b.div(t, d)]), out_dir=None)
+        got = _run(kernel, [x, divisors.reshape(6, 1)])[0]
+        with np.errstate(all="ignore"):
+            want = x / divisors.reshape(6, 1)
+        same = (got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))
+        assert same.all(), np.argwhere(~same)[:5]
+
+
+def test_division_by_a_row_maximum_is_the_ieee_quotient():
+    """The row kernel's form: the divisor is a reduction, the dividends come in chunks."""
+    rng = np.random.default_rng(13)
+    x = np.abs(rng.standard_normal((33, 1030))).astype(np.float32)
+    x[:, ::3] = 0.0
+    x[7, 5:9] = np.float32([1e-40, -0.0, 1e-25, -3.0])
+    x[8] = 0.0
+    x[9, 4] = np.inf
+    b = op_desc.DescBuilder("row_by_maximum")
+    t = b.input(list(x.shape), "float32")
+    kernel = driver.HipKernel(b.dumps([b.div(t, b.reduce("ReduceMax", t, [1], True))]), out_dir=None)
+    assert kernel.family == "row_reduce"
+    got = _run(kernel, [x])[0]
+    with np.errstate(all="ignore"):
+        want = x / x.max(1, keepdims=True)
+    same = (got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))
+    assert same.all(), np.argwhere(~same)[:5]
+
+
+@pytest.mark.parametrize("cols", [257, 300, 383, 385, 509, 511, 1025, 1535, 2047])
+def test_rows_that_leave_out_chunks(cols):
+    """One code object for every length of the bucket; softmax with a shared mask against float64: relative error of the
+    exponential's argument (2^-24 * 130), of the exponential (2^-23) and of a sum of `cols` terms in trees of four."""
+    b = op_desc.DescBuilder("chunks_left_out")
+    mask, x = b.input([7777, 1, 7778], "float32"), b.input([7777, 5, 7778], "float32")
+    s = b.add(x, mask)
+    e = b.unary("Exp", b.sub(s, b.reduce("ReduceMax", s, [2], True)))
+    doc = json.loads(b.dumps([b.div(e, b.reduce("ReduceSum", e, [2], True))]))
+    text = json.dumps(doc).replace("7777", "-1").replace("7778", "-1")
+    kernel = driver.HipDynamicKernel(text, None).specialize([[3, 1, cols], [3, 5, cols]])
+    rng = np.random.default_rng(cols)
+    m = np.where(rng.random((3, 1, cols)) < 0.3, -10000.0, 0.0).astype(np.float32)
+    a = (rng.standard_normal((3, 5, cols)) * 4).astype(np.float32)
+    got = _run(kernel, [m, a])[0]
+    t = a.astype(np.float64) + m
+    want = np.exp(t - t.max(2, keepdims=True))
+    want /= want.sum(2, keepdims=True)
+    assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max() and (np.abs(got - want) <= 2e-5 * want + 1e-30).all()
