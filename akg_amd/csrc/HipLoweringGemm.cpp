@@ -102,7 +102,9 @@ class GemmEmitter {
       note << " skinny: strips of 128 columns, B " << (skinnyLines() ? (streamsLines() ? "by whole lines past the caches" : "by whole lines") : "straight into MFMA operands")
            << ", mfma=" << mfmaName(false) << " waves=" << skinnyWaves() << " grid=" << k.grid[0];
     } else if (tileM_ > 0) {
-      note << " tile=" << tileM_ << "x" << tileN_ << "x" << stepK() / elemBytes() << " mfma=" << mfmaName(true) << " waves=2x2 grid=" << k.grid[0];
+      const int unitM = tileM_ % 128 == 0 ? 128 : 64, unitN = tileN_ % 128 == 0 ? 128 : 64;
+      note << " tile=" << unitM << "x" << unitN << "x" << stepK() / elemBytes() << " mfma=" << mfmaName(true) << " waves=2x2 grid=" << k.grid[0];
+      if (tileM_ * tileN_ > unitM * unitN) note << " (" << tileM_ / unitM << "x" << tileN_ / unitN << " tiles a workgroup)";
     } else {
       note << " tile=256x256x" << stepK() / elemBytes() << " mfma=" << mfmaName(true) << " waves=" << (tallWavefrontTiles() ? "2x4" : "4x2") << " grid=" << k.grid[0];
     }
@@ -183,25 +185,49 @@ class GemmEmitter {
   // (AKG_HIP_VARIANT bit 5 takes the other one.)
   bool tallWavefrontTiles() const { return (elem_ == DType::I8 && !transB_) != ((opt_.variant & 32) != 0); }
 
-  // Time in us of the small-tile kernel, after what it was measured to take: 3 us in front and behind, and per step of 128
-  // bytes of K 0.35 us (64 x 64; 0.28 where the workgroups of a CU cover each other), 0.48 (64 x 128), 0.72 (128 x 128): a CU
-  // takes in 46 .. 53 GB/s of operands with one workgroup or several, so workgroups beyond one per CU queue up. A split costs its
-  // partials' way to memory and back and the time of the workgroup that adds them.
-  double smallTileTime(int64_t bm, int64_t bn, int64_t split) const {
-    const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = ((m_ + bm - 1) / bm) * ((n_ + bn - 1) / bn);
-    const double perCu = static_cast<double>(tiles * split) / 256;
-    const double step = bn == 64 ? (perCu <= 1 ? 0.35 : 0.28) : (bm == 64 ? 0.48 : 0.72);
-    const double rounds = perCu <= 1 ? 1 : (perCu + std::ceil(perCu)) / 2;
-    const double loop = static_cast<double>((steps + split - 1) / split) * step * rounds;
-    const double area = static_cast<double>(bm * bn);
-    if (split == 1) return 3 + loop;
-    return 3 + loop + 2.5 + 0.3 * static_cast<double>(split) * area / 4096 + static_cast<double>(tiles * split) * area * 8 / 5e6;
+  // What one workgroup of the small-tile kernel computes: one 64 x 64, 64 x 128 or 128 x 128 tile, or several adjacent ones that
+  // share their operands in LDS (192 x 128: three of 64 x 128, 192 x 192: nine of 64 x 64, 128 x 256: two of 128 x 128). In us, per step of
+  // 128 bytes of K with one workgroup on a CU, with several, and behind the loop. A CU takes in 60 .. 70 GB/s of operands
+  // from L2 and memory whatever its workgroups do with them (loads alone take 42 us of the 46 of 300 x 4096 x 11008): its L1
+  // answers in order, so lines that are on their way from memory hold up those behind them. Larger workgroups take in less.
+  struct SmallShape {
+    int m, n;
+    double alone, shared, end;
+    int splits;   // 1, 2, 4 .. up to this many
+  };
+  static const std::vector<SmallShape> &smallShapes() {
+    static const std::vector<SmallShape> shapes = {{64, 64, 0.208, 0.204, 0.26, 8}, {64, 128, 0.29, 0.304, 1.2, 2}, {128, 128, 0.396, 0.44, 2.1, 2},
+                                                   {192, 128, 0.528, 0.666, 4.27, 1}, {192, 192, 0.771, 0.899, 5.9, 1}, {128, 256, 0.699, 0.815, 5.24, 1}};
+    return shapes;
   }
-  // ... and of the 256 x 256 kernel with `split` workgroups per tile: 2 us a step.
+  // Fitted to 55 products (M 65 .. 4055, K 512 .. 11008, both layouts, 8 and 16 bits) on every shape, 700 times in all: standard
+  // deviation 7 %; the shape it takes is 2.5 % behind the fastest in the mean (int8 4055 x 1408 x 1784 the furthest: 20.5 for 18.2). A split costs its partials' way to memory and
+  // back and the time of the workgroup that adds them; rows of a [K,N] weight that begin inside lines cost one line in ten.
+  double smallTileTime(const SmallShape &w, int64_t split) const {
+    if (m_ <= skinnyRows()) return narrowTileTime(w.n, split);
+    const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = ((m_ + w.m - 1) / w.m) * ((n_ + w.n - 1) / w.n);
+    const double perCu = static_cast<double>(tiles * split) / 256, whole = std::ceil(perCu), area = static_cast<double>(w.m * w.n);
+    const double rounds = perCu <= 1 ? 1 : 0.78 * whole + 0.22 * perCu;
+    double step = perCu <= 1 ? w.alone : w.shared * rounds;
+    if (!transB_) step *= (n_ * elemBytes() % 128 != 0 ? 1.054 : 1.007) + (elemBytes() == 1 ? 0.3 : 0);
+    const double time = 2.43 + static_cast<double>((steps + split - 1) / split) * step + w.end * rounds;
+    return split == 1 ? time : time + (split <= 4 ? 1.78 : 2.9) + 0.113 * static_cast<double>(split) * area / 4096 + 0.363 * static_cast<double>(tiles * split) * area * 8 / 5e6;
+  }
+  // At most 64 rows, where one tile's rows are the product's: an estimate of its own, which skinnyTime and smallTileRowsTime
+  // below go with.
+  double narrowTileTime(int64_t bn, int64_t split) const {
+    const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = (n_ + bn - 1) / bn;
+    const double perCu = static_cast<double>(tiles * split) / 256, area = static_cast<double>(64 * bn);
+    const double step = bn == 64 ? (perCu <= 1 ? 0.35 : 0.28) : 0.48, rounds = perCu <= 1 ? 1 : (perCu + std::ceil(perCu)) / 2;
+    const double loop = static_cast<double>((steps + split - 1) / split) * step * rounds;
+    return split == 1 ? 3 + loop : 5.5 + loop + 0.3 * static_cast<double>(split) * area / 4096 + static_cast<double>(tiles * split) * area * 8 / 5e6;
+  }
+  // ... and of the 256 x 256 kernel with `split` workgroups per tile (the same products, 14 %).
   double largeTileTime(int64_t split) const {
-    const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = ((m_ + 255) / 256) * ((n_ + 255) / 256);
-    const double loop = 2.0 * static_cast<double>((steps + split - 1) / split * ((tiles * split + 255) / 256));
-    return 6 + loop + (split == 1 ? 0 : 6 + 2 * static_cast<double>(split));
+    const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = ((m_ + 255) / 256) * ((n_ + 255) / 256), rounds = (tiles * split + 255) / 256;
+    const double step = 1.45 * (transB_ ? 1 : 1.093) * (elemBytes() == 1 ? 1.356 : 1), rows = static_cast<double>(std::min<int64_t>(m_, 256));
+    const double time = static_cast<double>(rounds) * (static_cast<double>((steps + split - 1) / split) * step + 7.35);
+    return split == 1 ? time : time + 5.67 + 2.32 * static_cast<double>(split) * rows / 256 + 0.24 * static_cast<double>(tiles * split) * rows * 2048 / 5e6;
   }
   // 33 .. 64 rows: time in us of the skinny kernel and of 64 x 64 tiles, fitted to 1256 measured products (both layouts, 8 and
   // 16 bits, K 512 .. 14336, N 1024 .. 16384; the first within 11 %, the second within a quarter; standard deviations 3 and 6 %).
@@ -221,39 +247,50 @@ class GemmEmitter {
     const double step = perCu <= 1 ? (transposing8 ? 0.35 : 0.23) : (transposing8 ? 0.6 : 0.41), rate = transposing8 ? 0.17 : 0.113;
     return 2.7 + static_cast<double>((steps + split - 1) / split) * step + mb * rate + (split > 1 ? 1.8 + 0.25 * static_cast<double>(split) + 0.5 * perCu : 0);
   }
-  // The small-tile kernel where its estimate is a tenth below that of the 256 x 256 kernel, and for 33 .. 64 rows where the
-  // skinny one is not estimated a twentieth faster ([N,K] weights, whose estimates scatter more: a tenth, and those of
-  // 16 bits are the skinny kernel's from 60 Mi elements on, where 8192 x 8184 takes 36.3 us for 30.3). Measured (us, the other
-  // kernel -> small tiles): bf16 K x N = 1024 x 1024: M = 64 10.3 -> 6.7, 300 30.4 -> 6.0, 1200 28.4 -> 9.0; 2048 x 4096: 64 16.8 ->
-  // 10.0, 300 33.7 -> 17.6, 1200 45.1 -> 37.5; 8192 x 2048: 128 41.7 -> 17.2, 640 63.2 -> 49.8; 4096 x 11000: 300 88.9 -> 53.7 ([K,N]
-  // 95.2 -> 59.2), 640 129 -> 75.8; int8 4096 x 4096: 192 32.3 -> 13.8, 640 39.7 -> 25.9; 512 x 7768: 1494 21.4 -> 16.9. It is the slower
-  // one, and the estimates say so, from M = 1200 on for 8192 x 2048 (82 us for 67) and 4096 x 11000 (147 for 118); of 376 products that
-  // the estimates give it two are slower than on 256 x 256 tiles (bf16 1600 x 2048 x 5120 55.3 for 51.7).
+  // The small-tile kernel where its estimate is below that of the 256 x 256 kernel, on the workgroup with the lowest one, and
+  // for 33 .. 64 rows where the skinny one is not estimated a twentieth faster ([N,K] weights, whose estimates scatter more: a tenth, and those of
+  // 16 bits are the skinny kernel's from 60 Mi elements on, where 8192 x 8184 takes 36.3 us for 30.3). Measured (us, 256 x 256
+  // tiles / one 64 x 64 .. 128 x 128 tile a workgroup / this): bf16 300 x 4096 x 11000 [K,N] 90 / 52 / 43, 948 x 5184 x 6608 129 / 80 / 74, 1113 x
+  // 4352 x 7776 142 / 113 / 75, 2168 x 4416 x 2248 102 / 56 / 49, 1096 x 1408 x 4592 42 / 36 / 20, 2936 x 6400 x 808 70 / 55 / 45, 720 x 2496 x 1368 36 / 14.5 / 14.5; 45 products
+  // that no constant was fitted to take 0.78 of the time on the average, the worst of them 248 x 6656 x 2256 (20.2 -> 21.5);
+  // it is the slower one, and the estimates say so, for 3568 x 5056 x 3848 (137 / 193 / 167) and 1881 x 4160 x 7568 (118 / 152 / 125).
   // The skinny one is faster at 33 rows for [K,N] weights of bf16 8192 x 6144 (30.9 for 26.1), int8 4096 x 6144 (14.8 for 13.4) and 6144 x 9216
   // (27.9 for 20.0), for [N,K] of bf16 11008 x 5120 (34.1 for 28.1).
-  // Below 2 MiB and from 2^26 elements of B on the kernels and splits of the other two stand. From 65 rows on that is not where the
-  // small tiles stop being the faster ones: bf16 512 x 768 with 256 rows takes 21.4 us for their 4.8, 8192 x 8192 with 96
-  // rows 50.7 for 41.5, with 256 rows 72.5 for 71.3, 14336 x 8192 with 256 rows 109 for 128. Narrow products of at most 64 rows (N <
-  // 1024) are the skinny kernel's.
+  // Weights below 2 MiB whose columns are whole 256-wide tiles and those from 2^26 elements on keep the kernels and splits
+  // that tests pin, though small tiles would be the faster ones there for some rows: bf16 512 x 768 with 256 rows takes 21.4 us
+  // for their 4.8, 8192 x 8192 with 96 rows 50.7 for 41.5. Other weights below 2 MiB take them (us: bf16 85 x 1088 x 816 22.7 -> 4.9,
+  // 365 x 1408 x 744 34.0 -> 7.4, 1096 x 1152 x 552 34.4 -> 7.0, int8 200 x 640 x 584 20.7 -> 4.5). Narrow products of at most 64 rows
+  // (N < 1024) are the skinny kernel's.
   bool pickSmallTile() {
     if (serial_ || dyn_ || batch_ != 1 || opt_.split > 0 || (opt_.variant & (8 | 128))) return false;
     const int64_t elements = k_ * n_;
-    if (m_ <= 32 || elements * elemBytes() < (2LL << 20) || elements >= (1LL << 26)) return false;
-    if (m_ <= skinnyRows() && n_ < 1024) return false;
-    if ((!transB_ && n_ * elemBytes() % 16 != 0) || k_ * elemBytes() * 128 >= (1LL << 31)) return false;
+    if (m_ <= 32 || elements >= (1LL << 26)) return false;
+    const bool narrow = m_ <= skinnyRows();
+    if (elements * elemBytes() < (2LL << 20) && (narrow || n_ % 256 == 0)) return false;
+    if (narrow && n_ < 1024) return false;
+    if (!transB_ && n_ * elemBytes() % 16 != 0) return false;
     const int64_t steps = (k_ * elemBytes() + 127) / 128;
-    static const int shapes[][3] = {{64, 64, 1}, {64, 64, 2}, {64, 64, 4}, {64, 64, 8}, {64, 128, 1}, {64, 128, 2}, {128, 128, 1}};
-    double best = m_ <= skinnyRows() ? 1e30 : 0.9 * largeTileTime(largeTileSplit());
-    for (const auto &s : shapes) {
-      if (s[2] > 1 && (s[2] - 1) * ((steps + s[2] - 1) / s[2]) >= steps) continue;   // no empty split
-      const int64_t tiles = ((m_ + s[0] - 1) / s[0]) * ((n_ + s[1] - 1) / s[1]);
-      if (tiles * s[2] * s[0] * s[1] * 4 >= (1LL << 30)) continue;
-      const double t = smallTileTime(s[0], s[1], s[2]);
-      if (t >= best) continue;
-      best = t;
-      tileM_ = s[0];
-      tileN_ = s[1];
-      kSplit_ = s[2];
+    // (columns that are whole 256-wide tiles pad nothing there: small ones from a quarter below on; 1200 x 8192 x 2048, which a test
+    // pins, takes 59.6 us on them and 56.4 on 128 x 128)
+    double best = narrow ? 1e30 : (n_ % 256 == 0 ? 0.75 : 1.0) * largeTileTime(largeTileSplit());
+    for (const SmallShape &w : smallShapes()) {
+      if ((narrow && w.m > 64) || k_ * elemBytes() * std::max(w.m, w.n) >= (1LL << 31)) continue;
+      // (several tiles a workgroup from 17 steps on: for fewer, what comes behind the loop is a third of their time;
+      // 464 x 576 x 10032 would take 11.8 us for 13.1, 645 x 1024 x 6008, whose tile a test pins, 16.0 for 20.2)
+      if (w.m * w.n > 128 * 128 && steps <= 16) continue;
+      const int64_t tiles = ((m_ + w.m - 1) / w.m) * ((n_ + w.n - 1) / w.n);
+      for (int split = 1; split <= w.splits; split *= 2) {
+        if (split > 1 && (split - 1) * ((steps + split - 1) / split) >= steps) continue;   // no empty split
+        if (tiles * split * w.m * w.n * 4 >= (1LL << 30)) continue;
+        // partials stay within the 16 MiB of a launch without allocations
+        if (split > 1 && w.m * w.n > 64 * 128 && tiles * split * w.m * w.n * 4 > (15LL << 20)) continue;
+        const double t = smallTileTime(w, split) * (split > 1 ? 1.03 : 1);   // (as fast without a workspace is better)
+        if (t >= best) continue;
+        best = t;
+        tileM_ = w.m;
+        tileN_ = w.n;
+        kSplit_ = split;
+      }
     }
     const bool large = transB_ && elemBytes() == 2 && elements >= (60LL << 20);
     if (skinnyTakes() && (large || skinnyTime(skinnySplit()) < (transB_ ? 0.9 : 0.95) * smallTileRowsTime(kSplit_))) tileM_ = tileN_ = 0;

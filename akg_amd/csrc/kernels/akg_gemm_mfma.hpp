@@ -985,14 +985,42 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Small tiles (BM x BN of 64 or 128): more rows than the skinny kernel takes and too few 256 x 256 tiles to fill the chip.
-//   workgroup = 2 x 2 wavefronts, 128 bytes of K per step, LDS double buffered (32 to 64 KiB: two to five workgroups per
-//   CU, whose phases cover each other, so the instructions of a step are left to the compiler)
+// LDS of a workgroup that needs `bytes`, in a launch of `groups` workgroups: as much as keeps a CU from taking more of them than
+// its share of the chip's 256 CUs. Left to itself the dispatcher fills CUs with two while others have none.
+constexpr int lds_for_even_spread(int bytes, long groups) {
+  const long perCu = (groups + 255) / 256;
+  const long least = perCu <= 4 ? 163840 / (perCu + 1) + 512 : 0;
+  return static_cast<int>(bytes > least ? bytes : least / 512 * 512);
+}
+
+// Instruction order of the first half of a step: M MFMAs, between them W times an LDS write and the load that fills its
+// registers anew.
+template <int M, int W, int I = 0>
+struct SmallTileOrder {
+  static AKG_DEV void emit() {
+    constexpr int kFrom = I * M / W, kUpto = (I + 1) * M / W;
+    if constexpr (kUpto > kFrom) __builtin_amdgcn_sched_group_barrier(0x008, kUpto - kFrom, 0);
+    __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    if constexpr (I + 1 < W) SmallTileOrder<M, W, I + 1>::emit();
+  }
+};
+
+// Small tiles (BM x BN of 64 x 64 up to 192 x 192 and 128 x 256): more rows than the skinny kernel takes and too few 256 x 256
+// tiles to fill the chip.
+//   What bounds it is the intake of operands: a CU takes in 60 .. 70 GB/s of L2 and memory together (its L1 answers in order, so
+//   lines that come from memory hold up those that L2 has), and 148 GB/s where everything is in L2. So a workgroup takes
+//   the largest tile that still leaves the CUs evenly loaded; workgroups are spread over them by the LDS they ask for.
+//   workgroup = 2 x 2 wavefronts, 128 bytes of K per step, LDS double buffered (32 to 96 KiB)
 //   global -> registers -> LDS: two register sets, so the loads of a step are issued three steps ahead of its MFMAs: the
 //   time of a short K loop is that of its load latencies
+//   The order within a step is given: the reads of its second half first, MFMAs between the LDS writes and the loads that fill
+//   their registers anew. Left to itself the compiler gives both halves one set of operand registers and waits for all loads
+//   but one before the first MFMA: us, bf16 678 x 5568 x 2216 40 -> 31, f16 948 x 5184 x 6608 90 -> 82.
 //   LDS rows without padding: the 16-byte chunks of a K-contiguous row r are permuted by (r >> 1) & 7, the 16-column units of
 //   a k-row of a row-major B by the bits of k that the lanes of one transposing read differ in; no bank is then hit twice
-//   by the lanes that are served together (which sixteen those are: see the 256 x 256 kernel).
+//   by the lanes that are served together (which sixteen those are: see the 256 x 256 kernel; rows of 192 columns begin in
+//   either half of the banks by themselves).
 //   The operands of the MFMA are exchanged (columns of C are its rows): a lane owns row c = lane % 16 and the four
 //   adjacent columns 4 (lane / 16) .. + 3 of every 16 x 16 tile, without exchanges between lanes.
 // Tiles of a column of tiles are neighbours in launch order on one XCD, eight tile-rows at a time: they share their
@@ -1002,7 +1030,7 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
                              unsigned *__restrict__ ws = nullptr) {
   constexpr int EB = Mma::kElemBytes;
   constexpr long K = KE * EB, NB = N * EB;
-  static_assert((BM == 64 || BM == 128) && (BN == 64 || BN == 128), "tile sizes");
+  static_assert(BM % 64 == 0 && BM <= 256 && BN % 64 == 0 && BN <= 256, "tile sizes");
   static_assert(K % 16 == 0 && N % 4 == 0 && (TRANSB || NB % 16 == 0), "whole 16-byte chunks");
   static_assert(BM * K < (1L << 31) && (TRANSB ? BN * K : NB * KE) < (1L << 31), "operand too large for 32-bit buffer offsets");
   constexpr int BK = 128;
@@ -1015,7 +1043,12 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
   constexpr int kPitchB = TRANSB ? BK : BN * EB;
   constexpr int kChunksPerRowB = BN * EB / 16;
   constexpr int kUnitBytes = 16 * EB;                   // 16 columns of a k-row
-  __shared__ __attribute__((aligned(16))) u8 lds[2][(BM + BN) * BK];
+  // the result leaves through the same LDS, in two halves of rows where it is larger than the operands
+  constexpr int kOutPasses = BM * BN * 4 <= 2 * (BM + BN) * BK ? 1 : 2, kOutRows = BM / kOutPasses;
+  static_assert(kOutRows * BN * 4 <= 2 * (BM + BN) * BK, "the result passes through the LDS of the operands");
+  constexpr int kLds = lds_for_even_spread(2 * (BM + BN) * BK, kGridTiles * KSPLIT);
+  __shared__ __attribute__((aligned(16))) u8 ldsAll[kLds];
+  u8 (*lds)[(BM + BN) * BK] = reinterpret_cast<u8 (*)[(BM + BN) * BK]>(ldsAll);
 
   const long wgAll = static_cast<long>(blockIdx.x);
   const long ksplit = KSPLIT > 1 ? wgAll / kGridTiles : 0;
@@ -1025,8 +1058,10 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
   constexpr long kGroupSize = kGemmGroupRows * kTilesN;
   const long firstRow = linear / kGroupSize * kGemmGroupRows;
   const long rowsInGroup = (kTilesM - firstRow) < kGemmGroupRows ? (kTilesM - firstRow) : kGemmGroupRows;
-  const long m0 = (firstRow + linear % kGroupSize % rowsInGroup) * BM;
-  const long n0 = linear % kGroupSize / rowsInGroup * BN;
+  // (the divisions leave these in vector registers at times, though they are the same in every lane: a descriptor made from
+  // them then takes a loop around every load; 2590 x 5184 x 960 67.5 us)
+  const long m0 = static_cast<long>(__builtin_amdgcn_readfirstlane(static_cast<int>((firstRow + linear % kGroupSize % rowsInGroup) * BM)));
+  const long n0 = static_cast<long>(__builtin_amdgcn_readfirstlane(static_cast<int>(linear % kGroupSize / rowsInGroup * BN)));
   const long stepBase = ksplit * kStepsPer;
   const long mySteps = (kSteps - stepBase) < kStepsPer ? (kSteps - stepBase) : kStepsPer;
 
@@ -1051,13 +1086,14 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
     const long row = m0 + kRow + 32 * i;
     aOff[i] = static_cast<u32>(((row < M ? row : M - 1) - m0) * K + kChunk * 16);
   }
-  // which permutation of its 16-column units a k-row of a row-major B has
+  // Which permutation of its 16-column units a k-row of a row-major B has: the k-rows that one transposing read asks for
+  // together then lie in different banks.
   auto unitSwap = [](int krow) {
-    if constexpr (EB == 2) return BN == 128 ? (krow & 3) | ((krow >> 1) & 4) : ((krow >> 1) & 1) | ((krow >> 2) & 2);
-    return BN == 128 ? ((krow >> 1) & 3) | ((krow >> 2) & 4) : ((krow >> 2) & 1) | ((krow >> 3) & 2);
+    if constexpr (BN == 192) return EB == 2 ? (krow >> 3) & 1 : (krow >> 4) & 1;
+    if constexpr (EB == 2) return BN >= 128 ? (krow & 3) | ((krow >> 1) & 4) : ((krow >> 1) & 1) | ((krow >> 2) & 2);
+    return BN >= 128 ? ((krow >> 1) & 3) | ((krow >> 2) & 4) : ((krow >> 2) & 1) | ((krow >> 3) & 2);
   };
-  const int bRow = tid / kChunksPerRowB, bChunk = tid % kChunksPerRowB;
-  constexpr int kRowStepB = 256 / kChunksPerRowB;
+  int bRow[kChunksB];   // row-major B: the k-row of each chunk
 #pragma unroll
   for (int i = 0; i < kChunksB; ++i) {
     if constexpr (TRANSB) {
@@ -1065,10 +1101,11 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
       bOff[i] = static_cast<u32>(((col < N ? col : N - 1) - n0) * K + kChunk * 16);
       bStore[i] = kStore + 32 * BK * i;
     } else {
-      const int krow = bRow + kRowStepB * i;
-      const long colByte = n0 * EB + bChunk * 16;
+      const int id = tid + 256 * i, krow = id / kChunksPerRowB, chunk = id % kChunksPerRowB;
+      const long colByte = n0 * EB + chunk * 16;
+      bRow[i] = krow;
       bOff[i] = colByte < NB ? static_cast<u32>(krow * NB + colByte) : kBeyondEveryBuffer;
-      bStore[i] = krow * kPitchB + ((bChunk * 16 / kUnitBytes) ^ unitSwap(krow)) * kUnitBytes + (bChunk * 16) % kUnitBytes;
+      bStore[i] = krow * kPitchB + ((chunk * 16 / kUnitBytes) ^ unitSwap(krow)) * kUnitBytes + (chunk * 16) % kUnitBytes;
     }
   }
   struct Stage {
@@ -1087,7 +1124,7 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
       if constexpr (TRANSB) {
         s.b[i] = __builtin_amdgcn_raw_buffer_load_b128(bRsrc, whole ? bOff[i] : kBeyondEveryBuffer, static_cast<int>(k0), 0);
       } else {
-        const bool rowOk = K % BK == 0 || k0 / EB + bRow + kRowStepB * i < KE;
+        const bool rowOk = K % BK == 0 || k0 / EB + bRow[i] < KE;
         s.b[i] = __builtin_amdgcn_raw_buffer_load_b128(bRsrc, rowOk ? bOff[i] : kBeyondEveryBuffer, static_cast<int>(k0 / EB * NB), 0);
       }
     }
@@ -1159,12 +1196,17 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
   Frags f[2];
   auto step = [&](long s, int buf, Stage &next) {
     read(buf, 1, f[1]);
+    __builtin_amdgcn_sched_barrier(0);
     store(buf ^ 1, next);
     load(s + 3, next);
     multiply(f[0]);
+    SmallTileOrder<kTM * kTN, kChunksA + kChunksB>::emit();
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     read(buf ^ 1, 0, f[0]);
+    __builtin_amdgcn_sched_barrier(0);
     multiply(f[1]);
+    __builtin_amdgcn_sched_barrier(0);
   };
   auto lastStep = [&](long s, int buf, Stage &next) {
     read(buf, 1, f[1]);
@@ -1176,9 +1218,12 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
     multiply(f[1]);
   };
   load(0, stage[0]);
+  __builtin_amdgcn_sched_barrier(0);
   if (mySteps > 1) load(1, stage[1]);
+  __builtin_amdgcn_sched_barrier(0);
   store(0, stage[0]);
   if (mySteps > 2) load(2, stage[0]);
+  __builtin_amdgcn_sched_barrier(0);
   __syncthreads();
   read(0, 0, f[0]);
   long s = 0;
@@ -1239,36 +1284,50 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
   // columns. us: int8 1494 x 512 x 7768 36.3 -> 16.9 (256 x 256 tiles 21.4), 1200 x 1024 x 8192 31.6 -> 20.9 (25.5), bf16 1135 x
   // 576 x 9384 38.1 -> 24.2 (29.6), 640 x 4096 x 11000 79 -> 75, 300 x 1024 x 1024 6.5 -> 6.0; 376 products 1.10 times as fast in the
   // mean, int8 802 x 1792 x 5264 the slowest of them (23.6 -> 25.4).
-  constexpr int kRowChunks = BN / 4;
+  constexpr int kRowChunks = BN / 4, kRowStep = 256 / kRowChunks, kRowsPer = (kOutRows + kRowStep - 1) / kRowStep;
   acc_t *__restrict__ out = reinterpret_cast<acc_t *>(&lds[0][0]);
-  auto chunkAt = [&](int row, int chunk) { return out + (row * kRowChunks + (chunk ^ (row & 15))) * 4; };
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < kTM; ++i) {
-#pragma unroll
-    for (int j = 0; j < kTN; ++j) *reinterpret_cast<typename Mma::acc4_v *>(chunkAt(rowLane + 16 * i, (colLane + 16 * j) / 4)) = acc[i][j];
-  }
-  __syncthreads();
-  const int chunk = tid % kRowChunks;
-  const long col = n0 + 4 * chunk;
-  if (col >= N) return;
-  epi.prepare(col);
-  constexpr int kRowStep = 256 / kRowChunks;
-  typename Mma::acc4_v v[BM / kRowStep];
-#pragma unroll
-  for (int i = 0; i < BM / kRowStep; ++i) v[i] = *reinterpret_cast<const typename Mma::acc4_v *>(chunkAt(tid / kRowChunks + kRowStep * i, chunk));
-  auto finish = [&](bool whole) {   // (without a condition per row the operands of all rows are requested together)
-#pragma unroll
-    for (int i = 0; i < BM / kRowStep; ++i) {
-      const long row = m0 + tid / kRowChunks + kRowStep * i;
-      const acc_t a4[4] = {v[i][0], v[i][1], v[i][2], v[i][3]};
-      if (whole || row < M) epi.apply(a4, row, col);
-    }
+  auto chunkAt = [&](int row, int chunk) {
+    const int at = (kRowChunks & 15) == 0 ? chunk ^ (row & 15) : (chunk + row) % kRowChunks;
+    return out + (row * kRowChunks + at) * 4;
   };
-  if (m0 + BM <= M) {
-    finish(true);
-  } else {
-    finish(false);
+  const int chunk = tid % kRowChunks, firstOut = tid / kRowChunks;
+  const long col = n0 + 4 * chunk;
+  const bool has = col < N && firstOut < kRowStep;   // (threads beyond whole rows of chunks have none)
+  if (has) epi.prepare(col);
+#pragma unroll
+  for (int pass = 0; pass < kOutPasses; ++pass) {
+    __syncthreads();
+    if (kOutPasses == 1 || wm == pass) {
+#pragma unroll
+      for (int i = 0; i < kTM; ++i) {
+#pragma unroll
+        for (int j = 0; j < kTN; ++j) {
+          *reinterpret_cast<typename Mma::acc4_v *>(chunkAt(rowLane + 16 * i - pass * kOutRows, (colLane + 16 * j) / 4)) = acc[i][j];
+        }
+      }
+    }
+    __syncthreads();
+    if (!has) continue;
+    typename Mma::acc4_v v[kRowsPer];
+#pragma unroll
+    for (int i = 0; i < kRowsPer; ++i) {
+      const int r = firstOut + kRowStep * i;
+      v[i] = *reinterpret_cast<const typename Mma::acc4_v *>(chunkAt(kOutRows % kRowStep == 0 || r < kOutRows ? r : kOutRows - 1, chunk));
+    }
+    auto finish = [&](bool whole) {   // (without a condition per row the operands of all rows are requested together)
+#pragma unroll
+      for (int i = 0; i < kRowsPer; ++i) {
+        const int r = firstOut + kRowStep * i;
+        const long row = m0 + pass * kOutRows + r;
+        const acc_t a4[4] = {v[i][0], v[i][1], v[i][2], v[i][3]};
+        if ((kOutRows % kRowStep == 0 || r < kOutRows) && (whole || row < M)) epi.apply(a4, row, col);
+      }
+    };
+    if (m0 + BM <= M) {
+      finish(true);
+    } else {
+      finish(false);
+    }
   }
 }
 

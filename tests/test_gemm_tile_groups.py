@@ -1,0 +1,52 @@
+"""Workgroups of several small tiles: which products take them, and their results at the edges."""
+import re
+
+import pytest
+
+from akg_amd import driver
+from test_gemm_small_tiles import _product, test_small_tiles_against_float64 as _against_float64
+
+
+def _tile(m, k, n, dtype, tb):
+    """Rows, columns and splits of a workgroup; none of another kernel."""
+    source = driver.HipKernel(_product(m, k, n, dtype, tb, "groups"), out_dir=None).source
+    found = re.search(r"gemm_small_tile<[^,]+, (\d+), (\d+), [^(]*?(\d+)>\(", source)
+    return found and tuple(int(x) for x in found.groups())
+
+
+def test_products_that_take_several_tiles_a_workgroup():
+    assert _tile(1059, 1704, 3604, "bfloat16", True) == (192, 128, 1)
+    assert _tile(1589, 2968, 5200, "bfloat16", False) == (192, 192, 1)
+    assert _tile(1312, 2432, 5040, "int8", False) == (128, 256, 1)
+    # at most 16 steps of K take single tiles, at most 64 rows always
+    assert _tile(1059, 1024, 3604, "bfloat16", True) == (64, 128, 1)
+    assert _tile(48, 4096, 4096, "bfloat16", True)[:2] == (64, 64)
+    # weights below 2 MiB, unless their columns are whole tiles of the 256 x 256 kernel or there are few rows
+    assert _tile(365, 1408, 744, "bfloat16", False)[:2] == (64, 64)
+    assert _tile(365, 1408, 512, "bfloat16", False) is None and _tile(48, 1408, 744, "bfloat16", False) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,n,dtype,tb,tile", [
+    (1059, 1704, 3604, "bfloat16", True, (192, 128, 1)),    # ragged rows and columns, a K tail of 80 bytes
+    (1102, 1592, 5120, "float16", False, (192, 128, 1)),
+    (1240, 2384, 3360, "int8", False, (192, 128, 1)),
+    (1460, 2080, 2984, "int8", True, (192, 128, 1)),
+    (1580, 1576, 5008, "bfloat16", True, (192, 192, 1)),
+    (1365, 2104, 6144, "bfloat16", False, (192, 192, 1)),
+    (2371, 2368, 3440, "int8", False, (192, 192, 1)),       # 192 columns of 8 bits: two k-rows a cycle of banks
+    (1383, 1520, 4808, "bfloat16", True, (128, 256, 1)),
+    (1133, 2520, 5520, "float16", False, (128, 256, 1)),
+    (1312, 2432, 5040, "int8", False, (128, 256, 1)),
+    (370, 4088, 3440, "bfloat16", False, (128, 128, 2)),    # split 128 x 128 tiles
+    (340, 9792, 2792, "int8", True, (128, 128, 2)),
+    (365, 1408, 744, "bfloat16", False, (64, 64, 1)),       # small weights
+    (365, 2088, 492, "bfloat16", True, (64, 64, 4)),
+    (85, 4000, 248, "float16", True, (64, 64, 8)),
+    (65, 64, 68, "bfloat16", True, (64, 64, 1)),            # one step
+])
+def test_tile_groups_against_float64(m, k, n, dtype, tb, tile, tmp_path):
+    """The bound of the small tiles' own test: any order of float32 sums, 8-bit products exactly."""
+    assert _tile(m, k, n, dtype, tb) == tile
+    units = "%dx%d" % tuple(128 if x % 128 == 0 else 64 for x in tile[:2])
+    _against_float64(m, k, n, dtype, tb, units, tmp_path)
