@@ -27,7 +27,7 @@ namespace akg {
 
 namespace {
 
-// The shapes both schedules need.
+// The shapes all schedules need.
 struct SegmentShapes {
   const OpNode *op = nullptr;
   const TensorValue *data = nullptr, *ids = nullptr, *out = nullptr;
@@ -1257,6 +1257,301 @@ LoweredKernel lowerSegmentScan(const OpGraph &g, const LoweringOptions &options,
   return k;
 }
 
+// Wide rows and at most 2^16 positions, as gradients of embedding tables have: one launch without a workspace. Workgroup (g, t)
+// sums the segments congruent to g modulo GROUPS in column tile t, one column a thread:
+//   it counts its positions per segment, lists them by segment and in their order (LDS), and walks the list with 64 rows in flight,
+//   whatever segments they belong to.
+// Frequent ids are often neighbours (tokens by rank), so neighbouring segments go to different workgroups, and a workgroup's
+// columns are at most 256. More positions than the list holds: by windows of the positions, the sums wait in the result
+// between them.
+// What bounds it is the chain of a frequent segment's rows where there is one (16000 x 128 into 1000: 1600 rows, 69 us, 40 ns a
+// row with 64 in flight; 112 us where the waits were for all 64) and two scans of the ids by every workgroup where there is none.
+// 1024 workgroups: 512 and 2048 take 98 and 102 us for 89 (32768 x 1024 into 32768, uniform ids). All tiles of a group on one CU,
+// as they were launched, took 225 us for 124 (ids as frequent as words).
+struct ListedPlan {
+  int64_t tiles = 0, block = 0, groupBits = 0, keys = 0;
+  bool possible = false;
+};
+
+ListedPlan planListed(const SegmentShapes &sh, const LoweringOptions &options) {
+  ListedPlan plan;
+  if (sh.slice <= 64 || sh.positions > (1 << 20) || options.block > 0) return plan;
+  plan.tiles = (sh.slice + 255) / 256;
+  plan.block = ((sh.slice + plan.tiles - 1) / plan.tiles + 63) / 64 * 64;
+  plan.tiles = (sh.slice + plan.block - 1) / plan.block;
+  const int64_t want = options.split > 0 ? options.split : 1024;
+  while (plan.groupBits < 24 && (1LL << plan.groupBits) * plan.tiles < want && (1LL << plan.groupBits) < sh.segments) ++plan.groupBits;
+  while (((sh.segments + (1LL << plan.groupBits) - 1) >> plan.groupBits) > 512) ++plan.groupBits;
+  plan.keys = (sh.segments + (1LL << plan.groupBits) - 1) >> plan.groupBits;
+  plan.possible = plan.tiles < 65536;
+  return plan;
+}
+
+LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, const ListedPlan &plan) {
+  using lowering::computeTypeName;
+  using lowering::dtypeTag;
+  const TensorValue &ids = *sh.ids, &out = *sh.out;
+  const std::string ct = computeTypeName(out.dtype), tag = dtypeTag(out.dtype), idTag = dtypeTag(ids.dtype);
+  const bool narrow = out.dtype == DType::F16 || out.dtype == DType::BF16 || out.dtype == DType::I8 || out.dtype == DType::I16;
+  std::ostringstream s;
+  s << "// Generated by the akg HIP lowering for gfx950. Op description: " << g.name << "\n";
+  s << "// family: segment_sum (positions listed by segment), fusion class: " << operatorTemplateName(g.operatorTemplate) << "\n";
+  s << "#include \"akg_rt.hpp\"\n\n";
+  s << "extern \"C\" __global__ __launch_bounds__(" << plan.block << ") void " << g.name << "_kernel(";
+  for (size_t i = 0; i < g.inputs.size(); ++i) {
+    s << (i ? ", " : "") << "const " << dtypeTag(g.tensor(g.inputs[i]).dtype) << "::storage *__restrict__ in" << i;
+  }
+  s << ", " << tag << "::storage *__restrict__ out0) {\n";
+  s << "  constexpr int POSITIONS = " << sh.positions << ", SEGMENTS = " << sh.segments << ", BLOCK = " << plan.block << ", NW = BLOCK / 64;\n";
+  s << "  constexpr int BITS = " << plan.groupBits << ", GROUPS = 1 << BITS, KEYS = " << plan.keys << ", LIST = 4096;\n";
+  s << "  constexpr int IDV = " << (ids.dtype == DType::I32 ? 4 : ids.dtype == DType::I64 ? 2 : 1) << ", U = 8;\n";
+  s << "  constexpr long SLICE = " << sh.slice << ";\n";
+  s << "  using id_t = " << idTag << "::storage;\n";
+  s << "  using T = " << tag << ";\n  using ID = " << idTag << ";\n";
+  s << "  using acc_t = " << ct << ";\n";
+  s << "  const id_t *__restrict__ ids = in" << ids.inputIndex << ";\n";
+  s << "  const T::storage *__restrict__ data = in" << sh.data->inputIndex << ";\n";
+  s << "  const acc_t zero = " << lowering::literalFor(out.dtype, 0.0) << ";\n";
+  // ids as int: anything outside [0, SEGMENTS) is nobody's
+  s << "  const auto as_int = " << (ids.dtype == DType::I64 ? "[](long v) { return v < 0 || v >= SEGMENTS ? -1 : static_cast<int>(v); }"
+                                                            : "[](int v) { return v; }") << ";\n";
+  s << "  const auto add = [](acc_t v, acc_t acc) -> acc_t { return " << (narrow ? "T::rnd(" : "(") << "akg::op_add(v, acc)); };\n";
+  s << R"(  struct __attribute__((aligned(sizeof(id_t) * IDV))) id_chunk { id_t v[IDV]; };
+  __shared__ unsigned akg_count[NW * KEYS];   // [wavefront][key]: its positions, then where it lists the next one
+  __shared__ unsigned akg_has[KEYS], akg_total;
+  __shared__ unsigned akg_list[LIST];         // key << 20 | position, by key
+  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // (the tiles of a group, of which all may be long, on different XCDs and CUs)
+  const int group = static_cast<int>(blockIdx.x + 37 * blockIdx.y) & (GROUPS - 1);
+  const long col = static_cast<long>(blockIdx.y) * BLOCK + tid;
+  const bool has = col < SLICE;
+  const unsigned from_col = static_cast<unsigned>(has ? col : SLICE - 1);
+  const auto mine = [&](int id) { return static_cast<unsigned>(id) < static_cast<unsigned>(SEGMENTS) && (id & (GROUPS - 1)) == group; };
+  // ids that fit are loaded once
+  constexpr bool ONCE = POSITIONS <= LIST && POSITIONS <= NW * 64 * IDV * U;
+  id_chunk chunk[U];
+  const auto load = [&](int base) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = base + (u * 64 + lane) * IDV;
+      if constexpr (POSITIONS % IDV == 0) {
+        chunk[u] = *reinterpret_cast<const id_chunk *>(ids + (p < POSITIONS ? p : 0));
+      } else if (p + IDV <= POSITIONS) {
+        chunk[u] = *reinterpret_cast<const id_chunk *>(ids + p);
+      } else {
+#pragma unroll
+        for (int e = 0; e < IDV; ++e) {
+          if (p + e < POSITIONS) chunk[u].v[e] = ids[p + e];
+        }
+      }
+    }
+  };
+  constexpr int SHARE = (POSITIONS + NW * 64 * IDV - 1) / (NW * 64 * IDV) * (64 * IDV);
+  if (ONCE) load(wave * SHARE);
+  // the ids of positions [from, upto), a contiguous share per wavefront, 64 * IDV at a time in ascending order
+  const auto scan = [&](int from, int upto, auto &&visit) {
+    const int share = (upto - from + NW * 64 * IDV - 1) / (NW * 64 * IDV) * (64 * IDV);
+    const int first = from + wave * share, end = first + share < upto ? first + share : upto;
+    for (int base = first; base < end; base += 64 * IDV * U) {
+      if (!ONCE) load(base);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int p = base + (u * 64 + lane) * IDV;
+        int key[IDV];
+        bool any = false;
+#pragma unroll
+        for (int e = 0; e < IDV; ++e) {
+          const int id = p + e < end ? as_int(ID::load(chunk[u].v[e])) : -1;
+          key[e] = mine(id) ? id >> BITS : -1;
+          any = any || key[e] >= 0;
+        }
+        if (__ballot(any) != 0) visit(p, key);
+      }
+    }
+  };
+  const auto count = [&](int from, int upto) {
+    for (int k = tid; k < NW * KEYS; k += BLOCK) akg_count[k] = 0;
+    __syncthreads();
+    scan(from, upto, [&](int, const int (&key)[IDV]) {
+#pragma unroll
+      for (int e = 0; e < IDV; ++e) {
+        if (key[e] >= 0) atomicAdd(&akg_count[wave * KEYS + key[e]], 1u);
+      }
+    });
+    __syncthreads();
+    if (wave == 0) {
+      unsigned run = 0;
+      for (int k0 = 0; k0 < KEYS; k0 += 64) {
+        const int k = k0 + lane;
+        unsigned c[NW], sum = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          c[w] = k < KEYS ? akg_count[w * KEYS + k] : 0;
+          sum += c[w];
+        }
+        unsigned upto_here = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const unsigned below = __shfl_up(upto_here, d);
+          if (lane >= d) upto_here += below;
+        }
+        unsigned at = run + upto_here - sum;
+        if (k < KEYS) {
+          akg_has[k] = sum;
+#pragma unroll
+          for (int w = 0; w < NW; ++w) {
+            akg_count[w * KEYS + k] = at;
+            at += c[w];
+          }
+        }
+        run += __builtin_amdgcn_readlane(upto_here, 63);
+      }
+      if (lane == 0) akg_total = run;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(static_cast<int>(akg_total));
+  };
+  const auto place = [&](int from, int upto) {
+    scan(from, upto, [&](int p, int (&key)[IDV]) {
+      for (;;) {   // one key at a time; its positions go up with the lanes, then with the elements
+        int pick = -1;
+#pragma unroll
+        for (int e = 0; e < IDV; ++e) pick = key[e] >= 0 ? key[e] : pick;
+        const unsigned long long left = __ballot(pick >= 0);
+        if (left == 0) break;
+        const int one = __builtin_ctzll(left), k = __builtin_amdgcn_readlane(pick, one);
+        unsigned before = 0, all = 0;
+#pragma unroll
+        for (int e = 0; e < IDV; ++e) {
+          const unsigned long long same = __ballot(key[e] == k);
+          before += __builtin_popcountll(same & ((1ULL << lane) - 1));
+          all += __builtin_popcountll(same);
+        }
+        unsigned at = 0;
+        if (lane == one) at = atomicAdd(&akg_count[wave * KEYS + k], all);
+        at = __builtin_amdgcn_readlane(at, one) + before;
+#pragma unroll
+        for (int e = 0; e < IDV; ++e) {
+          if (key[e] == k) {
+            akg_list[at++] = static_cast<unsigned>(k) << 20 | static_cast<unsigned>(p + e);
+            key[e] = -1;
+          }
+        }
+      }
+    });
+    __syncthreads();
+  };
+  const auto row_of = [&](int k) { return (static_cast<long>(k) << BITS | group) * SLICE + from_col; };
+  struct AllAtOnce { enum { kGoesOn = 0 }; };
+  struct ByWindows { enum { kGoesOn = 1 }; };
+  const auto sum = [&](int n, auto how) {
+    int current = -1;
+    acc_t acc = zero, v[64];
+    const auto fetch = [&](int q, unsigned entries) {   // eight rows of a chunk of 64 entries
+#pragma unroll
+      for (int u = q; u < q + 8; ++u) {
+        const unsigned p = __builtin_amdgcn_readlane(entries, u) & 0xfffffu;
+        v[u] = T::load((data + static_cast<long>(p) * SLICE)[from_col]);
+      }
+    };
+    const auto fold = [&](int q, unsigned entries, int left) {
+      // (the list ascends: the last of eight in the current segment, all are)
+      if (static_cast<int>(__builtin_amdgcn_readlane(entries, q + 7) >> 20) == current && q + 8 <= left) {
+#pragma unroll
+        for (int u = q; u < q + 8; ++u) acc = add(v[u], acc);
+        return;
+      }
+#pragma unroll
+      for (int u = q; u < q + 8; ++u) {
+        if (u >= left) continue;
+        const int k = static_cast<int>(__builtin_amdgcn_readlane(entries, u) >> 20);
+        if (k != current) {
+          if (current >= 0 && has) out0[row_of(current)] = T::store(acc);
+          current = k;
+          acc = zero;
+          if constexpr (decltype(how)::kGoesOn) acc = T::load(out0[row_of(k)]);
+        }
+        acc = add(v[u], acc);
+      }
+    };
+    const auto entries_at = [&](int i) { return akg_list[i + lane < n ? i + lane : n - 1]; };
+    unsigned entries = entries_at(0);
+    int i = 0;
+    if (n >= 128) {
+      // eight rows are summed, the eight 64 behind them requested; no load is conditional, or the waits would be for all of them
+#pragma unroll
+      for (int q = 0; q < 64; q += 8) fetch(q, entries);
+      for (; i + 128 <= n; i += 64) {
+        const unsigned next = entries_at(i + 64);
+#pragma unroll
+        for (int q = 0; q < 64; q += 8) {
+          fold(q, entries, 64);
+          fetch(q, next);
+        }
+        entries = next;
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 64; q += 8) {
+        if (q < n) fetch(q, entries);   // (entries beyond the list repeat its last one)
+      }
+    }
+    for (; i < n; i += 64) {
+      const unsigned next = entries_at(i + 64);
+#pragma unroll
+      for (int q = 0; q < 64; q += 8) {
+        if (i + q < n) fold(q, entries, n - i);
+        if (i + 64 + q < n) fetch(q, next);
+      }
+      entries = next;
+    }
+    if (has) out0[row_of(current)] = T::store(acc);
+  };
+  // zeros for the segments without positions, or for all
+  const auto clear = [&](bool all) {
+    for (int k0 = 0; k0 < KEYS; k0 += 64) {
+      const int k = k0 + lane;
+      unsigned long long empty = __ballot(k < KEYS && (static_cast<long>(k) << BITS | group) < SEGMENTS && (all || akg_has[k] == 0));
+      while (empty) {
+        if (has) out0[row_of(k0 + __builtin_ctzll(empty))] = T::store(zero);
+        empty &= empty - 1;
+      }
+    }
+  };
+  const int n = count(0, POSITIONS);
+  if (POSITIONS <= LIST || n <= LIST) {
+    clear(false);
+    place(0, POSITIONS);
+    if (n > 0) sum(n, AllAtOnce());
+    return;
+  }
+  clear(true);
+  for (int from = 0; from < POSITIONS; from += LIST) {
+    const int upto = from + LIST < POSITIONS ? from + LIST : POSITIONS;
+    const int here = count(from, upto);
+    place(from, upto);
+    if (here > 0) sum(here, ByWindows());
+    __syncthreads();
+  }
+}
+)";
+
+  LoweredKernel k;
+  k.kernelName = g.name + "_kernel";
+  k.source = s.str();
+  k.family = KernelFamily::SegmentSum;
+  k.grid[0] = static_cast<unsigned>(1LL << plan.groupBits);
+  k.grid[1] = static_cast<unsigned>(plan.tiles);
+  k.block[0] = static_cast<unsigned>(plan.block);
+  k.algorithmicBytes = lowering::countAlgorithmicBytes(g);
+  k.shapeArgs = lowering::buildShapeArgs(g);
+  std::ostringstream note;
+  note << "segment_sum positions=" << sh.positions << " segments=" << sh.segments << " slice=" << sh.slice << " positions listed by segment: "
+       << plan.keys << " segments/workgroup, column tiles=" << plan.tiles << " of " << plan.block;
+  k.scheduleNote = note.str();
+  return k;
+}
+
 }  // namespace
 
 LoweredKernel lowerSegmentSumToHip(const OpGraph &g, const LoweringOptions &options) {
@@ -1265,7 +1560,7 @@ LoweredKernel lowerSegmentSumToHip(const OpGraph &g, const LoweringOptions &opti
   // (69 thousand positions into 4954 segments: 0.050 ms grouped, 0.069 ms scanned). Its LDS counters
   // hold one word per segment.
   const bool canGroup = sh.segments <= 16384 && sh.segments * sh.slice + 256 < (1LL << 31);
-  const bool group = options.variant >= 2 ? canGroup : options.variant == 1 ? false : canGroup && sh.positions >= (1 << 16);
+  const bool group = options.variant == 5 ? false : options.variant >= 2 ? canGroup : options.variant == 1 ? false : canGroup && sh.positions >= (1 << 16);
   // Short rows (4, 8 or 12 bytes, 4-byte arithmetic) into many segments: by bucket first. The bucket is the largest power
   // of two of segments whose output elements number at most 32; there are at most 640 buckets (the counters of a chunk
   // must leave room for two workgroups per CU) and, unless asked for, at least 96 (the last launch has one workgroup
@@ -1298,7 +1593,15 @@ LoweredKernel lowerSegmentSumToHip(const OpGraph &g, const LoweringOptions &opti
   }
   if (byChunk) return lowerSegmentChunked(g, options, sh, chunked);
   if (bucketed) return lowerSegmentBucketed(g, options, sh, bucketBits);
-  return group ? lowerSegmentSorted(g, options, sh) : lowerSegmentScan(g, options, sh);
+  if (group) return lowerSegmentSorted(g, options, sh);
+  // Wide rows listed by segment. us, ids as frequent as words (the k-th with 1 / k) and uniform ones, scanned -> listed: 32768 x 1024
+  // into 32768 11600 -> 124 and 199 -> 89, 20000 x 768 into 30522 6020 -> 97 and 98 -> 62, 8192 x 256 into 8000 735 -> 28 and
+  // 17.5 -> 12.4, 2048 x 1024 into 32000 802 -> 38 and 48 -> 35, 60000 x 200 into 9000 5650 -> 340 and 89 -> 56. Uniform ids lose
+  // 1.5 to 2.5 us (at 130 MB of zeros 8) below some 2000 positions, where others gain far more: 600 x 128 into 30000 46.8 ->
+  // 9.8 and 8.1 -> 9.6, 512 x 1000 into 32768 212 -> 40 and 31 -> 40, 1500 x 400 into 3000 95 -> 11.5 and 6.8 -> 9.1.
+  const ListedPlan listed = planListed(sh, options);
+  if (listed.possible && (options.variant == 5 || (options.variant == 0 && sh.positions >= 512))) return lowerSegmentListed(g, sh, listed);
+  return lowerSegmentScan(g, options, sh);
 }
 
 }  // namespace akg
