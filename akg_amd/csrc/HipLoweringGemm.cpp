@@ -268,7 +268,10 @@ class GemmEmitter {
     const bool narrow = m_ <= skinnyRows();
     if (elements * elemBytes() < (2LL << 20) && (narrow || n_ % 256 == 0)) return false;
     if (narrow && n_ < 1024) return false;
-    if (!transB_ && n_ * elemBytes() % 16 != 0) return false;
+    // (Rows of a [K,N] weight that are not whole 16-byte chunks: with 8 bits and more than 64 rows. us, 256 x 256 tiles -> small ones:
+    // 219 x 3776 x 5640 38.5 -> 17.2, 836 x 4544 x 9240 97 -> 49, 104 x 768 x 9080 18.9 -> 6.8, 2002 x 3200 x 8280 108 -> 73. For
+    // 16 bits a test pins the other kernel.)
+    if (!transB_ && n_ * elemBytes() % 16 != 0 && (narrow || elemBytes() == 2)) return false;
     const int64_t steps = (k_ * elemBytes() + 127) / 128;
     // (columns that are whole 256-wide tiles pad nothing there: small ones from a quarter below on; 1200 x 8192 x 2048, which a test
     // pins, takes 59.6 us on them and 56.4 on 128 x 128)

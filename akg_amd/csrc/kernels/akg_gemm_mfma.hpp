@@ -1031,7 +1031,7 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
   constexpr int EB = Mma::kElemBytes;
   constexpr long K = KE * EB, NB = N * EB;
   static_assert(BM % 64 == 0 && BM <= 256 && BN % 64 == 0 && BN <= 256, "tile sizes");
-  static_assert(K % 16 == 0 && N % 4 == 0 && (TRANSB || NB % 16 == 0), "whole 16-byte chunks");
+  static_assert(K % 16 == 0 && N % 4 == 0, "whole 16-byte chunks of K, whole words of B's rows");
   static_assert(BM * K < (1L << 31) && (TRANSB ? BN * K : NB * KE) < (1L << 31), "operand too large for 32-bit buffer offsets");
   constexpr int BK = 128;
   constexpr int kTM = BM / 32, kTN = BN / 32;          // 16 x 16 tiles per wavefront
@@ -1070,7 +1070,8 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
   const int c = lane & 15, g = lane >> 4;
 
   // ---- staging. A row beyond M (a column of a [N,K] B beyond N) repeats the last one, its results are dropped; a chunk
-  // beyond K, or beyond the columns of a row-major B, is asked for beyond the buffer and reads zero.
+  // beyond K, or beyond the columns of a row-major B, is asked for beyond the buffer and reads zero. (Where B's rows are not whole chunks,
+  // the last one of a row goes on in the next row, and in the last row beyond the buffer, which is checked word by word.)
   auto bytesLeft = [](long bytes) { return static_cast<int>(bytes < 0x7fffffffL ? bytes : 0x7fffffffL); };
   const __amdgpu_buffer_rsrc_t aRsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<char *>(static_cast<const char *>(A)) + m0 * K, 0, bytesLeft((M - m0) * K), 0x00020000);
