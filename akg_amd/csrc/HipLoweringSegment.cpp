@@ -1264,10 +1264,11 @@ LoweredKernel lowerSegmentScan(const OpGraph &g, const LoweringOptions &options,
 // Frequent ids are often neighbours (tokens by rank), so neighbouring segments go to different workgroups, and a workgroup's
 // columns are at most 256. More positions than the list holds: by windows of the positions, the sums wait in the result
 // between them.
-// What bounds it is the chain of a frequent segment's rows where there is one (16000 x 128 into 1000: 1600 rows, 69 us, 40 ns a
-// row with 64 in flight; 112 us where the waits were for all 64) and two scans of the ids by every workgroup where there is none.
-// 1024 workgroups: 512 and 2048 take 98 and 102 us for 89 (32768 x 1024 into 32768, uniform ids). All tiles of a group on one CU,
-// as they were launched, took 225 us for 124 (ids as frequent as words).
+// What bounds it is the chain of a frequent segment's rows where there is one (16000 x 128 into 1000: 1600 rows, 43 us; 69 us with
+// addresses in vector registers, 112 us where every wait was for all 64 rows) and two scans of the ids by every workgroup where there
+// is none. At most 1024 workgroups, four a CU: 512 and 2048 take 98 and 102 us for 89 (32768 x 1024 into 32768, uniform ids), 1536 take
+// 85 for 72 (20000 x 768 into 30522). All tiles of a group on one CU, as they were launched, took 225 us for 124 (ids as frequent
+// as words).
 struct ListedPlan {
   int64_t tiles = 0, block = 0, groupBits = 0, keys = 0;
   bool possible = false;
@@ -1279,8 +1280,9 @@ ListedPlan planListed(const SegmentShapes &sh, const LoweringOptions &options) {
   plan.tiles = (sh.slice + 255) / 256;
   plan.block = ((sh.slice + plan.tiles - 1) / plan.tiles + 63) / 64 * 64;
   plan.tiles = (sh.slice + plan.block - 1) / plan.block;
+  if (plan.tiles == 1) plan.block = 256;   // (four wavefronts for the ids, whatever the columns)
   const int64_t want = options.split > 0 ? options.split : 1024;
-  while (plan.groupBits < 24 && (1LL << plan.groupBits) * plan.tiles < want && (1LL << plan.groupBits) < sh.segments) ++plan.groupBits;
+  while (plan.groupBits < 24 && (2LL << plan.groupBits) * plan.tiles <= want && (1LL << plan.groupBits) < sh.segments) ++plan.groupBits;
   while (((sh.segments + (1LL << plan.groupBits) - 1) >> plan.groupBits) > 512) ++plan.groupBits;
   plan.keys = (sh.segments + (1LL << plan.groupBits) - 1) >> plan.groupBits;
   plan.possible = plan.tiles < 65536;
@@ -1303,7 +1305,7 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
   }
   s << ", " << tag << "::storage *__restrict__ out0) {\n";
   s << "  constexpr int POSITIONS = " << sh.positions << ", SEGMENTS = " << sh.segments << ", BLOCK = " << plan.block << ", NW = BLOCK / 64;\n";
-  s << "  constexpr int BITS = " << plan.groupBits << ", GROUPS = 1 << BITS, KEYS = " << plan.keys << ", LIST = 4096;\n";
+  s << "  constexpr int BITS = " << plan.groupBits << ", GROUPS = 1 << BITS, KEYS = " << plan.keys << ", LIST = 8192;\n";
   s << "  constexpr int IDV = " << (ids.dtype == DType::I32 ? 4 : ids.dtype == DType::I64 ? 2 : 1) << ", U = 8;\n";
   s << "  constexpr long SLICE = " << sh.slice << ";\n";
   s << "  using id_t = " << idTag << "::storage;\n";
@@ -1441,6 +1443,8 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
     });
     __syncthreads();
   };
+  const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<T::storage *>(data), 0,
+      static_cast<int>(POSITIONS * SLICE * sizeof(T::storage) < 0x7fffffffUL ? POSITIONS * SLICE * sizeof(T::storage) : 0x7fffffffUL), 0x00020000);
   const auto row_of = [&](int k) { return (static_cast<long>(k) << BITS | group) * SLICE + from_col; };
   struct AllAtOnce { enum { kGoesOn = 0 }; };
   struct ByWindows { enum { kGoesOn = 1 }; };
@@ -1448,10 +1452,36 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
     int current = -1;
     acc_t acc = zero, v[64];
     const auto fetch = [&](int q, unsigned entries) {   // eight rows of a chunk of 64 entries
+      constexpr long BYTES = sizeof(T::storage);
+      if constexpr (POSITIONS * SLICE * BYTES < (1L << 31)) {
+        // one address for all lanes and one offset of a lane for all rows: two instructions a row
+        const unsigned at = (entries & 0xfffffu) * static_cast<unsigned>(SLICE * BYTES);
+        const int lane_at = static_cast<int>(from_col * BYTES);
 #pragma unroll
-      for (int u = q; u < q + 8; ++u) {
-        const unsigned p = __builtin_amdgcn_readlane(entries, u) & 0xfffffu;
-        v[u] = T::load((data + static_cast<long>(p) * SLICE)[from_col]);
+        for (int u = q; u < q + 8; ++u) {
+          const int row = __builtin_amdgcn_readlane(static_cast<int>(at), u);
+          T::storage x;
+          if constexpr (BYTES == 8) {
+            const auto w = __builtin_amdgcn_raw_buffer_load_b64(rows, lane_at, row, 0);
+            __builtin_memcpy(&x, &w, BYTES);
+          } else if constexpr (BYTES == 4) {
+            const auto w = __builtin_amdgcn_raw_buffer_load_b32(rows, lane_at, row, 0);
+            __builtin_memcpy(&x, &w, BYTES);
+          } else if constexpr (BYTES == 2) {
+            const auto w = __builtin_amdgcn_raw_buffer_load_b16(rows, lane_at, row, 0);
+            __builtin_memcpy(&x, &w, BYTES);
+          } else {
+            const auto w = __builtin_amdgcn_raw_buffer_load_b8(rows, lane_at, row, 0);
+            __builtin_memcpy(&x, &w, BYTES);
+          }
+          v[u] = T::load(x);
+        }
+      } else {
+#pragma unroll
+        for (int u = q; u < q + 8; ++u) {
+          const unsigned p = __builtin_amdgcn_readlane(entries, u) & 0xfffffu;
+          v[u] = T::load((data + static_cast<long>(p) * SLICE)[from_col]);
+        }
       }
     };
     const auto fold = [&](int q, unsigned entries, int left) {
@@ -1595,10 +1625,10 @@ LoweredKernel lowerSegmentSumToHip(const OpGraph &g, const LoweringOptions &opti
   if (bucketed) return lowerSegmentBucketed(g, options, sh, bucketBits);
   if (group) return lowerSegmentSorted(g, options, sh);
   // Wide rows listed by segment. us, ids as frequent as words (the k-th with 1 / k) and uniform ones, scanned -> listed: 32768 x 1024
-  // into 32768 11600 -> 124 and 199 -> 89, 20000 x 768 into 30522 6020 -> 97 and 98 -> 62, 8192 x 256 into 8000 735 -> 28 and
-  // 17.5 -> 12.4, 2048 x 1024 into 32000 802 -> 38 and 48 -> 35, 60000 x 200 into 9000 5650 -> 340 and 89 -> 56. Uniform ids lose
-  // 1.5 to 2.5 us (at 130 MB of zeros 8) below some 2000 positions, where others gain far more: 600 x 128 into 30000 46.8 ->
-  // 9.8 and 8.1 -> 9.6, 512 x 1000 into 32768 212 -> 40 and 31 -> 40, 1500 x 400 into 3000 95 -> 11.5 and 6.8 -> 9.1.
+  // into 32768 11600 -> 115 and 199 -> 92, 20000 x 768 into 30522 6020 -> 72 and 98 -> 52, 8192 x 256 into 8000 735 -> 22 and
+  // 17.4 -> 12.0, 2048 x 1024 into 32000 805 -> 38 and 48 -> 36, 60000 x 200 into 9000 5690 -> 129 and 89 -> 56. Uniform ids lose
+  // 2 to 3 us (at 130 MB of zeros 9) below some 2000 positions, where others gain far more: 600 x 128 into 30000 46.4 ->
+  // 10.2 and 8.1 -> 10.3, 512 x 1000 into 32768 214 -> 41 and 31 -> 40, 1500 x 400 into 3000 94 -> 10.6 and 6.8 -> 9.1.
   const ListedPlan listed = planListed(sh, options);
   if (listed.possible && (options.variant == 5 || (options.variant == 0 && sh.positions >= 512))) return lowerSegmentListed(g, sh, listed);
   return lowerSegmentScan(g, options, sh);

@@ -25,8 +25,8 @@ def test_sizes_whose_positions_are_listed():
     (1, 65, 1, "float32", "int32", "uniform"), (3, 256, 7, "float32", "int64", "uniform"),
     (700, 257, 50, "float32", "int32", "uniform"),             # one column beyond a tile
     (4097, 128, 1000, "float32", "int32", "words"), (32768, 264, 32768, "float32", "int32", "words"),
-    (4096, 200, 3000, "float32", "int32", "one_segment"),      # as many as the list holds
-    (4097, 200, 3000, "float32", "int32", "one_segment"), (30001, 130, 3000, "float32", "int32", "one_group"),   # by windows
+    (8192, 200, 3000, "float32", "int32", "one_segment"),      # as many as the list holds
+    (8193, 200, 3000, "float32", "int32", "one_segment"), (30001, 130, 3000, "float32", "int32", "one_group"),   # by windows
     (9000, 100, 40000, "float32", "int32", "sorted"), (5000, 96, 3000, "float32", "int32", "outside"),
     (2000, 80, 77, "float32", "int32", "nobody"),
     (30001, 72, 900, "float16", "int32", "words"), (9000, 520, 1300, "bfloat16", "int64", "one_segment"),   # additions that round
