@@ -845,11 +845,13 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
   const std::string ct = computeTypeName(out.dtype), tag = dtypeTag(out.dtype), idTag = dtypeTag(ids.dtype);
   const bool narrow = out.dtype == DType::F16 || out.dtype == DType::BF16 || out.dtype == DType::I8 || out.dtype == DType::I16;
   const std::string rndOpen = narrow ? tag + "::rnd(" : std::string("(");
-  // rounds of the last launch: 4096 entries on eight wavefronts; few entries per bucket: one chunk's worth on two or four
+  // Rounds of the last launch: 4096 entries on eight wavefronts; few entries per bucket: one chunk's worth on two or four, as many
+  // as have a lane for every output element of the bucket (of which there are at most 256).
   const bool small = sh.positions / plan.buckets < 1024 && plan.tiles <= 4;
-  const int nw = small ? (plan.tiles <= 2 ? 2 : 4) : 8, tiles = small ? static_cast<int>(plan.chunk) / (nw * 64) : 8;
+  const int64_t perBucket = plan.perBucket, chains = perBucket * sh.slice;
+  const int nw = small ? (plan.tiles <= 2 && chains <= 128 ? 2 : 4) : 8, tiles = small ? static_cast<int>(plan.chunk) / (nw * 64) : 8;
   // (at least sixteen chains a wavefront: an addition is an instruction of the whole wavefront however few lanes add)
-  const int64_t perBucket = plan.perBucket, chains = perBucket * sh.slice, chainsPerWave = std::max<int64_t>(16, (chains + nw - 1) / nw);
+  const int64_t chainsPerWave = std::max<int64_t>(16, (chains + nw - 1) / nw);
   int keyBits = 1;
   while ((1LL << keyBits) < perBucket) ++keyBits;
   std::ostringstream s;
@@ -940,6 +942,7 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
   s << "  constexpr int W = " << nw << ", T = " << tiles << ", CAP = W * T * 64, PLANE = CAP + 4 * S + 40, CHAINS = " << chains
     << ", PER_WAVE = " << chainsPerWave << ";\n";
   s << "  static_assert(CAP >= CHUNK, \"a chunk's run of one bucket fits a round\");\n";
+  s << "  static_assert(PER_WAVE <= 64 && W * PER_WAVE >= CHAINS, \"a lane for every output element\");\n";
   s << "  // a round's entries: whose run each is, and where entry k of the round is less k for every run\n";
   s << "  __shared__ unsigned short akg_run[CAP];\n  __shared__ unsigned akg_base[W * 64];\n";
   s << "  __shared__ __attribute__((aligned(16))) " << ct << " akg_plane[ROW][PLANE];   // column c of a round's rows, lists per segment\n";

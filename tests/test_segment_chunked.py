@@ -1,6 +1,7 @@
 """UnsortedSegmentSum of short rows, chunks of positions grouped by bucket of segments where they lie: which sizes take it, and
 its results bit for bit the serial loop's."""
 import os
+import re
 
 import numpy as np
 import pytest
@@ -23,25 +24,9 @@ def test_sizes_that_are_taken_by_chunk():
     assert not by_chunk(1020000, 4, 100) and by_chunk(980000, 4, 100) and by_chunk(1100000, 4, 100)
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("positions,width,segments,dtype,ids,pattern,chunks", [
-    (1, 1, 1, "float32", "int32", "uniform", 0),
-    (511, 3, 700, "float32", "int32", "uniform", 1), (513, 4, 513, "float32", "int64", "uniform", 1),   # edges of a chunk
-    (4097, 2, 1025, "float32", "int32", "uniform", 8), (33000, 3, 4954, "float32", "int32", "uniform", 0),
-    (300000, 1, 512, "float32", "int32", "uniform", 2),      # more chunks than a round looks up
-    (9000, 4, 32768, "int32", "int32", "uniform", 4),        # 64 segments a bucket
-    (150000, 3, 9000, "float32", "int32", "one_segment", 8), (70000, 4, 600, "float32", "int32", "one_segment", 1),
-    (100000, 3, 4954, "float32", "int32", "one_bucket", 4), (40000, 2, 3000, "float32", "int32", "sorted", 0),
-    (40000, 2, 3000, "float32", "int32", "outside", 2), (20000, 1, 77, "float32", "int32", "nobody", 0),
-    (70001, 2, 5000, "float16", "int32", "uniform", 0), (66000, 4, 1300, "bfloat16", "int64", "uniform", 0),   # additions that round
-    (33333, 4, 999, "int8", "int32", "uniform", 0), (540000, 3, 16384, "float32", "int32", "uniform", 0),
-])
-def test_bit_for_bit_the_serial_loop(positions, width, segments, dtype, ids, pattern, chunks, monkeypatch, tmp_path):
+def _check_bits(positions, width, segments, dtype, ids, pattern, tmp_path):
     import torch
     from oracle import cpu_ref
-    monkeypatch.setenv("AKG_HIP_VARIANT", "4")
-    if chunks:
-        monkeypatch.setenv("AKG_HIP_CHUNKS", str(chunks))
     name = "by_chunk_%s_%d_%d_%d_%s" % (dtype, positions, width, segments, pattern)
     text = op_desc.unsorted_segment_sum([positions], [width], segments, dtype, ids, name)
     path = os.path.join(str(tmp_path), name + ".info")
@@ -62,3 +47,49 @@ def test_bit_for_bit_the_serial_loop(positions, width, segments, dtype, ids, pat
         kernel.launch(on_device + [out])
         torch.cuda.synchronize()
         assert np.array_equal(out.cpu().numpy(), np.ascontiguousarray(want).reshape(-1).view(np.uint8)), name
+
+
+@pytest.mark.parametrize("positions,width,segments,dtype,split", [
+    (33000, 1, 32768, "float32", 0), (33000, 3, 32768, "float32", 0), (65535, 4, 32768, "float32", 0), (40000, 4, 20000, "float32", 0),
+    (40000, 3, 25000, "float32", 0), (33000, 4, 30000, "bfloat16", 0), (65535, 3, 32204, "int32", 0), (70000, 4, 16384, "float32", 0),
+    (540000, 4, 16384, "float32", 0), (40000, 4, 300, "float32", 0), (33000, 3, 6400, "float32", 100), (140000, 4, 6400, "float32", 100),
+])
+def test_every_output_element_has_a_lane(positions, width, segments, dtype, split, monkeypatch):
+    """One lane adds one output element: the wavefronts of the last launch have a lane for each element of a bucket."""
+    monkeypatch.setenv("AKG_HIP_VARIANT", "4" if split else "0")
+    monkeypatch.setenv("AKG_HIP_SPLIT", str(split))
+    source = driver.HipKernel(op_desc.unsorted_segment_sum([positions], [width], segments, dtype, "int32", "lanes_%s_%d_%d_%d" % (
+        dtype, positions, width, segments)), out_dir=None).source
+    assert BY_CHUNK in source
+    waves, rounds, chains, per_wave = map(int, re.search(r"W = (\d+), T = (\d+), CAP = .*CHAINS = (\d+), PER_WAVE = (\d+);", source).groups())
+    chunk = 512 * int(re.search(r"NW = 8, TILES = (\d+)", source).group(1))
+    assert chains >= width and per_wave <= 64 and waves * per_wave >= chains and waves * rounds * 64 >= chunk
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("positions,width,segments,dtype", [(40000, 4, 20000, "float32"), (40000, 4, 32768, "float32"), (65535, 3, 32204, "float32"),
+                                                            (33000, 4, 30000, "bfloat16"), (70000, 4, 16384, "int32")])
+def test_buckets_of_many_output_elements(positions, width, segments, dtype, monkeypatch, tmp_path):
+    """More than 128 output elements a bucket, through the default choice of the schedule."""
+    monkeypatch.delenv("AKG_HIP_VARIANT", raising=False)
+    _check_bits(positions, width, segments, dtype, "int32", "uniform", tmp_path)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("positions,width,segments,dtype,ids,pattern,chunks", [
+    (1, 1, 1, "float32", "int32", "uniform", 0),
+    (511, 3, 700, "float32", "int32", "uniform", 1), (513, 4, 513, "float32", "int64", "uniform", 1),   # edges of a chunk
+    (4097, 2, 1025, "float32", "int32", "uniform", 8), (33000, 3, 4954, "float32", "int32", "uniform", 0),
+    (300000, 1, 512, "float32", "int32", "uniform", 2),      # more chunks than a round looks up
+    (9000, 4, 32768, "int32", "int32", "uniform", 4),        # 64 segments a bucket
+    (150000, 3, 9000, "float32", "int32", "one_segment", 8), (70000, 4, 600, "float32", "int32", "one_segment", 1),
+    (100000, 3, 4954, "float32", "int32", "one_bucket", 4), (40000, 2, 3000, "float32", "int32", "sorted", 0),
+    (40000, 2, 3000, "float32", "int32", "outside", 2), (20000, 1, 77, "float32", "int32", "nobody", 0),
+    (70001, 2, 5000, "float16", "int32", "uniform", 0), (66000, 4, 1300, "bfloat16", "int64", "uniform", 0),   # additions that round
+    (33333, 4, 999, "int8", "int32", "uniform", 0), (540000, 3, 16384, "float32", "int32", "uniform", 0),
+])
+def test_bit_for_bit_the_serial_loop(positions, width, segments, dtype, ids, pattern, chunks, monkeypatch, tmp_path):
+    monkeypatch.setenv("AKG_HIP_VARIANT", "4")
+    if chunks:
+        monkeypatch.setenv("AKG_HIP_CHUNKS", str(chunks))
+    _check_bits(positions, width, segments, dtype, ids, pattern, tmp_path)
