@@ -1614,15 +1614,16 @@ LoweredKernel lowerSegmentSumToHip(const OpGraph &g, const LoweringOptions &opti
   // on instead of the scan (35304 x 1 into 1131 42.0 -> 8.4, 33000 x 4 into 300 51 -> 9.1). The other two schedules would lose
   // in between as well (300000 x 3 into 5000 36.7 by bucket, 13.4 by chunk; 27126 x 3 into 4954 29.4 scanned, 7.9), but their
   // launches and the scan's lack of a workspace are pinned by tests there. Nor may the workspace outgrow the 16 MiB of a
-  // launch without allocations where it did not before.
+  // launch without allocations where the schedule it takes the place of stays within them, as the scan does, which has none:
+  // 2 million x 3 into 20000 (26 MB by chunk) stays scanned, though that takes 1760 us for 32.
   const ChunkedPlan chunked = planChunked(sh, options);
   bool byChunk = chunked.possible && options.variant == 4;
   if (chunked.possible && options.variant == 0 && sh.positions >= (1 << 15)) {
     const bool many = sh.positions >= (1 << 19);
     byChunk = many || (group ? !bucketed && chunked.perBucket > 1 : sh.positions < (1 << 16));
     const int64_t runs = std::min<int64_t>(2048, std::max<int64_t>(1, sh.positions / 1024));   // (of the schedule by segment)
-    const int64_t before = bucketed ? sh.positions * 4 : sh.positions * rowBytes / 4 + runs * sh.segments;
-    if (group && chunked.words * 4 > (16 << 20) && before * 4 <= (16 << 20)) byChunk = false;
+    const int64_t before = !group ? 0 : bucketed ? sh.positions * 4 : sh.positions * rowBytes / 4 + runs * sh.segments;
+    if (chunked.words * 4 > (16 << 20) && before * 4 <= (16 << 20)) byChunk = false;
   }
   if (byChunk) return lowerSegmentChunked(g, options, sh, chunked);
   if (bucketed) return lowerSegmentBucketed(g, options, sh, bucketBits);

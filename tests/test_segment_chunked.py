@@ -24,6 +24,16 @@ def test_sizes_that_are_taken_by_chunk():
     assert not by_chunk(1020000, 4, 100) and by_chunk(980000, 4, 100) and by_chunk(1100000, 4, 100)
 
 
+@pytest.mark.parametrize("positions,width,segments", [(2000000, 3, 20000), (4000000, 4, 30000), (1200000, 3, 16385), (1 << 20, 4, 32768), (3000000, 1, 20000),
+                                                      (600000, 3, 20000), (540000, 1, 32768)])
+def test_more_segments_than_are_grouped_need_no_scratch_beyond_the_static_one(positions, width, segments):
+    """More than 16384 segments were scanned, without a workspace: a launch that allocates nothing serves these still."""
+    kernel = driver.HipKernel(op_desc.unsorted_segment_sum([positions], [width], segments, "float32", "int32", "ws_%d_%d_%d" % (
+        positions, width, segments)), out_dir=None)
+    assert kernel.workspace_bytes <= 16 << 20
+    assert (BY_CHUNK in kernel.source) == (kernel.workspace_bytes > 0)
+
+
 def _check_bits(positions, width, segments, dtype, ids, pattern, tmp_path):
     import torch
     from oracle import cpu_ref
