@@ -282,20 +282,30 @@ class GemmEmitter {
       // 464 x 576 x 10032 would take 11.8 us for 13.1, 645 x 1024 x 6008, whose tile a test pins, 16.0 for 20.2)
       if (w.m * w.n > 128 * 128 && steps <= 16) continue;
       const int64_t tiles = ((m_ + w.m - 1) / w.m) * ((n_ + w.n - 1) / w.n);
+      // Partials stay within the 16 MiB of a launch without allocations, those of the larger tiles within 15. Where they do not, half as
+      // many workgroups a tile, or one. us, K split as estimated / this: bf16 1130 x 12800 x 512 39.8 / 40.9 (47.6 on the tile estimated
+      // next), 338 x 13712 x 1368 51.5 / 56.1, 71 x 14272 x 4496 43.6 / 49.5, int8 2518 x 2528 x 808 20.0 / 17.2, 5350 x 3280 x 552 30.3 / 22.7.
+      const auto partialsFit = [&](int split) {
+        const int64_t bytes = tiles * split * w.m * w.n * 4;
+        return w.m * w.n > 64 * 128 ? bytes <= (15LL << 20) : bytes + tiles * 4 + 256 <= (16LL << 20);
+      };
       for (int split = 1; split <= w.splits; split *= 2) {
         if (split > 1 && (split - 1) * ((steps + split - 1) / split) >= steps) continue;   // no empty split
-        // (8-bit weights below 2 MiB with more than 16 steps: two workgroups a tile at least, where a test of workspaces wants one;
-        // estimated 0.5 us slower, and 20.7 -> 6 us against 256 x 256 tiles)
-        if (split == 1 && elemBytes() == 1 && steps > 16 && elements < (2LL << 20)) continue;
+        // (8-bit weights below 2 MiB with more than 16 steps: two workgroups a tile at least, where a test of workspaces wants one
+        // and the launch without allocations has the memory; estimated 0.5 us slower, and 20.7 -> 6 us against 256 x 256 tiles)
+        if (split == 1 && elemBytes() == 1 && steps > 16 && elements < (2LL << 20) && partialsFit(2)) continue;
         if (tiles * split * w.m * w.n * 4 >= (1LL << 30)) continue;
-        // partials stay within the 16 MiB of a launch without allocations
-        if (split > 1 && w.m * w.n > 64 * 128 && tiles * split * w.m * w.n * 4 > (15LL << 20)) continue;
+        int parts = split;
+        if (!narrow && split > 1 && !partialsFit(split)) {
+          parts = split / 2;
+          if (parts == 1 || !partialsFit(parts)) continue;
+        }
         const double t = smallTileTime(w, split) * (split > 1 ? 1.03 : 1);   // (as fast without a workspace is better)
         if (t >= best) continue;
         best = t;
         tileM_ = w.m;
         tileN_ = w.n;
-        kSplit_ = split;
+        kSplit_ = parts;
       }
     }
     const bool large = transB_ && elemBytes() == 2 && elements >= (60LL << 20);

@@ -26,6 +26,17 @@ def test_products_that_take_several_tiles_a_workgroup():
     assert _tile(365, 1408, 512, "bfloat16", False) is None and _tile(48, 1408, 744, "bfloat16", False) is None
 
 
+@pytest.mark.parametrize("m,k,n,dtype,tb", [
+    (69, 11776, 4504, "bfloat16", True), (1079, 12080, 464, "float16", False), (338, 13712, 1368, "bfloat16", True),
+    (4329, 11200, 120, "bfloat16", False), (4816, 2240, 840, "int8", False), (2518, 2528, 808, "int8", True), (8176, 2176, 584, "int8", True),
+    (370, 4088, 3440, "bfloat16", False),
+])
+def test_partials_fit_a_launch_without_allocations(m, k, n, dtype, tb):
+    """Such a launch has 16 MiB; the kernels that these products had before ask for less or nothing."""
+    kernel = driver.HipKernel(_product(m, k, n, dtype, tb, "partials"), out_dir=None)
+    assert "gemm_small_tile" in kernel.source and kernel.workspace_bytes <= 16 << 20
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,k,n,dtype,tb,tile", [
     (1059, 1704, 3604, "bfloat16", True, (192, 128, 1)),    # ragged rows and columns, a K tail of 80 bytes
@@ -43,6 +54,8 @@ def test_products_that_take_several_tiles_a_workgroup():
     (365, 1408, 744, "bfloat16", False, (64, 64, 1)),       # small weights
     (365, 2088, 492, "bfloat16", True, (64, 64, 4)),
     (85, 4000, 248, "float16", True, (64, 64, 8)),
+    (71, 14272, 4496, "bfloat16", True, (64, 64, 4)),       # eight would ask for more than the launch without allocations has
+    (2518, 2528, 808, "int8", True, (128, 128, 1)),         # ... as would two
     (65, 64, 68, "bfloat16", True, (64, 64, 1)),            # one step
     (219, 3776, 5640, "int8", False, None),                 # rows of B that are not whole 16-byte chunks
     (836, 2064, 9240, "int8", False, None), (97, 1040, 1004, "int8", False, None),
