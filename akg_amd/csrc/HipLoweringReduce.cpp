@@ -638,13 +638,14 @@ class StreamReduceEmitter {
     // neighbours read as well. The strips of the same rows then run on one XCD and the lines stay in its L2 (no hint); in
     // launch order and past the caches every such line came from memory twice. Two column sums of bf16 [4100,3000]
     // 14.9 -> 12.0 us, [16400,3000] 45.9 -> 34.8, [16400,1111] 21.0 -> 15.8; rows of whole lines keep the hint ([16400,3072]
-    // 32.9, 34.5 this way).
+    // 32.9, 34.5 this way). So does a single strip, whose lines no other workgroup reads but at the rows' edges (f32
+    // [400000,60] 33.8, 36.0 without it).
     sharedLines_ = false;
     for (int id : g_.inputs) {
       const TensorValue &t = g_.tensor(id);
-      if (dirY_ && t.used && t.numel() == O_ * R_ * I_) sharedLines_ = sharedLines_ || (I_ * static_cast<int64_t>(dtypeSize(t.dtype))) % 128 != 0;
+      if (dirY_ && strips_ > 1 && t.used && t.numel() == O_ * R_ * I_) sharedLines_ = sharedLines_ || (I_ * static_cast<int64_t>(dtypeSize(t.dtype))) % 128 != 0;
     }
-    if (dirY_) xcdContiguous_ = sharedLines_ && strips_ > 1;
+    if (dirY_) xcdContiguous_ = sharedLines_;
     // workspace: one arrival counter per group, then the partials of every reduction
     workspaceBytes_ = 0;
     partialOffset_.assign(reduces_.size(), 0);

@@ -12,10 +12,12 @@ def test_rows_of_whole_lines_keep_the_hint():
     assert "xcd_contiguous_id" in ragged and "V, true>(b_in" not in ragged
     whole = driver.HipKernel(op_desc.bias_grad(4100, 3072, "bfloat16"), out_dir=None).source
     assert "xcd_contiguous_id" not in whole and "V, true>(b_in" in whole
+    one_strip = driver.HipKernel(op_desc.bias_grad(40000, 60, "float32"), out_dir=None).source   # nothing that another strip reads
+    assert "xcd_contiguous_id" not in one_strip and "V, true>(b_in" in one_strip
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,cols,dtype", [(700, 1111, "bfloat16"), (4100, 130, "float32"), (3000, 4095, "float16"), (257, 72, "bfloat16")])
+@pytest.mark.parametrize("rows,cols,dtype", [(700, 1111, "bfloat16"), (4100, 130, "float32"), (3000, 4095, "float16"), (257, 72, "bfloat16"), (5000, 60, "float32")])
 def test_column_sums_of_ragged_rows(rows, cols, dtype):
     """Against float64, with the bound of a reassociated float32 sum of `rows` terms; an elementwise result stored beside it
     bit for bit."""
