@@ -95,12 +95,14 @@ class PlaneEmitter {
   int lastWalk_ = 0;               // walks 0 .. lastWalk_: one per level of reductions, the last one stores
   bool fullOutputs_ = false;
   int vec_ = 8, block_ = 256, chunks_ = 1, overlap_ = 0;
+  bool chunkBranch_ = false;       // a chunk beyond the channel is left out by a branch, not element by element
   int64_t slots_ = 1, parts_ = 0;  // slots of a run; workgroups per channel of the form with one launch per level (0: one, resident)
   std::vector<uint64_t> partialAt_;   // per tensor: byte offset of a reduction's partial results in the workspace
   uint64_t workspaceBytes_ = 0;
   int reduceCount_ = 0;
 
   void line(const std::string &s) { src_ << s << "\n"; }
+  static bool isExtremum(const lowering::ReduceSpec &spec) { return spec.combiner == "akg::RedMax" || spec.combiner == "akg::RedMin"; }
   static std::string id(const char *prefix, int t) { return std::string(prefix) + std::to_string(t); }
 
   std::vector<int64_t> padded(const TensorValue &t, const std::string &what) const {
@@ -243,9 +245,27 @@ class PlaneEmitter {
     while (block < 1024 && chunksFor(perChannel, block) > 8) block *= 2;
     if (opt_.block >= 64 && opt_.block <= 1024 && (opt_.block & (opt_.block - 1)) == 0) block = opt_.block;
     const int64_t resident = chunksFor(perChannel, block);
-    // The line between the forms: 64 registers of a 1024-thread workgroup hold 256 KiB; there both take the same time (bf16
-    // [32,16,64,64], exactly 64: 9.6 us resident, 9.7 by level), below the resident form wins (f32 [32,16,40,40] 6.5 / 9.8).
-    if (resident * regsPerChunk <= 64 && opt_.split <= 1) {
+    // Extrema of chunks of eight and sixteen: with a condition per element the compiler unpacks all chunks in front of it and spills
+    // (range of f16 [125,700,28,28] 83.9 us, 62.2 with a branch per chunk; int8 53.6 -> 44.8). Not 8-bit chunks that share elements (int8
+    // [2048,700,7,7] 48.3, 50.6 by branches) nor chunks of four (i32 [10,700,28,28]
+    // 9.0, 10.1).
+    for (const OpNode &op : g_.ops) {
+      if (lowering::isReduceKind(op.kind) && isExtremum(lowering::reduceSpec(op, g_.tensor(op.outputs[0]).dtype))) chunkBranch_ = true;
+    }
+    chunkBranch_ = chunkBranch_ && vec_ >= 8 && (overlap_ == 0 || widest == 2);
+    // The line between the forms. 64 registers of a 1024-thread workgroup hold 256 KiB as they came from memory. (Offsets and
+    // flags are a few more per chunk: where narrow types or short runs make 24 and more small chunks a thread some of them
+    // spill; with 256 channels and more that is still the faster form: range of int8 [32000,700,6] 352 us, 491 by level, 390 by one kernel
+    // per level and value as before. It is the slower one for f32 results of int8 runs of six: [12288,700,6] 174, by such kernels 161.)
+    // Few channels leave CUs idle in the resident form, and more than eight chunks a thread make that the longer way. us,
+    // resident / by level / one kernel per level and value, 16 channels: bf16 batch norm of [83,16,28,28] (8 chunks) 6.3 / 6.0 / 14.2, of 16
+    // chunks 11.0 / 7.2 / 16.8, f32 10.3 / 6.8 / 16.5; 32 channels: int8 range of [64,32,64,64] 17.2 / 7.0 / 11.5, [30000,32,2,3] 91.7 / 24 / 25.4;
+    // 128 channels, 16 chunks: 18.0 / 24.4, 13.3 / 19.0. Short runs, which share their lines, earlier: i32 range of [3072,16,6] 11.9 / 5.2 / 9.1,
+    // with 128 channels and one level range of f16 [12288,128,6] 62 / 33 / 46, of i32 [6144,128,6] 33.5 / 20.6 / 30.5 (batch norms, of two
+    // levels, stay: bf16 [16384,128,6] 54.6 / 61).
+    const int64_t runBytes = inner_ * widest;
+    const bool fewChannels = runBytes < 64 ? (kept_ <= 32 && perChannel > 4096) || (kept_ < 256 && resident > 8 && lastWalk_ == 1) : kept_ <= 32 && resident > 8;
+    if (resident * regsPerChunk <= 64 && opt_.split <= 1 && (!fewChannels || opt_.split == 1)) {
       block_ = block;
       chunks_ = static_cast<int>(resident);
       parts_ = 0;
@@ -254,11 +274,12 @@ class PlaneEmitter {
     // One launch per level: 128 bytes of loads in flight per thread, less where that leaves less than four workgroups per
     // CU. Bound by the passes over the tensor, one per level and one to store (a later pass is served by the last-level
     // cache in part): f32 [112,32,79,79] 90.5 -> 64.4 us (56 for the 3 + 1 passes), f16 [24,112,80,80] 33.3 -> 20.0, bf16
-    // [100,16,100,100] 33.8 -> 19.0, [128,64,56,56] 42.4 -> 32.5; 512 threads or half the chunks are within 5 % of it.
+    // [100,16,100,100] 33.8 -> 19.0, [128,64,56,56] 42.4 -> 32.5; 512 threads or half the chunks are within 5 % of it. Short runs of few
+    // channels: one workgroup per CU, as neighbours in a channel ask for the same lines (int8 [30000,32,2,3] 33 us with four, 24).
     block_ = opt_.block >= 64 && opt_.block <= 1024 && (opt_.block & (opt_.block - 1)) == 0 ? opt_.block : 256;
     int chunks = std::max(1, 32 / regsPerChunk);
     if (opt_.chunks > 0) chunks = opt_.chunks;
-    while (opt_.chunks == 0 && chunks > 1 && kept_ * chunksFor(perChannel, block_ * chunks) < 4 * opt_.computeUnits) chunks /= 2;
+    while (opt_.chunks == 0 && chunks > 1 && kept_ * chunksFor(perChannel, block_ * chunks) < (runBytes < 64 && kept_ <= 32 ? 1 : 4) * opt_.computeUnits) chunks /= 2;
     if (opt_.split > 1) chunks = static_cast<int>(chunksFor(perChannel, static_cast<int>(std::min<int64_t>(opt_.split, 1 << 16)) * block_));
     if (chunks * regsPerChunk > 128) throw LoweringError("plane kernel: too many chunks per thread");
     chunks_ = chunks;
@@ -442,6 +463,7 @@ class PlaneEmitter {
     }
     line("#pragma unroll");
     line("  for (int j = 0; j < CH; ++j) {");
+    if (chunkBranch_) line("    if (!akg_ok[j]) continue;");
     for (size_t i = 0; i < g_.inputs.size(); ++i) {
       const int t = g_.inputs[i];
       const TensorValue &tv = g_.tensor(t);
@@ -460,8 +482,9 @@ class PlaneEmitter {
       const std::string acc = id("acc", op->outputs[0]);
       line("#pragma unroll");
       src_ << "    for (int e = 0; e < V; ++e) {\n";
-      src_ << "      if (" << (overlap_ ? "e >= akg_skip[j]" : "akg_ok[j]") << ") " << acc << " = " << spec.combiner << "::apply(" << acc << ", "
-           << operandExpr(op->inputs[0]) << ");\n";
+      // (in a walk by branches an extremum takes the elements a chunk shares with its neighbour twice)
+      const std::string taken = chunkBranch_ && (overlap_ == 0 || isExtremum(spec)) ? "" : overlap_ ? "if (e >= akg_skip[j]) " : "if (akg_ok[j]) ";
+      src_ << "      " << taken << acc << " = " << spec.combiner << "::apply(" << acc << ", " << operandExpr(op->inputs[0]) << ");\n";
       src_ << "    }\n";
     }
     if (stores) {

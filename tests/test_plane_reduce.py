@@ -64,6 +64,33 @@ def test_descriptions_that_take_the_plane_kernel_and_those_that_do_not():
     assert family(b.dumps([b.sub(y, b.reduce("ReduceMax", y, [0, 2, 3], True))])) == "staged"
 
 
+def _mixed(shape, dtype):
+    """float32 results of a narrow input: chunks of four elements, less than 16 bytes each."""
+    b = op_desc.DescBuilder("mixed_%s_%s" % (dtype, "x".join(map(str, shape))))
+    x = b.cast(b.input(shape, dtype), "float32")
+    return b.dumps([b.sub(x, b.reduce("ReduceMax", x, [0, 2, 3], True))])
+
+
+def _peak_and_sum(n, c, h, w):
+    """A maximum and a sum of one walk."""
+    b = op_desc.DescBuilder("peak_and_sum_%dx%dx%dx%d" % (n, c, h, w))
+    x = b.input([n, c, h, w], "float16")
+    f = b.cast(x, "float32")
+    s = b.reduce("ReduceSum", b.mul(f, f), [0, 2, 3], True)
+    return b.dumps([b.sub(x, b.reduce("ReduceMax", x, [0, 2, 3], True)), s])
+
+
+def test_few_channels_of_many_chunks_take_a_launch_per_level():
+    def by_level(text):
+        kernel = driver.HipKernel(text, out_dir=None)
+        assert kernel.family == "plane_reduce"
+        return "_level0" in kernel.source
+    assert by_level(_range([30000, 32, 2, 3], [0, 2, 3], "int8")) and by_level(_range([64, 32, 64, 64], [0, 2, 3], "int8"))
+    assert by_level(_range([8000, 128, 2, 3], [0, 2, 3], "float16")) and by_level(_mixed([64, 16, 63, 63], "int8"))
+    assert not by_level(_bn(64, 128, 28, 28, "bfloat16")) and not by_level(_range([64, 128, 64, 64], [0, 2, 3], "int8"))
+    assert not by_level(_bn(80, 16, 28, 28, "bfloat16"))    # eight chunks a thread
+
+
 CASES = [
     (_bn(64, 16, 7, 7, "bfloat16"), "1"),            # a chunk shared by two slots of a run of 49
     (_bn(33, 17, 28, 28, "bfloat16"), "1"),          # whole chunks, the last ones of a thread beyond the channel
@@ -78,6 +105,9 @@ CASES = [
     (_backward(12, 20, 14, 14), "1"), (_backward(12, 20, 14, 14), "4"),
     (_range([8, 40, 5, 7], [0, 2, 3], "int32"), "1"), (_range([3, 4, 2, 9, 1, 70], [0, 1, 4, 5], "float16"), "2"),
     (_statistics(8, 24, 30, 30), "1"), (_statistics(8, 24, 30, 30), "5"),
+    # extrema: a chunk beyond the channel by a branch, whole and shared ones
+    (_range([41, 20, 7, 7], [0, 2, 3], "float16"), "1"), (_range([33, 17, 8, 8], [0, 2, 3], "int8"), "1"), (_range([130, 18, 5, 5], [0, 2, 3], "int8"), "1"),
+    (_peak_and_sum(40, 16, 7, 9), "1"), (_peak_and_sum(40, 16, 7, 9), "3"), (_mixed([600, 16, 9, 9], "int8"), "0"), (_range([5000, 16, 2, 3], [0, 2, 3], "int8"), "0"),
 ]
 
 
@@ -106,7 +136,7 @@ def test_results_against_the_oracle(index, monkeypatch):
     on_device = [torch.from_numpy(np.ascontiguousarray(a).view(np.int16) if a.dtype == np.uint16 else np.ascontiguousarray(a)).cuda() for a in inputs]
     first = None
     for _ in range(3):
-        outs = [torch.full(d.shape, 77, dtype={"bfloat16": torch.int16, "float16": torch.float16, "float32": torch.float32, "int32": torch.int32}[d.dtype],
+        outs = [torch.full(d.shape, 77, dtype={"bfloat16": torch.int16, "float16": torch.float16, "float32": torch.float32, "int32": torch.int32, "int8": torch.int8}[d.dtype],
                            device="cuda") for d in kernel.outputs]
         kernel.launch(on_device + outs)
         torch.cuda.synchronize()
