@@ -52,7 +52,8 @@ struct LoweringOptions {
   //   column_reduce  5: one strip per workgroup (no second set of resident registers)
   //   segment_sum    1: every workgroup scans all ids, 2: positions grouped by segment first (whatever the size),
   //                  3: grouped by bucket of segments first (whatever the number of buckets),
-  //                  4: chunks grouped by bucket where they lie (short rows, whatever the size)
+  //                  4: chunks grouped by bucket where they lie (short rows, whatever the size),
+  //                  5: wide rows listed by segment (whatever the number of positions up to 2^20)
   //   indexed        1: no LDS-tiled transposes, 2: no chunk-wide loads
   int variant = 0;
   int nonTemporal = 1;  // stream once-touched tensors with non-temporal accesses (AKG_HIP_NT=0 turns it off)

@@ -1263,7 +1263,7 @@ LoweredKernel lowerSegmentScan(const OpGraph &g, const LoweringOptions &options,
 // Wide rows and at most 2^16 positions, as gradients of embedding tables have: one launch without a workspace. Workgroup (g, t)
 // sums the segments congruent to g modulo GROUPS in column tile t, one column a thread:
 //   it counts its positions per segment, lists them by segment and in their order (LDS), and walks the list with 64 rows in flight,
-//   whatever segments they belong to.
+//   whatever segments they belong to; zeros for segments without positions it writes for its own or for a share of adjacent ones.
 // Frequent ids are often neighbours (tokens by rank), so neighbouring segments go to different workgroups, and a workgroup's
 // columns are at most 256. More positions than the list holds: by windows of the positions, the sums wait in the result
 // between them.
@@ -1309,7 +1309,22 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
   s << ", " << tag << "::storage *__restrict__ out0) {\n";
   s << "  constexpr int POSITIONS = " << sh.positions << ", SEGMENTS = " << sh.segments << ", BLOCK = " << plan.block << ", NW = BLOCK / 64;\n";
   s << "  constexpr int BITS = " << plan.groupBits << ", GROUPS = 1 << BITS, KEYS = " << plan.keys << ", LIST = 8192;\n";
-  s << "  constexpr int IDV = " << (ids.dtype == DType::I32 ? 4 : ids.dtype == DType::I64 ? 2 : 1) << ", U = 8;\n";
+  const int64_t idv = ids.dtype == DType::I32 ? 4 : ids.dtype == DType::I64 ? 2 : 1;
+  // chunks of ids a lane has in flight: no more than there are, as every workgroup loads them all (eight for 2000 x 128 into 2000,
+  // where there are two: 33 MB from L2, 2.5 of 8.5 us)
+  const int64_t inFlight = std::min<int64_t>(8, (sh.positions + plan.block * idv - 1) / (plan.block * idv));
+  s << "  constexpr int IDV = " << idv << ", U = " << inFlight << ";\n";
+  // Segments without positions: a share of adjacent ones per workgroup, in pieces of up to 16 bytes, so that lines are written whole and by
+  // one XCD. Finding out which ones have none costs two instructions an id and workgroup: with more than 4096 positions a workgroup
+  // writes zeros for its own segments. us, uniform ids, own / share: 512 x 1000 into 32768 43.4 / 31.2 (rows of 4000 bytes), 800 x 1544
+  // into 16000 34.7 / 27.0, 4096 x 128 into 4096 9.4 / 7.8, 8192 x 256 into 8000 11.8 / 13.1, 60000 x 200 into 9000 58 / 64.
+  const bool byShare = sh.positions <= 4096;
+  int64_t piece = 16 / static_cast<int64_t>(dtypeSize(out.dtype));
+  while (sh.slice % piece != 0) piece /= 2;
+  const int64_t workgroups = (1LL << plan.groupBits) * plan.tiles;
+  s << "  constexpr int WORKGROUPS = " << workgroups << ", SHARE_ROWS = " << (sh.segments + workgroups - 1) / workgroups << ", PIECE = " << piece
+    << ", PIECES = " << sh.slice / piece << ";\n";
+  s << "  constexpr bool BY_SHARE = " << (byShare ? "true" : "false") << ";\n";
   s << "  constexpr long SLICE = " << sh.slice << ";\n";
   s << "  using id_t = " << idTag << "::storage;\n";
   s << "  using T = " << tag << ";\n  using ID = " << idTag << ";\n";
@@ -1324,6 +1339,7 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
   s << R"(  struct __attribute__((aligned(sizeof(id_t) * IDV))) id_chunk { id_t v[IDV]; };
   __shared__ unsigned akg_count[NW * KEYS];   // [wavefront][key]: its positions, then where it lists the next one
   __shared__ unsigned akg_has[KEYS], akg_total;
+  __shared__ unsigned akg_met[BY_SHARE ? SHARE_ROWS : 1];    // this workgroup's share of adjacent segments: which ones have positions
   __shared__ unsigned akg_list[LIST];         // key << 20 | position, by key
   const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // (the tiles of a group, of which all may be long, on different XCDs and CUs)
@@ -1331,6 +1347,7 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
   const long col = static_cast<long>(blockIdx.y) * BLOCK + tid;
   const bool has = col < SLICE;
   const unsigned from_col = static_cast<unsigned>(has ? col : SLICE - 1);
+  const unsigned share_first = static_cast<unsigned>(akg::xcd_contiguous_id(static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x), WORKGROUPS)) * SHARE_ROWS;
   const auto mine = [&](int id) { return static_cast<unsigned>(id) < static_cast<unsigned>(SEGMENTS) && (id & (GROUPS - 1)) == group; };
   // ids that fit are loaded once
   constexpr bool ONCE = POSITIONS <= LIST && POSITIONS <= NW * 64 * IDV * U;
@@ -1354,7 +1371,7 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
   constexpr int SHARE = (POSITIONS + NW * 64 * IDV - 1) / (NW * 64 * IDV) * (64 * IDV);
   if (ONCE) load(wave * SHARE);
   // the ids of positions [from, upto), a contiguous share per wavefront, 64 * IDV at a time in ascending order
-  const auto scan = [&](int from, int upto, auto &&visit) {
+  const auto scan = [&](int from, int upto, auto &&meet, auto &&visit) {
     const int share = (upto - from + NW * 64 * IDV - 1) / (NW * 64 * IDV) * (64 * IDV);
     const int first = from + wave * share, end = first + share < upto ? first + share : upto;
     for (int base = first; base < end; base += 64 * IDV * U) {
@@ -1367,6 +1384,7 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
 #pragma unroll
         for (int e = 0; e < IDV; ++e) {
           const int id = p + e < end ? as_int(ID::load(chunk[u].v[e])) : -1;
+          meet(static_cast<unsigned>(id) - share_first);
           key[e] = mine(id) ? id >> BITS : -1;
           any = any || key[e] >= 0;
         }
@@ -1374,10 +1392,10 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
       }
     }
   };
-  const auto count = [&](int from, int upto) {
+  const auto count = [&](int from, int upto, auto &&meet) {
     for (int k = tid; k < NW * KEYS; k += BLOCK) akg_count[k] = 0;
     __syncthreads();
-    scan(from, upto, [&](int, const int (&key)[IDV]) {
+    scan(from, upto, meet, [&](int, const int (&key)[IDV]) {
 #pragma unroll
       for (int e = 0; e < IDV; ++e) {
         if (key[e] >= 0) atomicAdd(&akg_count[wave * KEYS + key[e]], 1u);
@@ -1396,7 +1414,7 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
         }
         unsigned upto_here = sum;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
+        for (int d = 1; d < (KEYS < 64 ? KEYS : 64); d <<= 1) {
           const unsigned below = __shfl_up(upto_here, d);
           if (lane >= d) upto_here += below;
         }
@@ -1409,15 +1427,16 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
             at += c[w];
           }
         }
-        run += __builtin_amdgcn_readlane(upto_here, 63);
+        run += __builtin_amdgcn_readlane(upto_here, KEYS < 64 ? KEYS - 1 : 63);
       }
       if (lane == 0) akg_total = run;
     }
     __syncthreads();
     return __builtin_amdgcn_readfirstlane(static_cast<int>(akg_total));
   };
+  const auto pass_by = [](unsigned) {};
   const auto place = [&](int from, int upto) {
-    scan(from, upto, [&](int p, int (&key)[IDV]) {
+    scan(from, upto, pass_by, [&](int p, int (&key)[IDV]) {
       for (;;) {   // one key at a time; its positions go up with the lanes, then with the elements
         int pick = -1;
 #pragma unroll
@@ -1510,6 +1529,13 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
     const auto entries_at = [&](int i) { return akg_list[i + lane < n ? i + lane : n - 1]; };
     unsigned entries = entries_at(0);
     int i = 0;
+    if (BY_SHARE && n <= 8) {
+      // (the ways below jump over a part for every eight rows: 512 x 128 into 1000 4.1 us, 3.3 this way)
+      fetch(0, entries);
+      fold(0, entries, n);
+      if (has) out0[row_of(current)] = T::store(acc);
+      return;
+    }
     if (n >= 128) {
       // eight rows are summed, the eight 64 behind them requested; no load is conditional, or the waits would be for all of them
 #pragma unroll
@@ -1540,8 +1566,26 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
     }
     if (has) out0[row_of(current)] = T::store(acc);
   };
-  // zeros for the segments without positions, or for all
-  const auto clear = [&](bool all) {
+  if constexpr (BY_SHARE) {
+    for (int r = tid; r < SHARE_ROWS; r += BLOCK) akg_met[r] = 0;   // (a barrier follows)
+  }
+  const int n = count(0, POSITIONS, [&](unsigned r) {
+    if (BY_SHARE && r < static_cast<unsigned>(SHARE_ROWS)) akg_met[r] = 1;
+  });
+  if constexpr (BY_SHARE) {
+    struct __attribute__((aligned(sizeof(T::storage)))) zeros { T::storage v[PIECE]; };
+    // (each workgroup begins elsewhere in its share: at a power-of-two distance they would all write to the same channels)
+    constexpr int TRIPS = (SHARE_ROWS * PIECES + BLOCK - 1) / BLOCK;
+    const int begin = static_cast<int>((blockIdx.x + blockIdx.y * gridDim.x) * 40503u % 65536u * TRIPS / 65536u);
+    for (int trip = 0; trip < TRIPS; ++trip) {
+      const int i = (trip + begin < TRIPS ? trip + begin : trip + begin - TRIPS) * BLOCK + tid, r = i / PIECES;
+      if (r < SHARE_ROWS && share_first + r < static_cast<unsigned>(SEGMENTS) && akg_met[r] == 0) {
+        *reinterpret_cast<zeros *>(out0 + static_cast<long>(share_first + r) * SLICE + (i - r * PIECES) * PIECE) = zeros{};
+      }
+    }
+  } else {
+    // (sums that go on from window to window begin with zeros)
+    const bool all = POSITIONS > LIST && n > LIST;
     for (int k0 = 0; k0 < KEYS; k0 += 64) {
       const int k = k0 + lane;
       unsigned long long empty = __ballot(k < KEYS && (static_cast<long>(k) << BITS | group) < SEGMENTS && (all || akg_has[k] == 0));
@@ -1550,18 +1594,15 @@ LoweredKernel lowerSegmentListed(const OpGraph &g, const SegmentShapes &sh, cons
         empty &= empty - 1;
       }
     }
-  };
-  const int n = count(0, POSITIONS);
+  }
   if (POSITIONS <= LIST || n <= LIST) {
-    clear(false);
     place(0, POSITIONS);
     if (n > 0) sum(n, AllAtOnce());
     return;
   }
-  clear(true);
   for (int from = 0; from < POSITIONS; from += LIST) {
     const int upto = from + LIST < POSITIONS ? from + LIST : POSITIONS;
-    const int here = count(from, upto);
+    const int here = count(from, upto, pass_by);
     place(from, upto);
     if (here > 0) sum(here, ByWindows());
     __syncthreads();
@@ -1629,10 +1670,11 @@ LoweredKernel lowerSegmentSumToHip(const OpGraph &g, const LoweringOptions &opti
   if (bucketed) return lowerSegmentBucketed(g, options, sh, bucketBits);
   if (group) return lowerSegmentSorted(g, options, sh);
   // Wide rows listed by segment. us, ids as frequent as words (the k-th with 1 / k) and uniform ones, scanned -> listed: 32768 x 1024
-  // into 32768 11600 -> 115 and 199 -> 92, 20000 x 768 into 30522 6020 -> 72 and 98 -> 52, 8192 x 256 into 8000 735 -> 22 and
-  // 17.4 -> 12.0, 2048 x 1024 into 32000 805 -> 38 and 48 -> 36, 60000 x 200 into 9000 5690 -> 129 and 89 -> 56. Uniform ids lose
-  // 2 to 3 us (at 130 MB of zeros 9) below some 2000 positions, where others gain far more: 600 x 128 into 30000 46.4 ->
-  // 10.2 and 8.1 -> 10.3, 512 x 1000 into 32768 214 -> 41 and 31 -> 40, 1500 x 400 into 3000 94 -> 10.6 and 6.8 -> 9.1.
+  // into 32768 11600 -> 117 and 198 -> 92, 20000 x 768 into 30522 5780 -> 72 and 98 -> 52, 8192 x 256 into 8000 710 -> 22 and
+  // 18.1 -> 11.8, 2048 x 1024 into 32000 745 -> 36 and 50 -> 33, 60000 x 200 into 9000 5690 -> 150 and 99 -> 58, 600 x 128 into 30000 48 ->
+  // 6.6 and 8.1 -> 6.5, 512 x 1000 into 32768 205 -> 31 and 31 -> 31, 1500 x 400 into 3000 150 -> 9.2 and 7.2 -> 6.6. The least
+  // there is, 512 x 128 into 1000, takes 14.5 -> 4.4 and 3.1 -> 3.3. Rows of 5 to 64 elements stay scanned, as a thread has a column of one row here:
+  // fewer than 64 of a wavefront would work (32768 x 64 into 32768 43 us with uniform ids, 3730 with ids as frequent as words).
   const ListedPlan listed = planListed(sh, options);
   if (listed.possible && (options.variant == 5 || (options.variant == 0 && sh.positions >= 512))) return lowerSegmentListed(g, sh, listed);
   return lowerSegmentScan(g, options, sh);

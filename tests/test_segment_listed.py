@@ -20,6 +20,13 @@ def test_sizes_whose_positions_are_listed():
     assert not listed(511, 128, 1000) and not listed(32768, 64, 1000) and not listed(65536, 128, 1000) and not listed((1 << 20) + 1, 128, 20000)
 
 
+def test_few_positions_load_their_ids_once_and_write_zeros_by_share():
+    def source(positions, width, segments):
+        return driver.HipKernel(op_desc.unsorted_segment_sum([positions], [width], segments, "float32", "int32", "f_%d" % positions), out_dir=None).source
+    assert "U = 1;" in source(512, 1000, 32768) and "U = 2;" in source(2000, 128, 2000) and "U = 8;" in source(8192, 256, 8000)
+    assert "BY_SHARE = true" in source(4096, 128, 2000) and "BY_SHARE = false" in source(4097, 128, 2000)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("positions,width,segments,dtype,ids,pattern", [
     (1, 65, 1, "float32", "int32", "uniform"), (3, 256, 7, "float32", "int64", "uniform"),
@@ -29,6 +36,10 @@ def test_sizes_whose_positions_are_listed():
     (8193, 200, 3000, "float32", "int32", "one_segment"), (30001, 130, 3000, "float32", "int32", "one_group"),   # by windows
     (9000, 100, 40000, "float32", "int32", "sorted"), (5000, 96, 3000, "float32", "int32", "outside"),
     (2000, 80, 77, "float32", "int32", "nobody"),
+    # zeros by share of adjacent segments: the last position count, pieces of 1 to 16 bytes, shares beyond the last segment
+    (4096, 128, 1000, "float32", "int32", "words"), (512, 65, 40001, "float32", "int32", "uniform"), (600, 129, 3000, "bfloat16", "int32", "words"),
+    (700, 130, 300, "int8", "int32", "uniform"), (1000, 68, 2000, "int64", "int64", "outside"), (520, 1026, 5000, "float16", "int32", "sorted"),
+    (2000, 300, 1025, "float32", "int32", "one_segment"), (4000, 72, 70000, "float32", "int32", "nobody"),
     (30001, 72, 900, "float16", "int32", "words"), (9000, 520, 1300, "bfloat16", "int64", "one_segment"),   # additions that round
     (3333, 100, 999, "int8", "int32", "uniform"), (5001, 70, 333, "int64", "int32", "words"), (100000, 66, 20000, "int32", "int32", "uniform"),
 ])
