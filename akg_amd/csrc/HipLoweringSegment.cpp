@@ -812,6 +812,8 @@ ChunkedPlan planChunked(const SegmentShapes &sh, const LoweringOptions &options)
   // Chunks: small ones while there are few, for workgroups; larger ones then, for longer runs. us with chunks of 512 / 1024 /
   // 2048 / 4096 positions: 35304 x 1 into 1131 8.4 / 9.0 / 10.3 / 11.4, 86700 x 3 into 8856 11.0 / 10.0 / 12.0 / 13.6, 138073 x 1
   // into 998 14.1 / 12.3 / 11.6 / 12.6, 300000 x 3 into 5000 22.7 / 18.6 / 14.4 / 16.0, 1536784 x 4 into 12654 91 / 56 / 42 / 34.
+  // (Rows of 16 bytes in chunks of 4096 spill 13 registers of <op>_place. Chunks of 2048 do not and are no faster: 12.5 million x 4 into
+  // 2216 224.9 us, 224.7 with 4096, 20 million x 4 into 16384 335 and 314, 2 million x 4 into 32768 48 and 42.)
   if (options.chunks == 0) p.tiles = sh.positions < (1 << 16) ? 1 : sh.positions < (1 << 17) ? 2 : sh.positions < (1 << 19) ? 4 : 8;
   p.chunk = 512LL * p.tiles;
   p.chunks = (sh.positions + p.chunk - 1) / p.chunk;

@@ -461,11 +461,12 @@ AKG_DEV double op_minimum(double a, double b) { return (a != a) ? a : ((b != b) 
 AKG_DEV int op_minimum(int a, int b) { return a < b ? a : b; }
 AKG_DEV long long op_minimum(long long a, long long b) { return a < b ? a : b; }
 
-// exp(x) = 2^f * 2^n with n = round(x log2 e), |f| <= 1/2: f as the rounded product less n plus what the rounding lost and
-// the part of log2 e below its float, one rounding in all; 2^f from the hardware, the scaling by ldexp, which rounds once
-// where the result is subnormal. n comes from the argument clamped to the range of results, the last term of f does not:
-// infinities, NaN and arguments beyond the range flow through it. Ten instructions, the device library's error (rms 2.62e-8,
-// 0.84 ulp at most) without its selects; float32 row kernels are bound by their vector instructions.
+// exp(x) = 2^f * 2^n with n = round(x log2 e), |f| <= 1/2 (Cody and Waite's reduction by a constant in two parts): f as the
+// rounded product less n plus what the rounding lost and the part of log2 e below its float, one rounding in all; 2^f from the
+// hardware, the scaling by ldexp, which rounds once where the result is subnormal. n comes from the argument clamped to the
+// range of results, the last term of f does not: infinities, NaN and arguments beyond the range flow through it. Ten
+// instructions, the device library's error (rms 2.62e-8, 0.84 ulp at most) without its selects; float32 row kernels are
+// bound by their vector instructions.
 AKG_DEV float op_exp(float x) {
   const float c = __builtin_amdgcn_fmed3f(x, -120.0f, 100.0f);
   const float p = c * 0x1.715476p+0f;
