@@ -429,7 +429,7 @@ class PlaneEmitter {
       src_ << "  " << ct << " " << acc << " = " << spec.init << ";  // " << op.name << " -> " << g_.tensor(out).name << "\n";
       src_ << "  for (unsigned p = tid; p < " << parts_ << "u; p += BLOCK) " << acc << " = " << spec.combiner << "::apply(" << acc
            << ", reinterpret_cast<const " << ct << " *>(akg_ws + " << partialAt_[static_cast<size_t>(out)] << "L)[akg_k * " << parts_ << "u + p]);\n";
-      src_ << "  " << acc << " = akg::group_reduce<" << spec.combiner << ", BLOCK>(" << acc << ", " << scratchExpr(ct) << ", tid);\n";
+      src_ << "  " << acc << " = akg::group_reduce<" << spec.combiner << ", BLOCK, true>(" << acc << ", " << scratchExpr(ct) << ", tid);\n";
       Val &v = vals_[static_cast<size_t>(out)];
       v.defined = true;
       v.ident = acc;
@@ -512,7 +512,7 @@ class PlaneEmitter {
       const DType od = g_.tensor(out).dtype;
       const lowering::ReduceSpec spec = lowering::reduceSpec(*op, od);
       const std::string ct = computeTypeName(od), acc = id("acc", out);
-      src_ << "  " << acc << " = akg::group_reduce<" << spec.combiner << ", BLOCK>(" << acc << ", " << scratchExpr(ct) << ", tid);\n";
+      src_ << "  " << acc << " = akg::group_reduce<" << spec.combiner << ", BLOCK, true>(" << acc << ", " << scratchExpr(ct) << ", tid);\n";
       if (parts_ != 0) {
         src_ << "  if (tid == 0) reinterpret_cast<" << ct << " *>(akg_ws + " << partialAt_[static_cast<size_t>(out)] << "L)[akg_wg] = " << acc << ";\n";
       }
