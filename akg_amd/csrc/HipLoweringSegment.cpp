@@ -847,11 +847,13 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
   const std::string ct = computeTypeName(out.dtype), tag = dtypeTag(out.dtype), idTag = dtypeTag(ids.dtype);
   const bool narrow = out.dtype == DType::F16 || out.dtype == DType::BF16 || out.dtype == DType::I8 || out.dtype == DType::I16;
   const std::string rndOpen = narrow ? tag + "::rnd(" : std::string("(");
-  // Rounds of the last launch: 4096 entries on eight wavefronts; few entries per bucket: one chunk's worth on two or four, as many
-  // as have a lane for every output element of the bucket (of which there are at most 256).
+  // Rounds of the last launch: 4096 entries on eight wavefronts; few entries per bucket: 2048 on four, or where chunks are 512 that many
+  // on two, if those have a lane for every output element of the bucket (of which there are at most 256). A frequent segment takes as
+  // many rounds as its positions: us, 100000 x 4 into 5000, rounds of 1024 / 2048 / 4096: ids as frequent as words 187 / 128 / 111 (136 by
+  // segment), uniform ones 10.1 / 10.4 / 11.4; chunks of 512, 60000 x 4 into 16000 uniform, rounds of 512 / 2048: 8.4 / 9.2.
   const bool small = sh.positions / plan.buckets < 1024 && plan.tiles <= 4;
   const int64_t perBucket = plan.perBucket, chains = perBucket * sh.slice;
-  const int nw = small ? (plan.tiles <= 2 && chains <= 128 ? 2 : 4) : 8, tiles = small ? static_cast<int>(plan.chunk) / (nw * 64) : 8;
+  const int nw = small ? (plan.tiles == 1 && chains <= 128 ? 2 : 4) : 8, tiles = small && plan.tiles == 1 ? static_cast<int>(plan.chunk) / (nw * 64) : 8;
   // (at least sixteen chains a wavefront: an addition is an instruction of the whole wavefront however few lanes add)
   const int64_t chainsPerWave = std::max<int64_t>(16, (chains + nw - 1) / nw);
   int keyBits = 1;

@@ -62,7 +62,7 @@ def _check_bits(positions, width, segments, dtype, ids, pattern, tmp_path):
 @pytest.mark.parametrize("positions,width,segments,dtype,split", [
     (33000, 1, 32768, "float32", 0), (33000, 3, 32768, "float32", 0), (65535, 4, 32768, "float32", 0), (40000, 4, 20000, "float32", 0),
     (40000, 3, 25000, "float32", 0), (33000, 4, 30000, "bfloat16", 0), (65535, 3, 32204, "int32", 0), (70000, 4, 16384, "float32", 0),
-    (540000, 4, 16384, "float32", 0), (40000, 4, 300, "float32", 0), (33000, 3, 6400, "float32", 100), (140000, 4, 6400, "float32", 100),
+    (540000, 4, 16384, "float32", 0), (40000, 4, 300, "float32", 0), (33000, 3, 6400, "float32", 100), (140000, 4, 6400, "float32", 100), (100000, 4, 5000, "float32", 0),
 ])
 def test_every_output_element_has_a_lane(positions, width, segments, dtype, split, monkeypatch):
     """One lane adds one output element: the wavefronts of the last launch have a lane for each element of a bucket."""
@@ -74,6 +74,7 @@ def test_every_output_element_has_a_lane(positions, width, segments, dtype, spli
     waves, rounds, chains, per_wave = map(int, re.search(r"W = (\d+), T = (\d+), CAP = .*CHAINS = (\d+), PER_WAVE = (\d+);", source).groups())
     chunk = 512 * int(re.search(r"NW = 8, TILES = (\d+)", source).group(1))
     assert chains >= width and per_wave <= 64 and waves * per_wave >= chains and waves * rounds * 64 >= chunk
+    assert waves * rounds * 64 >= (2048 if chunk > 512 else 512)   # a frequent segment takes as many rounds as its positions
 
 
 @pytest.mark.gpu
@@ -92,6 +93,7 @@ def test_buckets_of_many_output_elements(positions, width, segments, dtype, monk
     (4097, 2, 1025, "float32", "int32", "uniform", 8), (33000, 3, 4954, "float32", "int32", "uniform", 0),
     (300000, 1, 512, "float32", "int32", "uniform", 2),      # more chunks than a round looks up
     (9000, 4, 32768, "int32", "int32", "uniform", 4),        # 64 segments a bucket
+    (70001, 4, 5000, "float32", "int32", "uniform", 2), (70001, 2, 700, "bfloat16", "int32", "one_bucket", 2),   # rounds of two chunks
     (150000, 3, 9000, "float32", "int32", "one_segment", 8), (70000, 4, 600, "float32", "int32", "one_segment", 1),
     (100000, 3, 4954, "float32", "int32", "one_bucket", 4), (40000, 2, 3000, "float32", "int32", "sorted", 0),
     (40000, 2, 3000, "float32", "int32", "outside", 2), (20000, 1, 77, "float32", "int32", "nobody", 0),
