@@ -1014,9 +1014,8 @@ struct SmallTileOrder {
 //   workgroup = 2 x 2 wavefronts, 128 bytes of K per step, LDS double buffered (32 to 96 KiB)
 //   global -> registers -> LDS: two register sets, so the loads of a step are issued three steps ahead of its MFMAs: the
 //   time of a short K loop is that of its load latencies
-//   The order within a step is given: the reads of its second half first, MFMAs between the LDS writes and the loads that fill
-//   their registers anew. Left to itself the compiler gives both halves one set of operand registers and waits for all loads
-//   but one before the first MFMA: us, bf16 678 x 5568 x 2216 40 -> 31, f16 948 x 5184 x 6608 90 -> 82.
+//   The order within a step is given: MFMAs between the LDS writes and the loads that fill their registers anew. Left to itself
+//   the compiler waits for all loads but one before the first MFMA: us, bf16 678 x 5568 x 2216 40 -> 31, f16 948 x 5184 x 6608 90 -> 82.
 //   LDS rows without padding: the 16-byte chunks of a K-contiguous row r are permuted by (r >> 1) & 7, the 16-column units of
 //   a k-row of a row-major B by the bits of k that the lanes of one transposing read differ in; no bank is then hit twice
 //   by the lanes that are served together (which sixteen those are: see the 256 x 256 kernel; rows of 192 columns begin in
@@ -1034,6 +1033,10 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
   static_assert(K % 16 == 0 && N % 4 == 0, "whole 16-byte chunks of K, whole words of B's rows");
   static_assert(BM * K < (1L << 31) && (TRANSB ? BN * K : NB * KE) < (1L << 31), "operand too large for 32-bit buffer offsets");
   constexpr int BK = 128;
+  // Whether the operands of a half step are all read before its MFMAs begin. Larger tiles then hold more registers than they need: 128 x 128
+  // of a [K,N] weight of 8 bits 260 .. 284, one workgroup a CU for two (us, int8, 2282 x 1792 x 11456 91.7 -> 68.4, 1576 x 1728 x 2640 25.7 -> 21.5,
+  // 1602 x 1344 x 10624 52.2 -> 37.6; bf16 64 x 128 and larger 1 to 4 % in the mean). 64 x 64 of bf16 is up to 14 % faster with it.
+  constexpr bool kReadsFirst = BM * BN == 64 * 64;
   constexpr int kTM = BM / 32, kTN = BN / 32;          // 16 x 16 tiles per wavefront
   constexpr int kChunksA = BM / 32, kChunksB = BN / 32;  // 16-byte chunks per thread, step and operand
   constexpr long kTilesM = (M + BM - 1) / BM, kTilesN = (N + BN - 1) / BN, kTiles = kTilesM * kTilesN;
@@ -1197,7 +1200,7 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
   Frags f[2];
   auto step = [&](long s, int buf, Stage &next) {
     read(buf, 1, f[1]);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kReadsFirst) __builtin_amdgcn_sched_barrier(0);
     store(buf ^ 1, next);
     load(s + 3, next);
     multiply(f[0]);
@@ -1205,7 +1208,7 @@ AKG_DEV void gemm_small_tile(const void *__restrict__ A, const void *__restrict_
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     read(buf ^ 1, 0, f[0]);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kReadsFirst) __builtin_amdgcn_sched_barrier(0);
     multiply(f[1]);
     __builtin_amdgcn_sched_barrier(0);
   };

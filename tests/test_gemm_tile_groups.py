@@ -1,5 +1,6 @@
 """Workgroups of several small tiles: which products take them, and their results at the edges."""
 import re
+import subprocess
 
 import pytest
 
@@ -66,3 +67,14 @@ def test_tile_groups_against_float64(m, k, n, dtype, tb, tile, tmp_path):
     assert got == tile if tile else got
     units = "%dx%d" % tuple(128 if x % 128 == 0 else 64 for x in got[:2])
     _against_float64(m, k, n, dtype, tb, units, tmp_path)
+
+
+@pytest.mark.parametrize("m,k,n", [(1576, 1728, 2640), (2282, 1792, 11456), (801, 960, 11712), (1249, 1728, 9368)])
+def test_two_workgroups_of_128_x_128_fit_a_cu(m, k, n, tmp_path):
+    """Their four wavefronts have 256 registers each; with more a CU takes one of them only."""
+    assert _tile(m, k, n, "int8", False) == (128, 128, 1)
+    kernel = driver.HipKernel(_product(m, k, n, "int8", False, "registers"), out_dir=str(tmp_path))
+    code = next(str(f) for f in tmp_path.glob("*.hsaco") if kernel.kernel_name.startswith(f.stem))
+    notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", code], capture_output=True, text=True, check=True).stdout
+    assert int(re.search(r"\.vgpr_count:\s+(\d+)", notes).group(1)) <= 256
+    assert int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", notes).group(1)) == 0
