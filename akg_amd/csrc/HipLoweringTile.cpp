@@ -115,9 +115,9 @@ class TileEmitter {
   // the heads): the leading extents of the folded iteration space are kernel arguments too, and the operand's row
   // offset is computed from them, so the source does not carry them as numbers.
   bool dimsArg_ = false;
-  // The row length is an argument and a thread holds several chunks: chunk j of a short row of the bucket lies beyond the
-  // row for every lane of the wavefront. The elementwise ops and reduction steps between two row-wide results are then
-  // emitted chunk by chunk, and a wavefront leaves out the chunks none of its lanes has.
+  // Many rows of a length that is an argument, with much arithmetic, on half a wavefront each: a chunk of a short row of the bucket
+  // lies beyond the row for every lane of the wavefront. The elementwise ops and reduction steps between two row-wide results are
+  // then emitted chunk by chunk, and a wavefront leaves out the chunks none of its lanes has.
   bool chunkwise_ = false;
   std::ostringstream pending_;   // ... the steps of one chunk, until the next row-wide result
   int64_t bucketLow_ = 0, bucketHigh_ = 0;
@@ -437,12 +437,18 @@ class TileEmitter {
           if (ceilDiv(rowChunks, t) <= 8) break;
         }
       }
-      // Rows of any length in the bucket that a wavefront of two chunks a lane holds: two rows a wavefront with four chunks
-      // a lane instead, of which the wavefront leaves out those beyond the row (chunkwise_). Bound by its vector
-      // instructions, and the second chunk of 64 lanes costs a row of 257 elements as much as one of 512: float32 softmax
-      // with a shared mask, us, 64 x 2 -> 32 x 4: [32,12,333,333] 71 -> 67, [32,12,512,257] 95 -> 88, 300 wide 99 -> 93, 509 wide
-      // 78.4 -> 77.7; rows of whole 64-byte pieces stay (400 wide 105 -> 112).
-      if (colsArg_ && !colsWhole_ && !ordered_ && tpr == 64 && ceilDiv(rowChunks, tpr) == 2) tpr = 32;
+      // Rows of any length in the bucket that a wavefront of two chunks a lane holds: where vector instructions bound them, two rows a
+      // wavefront with four chunks a lane instead, of which the wavefront leaves out those beyond the row (chunkwise_). The second
+      // chunk of 64 lanes costs a row of 257 elements as much as one of 512. That takes many rows, as a row is a longer way for its
+      // lanes, and seven and more elementwise ops. us, 64 x 2 / 32 x 4: float32 softmax with scale and a shared mask,
+      // [32,12,333,257] 63 / 58, 333 wide 70.6 / 67.1, 450 wide 86 / 89, [16,12,200,333] 22.6 / 23.7, [3,12,2,471] 2.5 / 3.4; without them, of three ops,
+      // [60000,333] 30.4 / 31.1; scaling by the norm, which memory bounds, [60000,509] 43.7 / 50.
+      int arithmetic = 0;
+      for (const OpNode &op : g_.ops) {
+        if (lowering::isElementwiseKind(op.kind) && op.kind != OpKind::BroadcastTo && op.kind != OpKind::Reshape) ++arithmetic;
+      }
+      chunkwise_ = colsArg_ && !colsWhole_ && !ordered_ && rows_ >= 65536 && arithmetic >= 7 && tpr == 64 && ceilDiv(rowChunks, tpr) == 2;
+      if (chunkwise_) tpr = 32;
       tpr_ = tpr;
       int64_t perThread = ceilDiv(schedCols, static_cast<int64_t>(tpr_) * vec_);
       // More than 64 values per thread of one row-sized input, or 96 over all of them, do not stay in registers: walk the row in groups of
@@ -509,7 +515,6 @@ class TileEmitter {
       rowsPerBlock_ = block_ / tpr_;
       grid_ = ceilDiv(rows_, rowsPerBlock_);
       raggedCols_ = colsArg_ || (groups_ * chunks_ * tpr_ != rowChunks);
-      chunkwise_ = colsArg_ && !ordered_ && chunks_ > 1;
       raggedRows_ = (rows_ % rowsPerBlock_) != 0 || extentArg_;
     } else {
       block_ = opt_.block > 0 ? opt_.block : 256;
@@ -905,6 +910,18 @@ class TileEmitter {
     }
   }
 
+  // The step of every chunk: at once, or with the other steps up to the next row-wide result.
+  void emitChunks(const std::string &step) {
+    if (chunkwise_) {
+      pending_ << step;
+      return;
+    }
+    line("#pragma unroll");
+    line("  for (int j = 0; j < NCHUNK; ++j) {");
+    src_ << step;
+    line("  }");
+  }
+
   void flushChunks() {
     if (!chunkwise_ || pending_.str().empty()) return;
     line("#pragma unroll");
@@ -1219,7 +1236,7 @@ class TileEmitter {
     std::vector<std::string> operands;
     for (int in : op.inputs) operands.push_back(operandExpr(in));
     const bool relaxed = relaxed_[static_cast<size_t>(outId)];
-    std::string expr, chunkDivision;
+    std::string expr, chunkDivision, wholeDivision;
     // float32 division of a tile by a per-row (or constant) divisor: hoist the reciprocal out of the element loop
     const bool uniformDivisor = op.kind == OpKind::Div && rank == ValRank::Tile && op.inputs.size() == 2 &&
                                 vals_[static_cast<size_t>(op.inputs[1])].rank != ValRank::Tile &&
@@ -1242,7 +1259,11 @@ class TileEmitter {
         q = "akg::div_uniform(" + operands[0] + ", " + hoisted + ")";
         const ValInfo &dividend = vals_[static_cast<size_t>(op.inputs[0])];
         // (chunks of four: with eight the checks of a chunk hold its quotients back, int8 quantisation of bf16 rows 215 -> 222 us)
-        if (outT.dtype == DType::F32 && dividend.rank == ValRank::Tile && vec_ <= 4) chunkDivision = "akg::div_uniform(" + dividend.ident + "[j], " + hoisted + ", ";
+        if (outT.dtype == DType::F32 && dividend.rank == ValRank::Tile && vec_ <= 4) {
+          chunkDivision = "akg::div_uniform(" + dividend.ident + "[j], " + hoisted + ", ";
+          // (with more chunks their quotients wait for each other: softmax [32,12,333,700] 132 -> 138 us)
+          if (!chunkwise_ && chunks_ <= 2) wholeDivision = "akg::div_uniform(" + dividend.ident + ", " + hoisted + ", ";
+        }
       }
       const DType od = outT.dtype;
       expr = (od == DType::F16 || od == DType::BF16) ? std::string(dtypeTag(od)) + "::rnd(" + q + ")" : q;
@@ -1258,16 +1279,13 @@ class TileEmitter {
       nm << "t" << outId;
       v.ident = nm.str();
       src_ << "  " << ctOf(outId) << " " << v.ident << "[NCHUNK][V];  // " << op.name << " -> " << outT.name << "\n";
+      if (!wholeDivision.empty()) {
+        src_ << "  " << wholeDivision << v.ident << ");\n";
+        return;
+      }
       std::string step = "#pragma unroll\n    for (int e = 0; e < V; ++e) {\n      " + v.ident + "[j][e] = " + expr + ";\n    }\n";
       if (!chunkDivision.empty()) step = "    " + chunkDivision + v.ident + "[j]);\n";
-      if (chunkwise_) {
-        pending_ << step;
-      } else {
-        line("#pragma unroll");
-        line("  for (int j = 0; j < NCHUNK; ++j) {");
-        src_ << step;
-        line("  }");
-      }
+      emitChunks(step);
     } else {
       nm << "u" << outId;
       v.ident = nm.str();
@@ -1338,18 +1356,11 @@ class TileEmitter {
       fold << "#pragma unroll\n";
       fold << "    for (int e = 1; e < V; ++e) " << part << " = " << spec.combiner << "::apply(" << part << ", " << in.ident << "[j][e]);\n";
       fold << "    if (akg_ok[j]) " << acc << " = " << spec.combiner << "::apply(" << acc << ", " << part << ");\n";
-      if (chunkwise_) {
-        pending_ << fold.str();
-        return;
-      }
-      line("#pragma unroll");
-      line("  for (int j = 0; j < NCHUNK; ++j) {");
-      src_ << fold.str();
-      line("  }");
+      emitChunks(fold.str());
       return;
     }
     std::ostringstream fold;
-    if (chunkwise_ && spec.combiner == "akg::RedSum" && ct == "float" && !spec.roundEachStep) {
+    if (colsArg_ && chunks_ > 1 && spec.combiner == "akg::RedSum" && ct == "float" && !spec.roundEachStep) {
       // the chunk's sum as a tree (no more roundings in a row than a thread of two chunks had), elements of its neighbour as zeros
       const std::string part = "akg_part" + std::to_string(outId);
       fold << "    float " << part << "[V];\n";
@@ -1362,7 +1373,7 @@ class TileEmitter {
       fold << "      for (int e = 0; e + d < V; e += 2 * d) " << part << "[e] = akg::RedSum::apply(" << part << "[e], " << part << "[e + d]);\n";
       fold << "    }\n";
       fold << "    " << acc << " = akg::RedSum::apply(" << acc << ", " << part << "[0]);\n";
-      pending_ << fold.str();
+      emitChunks(fold.str());
       return;
     }
     fold << "#pragma unroll\n";
@@ -1379,14 +1390,7 @@ class TileEmitter {
       fold << "      " << acc << " = " << step << ";\n";
     }
     fold << "    }\n";
-    if (chunkwise_) {
-      pending_ << fold.str();
-      return;
-    }
-    line("#pragma unroll");
-    line("  for (int j = 0; j < NCHUNK; ++j) {");
-    src_ << fold.str();
-    line("  }");
+    emitChunks(fold.str());
   }
 
   void emitReduceFinish(const OpNode &op) {

@@ -576,6 +576,29 @@ AKG_DEV void div_uniform(const float (&a)[V], const UniformDivisor &d, float (&q
     for (int e = 0; e < V; ++e) q[e] = a[e] / d.b;
   }
 }
+// All dividends of a thread that has few: one branch for them (float32 softmax of 12 rows 2.1 -> 1.9 us). NaN is NaN on either way.
+template <int N, int V>
+AKG_DEV void div_uniform(const float (&a)[N][V], const UniformDivisor &d, float (&q)[N][V]) {
+  float least = 1.0f, most = 1.0f;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      const float aa = __builtin_fabsf(a[j][e]);
+      least = __builtin_fminf(least, aa <= d.zero ? 1.0f : aa);
+      most = __builtin_fmaxf(most, aa);
+      const float t = a[j][e] * d.rcp;
+      q[j][e] = __builtin_fmaf(-__builtin_fmaf(t, d.b, -a[j][e]), d.rcp, t);
+    }
+  }
+  if (__builtin_expect(!(d.safe && least >= 0x1p-60f && most <= 0x1p+60f), 0)) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) q[j][e] = a[j][e] / d.b;
+    }
+  }
+}
 
 // ---------------------------------------------------------------------------------------------------------
 // Relaxed math, used only for values whose every path to a kernel output passes through a cast to a 16-bit

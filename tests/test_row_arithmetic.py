@@ -1,13 +1,11 @@
 """Float32 arithmetic of the row kernels: the exponential over its whole range, division by a per-row value bit for bit the
-IEEE quotient, and rows of any length whose wavefronts leave out chunks."""
+IEEE quotient, and rows of any length in a bucket, among them those whose wavefronts leave out chunks."""
 import json
 
 import numpy as np
 import pytest
 
 from akg_amd import driver, op_desc
-
-pytestmark = pytest.mark.gpu
 
 
 def _run(kernel, arrays):
@@ -18,6 +16,7 @@ def _run(kernel, arrays):
     return [o.cpu().numpy() for o in outs]
 
 
+@pytest.mark.gpu
 def test_the_exponential_over_its_whole_range():
     """One unit in the last place at most where the result is normal, one step of 2^-149 where it is subnormal (the hardware's
     2^f is good to one unit, f to 2^-26); 0, infinity and NaN where they belong."""
@@ -39,6 +38,7 @@ def test_the_exponential_over_its_whole_range():
         assert (np.abs(got[finite].astype(np.float64) - want[finite]) / unit).max() <= 1.0
 
 
+@pytest.mark.gpu
 def test_division_by_a_row_value_is_the_ieee_quotient():
     """Zeros of both signs, subnormal and tiny dividends, infinities and NaN over positive, negative, tiny and huge divisors."""
     rng = np.random.default_rng(12)
@@ -57,6 +57,7 @@ def test_division_by_a_row_value_is_the_ieee_quotient():
         assert same.all(), np.argwhere(~same)[:5]
 
 
+@pytest.mark.gpu
 def test_division_by_a_row_maximum_is_the_ieee_quotient():
     """The row kernel's form: the divisor is a reduction, the dividends come in chunks."""
     rng = np.random.default_rng(13)
@@ -76,6 +77,7 @@ def test_division_by_a_row_maximum_is_the_ieee_quotient():
     assert same.all(), np.argwhere(~same)[:5]
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("cols", [257, 300, 383, 385, 509, 511, 1025, 1535, 2047])
 def test_rows_that_leave_out_chunks(cols):
     """One code object for every length of the bucket; softmax with a shared mask against float64: relative error of the
@@ -95,3 +97,46 @@ def test_rows_that_leave_out_chunks(cols):
     want = np.exp(t - t.max(2, keepdims=True))
     want /= want.sum(2, keepdims=True)
     assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max() and (np.abs(got - want) <= 2e-5 * want + 1e-30).all()
+
+
+def _scaled_masked_softmax():
+    """softmax(0.125 x + (1 - mask) * -10000) with every extent open."""
+    b = op_desc.DescBuilder("scaled_masked_softmax")
+    mask, x = b.input([7777, 1, 7778, 7779], "float32"), b.input([7777, 12, 7778, 7779], "float32")
+    s = b.add(b.mul(b.sub(b.const(1.0, "float32"), mask), b.const(-10000.0, "float32")), b.mul(b.const(0.125, "float32"), x))
+    e = b.unary("Exp", b.sub(s, b.reduce("ReduceMax", s, [3], True)))
+    text = b.dumps([b.div(e, b.reduce("ReduceSum", e, [3], True))])
+    return text.replace("7777", "-1").replace("7778", "-1").replace("7779", "-1")
+
+
+def test_rows_on_half_a_wavefront_are_many_and_full_of_arithmetic():
+    kernel = driver.HipDynamicKernel(_scaled_masked_softmax(), None)
+
+    def leaves_out(batch, rows, cols):
+        return "akg_some" in kernel.specialize([[batch, 1, rows, cols], [batch, 12, rows, cols]]).source
+    assert leaves_out(32, 333, 333) and leaves_out(16, 342, 509)
+    assert not leaves_out(16, 341, 333) and not leaves_out(32, 333, 400) and not leaves_out(32, 333, 255) and not leaves_out(32, 333, 700)
+    b = op_desc.DescBuilder("plain_softmax")
+    x = b.input([7777, 7778], "float32")
+    e = b.unary("Exp", b.sub(x, b.reduce("ReduceMax", x, [1], True)))
+    text = b.dumps([b.div(e, b.reduce("ReduceSum", e, [1], True))]).replace("7777", "-1").replace("7778", "-1")
+    assert "akg_some" not in driver.HipDynamicKernel(text, None).specialize([[100000, 333]]).source
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [257, 258, 383, 385, 509, 511])
+def test_many_rows_that_leave_out_chunks(cols):
+    """As above, 65664 rows; the argument of the exponential is at most 10000 + 2 wide where it is masked (then the exponential is
+    zero on both sides) and 4 elsewhere."""
+    import torch
+    shapes = [[16, 1, 342, cols], [16, 12, 342, cols]]
+    kernel = driver.HipDynamicKernel(_scaled_masked_softmax(), None).specialize(shapes)
+    assert "akg_some" in kernel.source
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    mask = (torch.rand(shapes[0], generator=g, device="cuda") > 0.3).float()
+    x = torch.randn(shapes[1], generator=g, device="cuda") * 4
+    out = torch.full(shapes[1], float("nan"), device="cuda")
+    kernel.launch([mask, x, out])
+    want = torch.softmax((1.0 - mask.double()) * -10000.0 + 0.125 * x.double(), -1)
+    wrong = (out.double() - want).abs()
+    assert bool((wrong <= 2e-5 * want + 1e-30).all())
