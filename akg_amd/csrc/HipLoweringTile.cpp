@@ -115,9 +115,9 @@ class TileEmitter {
   // the heads): the leading extents of the folded iteration space are kernel arguments too, and the operand's row
   // offset is computed from them, so the source does not carry them as numbers.
   bool dimsArg_ = false;
-  // Many rows of a length that is an argument, with much arithmetic, on half a wavefront each: a chunk of a short row of the bucket
-  // lies beyond the row for every lane of the wavefront. The elementwise ops and reduction steps between two row-wide results are
-  // then emitted chunk by chunk, and a wavefront leaves out the chunks none of its lanes has.
+  // Many rows of a length that is an argument, with much arithmetic: a chunk of a short row of the bucket lies beyond the row for
+  // every lane of the wavefront. The elementwise ops and reduction steps between two row-wide results are then emitted chunk by
+  // chunk, and a wavefront leaves out the chunks none of its lanes has.
   bool chunkwise_ = false;
   std::ostringstream pending_;   // ... the steps of one chunk, until the next row-wide result
   int64_t bucketLow_ = 0, bucketHigh_ = 0;
@@ -437,18 +437,18 @@ class TileEmitter {
           if (ceilDiv(rowChunks, t) <= 8) break;
         }
       }
-      // Rows of any length in the bucket that a wavefront of two chunks a lane holds: where vector instructions bound them, two rows a
-      // wavefront with four chunks a lane instead, of which the wavefront leaves out those beyond the row (chunkwise_). The second
-      // chunk of 64 lanes costs a row of 257 elements as much as one of 512. That takes many rows, as a row is a longer way for its
-      // lanes, and seven and more elementwise ops. us, 64 x 2 / 32 x 4: float32 softmax with scale and a shared mask,
-      // [32,12,333,257] 63 / 58, 333 wide 70.6 / 67.1, 450 wide 86 / 89, [16,12,200,333] 22.6 / 23.7, [3,12,2,471] 2.5 / 3.4; without them, of three ops,
+      // Rows of any length in the bucket that vector instructions bound: a wavefront leaves out the chunks beyond its row (chunkwise_), and
+      // where it would hold a row in two chunks a lane it takes two rows with four chunks a lane instead - the second chunk of 64
+      // lanes costs a row of 257 elements as much as one of 512. That takes many rows, as a row is a longer way for its lanes, and
+      // seven and more elementwise ops. us, all chunks on 64 lanes / this: float32 softmax with scale and a shared mask, [32,12,333,257] 63 / 58,
+      // 333 wide 70.6 / 67.1, 450 wide 86 / 89, 700 wide 141.5 / 134.4, [16,12,200,333] 22.6 / 23.7, [3,12,2,471] 2.5 / 3.4; without them, of three ops,
       // [60000,333] 30.4 / 31.1; scaling by the norm, which memory bounds, [60000,509] 43.7 / 50.
       int arithmetic = 0;
       for (const OpNode &op : g_.ops) {
         if (lowering::isElementwiseKind(op.kind) && op.kind != OpKind::BroadcastTo && op.kind != OpKind::Reshape) ++arithmetic;
       }
-      chunkwise_ = colsArg_ && !colsWhole_ && !ordered_ && rows_ >= 65536 && arithmetic >= 7 && tpr == 64 && ceilDiv(rowChunks, tpr) == 2;
-      if (chunkwise_) tpr = 32;
+      const bool manyHeavyRows = colsArg_ && !ordered_ && rows_ >= 65536 && arithmetic >= 7;
+      if (manyHeavyRows && !colsWhole_ && tpr == 64 && ceilDiv(rowChunks, tpr) == 2) tpr = 32;
       tpr_ = tpr;
       int64_t perThread = ceilDiv(schedCols, static_cast<int64_t>(tpr_) * vec_);
       // More than 64 values per thread of one row-sized input, or 96 over all of them, do not stay in registers: walk the row in groups of
@@ -515,6 +515,7 @@ class TileEmitter {
       rowsPerBlock_ = block_ / tpr_;
       grid_ = ceilDiv(rows_, rowsPerBlock_);
       raggedCols_ = colsArg_ || (groups_ * chunks_ * tpr_ != rowChunks);
+      chunkwise_ = manyHeavyRows && chunks_ > 1;
       raggedRows_ = (rows_ % rowsPerBlock_) != 0 || extentArg_;
     } else {
       block_ = opt_.block > 0 ? opt_.block : 256;
@@ -1261,8 +1262,9 @@ class TileEmitter {
         // (chunks of four: with eight the checks of a chunk hold its quotients back, int8 quantisation of bf16 rows 215 -> 222 us)
         if (outT.dtype == DType::F32 && dividend.rank == ValRank::Tile && vec_ <= 4) {
           chunkDivision = "akg::div_uniform(" + dividend.ident + "[j], " + hoisted + ", ";
-          // (with more chunks their quotients wait for each other: softmax [32,12,333,700] 132 -> 138 us)
-          if (!chunkwise_ && chunks_ <= 2) wholeDivision = "akg::div_uniform(" + dividend.ident + ", " + hoisted + ", ";
+          // Whole rows: float32 softmax of 8 x 100 3.7 us chunk by chunk, 2.6 (3.3 one by one), 8 x 10000 4.3, 3.6 (4.0). With more than two
+          // chunks of a row of any length the quotients wait for chunks beyond it: softmax with a mask [32,12,333,700] 132 -> 138 us.
+          if (!chunkwise_ && (chunks_ <= 2 || !colsArg_)) wholeDivision = "akg::div_uniform(" + dividend.ident + ", " + hoisted + ", ";
         }
       }
       const DType od = outT.dtype;
