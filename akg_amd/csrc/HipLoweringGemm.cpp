@@ -59,7 +59,7 @@ class GemmEmitter {
       k.grid[0] = static_cast<unsigned>(((m_ + 63) / 64) * ((n_ + 16 * epiWidth() - 1) / (16 * epiWidth())));
       k.block[0] = 256;
     } else if (skinny_) {
-      const int64_t strips = (n_ + 127) / 128;
+      const int64_t strips = (n_ + stripCols() - 1) / stripCols();
       k.grid[0] = static_cast<unsigned>(strips * kSplit_);
       if (kSplit_ > 1) {
         const int64_t groups = strips * batch_;
@@ -99,8 +99,8 @@ class GemmEmitter {
       note << " serial: the reference's k-ordered sum in the declared type on the vector ALUs, tile=64x" << 16 * epiWidth()
            << " grid=" << k.grid[0];
     } else if (skinny_) {
-      note << " skinny: strips of 128 columns, B " << (skinnyLines() ? (streamsLines() ? "by whole lines past the caches" : "by whole lines") : "straight into MFMA operands")
-           << ", mfma=" << mfmaName(false) << " waves=" << skinnyWaves() << " grid=" << k.grid[0];
+      note << " skinny: strips of " << stripCols() << " columns, B " << (narrowCols_ > 0 ? "straight into MFMA operands, all of K" : skinnyLines() ? (streamsLines() ? "by whole lines past the caches" : "by whole lines") : "straight into MFMA operands")
+           << ", mfma=" << mfmaName(narrowCols_ > 0) << " waves=" << skinnyWaves() << " grid=" << k.grid[0];
     } else if (tileM_ > 0) {
       const int unitM = tileM_ % 128 == 0 ? 128 : 64, unitN = tileN_ % 128 == 0 ? 128 : 64;
       note << " tile=" << unitM << "x" << unitN << "x" << stepK() / elemBytes() << " mfma=" << mfmaName(true) << " waves=2x2 grid=" << k.grid[0];
@@ -122,8 +122,9 @@ class GemmEmitter {
   int64_t m_ = 0, n_ = 0, k_ = 0, batch_ = 1;
   int kSplit_ = 1;  // workgroups per tile, each with a range of K steps (see pickSplit)
   int skinnyRows() const { return 64; }   // (96 rows: no faster than the tile kernel; 128: slower)
-  int skinnyWaves() const { return opt_.block == 512 ? 8 : 4; }
-  int skinnyUnroll() const { return opt_.chunks > 0 ? opt_.chunks : 2; }
+  int skinnyWaves() const { return narrowCols_ > 0 ? narrowWaves_ : (opt_.block == 512 ? 8 : 4); }
+  int skinnyUnroll() const { return opt_.chunks > 0 ? opt_.chunks : (narrowCols_ > 0 ? (transB_ ? 4 : 2) : 2); }
+  int stripCols() const { return narrowCols_ > 0 ? narrowCols_ : 128; }
   // A [N,K] weight with a short K is read in 32-byte pieces, four per cache line, by instructions that follow each other:
   // with the non-temporal hint the line is not kept for the next piece. (skinnyLines() reads whole lines.)
   bool skinnyNonTemporal() const { return opt_.nonTemporal != 0 && !transB_; }
@@ -148,12 +149,14 @@ class GemmEmitter {
   }
   // ... as the kernel's last argument, behind the other ones that have defaults
   std::string linesArgument(const std::string &before) const {
+    if (narrowCols_ > 0) return before + ", akg::NarrowStrips<" + std::to_string(narrowCols_) + ">()";
     if (!transB_) return "";
     return streamsLines() ? before + ", akg::StreamedLines()" : (skinnyLines() ? "" : before + ", akg::NoLines()");
   }
   bool serial_ = false;  // no MFMA kernel takes the description: gemm_serial (akg_gemm_serial.hpp)
   int epiWidth() const { return (serial_ && n_ % 4 != 0) ? 1 : 4; }   // adjacent result columns per epilogue call
   int tileM_ = 0, tileN_ = 0;   // gemm_small_tile: its tile (0: another kernel)
+  int narrowCols_ = 0, narrowWaves_ = 8;   // gemm_skinny_narrow: columns of a strip (0: another kernel), wavefronts
   bool skinny_ = false;  // M <= 64: the kernel that streams B, without barriers (gemm_skinny)
   // A dynamic description (extents bound per call): M and the K split are kernel arguments, so the source - and with it
   // the code object - is the same for every token count; the skinny kernel comes in three sizes (16, 32, 64 rows).
@@ -334,7 +337,10 @@ class GemmEmitter {
     kSplit_ = 1;
     if (serial_) return;
     dyn_ = opt_.extentAsArgument && batch_ == 1;
-    if (pickSmallTile()) return;
+    if (pickSmallTile()) {
+      if (m_ > skinnyRows() || !pickNarrow(0.8 * smallTileRowsTime(kSplit_))) return;
+      tileM_ = tileN_ = 0;
+    }
     kSplit_ = 1;
     // At most 64 rows of A (and K a multiple of 32 bytes): the time is that of streaming B, which gemm_skinny reads
     // straight into MFMA operands, or a [N,K] one by whole lines through LDS of each wavefront (skinnyLines()); 256
@@ -344,11 +350,62 @@ class GemmEmitter {
     // AKG_HIP_VARIANT bit 3 keeps the 256 x 256 tile kernel.
     skinny_ = skinnyTakes();
     if (skinny_) {
+      if (narrowCols_ > 0) return;   // (instead of small tiles)
       kSplit_ = static_cast<int>(skinnySplit());
+      if (pickNarrow(m_ <= 32 ? 0.92 * wideStripTime() : 0.85 * skinnyTime(kSplit_))) kSplit_ = 1;
       return;
     }
     if (batch_ != 1) return;
     kSplit_ = static_cast<int>(largeTileSplit());
+  }
+
+  // us of the narrow strips, fitted to 122 products of at most 64 rows on 16, 32 and 64 columns (575 in all, both layouts, 8 and 16
+  // bits, 0.4 to 96 MB of weight; standard deviation 12 %): a start, what a CU takes in of the weight and of A (32 columns of
+  // 16-bit k-rows are half lines), and the weight from memory.
+  double narrowTime(int64_t cols) const {
+    const double kb = static_cast<double>(k_ * elemBytes()) / 1024, mb = static_cast<double>(k_ * n_ * elemBytes()) * 1e-6;
+    const double strips = static_cast<double>((n_ + cols - 1) / cols) / 256;
+    const double perCu = (strips <= 1 ? 1 : 0.5 * (strips + std::ceil(strips))) * kb, rows = static_cast<double>(m_), width = static_cast<double>(cols);
+    if (transB_) return 3.02 + perCu * (0.0104 * width + 0.014 * rows) + 0.091 * mb;
+    if (elemBytes() == 1) return 2.74 + perCu * (0.0195 * width + 0.026 * rows) + 0.119 * mb;
+    return cols == 32 ? 2.33 + perCu * (0.0173 * width + 0.0172 * rows) + 0.107 * mb : 2.4 + perCu * (0.0145 * width + 0.019 * rows) + 0.102 * mb;
+  }
+  // ... and of the strips of 128 columns for at most 32 rows (90 of the same products, 6 %).
+  double wideStripTime() const {
+    const double mb = static_cast<double>(k_ * n_ * elemBytes()) * 1e-6, rows = static_cast<double>(m_), splits = static_cast<double>(skinnySplit());
+    const double idle = std::max(0.0, 224 / (static_cast<double>((n_ + 127) / 128) * splits) - 1);
+    if (transB_) return 5.41 + mb * ((elemBytes() == 1 ? 0.147 : 0.135) + 0.00174 * rows) + 0.0068 * splits * rows;
+    return 6.32 + mb * ((elemBytes() == 1 ? 0.235 : 0.15) + 0.00196 * rows - 0.094 * idle) + 0.0108 * splits * rows;
+  }
+  // Narrow strips, each the whole K of one workgroup, where they are estimated faster than the kernel that `other` us are the estimate
+  // of: they save the exchange of partials (3 of 6 us), and lose where few strips leave CUs idle with a long K, or where the rows of A,
+  // which every strip reads, weigh more than its columns. us, strips of 128 columns / narrow ones: bf16 [N,K] 8 x 640 x 1336 6.0 / 3.2,
+  // 4 x 5056 x 2176 10.0 / 6.2, 32 x 7040 x 1832 13.7 / 11.0, 16 x 7360 x 3536 15.5 / 13.5; [K,N] 2 x 512 x 2912 5.3 / 3.4, 25 x 896 x 5656 9.2 / 5.2,
+  // 16 x 2880 x 5408 11.3 / 7.7, 5 x 6592 x 560 8.1 / 12.7, 26 x 5248 x 8632 27 / 32; int8 [N,K] 9 x 2688 x 3760 7.7 / 4.4, [K,N] 1 x 1920 x
+  // 4808 8.2 / 6.3; small tiles / narrow strips: int8 [K,N] 49 x 1856 x 11256 16.6 / 10.0, bf16 [N,K] 62 x 1536 x 5880 7.7 / 8.1. Of the 122
+  // products 0.80 of the time in the geometric mean, the worst 1.1 of it.
+  // More than 32 rows only with the weights that were measured, up to 24 MiB. A weight that is read past the caches keeps its kernel, as does one of a description with an open
+  // row count or of several batches. (AKG_HIP_VARIANT bit 8 keeps the strips of 128 columns.)
+  bool pickNarrow(double other) {
+    narrowCols_ = 0;
+    if (dyn_ || batch_ != 1 || !skinnyTakes() || opt_.split > 0 || opt_.block > 0 || opt_.chunks > 0 || (opt_.variant & 256)) return false;
+    const int64_t kBytes = k_ * elemBytes();
+    if (kBytes % 64 != 0 || kBytes < 640 || weightBytes() >= ((m_ <= 32 ? 96LL : 24LL) << 20)) return false;
+    int64_t cols = 0;
+    double best = other;
+    for (const int64_t width : {16, 32, 64}) {
+      if (!transB_ && width * elemBytes() < 64) continue;
+      const double t = narrowTime(width);
+      if (t < best) {
+        best = t;
+        cols = width;
+      }
+    }
+    narrowCols_ = static_cast<int>(cols);
+    // (eight wavefronts where each has two to four units of K: us, 17 x 1280 x 1368 4.36 on four and 4.23, 2 x 3584 x 4192 7.3 and 7.7)
+    const int64_t units = (kBytes + 127) / 128;
+    narrowWaves_ = m_ <= 32 && units >= 12 && units <= 32 ? 8 : 4;
+    return cols > 0;
   }
 
   int64_t largeTileSplit() const {

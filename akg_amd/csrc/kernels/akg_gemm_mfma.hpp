@@ -668,19 +668,239 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
 // DYN: MS is the most rows the code object takes (16, 32 or 64), the actual row count and the number of K splits are
 // kernel arguments (`mDyn` <= MS, `ksDyn`); `ws` is always a valid pointer.
 // UNROLL and NT are those of the operands loaded as they are; whole lines of a [N,K] weight are one in flight, past the
-// caches with StreamedLines. With NoLines the operands are loaded as they are whatever the length of K.
+// caches with StreamedLines. With NoLines the operands are loaded as they are whatever the length of K. NarrowStrips is
+// gemm_skinny_narrow, whose strips have COLS columns and whose UNROLL is the units in flight.
 struct CachedLines {
   static constexpr bool kWhole = true, kPastCaches = false;
+  static constexpr int kNarrow = 0;
 };
 struct StreamedLines {
   static constexpr bool kWhole = true, kPastCaches = true;
+  static constexpr int kNarrow = 0;
 };
 struct NoLines {
   static constexpr bool kWhole = false, kPastCaches = false;
+  static constexpr int kNarrow = 0;
 };
+template <int COLS>
+struct NarrowStrips {
+  static constexpr bool kWhole = false, kPastCaches = false;
+  static constexpr int kNarrow = COLS;
+};
+
+// Few rows and a weight of which a CU's share is little: narrow strips of columns, each the whole K of one workgroup, so that
+// nothing is exchanged between workgroups (which took 3 of the 6 us of 8 x 640 x 1336: 6.0 -> 3.2; 16 x 2880 x 5408 [K,N] 11.3 -> 7.7).
+//   What bounds it is what one CU takes in: 32 KiB of lines on their way at a time, 54 GB/s from memory (146 from L2).
+//   workgroup = WAVES wavefronts, one strip of COLS columns; wavefront w takes the units w, w + WAVES, ... of K, DEPTH of them in flight
+//   a unit is 128 bytes of K, two MFMA steps. An instruction loads the lines of eight rows of A, or of eight columns of a [N,K]
+//   weight, and the operands are formed through LDS of the wavefront's own. (16 x 16 MFMAs take 64 bytes of K from 16 rows and
+//   columns: loading those as they are touches every line twice, and a CU then takes in 28 .. 35 GB/s of the 54 it can.)
+//   [K,N]: lane (c, g) loads COLS / 16 adjacent columns of its own 8 (16-bit) or 16 k-rows of a step and turns them into operands in
+//   registers
+// The operands of the MFMA are exchanged, as in gemm_small_tile. The wavefronts add their accumulators through LDS.
+template <typename Mma, long M, long N, long KE, bool TRANSB, typename Epilogue, int WAVES, int COLS, int DEPTH>
+AKG_DEV void gemm_skinny_narrow(const void *__restrict__ A, const void *__restrict__ B, Epilogue &epi) {
+  constexpr int EB = Mma::kElemBytes;
+  constexpr long K = KE * EB, NB = N * EB;
+  static_assert(M >= 1 && M <= 64 && K % 64 == 0 && N % 4 == 0, "few rows, whole steps of K, whole chunks of columns");
+  static_assert(COLS == 16 || COLS == 32 || COLS == 64, "one, two or four tiles of 16 columns");
+  static_assert(TRANSB || COLS * EB / 16 >= 4, "a lane's columns of a k-row fill a word");
+  static_assert(M * K < (1L << 31) && NB * KE < (1L << 31), "operand too large for 32-bit buffer offsets");
+  constexpr int kRowTiles = static_cast<int>((M + 15) / 16), kColTiles = COLS / 16, kThreads = WAVES * 64;
+  constexpr int kUnitSteps = 2;
+  constexpr long kSteps = K / 64, kUnits = (kSteps + kUnitSteps - 1) / kUnitSteps, kStrips = (N + COLS - 1) / COLS;
+  constexpr int kKRows = 16 / EB, kRowWords = TRANSB ? 1 : kColTiles * EB / 4;   // [K,N]: k-rows of a lane, words of one
+  typedef typename Mma::acc_t acc_t;
+  typedef typename Mma::acc4_v acc4_v;
+  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  // (neighbouring strips of a [K,N] weight share lines: on one XCD)
+  const long strip = TRANSB ? static_cast<long>(blockIdx.x) : xcd_contiguous_id(static_cast<int>(blockIdx.x), static_cast<int>(kStrips));
+  const __amdgpu_buffer_rsrc_t aRsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(A), 0, static_cast<int>(M * K), 0x00020000);
+  const __amdgpu_buffer_rsrc_t bRsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(B), 0, static_cast<int>(NB * KE), 0x00020000);
+  constexpr int kLoadsA = static_cast<int>((M + 7) / 8), kLoads = TRANSB ? 2 * kColTiles : 1;   // eight rows or columns each
+  u32 aOff[kLoadsA], bOff[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoadsA; ++i) {
+    const long row = 8 * i + (lane >> 3) < M ? 8 * i + (lane >> 3) : M - 1;   // (what lies in rows beyond M: their results are dropped)
+    aOff[i] = static_cast<u32>(row * K + (lane & 7) * 16);
+  }
+  if constexpr (TRANSB) {
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      const long col = strip * COLS + 8 * j + (lane >> 3);
+      bOff[j] = static_cast<u32>((col < N ? col : N - 1) * K + (lane & 7) * 16);
+    }
+  } else {
+    const long col = strip * COLS + kColTiles * c;   // (a chunk of columns beyond N reads zero, beyond the buffer)
+    bOff[0] = col < N ? static_cast<u32>(g * kKRows * NB + col * EB) : kBeyondEveryBuffer;
+  }
+  struct Unit {
+    v4i a[kLoadsA], b[kLoads];
+    u32 w[TRANSB ? 1 : kUnitSteps * kKRows][kRowWords];
+  };
+  constexpr int kChunks = COLS / 4;                                                   // of a row of the result
+  constexpr int kSumBytes = WAVES * static_cast<int>(M) * COLS * 4, kLines = 16 * kRowTiles + (TRANSB ? COLS : 0), kLineBytes = WAVES * kLines * 128;
+  __shared__ __attribute__((aligned(16))) u8 akg_narrow_lds[kSumBytes > kLineBytes ? kSumBytes : kLineBytes];
+  u8 *__restrict__ linesA = akg_narrow_lds + wave * (kLines * 128), *__restrict__ linesB = linesA + 16 * kRowTiles * 128;
+  // Strips begin at different units: the same unit of all strips of a [N,K] weight lies a multiple of the row pitch apart.
+  const long rot = strip % kUnits;
+  auto stepOf = [&](long i) {
+    const long u = wave + i * WAVES + rot;
+    return (u >= kUnits ? u - kUnits : u) * kUnitSteps;
+  };
+  auto load = [&](long i, Unit &u) {
+    const long t = stepOf(i);
+#pragma unroll
+    for (int j = 0; j < kLoadsA; ++j) u.a[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(aRsrc, aOff[j], static_cast<int>(t * 64), 0));
+    if constexpr (TRANSB) {
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) u.b[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(bRsrc, bOff[j], static_cast<int>(t * 64), 0));
+    } else {
+#pragma unroll
+      for (int j = 0; j < kUnitSteps * kKRows; ++j) {   // (k-rows behind the last one are beyond the buffer)
+        const int row = static_cast<int>((t * (64 / EB) + j / kKRows * (64 / EB) + j % kKRows) * NB);
+        if constexpr (kRowWords == 2) {
+          const auto q = __builtin_amdgcn_raw_buffer_load_b64(bRsrc, bOff[0], row, 0);
+          u.w[j][0] = q[0];
+          u.w[j][1] = q[1];
+        } else {
+          u.w[j][0] = __builtin_amdgcn_raw_buffer_load_b32(bRsrc, bOff[0], row, 0);
+        }
+      }
+    }
+  };
+  acc4_v acc[kRowTiles][kColTiles];
+#pragma unroll
+  for (int r = 0; r < kRowTiles; ++r) {
+#pragma unroll
+    for (int j = 0; j < kColTiles; ++j) acc[r][j] = acc4_v{0, 0, 0, 0};
+  }
+  auto multiply = [&](long i, const Unit &u) {
+    // (chunks permuted by the row as in gemm_small_tile; a wavefront's LDS accesses complete in program order)
+    const long t = stepOf(i);
+    const auto place = [&](u8 *to, int row, v4i v) { *reinterpret_cast<v4i *>(to + row * 128 + ((lane & 7) ^ ((row >> 1) & 7)) * 16) = v; };
+    const auto operand = [&](const u8 *from, int tile, int s) {
+      return *reinterpret_cast<const v4i *>(from + (16 * tile + c) * 128 + ((4 * s + g) ^ ((c >> 1) & 7)) * 16);
+    };
+#pragma unroll
+    for (int j = 0; j < kLoadsA; ++j) place(linesA, 8 * j + (lane >> 3), u.a[j]);
+    if constexpr (TRANSB) {
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) place(linesB, 8 * j + (lane >> 3), u.b[j]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int s = 0; s < kUnitSteps; ++s) {
+      if (kSteps % kUnitSteps != 0 && t + s >= kSteps) continue;   // (uniform: the half unit behind the last step)
+      v4i a[kRowTiles], b[kColTiles];
+#pragma unroll
+      for (int r = 0; r < kRowTiles; ++r) a[r] = operand(linesA, r, s);
+      const auto &w = u.w;
+      if constexpr (TRANSB) {
+#pragma unroll
+        for (int j = 0; j < kColTiles; ++j) b[j] = operand(linesB, j, s);
+      } else if constexpr (EB == 2) {
+#pragma unroll
+        for (int i2 = 0; i2 < 4; ++i2) {   // k-rows 2 i2 and the next one -> word i2 of every column's operand
+          const int k = s * kKRows + 2 * i2;
+#pragma unroll
+          for (int h = 0; h < kRowWords; ++h) {
+            b[2 * h][i2] = static_cast<int>(pack_lo16(w[k][h], w[k + 1][h]));
+            b[2 * h + 1][i2] = static_cast<int>(pack_hi16(w[k][h], w[k + 1][h]));
+          }
+        }
+      } else {
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const int k = s * kKRows + 4 * i4;
+          const u32 rows[4] = {w[k][0], w[k + 1][0], w[k + 2][0], w[k + 3][0]};
+          u32 cols[4];
+          transpose4x4_bytes(rows, cols);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) b[j][i4] = static_cast<int>(cols[j]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < kColTiles; ++j) {
+#pragma unroll
+        for (int r = 0; r < kRowTiles; ++r) acc[r][j] = Mma::mma16(b[j], a[r], acc[r][j]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  // DEPTH units in flight. Every wavefront has at least kLeast of them, requested without a condition.
+  constexpr long kLeast = kUnits / WAVES;
+  const long mine = wave < kUnits ? (kUnits - wave + WAVES - 1) / WAVES : 0;
+  Unit flight[DEPTH];
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) {
+    if (d < kLeast || d < mine) load(d, flight[d]);
+  }
+  long i = 0;
+  for (; i + 2 * DEPTH <= mine; i += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      multiply(i + d, flight[d]);
+      load(i + DEPTH + d, flight[d]);
+    }
+  }
+  for (; i < mine; i += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      if (i + d < mine) multiply(i + d, flight[d]);
+      if (i + DEPTH + d < mine) load(i + DEPTH + d, flight[d]);
+    }
+  }
+
+  // ---- the wavefronts' sums: chunks of four adjacent columns, permuted by the row
+  acc4_v (*akg_narrow_sum)[M][kChunks] = reinterpret_cast<acc4_v (*)[M][kChunks]>(akg_narrow_lds);
+  const int q = tid % kChunks;
+  const long col = strip * COLS + 4 * q;
+  if (col < N) epi.prepare(col);
+  __syncthreads();   // (the sums lie where the lines did)
+#pragma unroll
+  for (int r = 0; r < kRowTiles; ++r) {
+    const int row = 16 * r + c;
+    if (row < M) {
+#pragma unroll
+      for (int j = 0; j < kColTiles; ++j) {
+        acc4_v v;
+        int at;
+        if constexpr (TRANSB) {          // tile j, columns 4 g ..
+          v = acc[r][j];
+          at = 4 * j + g;
+        } else if constexpr (kColTiles == 4) {   // column 4 r' + j of operand row r' = 4 g + i
+          v = acc4_v{acc[r][0][j], acc[r][1][j], acc[r][2][j], acc[r][3][j]};
+          at = 4 * g + j;
+        } else {                         // column 2 r' + j
+          v = acc4_v{acc[r][0][2 * j], acc[r][1][2 * j], acc[r][0][2 * j + 1], acc[r][1][2 * j + 1]};
+          at = 2 * g + j;
+        }
+        akg_narrow_sum[wave][row][at ^ (row & (kChunks - 1))] = v;
+      }
+    }
+  }
+  __syncthreads();
+  for (int row = tid / kChunks; row < M; row += kThreads / kChunks) {
+    acc4_v sum = akg_narrow_sum[0][row][q ^ (row & (kChunks - 1))];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum += akg_narrow_sum[w][row][q ^ (row & (kChunks - 1))];
+    const acc_t a4[4] = {sum[0], sum[1], sum[2], sum[3]};
+    if (col < N) epi.apply(a4, row, col);
+  }
+}
+
 template <typename Mma, long MS, long N, long KE, bool TRANSB, typename Epilogue, int KSPLIT, int WAVES = 4, int UNROLL = 2, bool NT = false, bool DYN = false, typename Lines = CachedLines>
 AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ Bv, Epilogue &epi,
                          unsigned *__restrict__ ws, long group0, long mDyn = 0, int ksDyn = 1, Lines = Lines()) {
+  if constexpr (Lines::kNarrow > 0) {
+    static_assert(!DYN && KSPLIT == 1, "a strip is one workgroup's");
+    gemm_skinny_narrow<Mma, MS, N, KE, TRANSB, Epilogue, WAVES, Lines::kNarrow, UNROLL>(Av, Bv, epi);
+    return;
+  } else {
   const long M = DYN ? mDyn : MS;
   const int kSplits = DYN ? ksDyn : KSPLIT;
   constexpr bool kSplitPossible = DYN || KSPLIT > 1;
@@ -981,6 +1201,7 @@ AKG_DEV void gemm_skinny(const void *__restrict__ Av, const void *__restrict__ B
   for (int i = 0; i < kRowsPerThread; ++i) {
     const int row = r0 + 8 * i;
     if (row < M) epi.apply(sum[i], row, col);
+  }
   }
 }
 
