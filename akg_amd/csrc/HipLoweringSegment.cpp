@@ -432,25 +432,24 @@ __device__ inline void chunk_sort(const int (&key)[TILES], unsigned (&slot)[TILE
   const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, w = tid >> 6;
   for (int k = tid; k < NW * KEYS; k += THREADS) cnt[k] = 0;
   __syncthreads();
-  const unsigned long long below = (1ull << lane) - 1ull;
   unsigned short *mine = cnt + w * KEYS;
 #pragma unroll
   for (int u = 0; u < TILES; ++u) {
     const int k = key[u] >= 0 ? key[u] : 0;
-    unsigned long long same = __ballot(key[u] >= 0);
+    const unsigned long long part = __ballot(key[u] >= 0);
+    unsigned lo = static_cast<unsigned>(part), hi = static_cast<unsigned>(part >> 32);   // lanes with the same key
 #pragma unroll
     for (int bit = 0; bit < KEY_BITS; ++bit) {
-      const int mine_bit = __builtin_amdgcn_sbfe(k, bit, 1);   // 0 or all ones
-      const unsigned long long with = __ballot(mine_bit != 0);
-      const unsigned lo = ~(static_cast<unsigned>(with) ^ static_cast<unsigned>(mine_bit));
-      const unsigned hi = ~(static_cast<unsigned>(with >> 32) ^ static_cast<unsigned>(mine_bit));
-      same &= (static_cast<unsigned long long>(hi) << 32) | lo;   // lanes whose bit equals mine
+      const unsigned mine_bit = static_cast<unsigned>(__builtin_amdgcn_sbfe(k, bit, 1));   // 0 or all ones
+      const unsigned long long with = __ballot(mine_bit != 0u);
+      lo &= ~(static_cast<unsigned>(with) ^ mine_bit);
+      hi &= ~(static_cast<unsigned>(with >> 32) ^ mine_bit);   // lanes whose bit equals mine
     }
     slot[u] = 0u;
     if (key[u] >= 0) {
-      const unsigned at = mine[k] + static_cast<unsigned>(__popcll(same & below));
-      slot[u] = at;
-      if ((same >> lane) >> 1 == 0ull) mine[k] = static_cast<unsigned short>(at + 1u);   // the group's highest lane
+      const unsigned before = mine[k];
+      slot[u] = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, before));
+      mine[k] = static_cast<unsigned short>(before + static_cast<unsigned>(__popc(lo) + __popc(hi)));   // (the same from every lane of the key)
     }
   }
   __syncthreads();
@@ -497,6 +496,44 @@ __device__ inline void chunk_sort(const int (&key)[TILES], unsigned (&slot)[TILE
   for (int u = 0; u < TILES; ++u) {
     if (key[u] >= 0) slot[u] += mine[key[u]];
   }
+}
+)AKG";
+
+// Device code of the launches that add lists out of LDS.
+const char *const kAddList = R"AKG(
+// acc, then list[0] .. list[n - 1] added to it one after the other. `list` begins at a multiple of 16 bytes; up to 384 bytes behind its
+// end are read and not added. An addition takes 4.4 cycles and LDS up to 230, so every value is requested 44 additions ahead and the
+// order is given: left to itself the compiler requests values in front of the last two additions before them (13.7 cycles an addition).
+constexpr int ADD_BLOCK = 48;
+template <typename T, typename Add>
+__device__ inline T add_list(const T *list, int n, T acc, Add add) {
+  typedef T quad_t __attribute__((ext_vector_type(4)));
+  constexpr int BLOCK = ADD_BLOCK, QUADS = BLOCK / 4;
+  const quad_t *quads = reinterpret_cast<const quad_t *>(list);
+  quad_t q[QUADS];
+#pragma unroll
+  for (int i = 0; i < QUADS; ++i) q[i] = quads[i];
+  int j = 0;
+  for (; j + BLOCK <= n; j += BLOCK) {
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc = add(q[i][u], acc);
+      q[i] = quads[j / 4 + QUADS + i];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < BLOCK; h += 8) {
+    if (j + h < n) {
+#pragma unroll
+      for (int u = h; u < h + 8; ++u) {
+        const T sum = add(q[u / 4][u & 3], acc);
+        acc = j + u < n ? sum : acc;
+      }
+    }
+  }
+  return acc;
 }
 )AKG";
 
@@ -736,9 +773,8 @@ __device__ inline void chunk_rank(const int (&key)[TILES], unsigned (&slot)[TILE
       const unsigned before = mine[k];
       __builtin_amdgcn_wave_barrier();
       __hip_atomic_store(lanes + k, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      const unsigned at = before + static_cast<unsigned>(__popcll(same & (bit - 1ull)));
-      slot[u] = at;
-      if ((same >> lane) >> 1 == 0ull) mine[k] = static_cast<unsigned short>(at + 1u);   // the group's highest lane
+      slot[u] = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(same >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(same), before));
+      mine[k] = static_cast<unsigned short>(before + static_cast<unsigned>(__popcll(same)));   // (the same from every lane of the key)
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -875,7 +911,7 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
   }
   s << "struct __attribute__((aligned(4))) row_t { unsigned w[ROW_WORDS]; };\n";
   s << "typedef unsigned quad_words __attribute__((ext_vector_type(4)));\n";
-  s << kChunkSort << kChunkRank;
+  s << kChunkSort << kAddList << kChunkRank;
   s << "}  // namespace\n\n";
   std::ostringstream params;
   for (size_t i = 0; i < g.inputs.size(); ++i) {
@@ -943,13 +979,14 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
 
   // ---- chains ----
   s << "extern \"C\" __global__ __launch_bounds__(" << nw * 64 << (small ? "" : ", 4") << ") void " << g.name << "_kernel(" << params.str() << ") {\n";
-  s << "  constexpr int W = " << nw << ", T = " << tiles << ", CAP = W * T * 64, PLANE = CAP + 4 * S + 40, CHAINS = " << chains
+  s << "  constexpr int W = " << nw << ", T = " << tiles << ", CAP = W * T * 64, PLANE = CAP + 4 * S, CHAINS = " << chains
     << ", PER_WAVE = " << chainsPerWave << ";\n";
   s << "  static_assert(CAP >= CHUNK, \"a chunk's run of one bucket fits a round\");\n";
   s << "  static_assert(PER_WAVE <= 64 && W * PER_WAVE >= CHAINS, \"a lane for every output element\");\n";
   s << "  // a round's entries: whose run each is, and where entry k of the round is less k for every run\n";
   s << "  __shared__ unsigned short akg_run[CAP];\n  __shared__ unsigned akg_base[W * 64];\n";
-  s << "  __shared__ __attribute__((aligned(16))) " << ct << " akg_plane[ROW][PLANE];   // column c of a round's rows, lists per segment\n";
+  s << "  // column c of a round's rows from c * PLANE on, lists per segment; what add_list reads behind the last one\n";
+  s << "  __shared__ __attribute__((aligned(16))) " << ct << " akg_plane[ROW * PLANE + 2 * ADD_BLOCK];\n";
   s << "  __shared__ unsigned short akg_cnt[W * S];\n";
   s << "  __shared__ unsigned akg_start[S], akg_len[S], akg_scan[W], akg_sums[W], akg_taken[W], akg_total[W];\n";
   s << "  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, w = tid >> 6;\n";
@@ -962,7 +999,6 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
   s << "  const bool has = lane < PER_WAVE && chain < CHAINS;\n";
   s << "  const int cs = has ? chain / ROW : 0, cc = has ? chain - cs * ROW : 0;\n";
   s << "  union cell_t { row_t r; " << tag << "::storage v[ROW_WORDS * 4 / sizeof(" << tag << "::storage)]; };\n";
-  s << "  typedef " << ct << " quad_t __attribute__((ext_vector_type(4)));\n";
   s << "  " << ct << " acc = " << lowering::literalFor(out.dtype, 0.0) << ";\n";
   s << "  unsigned first = 0u, behind = 0u;   // this thread's run of the round: entries first .. behind - 1 of its chunk\n";
   s << "  const auto look_up = [&](int chunk) {\n";
@@ -1014,6 +1050,8 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
   s << "    }\n";
   s << "    chunk0 += taken;\n";
   s << "    look_up(chunk0 + tid);   // (the next round's runs)\n";
+  s << "  };\n";
+  s << "  const auto fetch_round = [&]() {\n";
   s << "#pragma unroll\n";
   s << "    for (int u = 0; u < T; ++u) {\n";
   s << "      const unsigned k = (w * T + u) * 64 + lane;\n";
@@ -1022,48 +1060,38 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
   s << "      segment[u] = segs[from];\n";
   s << "    }\n";
   s << "  };\n";
-  s << "  next_round();\n";
+  s << "  next_round();\n  fetch_round();\n";
   s << "  for (;;) {\n";
   s << "    int key[T];\n    unsigned slot[T];\n";
   s << "#pragma unroll\n";
   s << "    for (int u = 0; u < T; ++u) key[u] = static_cast<unsigned>((w * T + u) * 64 + lane) < total ? segment[u] : -1;\n";
-  s << "    chunk_sort<W, S, " << keyBits << ", T, 4>(key, slot, akg_cnt, akg_start, akg_len, akg_scan);\n";
+  if (perBucket == 1) {   // (nothing to sort)
+    s << "#pragma unroll\n";
+    s << "    for (int u = 0; u < T; ++u) slot[u] = static_cast<unsigned>((w * T + u) * 64 + lane);\n";
+    s << "    if (tid == 0) {\n      akg_start[0] = 0u;\n      akg_len[0] = total;\n    }\n";
+  } else {
+    s << "    chunk_sort<W, S, " << keyBits << ", T, 4>(key, slot, akg_cnt, akg_start, akg_len, akg_scan);\n";
+  }
   s << "#pragma unroll\n";
   s << "    for (int u = 0; u < T; ++u) {\n";
   s << "      if (key[u] >= 0) {\n";
   s << "#pragma unroll\n";
-  s << "        for (int c = 0; c < ROW; ++c) akg_plane[c][slot[u]] = " << tag << "::load(cur[u].v[c]);\n";
+  s << "        for (int c = 0; c < ROW; ++c) akg_plane[c * PLANE + slot[u]] = " << tag << "::load(cur[u].v[c]);\n";
   s << "      }\n";
   s << "    }\n";
   s << "    __syncthreads();\n";
-  s << "    // the next round's entries are on their way while this one's are added up\n";
+  s << "    // The next round's entries are requested while this one's are added up, by the wavefronts that add behind their additions: requests\n";
+  s << "    // wait for room in the CU's 32 KiB of lines on their way, and a round ends with its longest list.\n";
   s << "    const bool more = chunk0 < CHUNKS;   // (uniform)\n";
   s << "    if (more) next_round();\n";
   s << "    if (has) {\n";
-  s << "      const int n = static_cast<int>(akg_len[cs]);\n";
-  s << "      const quad_t *__restrict__ list = reinterpret_cast<const quad_t *>(&akg_plane[cc][akg_start[cs]]);   // (a multiple of 4)\n";
-  s << "      // sixteen additions at a time, the next sixteen values on their way (what lies behind the list's end is read,\n";
-  s << "      // inside the plane, and not added)\n";
-  s << "      quad_t q[4];\n";
-  s << "#pragma unroll\n";
-  s << "      for (int i = 0; i < 4; ++i) q[i] = list[i];\n";
-  s << "      int j = 0;\n";
-  s << "      for (; j + 16 <= n; j += 16) {\n";
-  s << "        quad_t next[4];\n";
-  s << "#pragma unroll\n";
-  s << "        for (int i = 0; i < 4; ++i) next[i] = list[j / 4 + 4 + i];\n";
-  s << "#pragma unroll\n";
-  s << "        for (int u = 0; u < 16; ++u) acc = " << rndOpen << "akg::op_add(q[u / 4][u & 3], acc));\n";
-  s << "#pragma unroll\n";
-  s << "        for (int i = 0; i < 4; ++i) q[i] = next[i];\n";
-  s << "      }\n";
-  s << "#pragma unroll\n";
-  s << "      for (int u = 0; u < 16; ++u) {\n";
-  s << "        const " << ct << " sum = " << rndOpen << "akg::op_add(q[u / 4][u & 3], acc));\n";
-  s << "        acc = j + u < n ? sum : acc;\n";
-  s << "      }\n";
+  s << "      __builtin_amdgcn_s_setprio(3);\n";
+  s << "      acc = add_list(akg_plane + cc * PLANE + akg_start[cs], static_cast<int>(akg_len[cs]), acc, [](" << ct << " v, " << ct << " sum) { return " << rndOpen
+    << "akg::op_add(v, sum)); });\n";
+  s << "      __builtin_amdgcn_s_setprio(0);\n";
   s << "    }\n";
   s << "    if (!more) break;\n";
+  s << "    fetch_round();\n";
   s << "    __syncthreads();\n";
   s << "  }\n";
   s << "  if (has && bucket * S + cs < SEGMENTS) out0[static_cast<long>(bucket * S + cs) * ROW + cc] = " << tag << "::store(acc);\n";
@@ -1086,6 +1114,353 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
   std::ostringstream note;
   note << "segment_sum positions=" << sh.positions << " segments=" << sh.segments << " slice=" << sh.slice << " chunks=" << plan.chunks << " of "
        << plan.chunk << " positions grouped by bucket of " << perBucket << " segments where they lie: " << plan.buckets << " buckets, 2 launches";
+  k.scheduleNote = note.str();
+  return k;
+}
+
+// Sizes of the schedule by records.
+struct RecordPlan {
+  bool possible = false;
+  int64_t chunks = 0, stride = 0, pitch = 0, wTable = 0, words = 0;   // words of a chunk's records, entries of a table row
+};
+
+RecordPlan planRecords(const ChunkedPlan &chunked) {
+  RecordPlan p;
+  if (!chunked.possible) return p;
+  p.chunks = chunked.chunks;
+  // (a record's segments take whole words)
+  p.stride = (chunked.chunk * chunked.rowWords + (chunked.chunk + 3 * chunked.buckets) / 4 + 4) / 4 * 4;
+  p.pitch = (chunked.buckets + 1 + 7) / 8 * 8;
+  p.wTable = p.chunks * p.stride;
+  p.words = p.wTable + p.chunks * p.pitch / 2;
+  p.possible = p.words < (1LL << 32) && p.stride <= 65535;   // (32-bit word numbers, 16-bit ones within a chunk)
+  return p;
+}
+
+// Device code of the schedule by records. The emitter defines the constants and types in front of it.
+const char *const kRecordCode = R"AKG(
+// Words of a record of n entries: n bytes, the segments within the bucket, in whole words, then n rows.
+__device__ inline unsigned record_words(unsigned n) { return n * ROW_WORDS + (n + 3u) / 4u; }
+// ... and the entries of a record of that many words.
+__device__ inline unsigned record_entries(unsigned words) { return words * 4u / (4u * ROW_WORDS + 1u); }
+
+__device__ inline void place_records(const id_store *__restrict__ ids, const unsigned *__restrict__ data, unsigned *__restrict__ ws) {
+  constexpr int THREADS = NW * 64, PER = (KEYS + THREADS - 1) / THREADS;
+  // the lane masks of the ranking, then (a barrier later) the chunk's records
+  constexpr int MASK_BYTES = NW * KEYS * 8, STAGE_BYTES = STRIDE * 4;
+  __shared__ __attribute__((aligned(16))) unsigned char akg_stage[MASK_BYTES > STAGE_BYTES ? MASK_BYTES : STAGE_BYTES];
+  __shared__ unsigned short akg_cnt[NW * KEYS];
+  __shared__ __attribute__((aligned(16))) unsigned short akg_start[PITCH];   // where a record begins, in words
+  __shared__ unsigned short akg_rows[KEYS];                                   // ... and its rows
+  __shared__ unsigned akg_scan[NW];
+  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, w = tid >> 6;
+  const row_t *__restrict__ rows = reinterpret_cast<const row_t *>(data);
+  const unsigned long long bit = 1ull << lane;
+  unsigned long long *masks = reinterpret_cast<unsigned long long *>(akg_stage), *lanes = masks + w * KEYS;
+  unsigned short *mine = akg_cnt + w * KEYS;
+  int next_id[TILES];
+  row_t next_row[TILES];
+  const auto fetch = [&](int chunk, int u) {   // (positions behind the last one read the last one's row and take no part)
+    const int p = chunk * CHUNK + (w * TILES + u) * 64 + lane, at = p < POSITIONS ? p : POSITIONS - 1;
+    const int id = as_segment(load_id(ids, at));
+    next_id[u] = p < POSITIONS ? id : -1;
+    next_row[u] = rows[at];
+  };
+#pragma unroll
+  for (int u = 0; u < TILES; ++u) fetch(static_cast<int>(blockIdx.x), u);
+  for (int chunk = static_cast<int>(blockIdx.x); chunk < CHUNKS; chunk += static_cast<int>(gridDim.x)) {
+    int key[TILES];   // the bucket, and the segment within it in the upper half
+    row_t row[TILES];
+    unsigned slot[TILES];
+#pragma unroll
+    for (int u = 0; u < TILES; ++u) {
+      const unsigned bucket = static_cast<unsigned>(next_id[u]) / S;
+      key[u] = next_id[u] >= 0 ? static_cast<int>(bucket | (static_cast<unsigned>(next_id[u]) - bucket * S) << 16) : -1;
+      row[u] = next_row[u];
+    }
+    for (int k = tid; k < NW * KEYS; k += THREADS) {
+      masks[k] = 0ull;
+      akg_cnt[k] = 0;
+    }
+    __syncthreads();
+    // rank among the wavefront's items of the bucket, as in chunk_rank; behind every tile its loads for the next chunk (all of them in
+    // front waited for the stores of the chunk before: 13 of the 28 thousand cycles of a chunk)
+    const int next = chunk + static_cast<int>(gridDim.x) < CHUNKS ? chunk + static_cast<int>(gridDim.x) : CHUNKS - 1;
+#pragma unroll
+    for (int u = 0; u < TILES; ++u) {
+      slot[u] = 0u;
+      if (key[u] >= 0) {
+        const int k = key[u] & 0xffff;
+        __hip_atomic_fetch_or(lanes + k, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __builtin_amdgcn_wave_barrier();
+        const unsigned long long same = __hip_atomic_load(lanes + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const unsigned before = mine[k];
+        __builtin_amdgcn_wave_barrier();
+        __hip_atomic_store(lanes + k, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        slot[u] = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(same >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(same), before));
+        mine[k] = static_cast<unsigned short>(before + static_cast<unsigned>(__popcll(same)));   // (the same from every lane of the key)
+      }
+      __builtin_amdgcn_wave_barrier();
+      fetch(next, u);
+    }
+    __syncthreads();
+    unsigned count[PER], words = 0u;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int k = tid * PER + j;
+      count[j] = 0u;
+      if (k < KEYS) {
+#pragma unroll
+        for (int h = 0; h < NW; ++h) {
+          const unsigned n = akg_cnt[h * KEYS + k];
+          akg_cnt[h * KEYS + k] = static_cast<unsigned short>(count[j]);
+          count[j] += n;
+        }
+      }
+      words += record_words(count[j]);
+    }
+    unsigned incl = words;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned o = __shfl_up(incl, d);
+      if (lane >= d) incl += o;
+    }
+    if (lane == 63) akg_scan[w] = incl;
+    __syncthreads();
+    unsigned at = incl - words;
+#pragma unroll
+    for (int j = 0; j < NW; ++j) at += j < w ? akg_scan[j] : 0u;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int k = tid * PER + j;
+      if (k < KEYS) {
+        akg_start[k] = static_cast<unsigned short>(at);
+        akg_rows[k] = static_cast<unsigned short>(at + (count[j] + 3u) / 4u);
+      }
+      at += record_words(count[j]);
+    }
+    if (tid == THREADS - 1) akg_start[KEYS] = static_cast<unsigned short>(at);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < TILES; ++u) {
+      if (key[u] >= 0) {
+        const int k = key[u] & 0xffff;
+        const unsigned rank = slot[u] + mine[k];
+        akg_stage[akg_start[k] * 4u + rank] = static_cast<unsigned char>(key[u] >> 16);
+        unsigned *to = reinterpret_cast<unsigned *>(akg_stage) + akg_rows[k] + rank * ROW_WORDS;
+#pragma unroll
+        for (int c = 0; c < ROW_WORDS; ++c) to[c] = row[u].w[c];
+      }
+    }
+    __syncthreads();
+    // whole 16-byte pieces; what lies behind the segments of a record and behind the last record is never looked at
+    const int pieces = (akg_start[KEYS] + 3) / 4;
+    quad_words *out = reinterpret_cast<quad_words *>(ws + static_cast<long>(chunk) * STRIDE);
+    for (int i = tid; i < pieces; i += THREADS) out[i] = reinterpret_cast<const quad_words *>(akg_stage)[i];
+    out = reinterpret_cast<quad_words *>(ws + W_TABLE + static_cast<long>(chunk) * (PITCH / 2));
+    for (int i = tid; i < PITCH / 8; i += THREADS) out[i] = reinterpret_cast<const quad_words *>(akg_start)[i];
+    __syncthreads();
+  }
+}
+
+__device__ inline void sum_records(const unsigned *__restrict__ ws, store_t *__restrict__ out0) {
+  constexpr int PLANE = CAP + 4 * S;
+  static_assert(PER_WAVE <= 64 && W * PER_WAVE >= CHAINS, "a lane for every output element");
+  // row of entry k of the round: rows + k * ROW_WORDS; its segment: byte k - first of the record, `words` words in front of the rows
+  struct run_t { unsigned rows; short first, words; };
+  __shared__ unsigned short akg_run[CAP];             // whose run each entry of the round is
+  __shared__ run_t akg_base[W * 64];
+  // column c of a round's rows from c * PLANE on, lists per segment; what add_list reads behind the last one
+  __shared__ __attribute__((aligned(16))) compute_t akg_plane[ROW * PLANE + 2 * ADD_BLOCK];
+  __shared__ unsigned short akg_cnt[W * S];
+  __shared__ unsigned akg_start[S], akg_len[S], akg_scan[W], akg_sums[W], akg_taken[W], akg_cut;
+  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, w = tid >> 6;
+  const int bucket = akg::xcd_contiguous_id(static_cast<int>(blockIdx.x), KEYS);
+  const unsigned char *__restrict__ segs = reinterpret_cast<const unsigned char *>(ws);
+  const unsigned short *__restrict__ table = reinterpret_cast<const unsigned short *>(ws + W_TABLE) + bucket;
+  // the output element of this lane, if it has one: wavefront w adds chains w * PER_WAVE ...
+  const int chain = w * PER_WAVE + lane;
+  const bool has = lane < PER_WAVE && chain < CHAINS;
+  const int cs = has ? chain / ROW : 0, cc = has ? chain - cs * ROW : 0;
+  compute_t acc = 0;
+  unsigned begin = 0u, behind = 0u;   // this thread's record of the round: words begin .. behind - 1 of its chunk
+  const auto look_up = [&](int chunk) {
+    const unsigned short *t = table + static_cast<long>(chunk < CHUNKS ? chunk : CHUNKS - 1) * PITCH;
+    begin = t[0];
+    behind = t[1];
+  };
+  look_up(tid);
+  cell_t cur[T];
+  int segment[T];
+  unsigned total = 0u, skip = 0u;   // entries of the round on its way; entries of its first run that earlier rounds had
+  int chunk0 = 0;
+  const auto next_round = [&]() {
+    const int chunk = chunk0 + tid;
+    const unsigned all = chunk < CHUNKS ? record_entries(behind - begin) : 0u, had = tid == 0 ? skip : 0u, len = all - had;
+    unsigned incl = len;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned o = __shfl_up(incl, d);
+      if (lane >= d) incl += o;
+    }
+    if (lane == 63) akg_sums[w] = incl;
+    if (tid == 0) akg_cut = 0u;
+    __syncthreads();
+    unsigned sum = 0u;
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+      incl += j < w ? akg_sums[j] : 0u;
+      sum += akg_sums[j];
+    }
+    // the round's last run may be cut; the next round begins inside it
+    const unsigned excl = incl - len, left = excl < static_cast<unsigned>(CAP) ? CAP - excl : 0u, take = len < left ? len : left;
+    const int whole = __popcll(__ballot(chunk < CHUNKS && incl <= static_cast<unsigned>(CAP)));
+    if (lane == 0) akg_taken[w] = static_cast<unsigned>(whole);
+    if (take > 0u && take < len) akg_cut = had + take;
+    const unsigned word = static_cast<unsigned>(chunk) * static_cast<unsigned>(STRIDE) + begin;
+    const int to_first = static_cast<int>(excl) - static_cast<int>(had);   // (a run beyond the round is not looked at)
+    akg_base[tid] = {word + (all + 3u) / 4u - static_cast<unsigned>(to_first) * ROW_WORDS, static_cast<short>(to_first), static_cast<short>((all + 3u) / 4u)};
+    // every run's entries, one after the other; runs of more than 32 by the whole wavefront
+    unsigned long long longer = __ballot(take > 32u);
+    if (take <= 32u) {
+      for (unsigned i = 0; i < take; ++i) akg_run[excl + i] = static_cast<unsigned short>(tid);
+    }
+    while (longer) {
+      const int b = __builtin_ctzll(longer);
+      longer &= longer - 1;
+      const unsigned n = __builtin_amdgcn_readlane(take, b), to = __builtin_amdgcn_readlane(excl, b);
+      for (unsigned i = lane; i < n; i += 64) akg_run[to + i] = static_cast<unsigned short>(w * 64 + b);
+    }
+    __syncthreads();
+    int taken = 0;
+#pragma unroll
+    for (int j = 0; j < W; ++j) taken += static_cast<int>(akg_taken[j]);
+    total = sum < static_cast<unsigned>(CAP) ? sum : CAP;
+    skip = akg_cut;
+    chunk0 += taken;
+    look_up(chunk0 + tid);   // (the next round's records)
+  };
+  const auto fetch_round = [&]() {
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const int k = (w * T + u) * 64 + lane;
+      const bool there = static_cast<unsigned>(k) < total;   // (the workspace's first words where there is no entry)
+      const run_t run = akg_base[there ? akg_run[k] : 0];
+      const unsigned from = there ? run.rows + static_cast<unsigned>(k) * ROW_WORDS : 0u;
+      cur[u].r = *reinterpret_cast<const row_t *>(ws + static_cast<unsigned long>(from));
+      const unsigned record = run.rows + static_cast<unsigned>(run.first * ROW_WORDS - run.words);
+      if constexpr (S > 1) segment[u] = segs[there ? static_cast<unsigned long>(record) * 4u + static_cast<unsigned>(k - run.first) : 0ul];
+    }
+  };
+  next_round();
+  fetch_round();
+  for (;;) {
+    int key[T];
+    unsigned slot[T];
+#pragma unroll
+    for (int u = 0; u < T; ++u) key[u] = static_cast<unsigned>((w * T + u) * 64 + lane) < total ? (S == 1 ? 0 : segment[u]) : -1;
+    if constexpr (S == 1) {   // (nothing to sort)
+#pragma unroll
+      for (int u = 0; u < T; ++u) slot[u] = static_cast<unsigned>((w * T + u) * 64 + lane);
+      if (tid == 0) {
+        akg_start[0] = 0u;
+        akg_len[0] = total;
+      }
+    } else {
+      chunk_sort<W, S, KEY_BITS, T, 4>(key, slot, akg_cnt, akg_start, akg_len, akg_scan);
+    }
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      if (key[u] >= 0) {
+#pragma unroll
+        for (int c = 0; c < ROW; ++c) akg_plane[c * PLANE + slot[u]] = load_value(cur[u].v[c]);
+      }
+    }
+    __syncthreads();
+    // The next round's entries are requested while this one's are added up, by the wavefronts that add behind their additions: requests
+    // wait for room in the CU's 32 KiB of lines on their way, and a round ends with its longest list.
+    const bool more = chunk0 < CHUNKS;   // (uniform)
+    if (more) next_round();
+    if (has) {
+      __builtin_amdgcn_s_setprio(3);
+      acc = add_list(akg_plane + cc * PLANE + akg_start[cs], static_cast<int>(akg_len[cs]), acc, [](compute_t v, compute_t sum) { return add_value(v, sum); });
+      __builtin_amdgcn_s_setprio(0);
+    }
+    if (!more) break;
+    fetch_round();
+    __syncthreads();
+  }
+  if (has && bucket * S + cs < SEGMENTS) out0[static_cast<long>(bucket * S + cs) * ROW + cc] = store_value(acc);
+}
+)AKG";
+
+/**
+ * As lowerSegmentChunked, for more positions: a bucket's run in a chunk is one record, a byte for the segment of every entry, in whole
+ * words, and the rows behind them. What bounds the last launch is not bytes but the lines its workgroups touch (a CU has 32
+ * KiB of lines on their way) and its phases: a run of eight entries touches two lines now, three with the segments elsewhere.
+ * The last run of a round may be cut, so rounds are full.
+ */
+LoweredKernel lowerSegmentRecords(const OpGraph &g, const LoweringOptions &options, const SegmentShapes &sh, const ChunkedPlan &plan, const RecordPlan &records) {
+  using lowering::computeTypeName;
+  using lowering::dtypeTag;
+  const TensorValue &data = *sh.data, &ids = *sh.ids, &out = *sh.out;
+  const std::string ct = computeTypeName(out.dtype), tag = dtypeTag(out.dtype), idTag = dtypeTag(ids.dtype);
+  const bool narrow = out.dtype == DType::F16 || out.dtype == DType::BF16 || out.dtype == DType::I8 || out.dtype == DType::I16;
+  const bool small = sh.positions / plan.buckets < 1024 && plan.tiles <= 4;
+  const int64_t perBucket = plan.perBucket, chains = perBucket * sh.slice;
+  const int nw = small ? (plan.tiles == 1 && chains <= 128 ? 2 : 4) : 8, tiles = small && plan.tiles == 1 ? static_cast<int>(plan.chunk) / (nw * 64) : 8;
+  const int64_t chainsPerWave = std::max<int64_t>(16, (chains + nw - 1) / nw);
+  int keyBits = 1;
+  while ((1LL << keyBits) < perBucket) ++keyBits;
+  std::ostringstream s;
+  s << "// Generated by the akg HIP lowering for gfx950. Op description: " << g.name << "\n";
+  s << "// family: segment_sum (positions grouped by bucket of segments, chunk by chunk, in records), fusion class: "
+    << operatorTemplateName(g.operatorTemplate) << "\n";
+  s << "#include \"akg_rt.hpp\"\n\n";
+  s << "namespace {\n";
+  s << "constexpr int POSITIONS = " << sh.positions << ", SEGMENTS = " << sh.segments << ", S = " << perBucket << ", KEYS = " << plan.buckets
+    << ", CHUNKS = " << records.chunks << ", PITCH = " << records.pitch << ", STRIDE = " << records.stride << ";\n";
+  s << "constexpr int ROW = " << sh.slice << ", ROW_WORDS = " << plan.rowWords << ", KEY_BITS = " << keyBits << ", NW = 8, TILES = " << plan.tiles
+    << ", CHUNK = NW * TILES * 64;\n";
+  s << "constexpr int W = " << nw << ", T = " << tiles << ", CAP = W * T * 64, CHAINS = " << chains << ", PER_WAVE = " << chainsPerWave << ";\n";
+  s << "constexpr long W_TABLE = " << records.wTable << ";\n";
+  s << "using id_store = " << idTag << "::storage;\nusing store_t = " << tag << "::storage;\nusing compute_t = " << ct << ";\n";
+  s << "__device__ inline auto load_id(const id_store *ids, int at) { return " << idTag << "::load(ids[at]); }\n";
+  s << "__device__ inline int as_segment(" << (ids.dtype == DType::I64 ? "long" : "int") << " v) { return v < 0 || v >= SEGMENTS ? -1 : static_cast<int>(v); }\n";
+  s << "__device__ inline compute_t load_value(store_t v) { return " << tag << "::load(v); }\n";
+  s << "__device__ inline store_t store_value(compute_t v) { return " << tag << "::store(v); }\n";
+  s << "__device__ inline compute_t add_value(compute_t v, compute_t acc) { return " << (narrow ? tag + "::rnd(" : "(") << "akg::op_add(v, acc)); }\n";
+  s << "struct __attribute__((aligned(4))) row_t { unsigned w[ROW_WORDS]; };\n";
+  s << "union cell_t { row_t r; store_t v[ROW_WORDS * 4 / sizeof(store_t)]; };\n";
+  s << "typedef unsigned quad_words __attribute__((ext_vector_type(4)));\n";
+  s << kChunkSort << kAddList << kRecordCode;
+  s << "}  // namespace\n\n";
+  std::ostringstream params;
+  for (size_t i = 0; i < g.inputs.size(); ++i) {
+    params << (i ? ", " : "") << "const " << dtypeTag(g.tensor(g.inputs[i]).dtype) << "::storage *__restrict__ in" << i;
+  }
+  params << ", " << tag << "::storage *__restrict__ out0, unsigned *__restrict__ akg_ws";
+  s << "extern \"C\" __global__ __launch_bounds__(512, 4) void " << g.name << "_place(" << params.str() << ") {\n  place_records(in" << ids.inputIndex
+    << ", reinterpret_cast<const unsigned *>(in" << data.inputIndex << "), akg_ws);\n}\n\n";
+  s << "extern \"C\" __global__ __launch_bounds__(" << nw * 64 << (small ? "" : ", 4") << ") void " << g.name << "_kernel(" << params.str() << ") {\n  sum_records(akg_ws, out0);\n}\n";
+
+  LoweredKernel k;
+  k.kernelName = g.name + "_kernel";
+  k.source = s.str();
+  k.family = KernelFamily::SegmentSum;
+  k.grid[0] = static_cast<unsigned>(plan.buckets);
+  k.block[0] = static_cast<unsigned>(nw * 64);
+  KernelPhase place;
+  place.kernelName = g.name + "_place";
+  place.grid[0] = static_cast<unsigned>(std::min<int64_t>(records.chunks, 2LL * options.computeUnits));
+  place.block[0] = 512;
+  k.earlierPhases.push_back(place);
+  k.workspaceBytes = static_cast<uint64_t>(records.words) * 4;
+  k.algorithmicBytes = lowering::countAlgorithmicBytes(g);
+  k.shapeArgs = lowering::buildShapeArgs(g);
+  std::ostringstream note;
+  note << "segment_sum positions=" << sh.positions << " segments=" << sh.segments << " slice=" << sh.slice << " chunks=" << records.chunks << " of "
+       << plan.chunk << " positions grouped by bucket of " << perBucket << " segments in records: " << plan.buckets << " buckets, 2 launches";
   k.scheduleNote = note.str();
   return k;
 }
@@ -1655,20 +2030,30 @@ LoweredKernel lowerSegmentSumToHip(const OpGraph &g, const LoweringOptions &opti
   // chunk: 24.5 million x 3 into 4954 413 -> 300, 12.5 million x 4 into 2216 401 -> 226, 20 million x 4 into 16384 1665 -> 314,
   // 1.5 million x 4 into 12654 261 -> 30, 5 million x 1 into 300 234 -> 180, 600000 x 1 into 300 49 -> 31, x 3 into 16000 227 -> 17.
   // Below, where the positions would be grouped by segment and a bucket has several segments (244664 x 4 into 9073 82 -> 13,
-  // 65974 x 1 into 13950 97 -> 8.9, 138073 x 1 into 998 29.6 -> 11.0, 200000 x 4 into 513 33.9 -> 14.5), and from 2^15 positions
-  // on instead of the scan (35304 x 1 into 1131 42.0 -> 8.4, 33000 x 4 into 300 51 -> 9.1). The other two schedules would lose
-  // in between as well (300000 x 3 into 5000 36.7 by bucket, 13.4 by chunk; 27126 x 3 into 4954 29.4 scanned, 7.9), but their
-  // launches and the scan's lack of a workspace are pinned by tests there. Nor may the workspace outgrow the 16 MiB of a
+  // 65974 x 1 into 13950 97 -> 8.9, 138073 x 1 into 998 29.6 -> 11.0, 200000 x 4 into 513 33.9 -> 14.5) or a row fewer than four elements
+  // from 3 * 2^15 positions on (124495 x 1 into 384 25.6 -> 9.9, 511656 x 2 into 344 46 -> 19.5; a test pins 70000 x 3 into 500), where they would be grouped into fewer than 512 buckets (149736 x 3
+  // into 2040 30.1 -> 11.4, 97239 x 2 into 3395 25.5 -> 10.2), and from 2^15 positions on instead of the scan (35304 x 1 into 1131
+  // 42.0 -> 8.4, 33000 x 4 into 300 51 -> 9.1). The other two schedules would lose in between as well (300000 x 3 into 5000 36.7 by
+  // bucket, 13.4 by chunk), but their launches are pinned by tests there. Nor may the workspace outgrow the 16 MiB of a
   // launch without allocations where the schedule it takes the place of stays within them, as the scan does, which has none:
   // 2 million x 3 into 20000 (26 MB by chunk) stays scanned, though that takes 1760 us for 32.
   const ChunkedPlan chunked = planChunked(sh, options);
-  bool byChunk = chunked.possible && options.variant == 4;
+  bool byChunk = chunked.possible && (options.variant == 4 || options.variant == 6);
   if (chunked.possible && options.variant == 0 && sh.positions >= (1 << 15)) {
     const bool many = sh.positions >= (1 << 19);
-    byChunk = many || (group ? !bucketed && chunked.perBucket > 1 : sh.positions < (1 << 16));
+    byChunk = many || (group ? (bucketed ? buckets < 512 : chunked.perBucket > 1 || (sh.slice < 4 && sh.positions >= (3 << 15))) : sh.positions < (1 << 16));
     const int64_t runs = std::min<int64_t>(2048, std::max<int64_t>(1, sh.positions / 1024));   // (of the schedule by segment)
     const int64_t before = !group ? 0 : bucketed ? sh.positions * 4 : sh.positions * rowBytes / 4 + runs * sh.segments;
     if (chunked.words * 4 > (16 << 20) && before * 4 <= (16 << 20)) byChunk = false;
+  }
+  // In records from 2^21 positions on. us, rows and segments apart / records: 24.5 million x 3 into 4954 283 / 261, 20 million x 4 into
+  // 16384 299 / 255, 14 million x 4 into 8656 208 / 180, 10.8 million x 1 into 5096 98 / 94, 2.7 million x 3 into 1909 42.2 / 41.5; below,
+  // 1.7 million x 3 into 520 43.8 / 44.7, 838736 x 4 into 1311 25.5 / 26.3. Not where only the whole words of the segments take the workspace
+  // beyond the 16 MiB of a launch without allocations. (AKG_HIP_VARIANT=6 takes them for any size.)
+  const RecordPlan records = planRecords(chunked);
+  const bool fits = records.words * 4 <= (16 << 20) || chunked.words * 4 > (16 << 20);
+  if (byChunk && records.possible && (options.variant == 6 || (options.variant == 0 && options.chunks == 0 && fits && sh.positions >= (1 << 21)))) {
+    return lowerSegmentRecords(g, options, sh, chunked, records);
   }
   if (byChunk) return lowerSegmentChunked(g, options, sh, chunked);
   if (bucketed) return lowerSegmentBucketed(g, options, sh, bucketBits);
