@@ -95,6 +95,7 @@ class PlaneEmitter {
   int lastWalk_ = 0;               // walks 0 .. lastWalk_: one per level of reductions, the last one stores
   bool fullOutputs_ = false;
   int vec_ = 8, block_ = 256, chunks_ = 1, overlap_ = 0;
+  bool keepsUnpacked_ = false;     // the elements of a channel stay in registers as they are computed with, from walk to walk
   bool chunkBranch_ = false;       // a chunk beyond the channel is left out by a branch, not element by element
   int64_t slots_ = 1, parts_ = 0;  // slots of a run; workgroups per channel of the form with one launch per level (0: one, resident)
   std::vector<uint64_t> partialAt_;   // per tensor: byte offset of a reduction's partial results in the workspace
@@ -216,13 +217,16 @@ class PlaneEmitter {
 
   void pickSchedule() {
     if (opt_.extentAsArgument) throw LoweringError("plane kernel: no open extents");
-    int widest = 1, fullBytes = 0;
+    int widest = 1, fullBytes = 0, fullInputs = 0;
     for (size_t t = 0; t < g_.tensors.size(); ++t) {
       const TensorValue &tv = g_.tensors[t];
       if (tv.isConst || span_[t] != Span::Full || (tv.inputIndex < 0 && tv.outputIndex < 0)) continue;
       if (tv.inputIndex >= 0 && !tv.used) continue;
       widest = std::max(widest, static_cast<int>(dtypeSize(tv.dtype)));
-      if (tv.inputIndex >= 0) fullBytes += static_cast<int>(dtypeSize(tv.dtype));
+      if (tv.inputIndex >= 0) {
+        fullBytes += static_cast<int>(dtypeSize(tv.dtype));
+        ++fullInputs;
+      }
     }
     if (fullBytes == 0) throw LoweringError("plane kernel: no full-sized input");
     vec_ = 16 / widest;
@@ -239,7 +243,7 @@ class PlaneEmitter {
     // One workgroup per channel: the smallest with at most eight chunks a thread, 1024 threads beyond. What bounds it is one
     // trip to memory and back with every load in flight, two workgroup-wide reductions and the store. Training batch
     // norm, us, one kernel per level and value -> this form (bytes of x and y at the rate of the largest streaming kernels):
-    // bf16 [64,128,28,28] 18.5 -> 7.8 (4.0), [8,936,23,23] 20.1 -> 5.4 (2.5), [27,136,27,27] 16.3 -> 5.1 (1.7),
+    // bf16 [64,128,28,28] 18.5 -> 7.5 (4.0), [8,936,23,23] 20.1 -> 5.4 (2.5), [27,136,27,27] 16.3 -> 5.1 (1.7),
     // [64,1024,7,7] 17.1 -> 4.8 (2.0), f16 [128,512,14,14] 27.2 -> 11.1 (8.0; 1024 threads 11.9, 256 with 13 chunks 11.3).
     int block = 128;
     while (block < 1024 && chunksFor(perChannel, block) > 8) block *= 2;
@@ -257,18 +261,23 @@ class PlaneEmitter {
     // flags are a few more per chunk: where narrow types or short runs make 24 and more small chunks a thread some of them
     // spill; with 256 channels and more that is still the faster form: range of int8 [32000,700,6] 352 us, 491 by level, 390 by one kernel
     // per level and value as before. It is the slower one for f32 results of int8 runs of six: [12288,700,6] 174, by such kernels 161.)
-    // Few channels leave CUs idle in the resident form, and more than eight chunks a thread make that the longer way. us,
-    // resident / by level / one kernel per level and value, 16 channels: bf16 batch norm of [83,16,28,28] (8 chunks) 6.3 / 6.0 / 14.2, of 16
-    // chunks 11.0 / 7.2 / 16.8, f32 10.3 / 6.8 / 16.5; 32 channels: int8 range of [64,32,64,64] 17.2 / 7.0 / 11.5, [30000,32,2,3] 91.7 / 24 / 25.4;
-    // 128 channels, 16 chunks: 18.0 / 24.4, 13.3 / 19.0. Short runs, which share their lines, earlier: i32 range of [3072,16,6] 11.9 / 5.2 / 9.1,
+    // Few channels leave CUs idle in the resident form, and many elements a thread make that the longer way. us, resident / by level,
+    // batch norms: bf16, 16 channels of 72 elements a thread 6.8 / 8.4, of 96 8.5 / 8.3, of 128 10.9 / 8.4; 32 channels 7.3 / 8.5, 9.3 / 8.6,
+    // 11.7 / 9.5; 48 channels of 96 9.9 / 10.0, of 128 12.3 / 11.5; 64 channels of 128 12.6 / 12.8; f32, 24 channels of 36 6.1 / 8.6, of 52 8.4 / 8.6.
+    // With one level of reductions, resident / by level / one kernel per level and value: int8 range of [64,32,64,64] 17.2 / 7.0 / 11.5,
+    // [30000,32,2,3] 91.7 / 24 / 25.4. Short runs, which share their lines, earlier: i32 range of [3072,16,6] 11.9 / 5.2 / 9.1,
     // with 128 channels and one level range of f16 [12288,128,6] 62 / 33 / 46, of i32 [6144,128,6] 33.5 / 20.6 / 30.5 (batch norms, of two
     // levels, stay: bf16 [16384,128,6] 54.6 / 61).
     const int64_t runBytes = inner_ * widest;
-    const bool fewChannels = runBytes < 64 ? (kept_ <= 32 && perChannel > 4096) || (kept_ < 256 && resident > 8 && lastWalk_ == 1) : kept_ <= 32 && resident > 8;
+    const bool fewChannels = runBytes < 64 ? (kept_ <= 32 && perChannel > 4096) || (kept_ < 256 && resident > 8 && lastWalk_ == 1)
+                             : lastWalk_ == 1 ? kept_ <= 32 && resident > 8 : kept_ <= 48 && resident * vec_ >= (kept_ <= 32 ? 96 : 120);
     if (resident * regsPerChunk <= 64 && opt_.split <= 1 && (!fewChannels || opt_.split == 1)) {
       block_ = block;
       chunks_ = static_cast<int>(resident);
       parts_ = 0;
+      // Half of the registers may hold the elements as they are computed with: the walks behind the first then neither unpack them nor
+      // compute what the walk before did (a batch norm's instructions are 4 of the 8 us of bf16 [64,128,28,28]: 809 -> 641, 8.0 -> 7.5 us).
+      keepsUnpacked_ = resident * vec_ * fullInputs <= 65536 / block_;
       return;
     }
     // One launch per level: 128 bytes of loads in flight per thread, less where that leaves less than four workgroups per
@@ -471,7 +480,7 @@ class PlaneEmitter {
       Val &v = vals_[static_cast<size_t>(t)];
       v.defined = v.full = true;
       v.ident = id("x", static_cast<int>(i));
-      if (again) src_ << "    akg::forget_unpacked(p_in" << i << "[j]);\n";
+      if (again && !keepsUnpacked_) src_ << "    akg::forget_unpacked(p_in" << i << "[j]);\n";
       src_ << "    " << computeTypeName(tv.dtype) << " " << v.ident << "[V];\n";
       src_ << "    akg::unpack_chunk(p_in" << i << "[j], " << v.ident << ");\n";
     }
