@@ -24,8 +24,8 @@
  *   back, per column, 8 or 4 consecutive k): no transposes in registers.
  *   SQ_LDS_BANK_CONFLICT reads 0 for both layouts (how the chunks are placed for that is said where they are written).
  *   Every lane ends up owning 4 ADJACENT output columns (by the order of the LDS rows of an [N,K] B; by a 4 x 4
- *   exchange inside each lane quad for a row-major B): the epilogue works on 4-element chunks and sixteen lanes store
- *   one aligned piece of 64 columns per output row.
+ *   exchange inside each lane quad for a row-major B): the epilogue works on 4-element chunks, and a store of a
+ *   wavefront writes two rows of 128 adjacent columns (four of 64 where its tile is 64 columns wide).
  *
  * Workgroup -> tile mapping: consecutive workgroup ids go round-robin to the 8 XCDs (each with its own L2), so
  * ids are first regrouped per XCD and then walked in column-major groups of 8 tile-rows, which keeps the A and B
@@ -194,13 +194,16 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
   const long kPerXcd = (kTiles + kGemmXcds - 1) / kGemmXcds;
   constexpr long kSteps = (K + BK - 1) / BK;
   constexpr bool kFull = !DYN && (MS % kGemmBM == 0) && (N % kGemmBN == 0) && (K % BK == 0);
-  // Whole tiles along N and K, and an M that is an argument or leaves a ragged last tile behind full ones: the loads need
-  // no checks either. Every thread clamps the rows of A it stages to the last row once, in front of the loop (the scalar
-  // offset of a buffer load takes no part in the descriptor's range check, so the descriptor alone would not keep the
-  // rows of a ragged last tile inside A); rows beyond M then hold copies of row M - 1 and their accumulators are
-  // dropped by the epilogue's row check. The main loop is the one of a whole shape: no compares, one basic block per K
-  // step. (A single ragged tile, M < 256, keeps the checks: there the wavefronts without rows skip their MFMAs.)
-  constexpr bool kClampRows = !kFull && (DYN || MS > kGemmBM) && (N % kGemmBN == 0) && (K % BK == 0);
+  // Ragged tiles behind full ones (and, with an M that is an argument, whole tiles along N and K): the loads need no checks either, so
+  // the main loop is the one of a whole shape, one basic block per K step. Every thread clamps the rows of A, and the columns of a
+  // [N,K] B, that it stages to the last one, once, in front of the loop (the scalar offset of a buffer load takes no part in the
+  // descriptor's range check, so the descriptor alone would not keep them inside); what lies beyond M and N then holds copies whose
+  // accumulators are dropped by the epilogue's checks. Chunks of a row-major B beyond N, and chunks beyond K, are asked for beyond the
+  // buffer and read zero. us, a branch around every load / this, with the epilogue's stores as they are below: f16 3584 x 896 x
+  // 8928 67.0 / 57.8, [N,K] 2048 x 4112 x 2052 int8 70.6 / 61.5, [N,K] 900 x 608 x 16380 f16 32.7 / 24.3; 42 products that take this kernel in
+  // 0.88 of the time in the mean, none slower by 3 %. (A single ragged tile, M <= 256, keeps the branches: there the wavefronts without
+  // rows skip their MFMAs.)
+  constexpr bool kClampRows = !kFull && (DYN ? (N % kGemmBN == 0) && (K % BK == 0) : MS > kGemmBM);
   constexpr bool kLoadsInRange = kFull || kClampRows;
   constexpr int kTileBytes = kGemmBM * kPitch;        // one operand tile in LDS
   static_assert(kRowChunks == 4, "the staging schedule is written for four 16-byte chunks per thread and operand");
@@ -289,7 +292,13 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
   const int bRowT = tid / kChunksPerRowB;     // + kRowStepB * i
   const int bChunkT = tid % kChunksPerRowB;
   const int bVoff = TRANSB ? static_cast<int>(aRow * K + aChunk * 16)
-                           : static_cast<int>(bRowT * NB + n0 * EB + bChunkT * 16);
+                           : static_cast<int>(kClampRows && n0 * EB + bChunkT * 16 >= NB ? static_cast<long>(kBeyondEveryBuffer) : bRowT * NB + n0 * EB + bChunkT * 16);
+  int bVoffClamped[kRowChunks];   // kClampRows, [N,K]: the same for the columns of B
+#pragma unroll
+  for (int i = 0; i < kRowChunks; ++i) {
+    const long col = n0 + aRow + kRowStep * i;
+    bVoffClamped[i] = static_cast<int>(((col < N ? col : N - 1) - n0) * K + aChunk * 16);
+  }
   // LDS write offsets. [N,K] B: the LDS row of a column is chosen so that the 16 lanes of a fragment read find, in the
   // four column tiles 4 q .. 4 q + 3, four ADJACENT columns (row 64 q + 16 t + c holds column 64 q + 4 c + t).
   // Row-major B: the 16-column units of a k-row are swapped in pairs for the k-rows of odd 16-lane groups.
@@ -314,8 +323,10 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
 
   auto loadChunk = [&](long step, int i) {
     const long k0 = (stepBase + step) * BK;
+    constexpr int kBeyond = static_cast<int>(kBeyondEveryBuffer);
+    const bool whole = K % BK == 0 || k0 + aChunk * 16 < K;   // (kClampRows: of a K-contiguous operand)
     if (kLoadsInRange || (m0 + aRow + kRowStep * i < M && k0 + aChunk * 16 < K)) {
-      const u32x4 v = kClampRows ? __builtin_amdgcn_raw_buffer_load_b128(aRsrc, aVoffClamped[i], static_cast<int>(k0), 0)
+      const u32x4 v = kClampRows ? __builtin_amdgcn_raw_buffer_load_b128(aRsrc, whole ? aVoffClamped[i] : kBeyond, static_cast<int>(k0), 0)
                                  : __builtin_amdgcn_raw_buffer_load_b128(aRsrc, aVoff, static_cast<int>((kRowStep * i) * K + k0), 0);
       stage.x[i] = v4i{static_cast<int>(v[0]), static_cast<int>(v[1]), static_cast<int>(v[2]), static_cast<int>(v[3])};
     } else {
@@ -323,7 +334,8 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
     }
     if constexpr (TRANSB) {
       if (kLoadsInRange || (n0 + aRow + kRowStep * i < N && k0 + aChunk * 16 < K)) {
-        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(bRsrc, bVoff, static_cast<int>((kRowStep * i) * K + k0), 0);
+        const u32x4 v = kClampRows ? __builtin_amdgcn_raw_buffer_load_b128(bRsrc, whole ? bVoffClamped[i] : kBeyond, static_cast<int>(k0), 0)
+                                   : __builtin_amdgcn_raw_buffer_load_b128(bRsrc, bVoff, static_cast<int>((kRowStep * i) * K + k0), 0);
         stage.y[i] = v4i{static_cast<int>(v[0]), static_cast<int>(v[1]), static_cast<int>(v[2]), static_cast<int>(v[3])};
       } else {
         stage.y[i] = v4i{0, 0, 0, 0};
@@ -331,7 +343,8 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
     } else {
       const long krow = k0 / EB + bRowT + kRowStepB * i;
       if (kLoadsInRange || (krow < KE && n0 * EB + bChunkT * 16 < NB)) {
-        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(bRsrc, bVoff, static_cast<int>((k0 / EB + kRowStepB * i) * NB), 0);
+        const bool there = !kClampRows || K % BK == 0 || krow < KE;
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(bRsrc, there ? bVoff : kBeyond, static_cast<int>((k0 / EB + kRowStepB * i) * NB), 0);
         stage.y[i] = v4i{static_cast<int>(v[0]), static_cast<int>(v[1]), static_cast<int>(v[2]), static_cast<int>(v[3])};
       } else {
         stage.y[i] = v4i{0, 0, 0, 0};
@@ -548,9 +561,32 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
       }
     }
   }
-  // first of the lane's four columns in column group q, and the row of accumulator v of row tile i inside the tile
-  const long colBase = n0 + wn * kWaveCols + (TRANSB ? 4 * fragC : 16 * (fragC & 3) + (fragC & ~3));
-  auto rowInTileOf = [&](int i, int v) { return static_cast<long>(wm * kWaveRows + i * 16 + fragG * 4 + v); };
+  // Two column groups (a wavefront's 64 x 128): the lanes of an even group of 16 take column group 0 of their own row and of that of the
+  // lanes 16 above, those column group 1 of both, so that a store of the wavefront writes 2 rows x 128 adjacent columns and not
+  // 4 x 64: where the rows of the result are not whole 64-byte pieces, half as many pieces are written in part. us, loads without
+  // branches, 4 x 64 / 2 x 128: bf16 [N,K] 3584 x 896 x 8936 81.1 / 60.4 (8960: 54.5 / 54.4), int8 -> bf16 64.0 / 43.1, f16 row-major
+  // 4096 x 2048 x 12280 206 / 178. (Stored without the streaming hint they meet in L2: 68.6, but the operands leave it: 60.0 for 8960.)
+  constexpr bool kPairs = kTN == 8;
+  if constexpr (kPairs) {
+#pragma unroll
+    for (int i = 0; i < kTM; ++i) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          typename Mma::acc_t lo = acc[i][j][v], hi = acc[i][4 + j][v];
+          swap_lanes16(lo, hi);
+          acc[i][j][v] = lo;
+          acc[i][4 + j][v] = hi;
+        }
+      }
+    }
+  }
+  // the lane's four columns, and the row of accumulator v of row tile i and group q inside the tile
+  const long col4 = n0 + wn * kWaveCols + (kPairs ? 64 * (fragG & 1) : 0) + (TRANSB ? 4 * fragC : 16 * (fragC & 3) + (fragC & ~3));
+  auto rowInTileOf = [&](int i, int q, int v) {
+    return static_cast<long>(wm * kWaveRows + i * 16 + (kPairs ? (fragG & 2) + q : fragG) * 4 + v);
+  };
   if (kSplitPossible && kSplits > 1) {
     const long kPartRows = M < kGemmBM ? M : kGemmBM;            // rows of a tile that can hold results
     const long kCounterBytes = (kGridTiles * 4 + 255) / 256 * 256;
@@ -559,19 +595,19 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
     const Buffer wsBuf = make_buffer(ws, kWsBytes);
     const u32 tileBase = static_cast<u32>(kCounterBytes + linear * kSplits * kPartBytes);
     auto partOffset = [&](int i, int q, int v) {
-      return static_cast<long>((rowInTileOf(i, v) * kGemmBN + (colBase + 64 * q - n0)) * static_cast<long>(sizeof(typename Mma::acc_t)));
+      return static_cast<long>((rowInTileOf(i, q, v) * kGemmBN + (col4 - n0)) * static_cast<long>(sizeof(typename Mma::acc_t)));
     };
-    auto rowOk = [&](int i, int v) { return rowInTileOf(i, v) < kPartRows && m0 + rowInTileOf(i, v) < M; };
+    auto rowOk = [&](int i, int q, int v) { return rowInTileOf(i, q, v) < kPartRows && m0 + rowInTileOf(i, q, v) < M; };
 #pragma unroll
     for (int q = 0; q < kTN / 4; ++q) {
-      if (!(kFull || colBase + 64 * q < N)) continue;
+      if (!(kFull || col4 < N)) continue;
 #pragma unroll
       for (int i = 0; i < kTM; ++i) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           // (a row beyond M stores to beyond the workspace, which drops it)
           const typename Mma::acc_t a4[4] = {acc[i][4 * q][v], acc[i][4 * q + 1][v], acc[i][4 * q + 2][v], acc[i][4 * q + 3][v]};
-          ws_store_chunk<4>(wsBuf, rowOk(i, v) ? tileBase + static_cast<u32>(ksplit * kPartBytes + partOffset(i, q, v)) : kBeyondEveryBuffer, a4);
+          ws_store_chunk<4>(wsBuf, rowOk(i, q, v) ? tileBase + static_cast<u32>(ksplit * kPartBytes + partOffset(i, q, v)) : kBeyondEveryBuffer, a4);
         }
       }
     }
@@ -580,16 +616,15 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
     if constexpr (!DYN) {
       // The number of splits is a constant: sum and epilogue per group of four accumulators, the loads of all splits of
       // the group in flight together (the compiler unrolls the splits and overlaps the groups).
+      if (!(kFull || col4 < N)) return;
+      epi.prepare(col4);
 #pragma unroll
       for (int q = 0; q < kTN / 4; ++q) {
-        const long col4 = colBase + 64 * q;
-        if (!(kFull || col4 < N)) continue;
-        epi.prepare(col4);
 #pragma unroll
         for (int i = 0; i < kTM; ++i) {
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            if (!rowOk(i, v)) continue;
+            if (!rowOk(i, q, v)) continue;
             typename Mma::acc_t sum[4] = {0, 0, 0, 0};
             for (int p = 0; p < kSplits; ++p) {
               typename Mma::acc_t part[4];
@@ -597,7 +632,7 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
 #pragma unroll
               for (int c = 0; c < 4; ++c) sum[c] += part[c];
             }
-            epi.apply(sum, m0 + rowInTileOf(i, v), col4);
+            epi.apply(sum, m0 + rowInTileOf(i, q, v), col4);
           }
         }
       }
@@ -619,13 +654,13 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
         const u32 splitBase = tileBase + static_cast<u32>(p * kPartBytes);
 #pragma unroll
         for (int q = 0; q < kTN / 4; ++q) {
-          if (!(kFull || colBase + 64 * q < N)) continue;
+          if (!(kFull || col4 < N)) continue;
 #pragma unroll
           for (int i = 0; i < kTM; ++i) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
               typename Mma::acc_t part[4];
-              ws_load_chunk<4>(wsBuf, rowOk(i, v) ? splitBase + static_cast<u32>(partOffset(i, q, v)) : kBeyondEveryBuffer, part);
+              ws_load_chunk<4>(wsBuf, rowOk(i, q, v) ? splitBase + static_cast<u32>(partOffset(i, q, v)) : kBeyondEveryBuffer, part);
 #pragma unroll
               for (int c = 0; c < 4; ++c) acc[i][4 * q + c][v] += part[c];
             }
@@ -634,17 +669,16 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
       }
     }
   }
+  if (!(kFull || col4 < N)) return;
+  epi.prepare(col4);
 #pragma unroll
   for (int q = 0; q < kTN / 4; ++q) {
-    const long col4 = colBase + 64 * q;
-    if (!(kFull || col4 < N)) continue;
-    epi.prepare(col4);
 #pragma unroll
     for (int i = 0; i < kTM; ++i) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const long row = m0 + rowInTileOf(i, v);
-        if (kFull || row < M) {
+        const long row = m0 + rowInTileOf(i, q, v);
+        if (kFull || (!DYN && MS % kGemmBM == 0) || row < M) {
           const typename Mma::acc_t a4[4] = {acc[i][4 * q][v], acc[i][4 * q + 1][v], acc[i][4 * q + 2][v], acc[i][4 * q + 3][v]};
           epi.apply(a4, row, col4);
         }

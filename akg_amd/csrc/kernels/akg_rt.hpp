@@ -841,6 +841,17 @@ AKG_DEV long long lane_partner(long long v) {
   return static_cast<long long>((static_cast<u64>(hi) << 32) | lo);
 }
 
+// Exchanges `hi` of the lanes of even groups of 16 with `lo` of the lanes 16 above them: afterwards `lo` holds (lo, hi) of the even
+// group in the two groups, `hi` those of the odd one.
+template <typename T>
+AKG_DEV void swap_lanes16(T &lo, T &hi) {
+  static_assert(sizeof(T) == 4, "one register per value");
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(u32, lo), __builtin_bit_cast(u32, hi), false, false);
+  const u32 r0 = r[0], r1 = r[1];
+  lo = __builtin_bit_cast(T, r0);
+  hi = __builtin_bit_cast(T, r1);
+}
+
 template <typename Red, int WIDTH, typename T>
 AKG_DEV T wave_group_reduce(T v) {
   static_assert(WIDTH <= kWaveSize && (WIDTH & (WIDTH - 1)) == 0, "group width must be a power of two <= 64");

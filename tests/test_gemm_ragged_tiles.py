@@ -1,0 +1,50 @@
+"""The 256 x 256 tile kernel on several rows of tiles whose last row, last column or last step of K is not whole."""
+import pytest
+
+from akg_amd import driver, op_desc
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tb", [True, False])
+@pytest.mark.parametrize("m,k,n,dtype", [
+    (257, 512, 260, "bfloat16"), (511, 40, 516, "float16"),         # one row, four columns behind a tile; less than a step of K
+    (512, 608, 8200, "bfloat16"), (300, 2056, 1016, "float16"),     # whole rows of tiles only; 16 bytes of K behind the last step, split
+    (770, 2104, 1276, "bfloat16"), (1500, 1088, 4092, "float16"),   # 112 bytes of K behind the last step; many tiles, none of them split
+    (300, 2064, 1028, "int8"), (513, 1136, 2296, "int8"), (768, 64, 4100, "int8"), (2048, 4112, 2052, "int8"),
+])
+def test_ragged_tiles_against_float64(m, k, n, dtype, tb, monkeypatch):
+    """float32 sums of k products differ from the exact sum by at most k * 2^-24 of the sum of the products' magnitudes, in
+    whatever order, and a result by one half unit of its type; 8-bit sums are exact."""
+    import torch
+    monkeypatch.setenv("AKG_HIP_VARIANT", "128")   # (small tiles take some of them)
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    dev = "cuda"
+    weight = (n, k) if tb else (k, n)
+    if dtype == "int8":
+        text = op_desc.gemm_int8_dequant_bias_gelu(m, k, n, transpose_b=tb)
+        a, w = (torch.randint(-127, 128, s, generator=g, device=dev).to(torch.int8) for s in ((m, k), weight))
+        scale, scale_n = torch.full((m, 1), 2.0 ** -6, device=dev), torch.full((n,), 2.0 ** -10, device=dev)
+        bias = torch.randn(n, generator=g, device=dev).bfloat16()
+        wide = w.double().t().contiguous() if tb else w.double()
+        y = a.double() @ wide * 2.0 ** -16 + bias.double()
+        y = y * (torch.tanh((y + y ** 3 * 0.044715) * 0.7978845608028654) + 1) * 0.5
+        # the factors are powers of two; float32 GELU: 2^-20 of the argument's magnitude, and the rounding to bfloat16
+        inputs, td, bound = [a, scale, w, scale_n, bias], torch.bfloat16, y.abs() * (2.0 ** -8 + 2.0 ** -19) + 2.0 ** -16
+    else:
+        td = getattr(torch, dtype)
+        text = op_desc.gemm_bias_act(m, k, n, dtype, "none", transpose_b=tb)
+        a, w, bias = (torch.randn(s, generator=g, device=dev).to(td) for s in ((m, k), weight, (n,)))
+        wide = w.double().t().contiguous() if tb else w.double()
+        y = a.double() @ wide + bias.double()
+        unit = 2.0 ** -8 if dtype == "bfloat16" else 2.0 ** -11
+        inputs, bound = [a, w, bias], (a.double().abs() @ wide.abs()) * (k * 2.0 ** -24) + y.abs() * (unit + 2.0 ** -23) + 2.0 ** -24
+    print("case", m, k, n, dtype, tb, flush=True)
+    kernel = driver.HipKernel(text, out_dir=None)
+    assert "gemm_256x256<" in kernel.source
+    # (behind the result: nothing of a row or column that the product does not have)
+    out = torch.full((m + 1, n), float("nan"), device=dev, dtype=td)
+    kernel.launch(inputs + [out[:m]])
+    torch.cuda.synchronize()
+    gap = (out[:m].double() - y).abs()
+    assert bool((gap <= bound).all()), float((gap / bound).max())
+    assert bool(out[m].isnan().all())
