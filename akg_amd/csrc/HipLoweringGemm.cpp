@@ -259,9 +259,11 @@ class GemmEmitter {
   // it is the slower one, and the estimates say so, for 3568 x 5056 x 3848 (137 / 193 / 167) and 1881 x 4160 x 7568 (118 / 152 / 125).
   // The skinny one is faster at 33 rows for [K,N] weights of bf16 8192 x 6144 (30.9 for 26.1), int8 4096 x 6144 (14.8 for 13.4) and 6144 x 9216
   // (27.9 for 20.0), for [N,K] of bf16 11008 x 5120 (34.1 for 28.1).
-  // Weights below 2 MiB whose columns are whole 256-wide tiles (or whose sums are rounded once by request) and those from 2^26 elements on keep the kernels and splits
-  // that tests pin, though small tiles would be the faster ones there for some rows: bf16 512 x 768 with 256 rows takes 21.4 us
-  // for their 4.8, 8192 x 8192 with 96 rows 50.7 for 41.5. Other weights below 2 MiB take them (us: bf16 85 x 1088 x 816 22.7 -> 4.9,
+  // Weights below 2 MiB with K from 1024 on that are at most 512 x 768 of whole 256-wide columns (or whose sums are rounded once by request) and those
+  // from 2^26 elements on keep the kernels and splits that tests pin, though small tiles would be the faster ones there for some rows: int8
+  // 121 x 1344 x 768 takes 26.9 us for their 5.5, bf16 8192 x 8192 with 96 rows 50.7 for 41.5. Other weights below 2 MiB take them (us: whole
+  // 256-wide columns f16 181 x 576 x 1280 27.8 -> 4.3, 8192 x 768 x 768 22.1 -> 17.5, int8 768 x 1408 x 512 31.3 -> 6.2, 2276 x 384 x 3072
+  // 20.3 -> 11.6, 200 such products a third of the time in the mean, none slower; others bf16 85 x 1088 x 816 22.7 -> 4.9,
   // 365 x 1408 x 744 34.0 -> 7.4, 1096 x 1152 x 552 34.4 -> 7.0, int8 200 x 640 x 584 20.7 -> 4.5). Narrow products of at most 64 rows
   // (N < 1024) are the skinny kernel's.
   bool pickSmallTile() {
@@ -269,7 +271,8 @@ class GemmEmitter {
     const int64_t elements = k_ * n_;
     if (m_ <= 32 || elements >= (1LL << 26)) return false;
     const bool narrow = m_ <= skinnyRows();
-    if (elements * elemBytes() < (2LL << 20) && (narrow || n_ % 256 == 0 || roundedOnce_)) return false;
+    const bool fewWhole = n_ % 256 == 0 && n_ <= 768 && m_ <= 512 && k_ >= 1024;
+    if (elements * elemBytes() < (2LL << 20) && (narrow || fewWhole || roundedOnce_)) return false;
     if (narrow && n_ < 1024) return false;
     // (Rows of a [K,N] weight that are not whole 16-byte chunks: with 8 bits and more than 64 rows. us, 256 x 256 tiles -> small ones:
     // 219 x 3776 x 5640 38.5 -> 17.2, 836 x 4544 x 9240 97 -> 49, 104 x 768 x 9080 18.9 -> 6.8, 2002 x 3200 x 8280 108 -> 73. For

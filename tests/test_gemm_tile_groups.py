@@ -78,3 +78,16 @@ def test_two_workgroups_of_128_x_128_fit_a_cu(m, k, n, tmp_path):
     notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", code], capture_output=True, text=True, check=True).stdout
     assert int(re.search(r"\.vgpr_count:\s+(\d+)", notes).group(1)) <= 256
     assert int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", notes).group(1)) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,n,dtype,tb", [
+    (65, 960, 256, "bfloat16", False), (257, 64, 512, "float16", True), (512, 1008, 768, "bfloat16", True),   # K below 1024
+    (513, 1024, 256, "float16", False), (300, 1024, 1024, "int8", False), (2048, 768, 768, "bfloat16", False),
+    (513, 2040, 512, "bfloat16", True), (1500, 1088, 1792, "int8", True),
+])
+def test_small_weights_of_whole_wide_columns(m, k, n, dtype, tb, tmp_path):
+    """Weights below 2 MiB whose columns are whole 256-wide tiles take small tiles too, but for a few products with a long K."""
+    got = _tile(m, k, n, dtype, tb)
+    assert got is not None
+    _against_float64(m, k, n, dtype, tb, "%dx%d" % tuple(128 if x % 128 == 0 else 64 for x in got[:2]), tmp_path)
