@@ -566,7 +566,8 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
   // 4 x 64: where the rows of the result are not whole 64-byte pieces, half as many pieces are written in part. us, loads without
   // branches, 4 x 64 / 2 x 128: bf16 [N,K] 3584 x 896 x 8936 81.1 / 60.4 (8960: 54.5 / 54.4), int8 -> bf16 64.0 / 43.1, f16 row-major
   // 4096 x 2048 x 12280 206 / 178. (Stored without the streaming hint they meet in L2: 68.6, but the operands leave it: 60.0 for 8960.)
-  constexpr bool kPairs = kTN == 8;
+  // Not where every row is whole pieces: 4096 x 8192 x 8192 419.5 / 420.6.
+  constexpr bool kPairs = kTN == 8 && N % 64 != 0;
   if constexpr (kPairs) {
 #pragma unroll
     for (int i = 0; i < kTM; ++i) {
@@ -582,8 +583,9 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
       }
     }
   }
-  // the lane's four columns, and the row of accumulator v of row tile i and group q inside the tile
-  const long col4 = n0 + wn * kWaveCols + (kPairs ? 64 * (fragG & 1) : 0) + (TRANSB ? 4 * fragC : 16 * (fragC & 3) + (fragC & ~3));
+  // the first of the lane's four columns in group q, and the row of accumulator v of row tile i and group q inside the tile
+  const long colBase = n0 + wn * kWaveCols + (kPairs ? 64 * (fragG & 1) : 0) + (TRANSB ? 4 * fragC : 16 * (fragC & 3) + (fragC & ~3));
+  auto colOf = [&](int q) { return colBase + (kPairs ? 0 : 64 * q); };
   auto rowInTileOf = [&](int i, int q, int v) {
     return static_cast<long>(wm * kWaveRows + i * 16 + (kPairs ? (fragG & 2) + q : fragG) * 4 + v);
   };
@@ -595,12 +597,12 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
     const Buffer wsBuf = make_buffer(ws, kWsBytes);
     const u32 tileBase = static_cast<u32>(kCounterBytes + linear * kSplits * kPartBytes);
     auto partOffset = [&](int i, int q, int v) {
-      return static_cast<long>((rowInTileOf(i, q, v) * kGemmBN + (col4 - n0)) * static_cast<long>(sizeof(typename Mma::acc_t)));
+      return static_cast<long>((rowInTileOf(i, q, v) * kGemmBN + (colOf(q) - n0)) * static_cast<long>(sizeof(typename Mma::acc_t)));
     };
     auto rowOk = [&](int i, int q, int v) { return rowInTileOf(i, q, v) < kPartRows && m0 + rowInTileOf(i, q, v) < M; };
 #pragma unroll
     for (int q = 0; q < kTN / 4; ++q) {
-      if (!(kFull || col4 < N)) continue;
+      if (!(kFull || colOf(q) < N)) continue;
 #pragma unroll
       for (int i = 0; i < kTM; ++i) {
 #pragma unroll
@@ -616,10 +618,10 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
     if constexpr (!DYN) {
       // The number of splits is a constant: sum and epilogue per group of four accumulators, the loads of all splits of
       // the group in flight together (the compiler unrolls the splits and overlaps the groups).
-      if (!(kFull || col4 < N)) return;
-      epi.prepare(col4);
 #pragma unroll
       for (int q = 0; q < kTN / 4; ++q) {
+        if (!(kFull || colOf(q) < N)) continue;
+        if (!kPairs || q == 0) epi.prepare(colOf(q));
 #pragma unroll
         for (int i = 0; i < kTM; ++i) {
 #pragma unroll
@@ -632,7 +634,7 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
 #pragma unroll
               for (int c = 0; c < 4; ++c) sum[c] += part[c];
             }
-            epi.apply(sum, m0 + rowInTileOf(i, q, v), col4);
+            epi.apply(sum, m0 + rowInTileOf(i, q, v), colOf(q));
           }
         }
       }
@@ -654,7 +656,7 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
         const u32 splitBase = tileBase + static_cast<u32>(p * kPartBytes);
 #pragma unroll
         for (int q = 0; q < kTN / 4; ++q) {
-          if (!(kFull || col4 < N)) continue;
+          if (!(kFull || colOf(q) < N)) continue;
 #pragma unroll
           for (int i = 0; i < kTM; ++i) {
 #pragma unroll
@@ -669,10 +671,10 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
       }
     }
   }
-  if (!(kFull || col4 < N)) return;
-  epi.prepare(col4);
 #pragma unroll
   for (int q = 0; q < kTN / 4; ++q) {
+    if (!(kFull || colOf(q) < N)) continue;
+    if (!kPairs || q == 0) epi.prepare(colOf(q));
 #pragma unroll
     for (int i = 0; i < kTM; ++i) {
 #pragma unroll
@@ -680,7 +682,7 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
         const long row = m0 + rowInTileOf(i, q, v);
         if (kFull || (!DYN && MS % kGemmBM == 0) || row < M) {
           const typename Mma::acc_t a4[4] = {acc[i][4 * q][v], acc[i][4 * q + 1][v], acc[i][4 * q + 2][v], acc[i][4 * q + 3][v]};
-          epi.apply(a4, row, col4);
+          epi.apply(a4, row, colOf(q));
         }
       }
     }

@@ -10,6 +10,7 @@ from akg_amd import driver, op_desc
     (257, 512, 260, "bfloat16"), (511, 40, 516, "float16"),         # one row, four columns behind a tile; less than a step of K
     (512, 608, 8200, "bfloat16"), (300, 2056, 1016, "float16"),     # whole rows of tiles only; 16 bytes of K behind the last step, split
     (770, 2104, 1276, "bfloat16"), (1500, 1088, 4092, "float16"),   # 112 bytes of K behind the last step; many tiles, none of them split
+    (300, 1056, 1024, "bfloat16"), (600, 544, 4160, "float16"), (513, 1040, 1088, "int8"),   # rows of whole 64-byte pieces
     (300, 2064, 1028, "int8"), (513, 1136, 2296, "int8"), (768, 64, 4100, "int8"), (2048, 4112, 2052, "int8"),
 ])
 def test_ragged_tiles_against_float64(m, k, n, dtype, tb, monkeypatch):
