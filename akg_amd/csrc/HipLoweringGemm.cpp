@@ -225,11 +225,18 @@ class GemmEmitter {
     const double loop = static_cast<double>((steps + split - 1) / split) * step * rounds;
     return split == 1 ? 3 + loop : 5.5 + loop + 0.3 * static_cast<double>(split) * area / 4096 + static_cast<double>(tiles * split) * area * 8 / 5e6;
   }
-  // ... and of the 256 x 256 kernel with `split` workgroups per tile (the same products, 14 %).
+  // ... and of the 256 x 256 kernel with `split` workgroups per tile: fitted to the same products (14 %), and with more than 256 rows and
+  // ragged columns to 200 such (K and N 512 .. 16384, 8 %; 8-bit ones with dequantisation and GELU behind the sums).
   double largeTileTime(int64_t split) const {
-    const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = ((m_ + 255) / 256) * ((n_ + 255) / 256), rounds = (tiles * split + 255) / 256;
-    const double step = 1.45 * (transB_ ? 1 : 1.093) * (elemBytes() == 1 ? 1.356 : 1), rows = static_cast<double>(std::min<int64_t>(m_, 256));
-    const double time = static_cast<double>(rounds) * (static_cast<double>((steps + split - 1) / split) * step + 7.35);
+    const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = ((m_ + 255) / 256) * ((n_ + 255) / 256), perTile = (steps + split - 1) / split;
+    const double perCu = static_cast<double>(tiles * split) / 256, whole = std::ceil(perCu), rows = static_cast<double>(std::min<int64_t>(m_, 256));
+    if (m_ > 256 && n_ % 256 != 0) {
+      const double step = 1.478 * (transB_ ? 1 : 1.068) * (elemBytes() == 1 ? (transB_ ? 0.949 : 0.967) : 1), rounds = perCu <= 1 ? 1 : 0.87 * whole + 0.13 * perCu;
+      const double time = rounds * (static_cast<double>(perTile) * step + (elemBytes() == 1 ? 13.45 : 7.54));
+      return split == 1 ? time : time + 6.45 + 1.35 * static_cast<double>(split);
+    }
+    const double step = 1.45 * (transB_ ? 1 : 1.093) * (elemBytes() == 1 ? 1.356 : 1);
+    const double time = whole * (static_cast<double>(perTile) * step + 7.35);
     return split == 1 ? time : time + 5.67 + 2.32 * static_cast<double>(split) * rows / 256 + 0.24 * static_cast<double>(tiles * split) * rows * 2048 / 5e6;
   }
   // 33 .. 64 rows: time in us of the skinny kernel and of 64 x 64 tiles, fitted to 1256 measured products (both layouts, 8 and
@@ -260,17 +267,20 @@ class GemmEmitter {
   // The skinny one is faster at 33 rows for [K,N] weights of bf16 8192 x 6144 (30.9 for 26.1), int8 4096 x 6144 (14.8 for 13.4) and 6144 x 9216
   // (27.9 for 20.0), for [N,K] of bf16 11008 x 5120 (34.1 for 28.1).
   // Weights below 2 MiB with K from 1024 on that are at most 512 x 768 of whole 256-wide columns (or whose sums are rounded once by request) and those
-  // from 2^26 elements on keep the kernels and splits that tests pin, though small tiles would be the faster ones there for some rows: int8
+  // of whole 256-wide columns from 2^26 elements on keep the kernels and splits that tests pin, though small tiles would be the faster ones there for some rows: int8
   // 121 x 1344 x 768 takes 26.9 us for their 5.5, bf16 8192 x 8192 with 96 rows 50.7 for 41.5. Other weights below 2 MiB take them (us: whole
   // 256-wide columns f16 181 x 576 x 1280 27.8 -> 4.3, 8192 x 768 x 768 22.1 -> 17.5, int8 768 x 1408 x 512 31.3 -> 6.2, 2276 x 384 x 3072
   // 20.3 -> 11.6, 200 such products a third of the time in the mean, none slower; others bf16 85 x 1088 x 816 22.7 -> 4.9,
-  // 365 x 1408 x 744 34.0 -> 7.4, 1096 x 1152 x 552 34.4 -> 7.0, int8 200 x 640 x 584 20.7 -> 4.5). Narrow products of at most 64 rows
+  // 365 x 1408 x 744 34.0 -> 7.4, 1096 x 1152 x 552 34.4 -> 7.0, int8 200 x 640 x 584 20.7 -> 4.5), and those of ragged columns from
+  // 2^26 elements on (us: int8 [N,K] 320 x 8192 x 8200 72 -> 38, f16 69 x 9728 x 13872 111 -> 60, [K,N] 845 x 8128 x 8560 206 -> 124; 103 products 0.75 of the
+  // time in the mean, f16 1600 x 12160 x 7408 the slowest of them, 275 -> 310). Narrow products of at most 64 rows
   // (N < 1024) are the skinny kernel's.
   bool pickSmallTile() {
     if (serial_ || dyn_ || batch_ != 1 || opt_.split > 0 || (opt_.variant & (8 | 128))) return false;
     const int64_t elements = k_ * n_;
-    if (m_ <= 32 || elements >= (1LL << 26)) return false;
     const bool narrow = m_ <= skinnyRows();
+    if (m_ <= 32 || (elements >= (1LL << 26) && (narrow || n_ % 256 == 0))) return false;
+    if (!transB_ && elements * elemBytes() >= (1LL << 31)) return false;   // (the row of a [K,N] weight is a 31-bit offset)
     const bool fewWhole = n_ % 256 == 0 && n_ <= 768 && m_ <= 512 && k_ >= 1024;
     if (elements * elemBytes() < (2LL << 20) && (narrow || fewWhole || roundedOnce_)) return false;
     if (narrow && n_ < 1024) return false;
@@ -281,7 +291,14 @@ class GemmEmitter {
     const int64_t steps = (k_ * elemBytes() + 127) / 128;
     // (columns that are whole 256-wide tiles pad nothing there: small ones from a quarter below on; 1200 x 8192 x 2048, which a test
     // pins, takes 59.6 us on them and 56.4 on 128 x 128)
-    double best = narrow ? 1e30 : (n_ % 256 == 0 ? 0.75 : 1.0) * largeTileTime(largeTileSplit());
+    // What the estimates above leave out, the operands' and the result's way from and to memory, is the same for every small tile: with it
+    // they are 2 % below 224 products measured, without 21 %. (Not those of 8-bit [K,N] weights, which are 5 % above as they are, nor with at most 256 rows or whole 256-wide
+    // columns, where the other estimate leaves it out too.) us, taken without it
+    // and on 256 x 256 tiles: f16 [N,K] 1600 x 12160 x 7408 311 / 277, 3931 x 2144 x 6224 123 / 111, int8 908 x 9600 x 12216 126 / 114; the other way round
+    // int8 [N,K] 2390 x 640 x 5184 20.4 / 21.0, f16 710 x 7104 x 15856 183 / 197.
+    const bool transposing8 = elemBytes() == 1 && !transB_;
+    const double traffic = transposing8 || m_ <= 256 || n_ % 256 == 0 ? 0 : (0.09 * static_cast<double>(elements * elemBytes()) + 0.19 * static_cast<double>(m_ * k_ * elemBytes()) + 0.18 * static_cast<double>(m_ * n_)) * 1e-6;
+    double best = narrow ? 1e30 : (n_ % 256 == 0 ? 0.75 : transposing8 ? 1.1 : 1.0) * largeTileTime(largeTileSplit()) - traffic;
     for (const SmallShape &w : smallShapes()) {
       if ((narrow && w.m > 64) || k_ * elemBytes() * std::max(w.m, w.n) >= (1LL << 31)) continue;
       // (several tiles a workgroup from 17 steps on: for fewer, what comes behind the loop is a third of their time;

@@ -85,9 +85,11 @@ def test_two_workgroups_of_128_x_128_fit_a_cu(m, k, n, tmp_path):
     (65, 960, 256, "bfloat16", False), (257, 64, 512, "float16", True), (512, 1008, 768, "bfloat16", True),   # K below 1024
     (513, 1024, 256, "float16", False), (300, 1024, 1024, "int8", False), (2048, 768, 768, "bfloat16", False),
     (513, 2040, 512, "bfloat16", True), (1500, 1088, 1792, "int8", True),
+    (65, 8192, 8196, "bfloat16", True), (300, 8192, 8200, "float16", False), (320, 8208, 8200, "int8", True), (129, 8208, 8196, "int8", False),   # large ones
 ])
-def test_small_weights_of_whole_wide_columns(m, k, n, dtype, tb, tmp_path):
-    """Weights below 2 MiB whose columns are whole 256-wide tiles take small tiles too, but for a few products with a long K."""
+def test_small_weights_of_whole_wide_columns_and_large_ones_of_ragged(m, k, n, dtype, tb, tmp_path):
+    """Weights below 2 MiB whose columns are whole 256-wide tiles take small tiles too, but for a few products with a long K,
+    and so do those from 2^26 elements on whose columns are not."""
     got = _tile(m, k, n, dtype, tb)
     assert got is not None
     _against_float64(m, k, n, dtype, tb, "%dx%d" % tuple(128 if x % 128 == 0 else 64 for x in got[:2]), tmp_path)
