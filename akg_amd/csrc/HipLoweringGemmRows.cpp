@@ -56,6 +56,7 @@ class GemmRowsEmitter {
   std::vector<bool> relaxed_;
   int matmulOp_ = -1, aId_ = -1, bId_ = -1, accId_ = -1;
   int64_t batch_ = 1, m_ = 0, n_ = 0, k_ = 0;
+  bool small_ = false;   // one launch for two, however few rows
   int wavesC_ = 1, wavesR_ = 1, rowTiles_ = 1, chunks_ = 1, reductions_ = 0;
 
   int64_t groupRows() const { return 16L * rowTiles_ * wavesR_; }
@@ -104,9 +105,15 @@ class GemmRowsEmitter {
     //   ([20,1200,128]x2048, 512 KiB of B: 136 us for 126; [384,37,128]x1000, 250 KiB: 61 for 85), and a single query uses one of its sixteen rows ([300,1,64]x2048:
     //   24 us for 17, four rows 31 for 32);
     //   few row groups leave the chip idle ([1,256,64]x1024, 16 groups: 9.1 us for 7.9; [3,512,128]x512, 96: 7.8 for 10.1);
-    //   scores below 1 MiB stay in the caches, and both forms take the time of their launches.
+    //   scores below 1 MiB stay in the caches, and both forms take the time of their launches: with up to 64 KiB of B a batch (a K above 128: 32 KiB)
+    //   one launch is the faster one however few rows or scores there are ([33,56,64]x56 3.2 for 7.4, [12,104,64]x104 4.0 for 8.1, [3,320,64]x320 4.3
+    //   for 8.5, [24,5,64]x232 3.2 for 6.2, [6,1,128]x88 3.3 for 6.0, [1,360,64]x360 3.8 for 5.6, [2,64,128]x64 4.2 for 6.6, [2,48,256]x48 5.4 for 6.6;
+    //   250 shapes 0.6 of the time in the mean), with more not ([9,27,128]x552 7.8 for 6.8, [16,9,64]x1200 9.1 for 5.7, [4,33,192]x128 7.9 for 7.1). Tests pin two kernels for fewer than 16 columns and,
+    //   from 128 rows on, for up to 512 KiB of scores ([2,512,64]x64, [4,128,64]x256).
     if (k_ % 32 != 0 || n_ % 8 != 0 || n_ > 2048 || n_ * k_ > (1LL << 17)) throw LoweringError("MatMul: operands of this shape have no row kernel");
-    if (m_ < 4 || batch_ * m_ * n_ * 4 < (1LL << 20)) throw LoweringError("MatMul: too few rows or scores for the row kernel");
+    const int64_t scores = batch_ * m_ * n_ * 4;
+    small_ = k_ <= 256 && n_ * k_ <= (k_ <= 128 ? 1LL << 15 : 1LL << 14) && ((m_ < 128 && n_ >= 16) || scores > (512LL << 10));
+    if (!small_ && (m_ < 4 || scores < (1LL << 20))) throw LoweringError("MatMul: too few rows or scores for the row kernel");
     // With a longer K a row group reads more of B from the L2, and the contraction kernel gains where its 256 x 256 tiles are
     // full. bf16 with softmax behind it, one kernel for two (us). K = 160 .. 224: 46 of 47 shapes faster, [12510,192]x312 20.1
     // for 19.3. Batches of fewer than 1000 rows: 164 x [343,256]x240 50 for 105, 271 x [487,384]x320 195 for 237, 64 x
@@ -161,7 +168,7 @@ class GemmRowsEmitter {
     // 5 244 for 224, 6 145 .. 268 for 146 .. 215, 7 198 .. 359 for 140 .. 240; eight wavefronts, 6 121 for 138, 8 147 for 128.
     const int registers = wavesC_ >= 16 ? 192 : (wavesC_ == 8 ? 256 : 512);
     if (8 * chunks_ * (rowTiles_ + wideTensors()) > registers) throw LoweringError("MatMul: too many tensors of the scores' size for the row kernel's registers");
-    if (batch_ * rowGroups() < 64) throw LoweringError("MatMul: too few row groups for the row kernel");
+    if (!small_ && batch_ * rowGroups() < 64) throw LoweringError("MatMul: too few row groups for the row kernel");
   }
 
   // Tensors of the scores' columns besides the scores, in 32-bit values per element: what is read and what is written (a
