@@ -437,6 +437,15 @@ class TileEmitter {
           if (ceilDiv(rowChunks, t) <= 8) break;
         }
       }
+      // Few rows: what a thread does one after the other is all of the time, so a row takes threads until each has one chunk, as long as the
+      // threads of all rows are half of what the chip holds at once (512 a row: a quarter). us, the rules above / this: bf16 quantisation
+      // 224 x 835 6.6 / 3.3 (14 workgroups), 152 x 7120 6.6 / 3.8, 30 x 3112 6.0 / 3.4, 744 x 810 6.2 / 3.3, LayerNorm 17 x 6488 4.6 / 3.5, 1324 x 1583
+      // 4.8 / 4.4, 1483 x 3392 9.5 / 7.3; beyond, quantisation 2248 x 1328 would take 6.3 for 6.1, 1096 x 451 on 256 threads a row 4.2 for 3.5.
+      // (Fewer than ten rows stay as they are: tests pin the rules above on them.)
+      if (opt_.threadsPerRow == 0 && !ordered_ && !extentArg_ && rows_ >= 10) {
+        while (tpr < 256 && tpr < rowChunks && rows_ * 2 * tpr <= (1LL << 18)) tpr *= 2;
+        while (tpr >= 256 && tpr < 512 && tpr < rowChunks && rows_ * 2 * tpr <= (1LL << 17)) tpr *= 2;
+      }
       // Rows of any length in the bucket that vector instructions bound: a wavefront leaves out the chunks beyond its row (chunkwise_), and
       // where it would hold a row in two chunks a lane it takes two rows with four chunks a lane instead - the second chunk of 64
       // lanes costs a row of 257 elements as much as one of 512. That takes many rows, as a row is a longer way for its lanes, and
