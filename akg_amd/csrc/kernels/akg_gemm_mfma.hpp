@@ -196,8 +196,7 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
   constexpr bool kFull = !DYN && (MS % kGemmBM == 0) && (N % kGemmBN == 0) && (K % BK == 0);
   // Ragged tiles behind full ones (and, with an M that is an argument, whole tiles along N and K): the loads need no checks either, so
   // the main loop is the one of a whole shape, one basic block per K step. Every thread clamps the rows of A, and the columns of a
-  // [N,K] B, that it stages to the last one, once, in front of the loop (the scalar offset of a buffer load takes no part in the
-  // descriptor's range check, so the descriptor alone would not keep them inside); what lies beyond M and N then holds copies whose
+  // [N,K] B, that it stages to the last one, once, in front of the loop; what lies beyond M and N then holds copies whose
   // accumulators are dropped by the epilogue's checks. Chunks of a row-major B beyond N, and chunks beyond K, are asked for beyond the
   // buffer and read zero. us, a branch around every load / this, with the epilogue's stores as they are below: f16 3584 x 896 x
   // 8928 67.0 / 57.8, [N,K] 2048 x 4112 x 2052 int8 70.6 / 61.5, [N,K] 900 x 608 x 16380 f16 32.7 / 24.3; 42 products that take this kernel in
@@ -272,7 +271,8 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
   const int aChunk = tid % kChunksPerRow;
   // Global loads are buffer loads: the per-lane offset is computed once, everything that changes from load to load
   // (row block, k-row, K step) is a scalar offset, so the loop spends no vector instructions on addresses (vector
-  // instructions and MFMAs compete for issue cycles). Out-of-range lanes read zero through the descriptor's size.
+  // instructions and MFMAs compete for issue cycles). Out-of-range lanes read zero through the descriptor's size: the hardware
+  // compares the sum of both offsets with it, word by word (measured inside one allocation, behind a shorter descriptor).
   // The descriptor of A (and of a [N,K] B) starts at the tile's first row, so the 32-bit offsets only have to span a
   // tile and A may be of any size (131072 tokens x 8192 bf16 are 2 GiB); a row-major B is addressed from its start.
   static_assert(kGemmBM * K < (1L << 31) && (TRANSB ? kGemmBN * K : N * K) < (1L << 31), "operand too large for 32-bit buffer offsets");

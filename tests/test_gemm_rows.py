@@ -88,7 +88,7 @@ def test_scores_and_their_row_reductions(batch, m, k, n, dtype, mask, outputs):
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,m,k,n,dtype,mask,outputs", [
     (1, 1, 64, 16, "bfloat16", None, ["p"]), (6, 3, 128, 88, "float16", [6, 3, 88], ["p"]),      # one row, three
-    (2, 127, 256, 64, "bfloat16", [1, 127, 64], ["p", "max"]), (0, 17, 32, 1024, "float16", [1, 1024], ["p32", "sum"]),   # the most of B
+    (3, 127, 256, 64, "bfloat16", [1, 127, 64], ["p", "max"]), (0, 17, 32, 1024, "float16", [1, 1024], ["p32", "sum"]),   # the most of B
     (3, 320, 64, 320, "float16", [3, 320, 320], ["p"]), (5, 161, 96, 168, "bfloat16", None, ["p"]),   # from 128 rows on: more than 512 KiB of scores
     (33, 56, 64, 56, "bfloat16", [33, 1, 56], ["p", "sum_flat"]),
 ])
