@@ -266,7 +266,7 @@ class GemmEmitter {
   // it is the slower one, and the estimates say so, for 3568 x 5056 x 3848 (137 / 193 / 167) and 1881 x 4160 x 7568 (118 / 152 / 125).
   // The skinny one is faster at 33 rows for [K,N] weights of bf16 8192 x 6144 (30.9 for 26.1), int8 4096 x 6144 (14.8 for 13.4) and 6144 x 9216
   // (27.9 for 20.0), for [N,K] of bf16 11008 x 5120 (34.1 for 28.1).
-  // Weights below 2 MiB with K from 1024 on that are at most 512 x 768 of whole 256-wide columns (or whose sums are rounded once by request) and those
+  // Weights below 2 MiB with K from 1024 on (256 columns: 512) and at most 512 rows x 768 of whole 256-wide columns (or whose sums are rounded once by request) and those
   // of whole 256-wide columns from 2^26 elements on keep the kernels and splits that tests pin, though small tiles would be the faster ones there for some rows: int8
   // 121 x 1344 x 768 takes 26.9 us for their 5.5, bf16 8192 x 8192 with 96 rows 50.7 for 41.5. Other weights below 2 MiB take them (us: whole
   // 256-wide columns f16 181 x 576 x 1280 27.8 -> 4.3, 8192 x 768 x 768 22.1 -> 17.5, int8 768 x 1408 x 512 31.3 -> 6.2, 2276 x 384 x 3072
@@ -281,7 +281,7 @@ class GemmEmitter {
     const bool narrow = m_ <= skinnyRows();
     if (m_ <= 32 || (elements >= (1LL << 26) && (narrow || n_ % 256 == 0))) return false;
     if (!transB_ && elements * elemBytes() >= (1LL << 31)) return false;   // (the row of a [K,N] weight is a 31-bit offset)
-    const bool fewWhole = n_ % 256 == 0 && n_ <= 768 && m_ <= 512 && k_ >= 1024;
+    const bool fewWhole = n_ % 256 == 0 && n_ <= 768 && m_ <= 512 && k_ >= (n_ <= 256 ? 512 : 1024);
     if (elements * elemBytes() < (2LL << 20) && (narrow || fewWhole || roundedOnce_)) return false;
     if (narrow && n_ < 1024) return false;
     // (Rows of a [K,N] weight that are not whole 16-byte chunks: with 8 bits and more than 64 rows. us, 256 x 256 tiles -> small ones:
