@@ -162,7 +162,12 @@ class GemmRowsEmitter {
       while (wavesC_ * wavesR_ < 4 && m_ > 16L * rowTiles_ * wavesR_) wavesR_ *= 2;
       return batch_ * rowGroups();
     };
-    if (m_ <= 16 || shape(2) < 512) shape(1);
+    // (Sixteen wavefronts are alone on their CU, where two row tiles take 1.75 of the time of one: [8,1824,64] x 1824, 912 and 456 workgroups,
+    // 63.0 / 55.3 us, [26,1160,64] x 1160 82.9 / 72.8, [100,96,64] x 1400, 600 and 300, 37.6 / 41.0.
+    // With more than a mask and a 16-bit result two tiles have no registers left: those as the others.)
+    const int64_t one = shape(1), two = shape(2);
+    const bool pays = wavesC_ >= 16 && wideTensors() <= 2 ? 7 * ((two + 255) / 256) < 4 * ((one + 255) / 256) : two >= 512;
+    if (m_ <= 16 || !pays) shape(1);
     // Every tensor of the scores' columns takes eight registers per unit, and a workgroup of sixteen wavefronts leaves 128 a
     // lane: beyond half as many again the spills cost more than the scores' way through memory. [*,*,64] x 2048 by the number
     // wideTensors() (us for two kernels): 3 (a float32 result and a mask) 122 .. 135 for 120 .. 136, 4 115 .. 179 for 139 .. 194,
@@ -171,6 +176,12 @@ class GemmRowsEmitter {
     if (8 * chunks_ * (rowTiles_ + wideTensors()) > registers) throw LoweringError("MatMul: too many tensors of the scores' size for the row kernel's registers");
     if (!small_ && batch_ * rowGroups() < 64) throw LoweringError("MatMul: too few row groups for the row kernel");
   }
+
+  // Eight wavefronts a row (513 .. 1024 columns): 32-bit tensors of the scores' size are read by whole lines of eight rows, and with two row
+  // tiles so is B. us, half lines of sixteen rows / the tensors / both: [60,640,64] x 640 48.5 / 45.7 / 44.9, [24,896,64] x 896 40.6 / 39.7 / 37.3,
+  // [20,2048,64] x 1024 68.6 / 67.2 / 63.5, [13,664,64] x 664 (one row tile) 16.3 / 15.9 / 16.4; four wavefronts [192,512,64] x 512 72.7 / 72.9 / 76.5,
+  // sixteen [26,1160,64] x 1160 73.0 / 74.2 / 74.0, two [300,256,64] x 256 33.9 / 34.6 / 34.7.
+  bool byLines() const { return wavesC_ == 8; }
 
   // Tensors of the scores' columns besides the scores, in 32-bit values per element: what is read and what is written (a
   // float32 result is computed by the longer forms of the functions in front of it: one more).
@@ -211,12 +222,12 @@ class GemmRowsEmitter {
     return s;
   }
 
-  // row of the tensor (in rows of its last extent) that belongs to row akg_mc of batch akg_b
-  std::string rowOf(const std::vector<int64_t> &s) const {
+  // row of the tensor (in rows of its last extent) that belongs to `row` (akg_mc: the lane's own) of batch akg_b
+  std::string rowOf(const std::vector<int64_t> &s, const std::string &row = "akg_mc") const {
     const bool b = s[0] != 1, m = s[1] != 1;
-    if (b && m) return "(akg_b * M + akg_mc)";
+    if (b && m) return "(akg_b * M + " + row + ")";
     if (b) return "akg_b";
-    return m ? "akg_mc" : "0L";
+    return m ? row : "0L";
   }
 
   void loops(const std::string &indent) {
@@ -238,6 +249,12 @@ class GemmRowsEmitter {
     }
     v.rank = Rank::Full;
     v.ident = "t_in" + std::to_string(i);
+    if (byLines() && s[1] != 1 && dtypeSize(t.dtype) == 4) {
+      src_ << "    " << ct << " " << v.ident << "[NCHUNK][8];\n#pragma unroll\n    for (int j = 0; j < NCHUNK; ++j) akg::load_own_row_if<" << tag
+           << ">(b_in" << i << ", akg_ok[j], " << rowOf(s, "akg_low") << " * N + akg_cols[j], " << rowOf(s, "akg_high")
+           << " * N + akg_cols[j], lane, " << v.ident << "[j]);\n";
+      return;
+    }
     src_ << "    " << ct << " " << v.ident << "[NCHUNK][8];\n#pragma unroll\n    for (int j = 0; j < NCHUNK; ++j) akg::load_chunk_if<" << tag
          << ", 8, false>(b_in" << i << ", akg_ok[j], " << rowOf(s) << " * N + akg_cols[j], " << v.ident << "[j]);\n";
   }
@@ -390,11 +407,14 @@ class GemmRowsEmitter {
       << "    akg_cols[j] = 32L * akg::row_unit<NCHUNK, WC>(j, wc) + 8 * (lane >> 4);\n    akg_ok[j] = "
       << (n_ % (32L * wavesC_) == 0 ? "true" : "akg_cols[j] < N") << ";\n  }\n"
       << "  float akg_s[RT][NCHUNK][8];\n" 
-      << "  akg::row_scores<" << mma() << ", M, N, " << k_ * 2 << "L, RT, NCHUNK, WC>(in" << g_.tensor(aId_).inputIndex << " + akg_b * "
+      << "  akg::row_scores<" << mma() << ", M, N, " << k_ * 2 << "L, RT, NCHUNK, WC, " << (byLines() && rowTiles_ == 2 ? "true" : "false") << ">(in" << g_.tensor(aId_).inputIndex << " + akg_b * "
       << m_ * k_ << "L, in" << g_.tensor(bId_).inputIndex << " + akg_b * " << n_ * k_ << "L, akg_row0, wc, lane, akg_s);\n"
       << "#pragma unroll\n  for (int rt = 0; rt < RT; ++rt) {\n"
       << "    const long akg_m = akg_row0 + 16 * rt + (lane & 15);\n    const bool akg_row_ok = akg_m < M;\n"
       << "    const long akg_mc = akg_row_ok ? akg_m : M - 1;\n    (void)akg_mc;\n"
+      << "    // the rows of lanes c % 8 and c % 8 + 8 of the sixteen (load_own_row_if)\n"
+      << "    const long akg_first = akg_row0 + 16 * rt + (lane & 7), akg_low = akg_first < M ? akg_first : M - 1, akg_high = akg_first + 8 < M ? akg_first + 8 : M - 1;\n"
+      << "    (void)akg_low, (void)akg_high;\n"
       << src_.str() << "  }\n}\n";
     return o.str();
   }

@@ -26,6 +26,38 @@ AKG_DEV constexpr int row_unit(int j, int wc) {
   return NCHUNK % 2 == 0 ? ((j / 2) * WC + wc) * 2 + j % 2 : j * WC + wc;
 }
 
+// Two loads of 16 bytes a lane that touch whole lines of eight rows each: in the first, the lanes c = lane % 16 below 8 have piece p of row c,
+// the others piece q of row c - 8; in the second piece p of row c + 8 and piece q of row c. Afterwards `first` is piece p and `second` piece
+// q of the lane's own row c. (Rows of their own in either load, all sixteen of them half a line each, take twice as many of a CU's
+// requests.)
+AKG_DEV void own_row_pieces(v4i &first, v4i &second) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int f = first[e], s = second[e];
+    first[e] = __builtin_amdgcn_update_dpp(f, s, 0x128, 0xF, 0xC, false);    // lanes 8 .. 15 take from the lane 8 below
+    second[e] = __builtin_amdgcn_update_dpp(s, f, 0x128, 0xF, 0x3, false);   // lanes 0 .. 7 from the lane 8 above
+  }
+}
+
+// load_chunk_if of the eight adjacent 32-bit columns of the lane's own row, by whole lines: `low` is the index of these columns in the row
+// of lane c % 8 of the sixteen, `high` in that of lane c % 8 + 8.
+template <typename DT>
+AKG_DEV void load_own_row_if(Buffer buf, bool ok, long low, long high, int lane, typename DT::compute (&dst)[8]) {
+  typedef typename DT::storage S;
+  static_assert(sizeof(S) == 4, "a chunk is two pieces");
+  typedef BufferIo<16, kAuxDefault> Io;
+  const u32 piece = 16u * ((static_cast<u32>(lane) >> 3) & 1u);
+  v4i p = __builtin_bit_cast(v4i, Io::load(buf, ok ? static_cast<u32>(low) * 4u + piece : kBeyondEveryBuffer));
+  v4i q = __builtin_bit_cast(v4i, Io::load(buf, ok ? static_cast<u32>(high) * 4u + piece : kBeyondEveryBuffer));
+  own_row_pieces(p, q);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int a = p[e], b = q[e];
+    dst[e] = DT::load(__builtin_bit_cast(S, a));
+    dst[4 + e] = DT::load(__builtin_bit_cast(S, b));
+  }
+}
+
 // A number (of 64-byte slabs of K) as a type.
 template <int N>
 struct SlabCount {
@@ -33,12 +65,13 @@ struct SlabCount {
 };
 
 // s[rt][j] = the eight columns of unit row_unit(j, wc) (columns beyond N hold copies of column N - 1) in row
-// row0 + 16 rt + lane % 16 (rows beyond M hold copies of row M - 1). KB: bytes of K per row, a multiple of 64.
+// row0 + 16 rt + lane % 16 (rows beyond M hold copies of row M - 1). KB: bytes of K per row, a multiple of 64. LINES: two slabs of K at a
+// time from whole lines of B.
 // Up to seven slabs of 64 bytes the rows of A stay in registers; a longer K is taken in blocks of four with the
 // accumulators live, so the registers do not grow with K (bf16, 512 x 256 with softmax: 200 a lane at K = 512, 332 with all of K
 // held, where K = 1024 and more spilled; K = 512 50 us either way, and the next block's rows requested beside the MFMAs of a block
 // gave nothing).
-template <typename Mma, long M, long N, long KB, int RT, int NCHUNK, int WC>
+template <typename Mma, long M, long N, long KB, int RT, int NCHUNK, int WC, bool LINES>
 AKG_DEV void row_scores(const void *__restrict__ A, const void *__restrict__ B, long row0, int wc, int lane,
                         float (&s)[RT][NCHUNK][8]) {
   static_assert(KB % 64 == 0 && M * KB < (1L << 31) && N * KB < (1L << 31), "operand shapes of the fragments");
@@ -72,16 +105,37 @@ AKG_DEV void row_scores(const void *__restrict__ A, const void *__restrict__ B, 
       for (int j = j0; j < j0 + kBatch && j < NCHUNK; ++j) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          long col = 32L * row_unit<NCHUNK, WC>(j, wc) + 8 * (c >> 2) + 4 * h + (c & 3);
-          if constexpr (N % (32L * WC) != 0) col = col < N ? col : N - 1;
-          const u32 off = static_cast<u32>(col * KB) + 16u * static_cast<u32>(g) + at;
+          auto offsetOf = [&](int cc) {
+            long col = 32L * row_unit<NCHUNK, WC>(j, wc) + 8 * (cc >> 2) + 4 * h + (cc & 3);
+            if constexpr (N % (32L * WC) != 0) col = col < N ? col : N - 1;
+            return static_cast<u32>(col * KB) + 16u * static_cast<u32>(g) + at;
+          };
+          constexpr int kPaired = LINES ? kCount / 2 * 2 : 0;   // eight columns a load, own_row_pieces below; the others sixteen
+          if constexpr (kPaired > 0) {
+            const u32 half = 64u * static_cast<u32>(c >> 3), low = offsetOf(c & 7) + half, high = offsetOf((c & 7) + 8) + half;
 #pragma unroll
-          for (int i = 0; i < kCount; ++i) kf[j - j0][h][i] = *reinterpret_cast<const v4i *>(b + off + 64 * i);
+            for (int i = 0; i < kPaired; i += 2) {
+              kf[j - j0][h][i] = *reinterpret_cast<const v4i *>(b + low + 64 * i);
+              kf[j - j0][h][i + 1] = *reinterpret_cast<const v4i *>(b + high + 64 * i);
+            }
+          }
+          if constexpr (kPaired < kCount) {
+            const u32 off = offsetOf(c);
+#pragma unroll
+            for (int i = kPaired; i < kCount; ++i) kf[j - j0][h][i] = *reinterpret_cast<const v4i *>(b + off + 64 * i);
+          }
         }
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = j0; j < j0 + kBatch && j < NCHUNK; ++j) {
+        if constexpr (LINES) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i + 1 < kCount; i += 2) own_row_pieces(kf[j - j0][h][i], kf[j - j0][h][i + 1]);
+          }
+        }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll

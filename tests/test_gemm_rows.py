@@ -97,6 +97,18 @@ def test_one_launch_for_few_rows_and_scores(batch, m, k, n, dtype, mask, outputs
     test_scores_and_their_row_reductions(batch, m, k, n, dtype, mask, outputs)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,m,k,n,dtype,mask,outputs", [
+    (40, 401, 64, 520, "bfloat16", [40, 401, 520], ["p"]),                  # eight wavefronts, two row tiles: a row and eight columns over
+    (64, 249, 96, 1000, "float16", [1, 249, 1000], ["p"]),                  # a slab of K without a second one
+    (40, 25, 128, 544, "bfloat16", [40, 25, 544], ["p", "max"]),              # one row tile
+    (3, 1985, 64, 1032, "float16", [3, 1985, 1032], ["p"]), (5, 1601, 64, 1960, "bfloat16", [1, 1, 1960], ["p"]),   # sixteen wavefronts
+])
+def test_whole_lines_and_two_row_tiles(batch, m, k, n, dtype, mask, outputs):
+    """32-bit tensors and B by whole lines of eight rows, rows and columns beyond the last; bounds as above."""
+    test_scores_and_their_row_reductions(batch, m, k, n, dtype, mask, outputs)
+
+
 def _scratch_bytes(directory):
     """Private bytes per lane of the code objects under `directory` (the kernel descriptor's note, a MessagePack map)."""
     import glob
