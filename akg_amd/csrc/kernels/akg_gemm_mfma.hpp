@@ -341,10 +341,14 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
         stage.y[i] = v4i{0, 0, 0, 0};
       }
     } else {
-      const long krow = k0 / EB + bRowT + kRowStepB * i;
+      const long first = k0 / EB + kRowStepB * i, krow = first + bRowT;
       if (kLoadsInRange || (krow < KE && n0 * EB + bChunkT * 16 < NB)) {
-        const bool there = !kClampRows || K % BK == 0 || krow < KE;
-        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(bRsrc, there ? bVoff : kBeyond, static_cast<int>((k0 / EB + kRowStepB * i) * NB), 0);
+        const bool whole = !kClampRows || K % BK == 0;
+        // (A scalar offset of 2 GiB and more, behind the last k-row of a weight of nearly that size, would meet kBeyond inside the buffer
+        // if their sum had 32 bits. It has more on the card this was tried on; no lane is there, so the offset is left out.)
+        constexpr bool kPast2Gib = kClampRows && (kSteps * BK / EB) * NB >= (1L << 31);
+        const long rows = kPast2Gib && first >= KE ? 0 : first;
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(bRsrc, whole || krow < KE ? bVoff : kBeyond, static_cast<int>(rows * NB), 0);
         stage.y[i] = v4i{static_cast<int>(v[0]), static_cast<int>(v[1]), static_cast<int>(v[2]), static_cast<int>(v[3])};
       } else {
         stage.y[i] = v4i{0, 0, 0, 0};

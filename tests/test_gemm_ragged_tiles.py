@@ -49,3 +49,25 @@ def test_ragged_tiles_against_float64(m, k, n, dtype, tb, monkeypatch):
     gap = (out[:m].double() - y).abs()
     assert bool((gap <= bound).all()), float((gap / bound).max())
     assert bool(out[m].isnan().all())
+
+
+@pytest.mark.gpu
+def test_k_rows_behind_a_weight_of_nearly_2_gib_read_zero(monkeypatch):
+    """The last step of K has 8 of its 64 k-rows; those from 4112 on would begin 2 GiB and more behind the weight's first byte. An infinity in
+    one place of the weight (row 7, where an offset that has wrapped around would lie) reaches its own columns only."""
+    import torch
+    monkeypatch.setenv("AKG_HIP_VARIANT", "128")
+    m, k, n, at = 257, 4104, 261632, 257536
+    assert 2 * n * k < 1 << 31 <= 2 * n * 4112 and 2 * n * 4112 - (1 << 31) == 2 * (7 * n + at)
+    kernel = driver.HipKernel(op_desc.gemm_bias_act(m, k, n, "bfloat16", "none", transpose_b=False), out_dir=None)
+    assert "gemm_256x256<" in kernel.source
+    print("case", m, k, n, flush=True)
+    dev = "cuda"
+    a, w = torch.ones((m, k), device=dev, dtype=torch.bfloat16), torch.zeros((k, n), device=dev, dtype=torch.bfloat16)
+    w[7, at:at + 8] = float("inf")
+    out = torch.zeros((m, n), device=dev, dtype=torch.bfloat16)
+    kernel.launch([a, w, torch.ones(n, device=dev, dtype=torch.bfloat16), out])
+    torch.cuda.synchronize()
+    own = torch.zeros(n, device=dev, dtype=torch.bool)
+    own[at:at + 8] = True
+    assert bool(out[:, own].isinf().all()) and bool((out[:, ~own] == 1).all())
