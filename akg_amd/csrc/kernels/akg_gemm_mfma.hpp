@@ -531,7 +531,10 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
   __syncthreads();
   readA(0, 0, 0, fa[0]);
   readB(0, 0, 0, fb[0]);
+  // (Left to itself the compiler unrolls this for up to eight steps, and with a [K,N] B whose last one is not whole spills two to eight
+  // registers: us, bf16 6986 x 384 x 12096 95.2 -> 89.4, 2804 x 304 x 9272 37.1 -> 34.7, 571 x 352 x 9424 16.8 / 16.9.)
   long step = 0;
+#pragma unroll 1
   for (; step + 2 < mySteps; ++step) stepSpread(step, BoolTag<true>(), BoolTag<true>());
   if (step + 1 < mySteps) {
     stepSpread(step, BoolTag<true>(), BoolTag<false>());

@@ -2,6 +2,7 @@
 import pytest
 
 from akg_amd import driver, op_desc
+from gemm_checks import compiled_notes
 
 
 @pytest.mark.gpu
@@ -71,3 +72,15 @@ def test_k_rows_behind_a_weight_of_nearly_2_gib_read_zero(monkeypatch):
     own = torch.zeros(n, device=dev, dtype=torch.bool)
     own[at:at + 8] = True
     assert bool(out[:, own].isinf().all()) and bool((out[:, ~own] == 1).all())
+
+
+@pytest.mark.parametrize("m,k,n,dtype", [
+    (3979, 360, 8780, "float16"), (571, 352, 9424, "bfloat16"), (2804, 304, 9272, "bfloat16"), (5850, 440, 11392, "float16"),
+    (4033, 272, 2376, "bfloat16"), (512, 232, 1024, "float16"), (300, 168, 516, "bfloat16"), (6986, 384, 12096, "bfloat16"), (7857, 448, 2368, "int8"),
+])
+def test_few_steps_of_k_stay_in_registers(m, k, n, dtype, monkeypatch, tmp_path):
+    """A [K,N] weight and three to eight steps of K, the last one ragged or not."""
+    monkeypatch.setenv("AKG_HIP_VARIANT", "128")
+    text = op_desc.gemm_int8_dequant_bias_gelu(m, k, n) if dtype == "int8" else op_desc.gemm_bias_act(m, k, n, dtype, "relu")
+    kernel, scratch, _ = compiled_notes(text, tmp_path)
+    assert "gemm_256x256<" in kernel.source and scratch == 0
