@@ -573,8 +573,10 @@ AKG_DEV void gemm_256x256(const void *__restrict__ A, const void *__restrict__ B
   // 4 x 64: where the rows of the result are not whole 64-byte pieces, half as many pieces are written in part. us, loads without
   // branches, 4 x 64 / 2 x 128: bf16 [N,K] 3584 x 896 x 8936 81.1 / 60.4 (8960: 54.5 / 54.4), int8 -> bf16 64.0 / 43.1, f16 row-major
   // 4096 x 2048 x 12280 206 / 178. (Stored without the streaming hint they meet in L2: 68.6, but the operands leave it: 60.0 for 8960.)
-  // Not where every row is whole pieces: 4096 x 8192 x 8192 419.5 / 420.6.
-  constexpr bool kPairs = kTN == 8 && N % 64 != 0;
+  // Not where every row is whole pieces: 4096 x 8192 x 8192 419.5 / 420.6. Nor up to 128 columns, where the lanes of the second group would
+  // have few columns or none and the others the rows of both (us, batches of bf16, 4 x 64 / 2 x 128: 200 x [158,128] x 12 61.0 / 102, 4 x [145,96] x 32
+  // with softmax 6.6 / 8.2, 4 x [578,64] x 80 18.5 / 19.2).
+  constexpr bool kPairs = kTN == 8 && N > 128 && N % 64 != 0;
   if constexpr (kPairs) {
 #pragma unroll
     for (int i = 0; i < kTM; ++i) {

@@ -1,4 +1,5 @@
 """What the tests of the contraction kernels share."""
+import os
 import re
 import subprocess
 
@@ -13,3 +14,10 @@ def compiled_notes(text, folder):
     scratch = max(int(x) for x in re.findall(r"\.private_segment_fixed_size:\s+(\d+)", notes))
     registers = max(int(x) for x in re.findall(r"\.vgpr_count:\s+(\d+)", notes))
     return kernel, scratch, registers
+
+
+def disassembled(text, folder):
+    """... and its code."""
+    kernel = driver.HipKernel(text, out_dir=str(folder))
+    objdump = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
+    return kernel, "".join(subprocess.run([objdump, "-d", str(f)], check=True, capture_output=True, text=True).stdout for f in folder.glob("*.hsaco"))

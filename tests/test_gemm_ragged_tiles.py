@@ -2,7 +2,7 @@
 import pytest
 
 from akg_amd import driver, op_desc
-from gemm_checks import compiled_notes
+from gemm_checks import compiled_notes, disassembled
 
 
 @pytest.mark.gpu
@@ -84,3 +84,11 @@ def test_few_steps_of_k_stay_in_registers(m, k, n, dtype, monkeypatch, tmp_path)
     text = op_desc.gemm_int8_dequant_bias_gelu(m, k, n) if dtype == "int8" else op_desc.gemm_bias_act(m, k, n, dtype, "relu")
     kernel, scratch, _ = compiled_notes(text, tmp_path)
     assert "gemm_256x256<" in kernel.source and scratch == 0
+
+
+@pytest.mark.parametrize("n,swaps", [(12, False), (64, False), (80, False), (124, False), (128, False), (132, True), (192, False), (200, True)])
+def test_up_to_128_columns_are_stored_by_every_lane(n, swaps, tmp_path):
+    """The exchange between column groups leaves the lanes of the second one idle where that has no columns."""
+    text = op_desc.batch_matmul_scale_mask(4, 158, 128, n, "bfloat16", True, "pairs_%d" % n)
+    kernel, code = disassembled(text, tmp_path)
+    assert "gemm_256x256<" in kernel.source and ("v_permlane16_swap" in code) == swaps
