@@ -4,7 +4,7 @@ import subprocess
 
 import pytest
 
-from akg_amd import driver
+from akg_amd import driver, op_desc
 from test_gemm_small_tiles import _product, test_small_tiles_against_float64 as _against_float64
 
 
@@ -93,3 +93,13 @@ def test_small_weights_of_whole_wide_columns_and_large_ones_of_ragged(m, k, n, d
     got = _tile(m, k, n, dtype, tb)
     assert got is not None
     _against_float64(m, k, n, dtype, tb, "%dx%d" % tuple(128 if x % 128 == 0 else 64 for x in got[:2]), tmp_path)
+
+
+@pytest.mark.parametrize("m,k,n,dtype,act,tb", [
+    (4630, 14424, 432, "bfloat16", "none", False), (1106, 13632, 2992, "bfloat16", "gelu", False), (5852, 8160, 368, "bfloat16", "gelu", True),
+    (8100, 8128, 384, "bfloat16", "none", False),
+])
+def test_products_of_small_tiles_fit_a_launch_without_allocations_still(m, k, n, dtype, act, tb):
+    """The 256 x 256 kernel would ask for 40 to 67 MB of partials here."""
+    kernel = driver.HipKernel(op_desc.gemm_bias_act(m, k, n, dtype, act, transpose_b=tb), out_dir=None)
+    assert kernel.workspace_bytes <= 16 << 20
