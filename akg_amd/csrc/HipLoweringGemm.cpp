@@ -226,13 +226,14 @@ class GemmEmitter {
     return split == 1 ? 3 + loop : 5.5 + loop + 0.3 * static_cast<double>(split) * area / 4096 + static_cast<double>(tiles * split) * area * 8 / 5e6;
   }
   // ... and of the 256 x 256 kernel with `split` workgroups per tile: fitted to the same products (14 %), and with more than 256 rows and
-  // ragged columns to 200 such (K and N 512 .. 16384, 8 %; 8-bit ones with dequantisation and GELU behind the sums).
+  // ragged columns to 200 such (K and N 512 .. 16384, 8 %; 8-bit ones with dequantisation and GELU behind the sums, whose eight wavefronts
+  // a CU have nothing to do beside it: 16-bit ones with GELU take 5 us a tile longer than without).
   double largeTileTime(int64_t split) const {
     const int64_t steps = (k_ * elemBytes() + 127) / 128, tiles = ((m_ + 255) / 256) * ((n_ + 255) / 256), perTile = (steps + split - 1) / split;
     const double perCu = static_cast<double>(tiles * split) / 256, whole = std::ceil(perCu), rows = static_cast<double>(std::min<int64_t>(m_, 256));
     if (m_ > 256 && n_ % 256 != 0 && !outgrowsLaunch(split)) {
       const double step = 1.478 * (transB_ ? 1 : 1.068) * (elemBytes() == 1 ? (transB_ ? 0.949 : 0.967) : 1), rounds = perCu <= 1 ? 1 : 0.87 * whole + 0.13 * perCu;
-      const double time = rounds * (static_cast<double>(perTile) * step + (elemBytes() == 1 ? 13.45 : 7.54));
+      const double time = rounds * (static_cast<double>(perTile) * step + (elemBytes() == 1 ? 13.45 : functionBehind() ? 12.54 : 7.54));
       return split == 1 ? time : time + 6.45 + 1.35 * static_cast<double>(split);
     }
     const double step = 1.45 * (transB_ ? 1 : 1.093) * (elemBytes() == 1 ? 1.356 : 1);
@@ -245,6 +246,12 @@ class GemmEmitter {
   bool outgrowsLaunch(int64_t split) const {
     const int64_t tiles = ((m_ + 255) / 256) * ((n_ + 255) / 256);
     return split > 1 && k_ * n_ < (1LL << 26) && tiles * split * std::min<int64_t>(m_, 256) * 256 * 4 + tiles * 4 > (16LL << 20);
+  }
+  bool functionBehind() const {
+    for (const OpNode &op : g_.ops) {
+      if (op.kind == OpKind::Exp || op.kind == OpKind::Tanh || op.kind == OpKind::Log || op.kind == OpKind::Pow) return true;
+    }
+    return false;
   }
   // 33 .. 64 rows: time in us of the skinny kernel and of 64 x 64 tiles, fitted to 1256 measured products (both layouts, 8 and
   // 16 bits, K 512 .. 14336, N 1024 .. 16384; the first within 11 %, the second within a quarter; standard deviations 3 and 6 %).
@@ -280,7 +287,8 @@ class GemmEmitter {
   // 20.3 -> 11.6, 200 such products a third of the time in the mean, none slower; others bf16 85 x 1088 x 816 22.7 -> 4.9,
   // 365 x 1408 x 744 34.0 -> 7.4, 1096 x 1152 x 552 34.4 -> 7.0, int8 200 x 640 x 584 20.7 -> 4.5), and those of ragged columns from
   // 2^26 elements on (us: int8 [N,K] 320 x 8192 x 8200 72 -> 38, f16 69 x 9728 x 13872 111 -> 60, [K,N] 845 x 8128 x 8560 206 -> 124; 103 products 0.75 of the
-  // time in the mean, f16 1600 x 12160 x 7408 the slowest of them, 275 -> 310). Narrow products of at most 64 rows (N < 1024) are the skinny kernel's.
+  // time in the mean, 130 others 0.74; f16 [N,K] 1600 x 12160 x 7408 the slowest of them, 274 -> 301; with at most 256 rows where they are estimated a
+  // fifth faster: f16 [K,N] 216 x 16128 x 8872, estimated 0.89, takes 141 on 256 x 256 tiles and 151). Narrow products of at most 64 rows (N < 1024) are the skinny kernel's.
   bool pickSmallTile() {
     if (serial_ || dyn_ || batch_ != 1 || opt_.split > 0 || (opt_.variant & (8 | 128))) return false;
     const int64_t elements = k_ * n_;
@@ -299,12 +307,14 @@ class GemmEmitter {
     // pins, takes 59.6 us on them and 56.4 on 128 x 128)
     // What the estimates above leave out, the operands' and the result's way from and to memory, is the same for every small tile: with it
     // they are 2 % below 224 products measured, without 21 %. (Not those of 8-bit [K,N] weights, which are 5 % above as they are, nor with at most 256 rows or whole 256-wide
-    // columns, where the other estimate leaves it out too.) us, taken without it
+    // columns, where the other estimate leaves it out too, nor with 16 steps and less, where single tiles wait for it beside each other: with it
+    // they are 14 % above for 16 bits and up to eight steps, without 3 % below.) us, taken without it
     // and on 256 x 256 tiles: f16 [N,K] 1600 x 12160 x 7408 311 / 277, 3931 x 2144 x 6224 123 / 111, int8 908 x 9600 x 12216 126 / 114; the other way round
-    // int8 [N,K] 2390 x 640 x 5184 20.4 / 21.0, f16 710 x 7104 x 15856 183 / 197.
-    const bool transposing8 = elemBytes() == 1 && !transB_, moved = !transposing8 && m_ > 256 && n_ % 256 != 0 && !outgrowsLaunch(largeTileSplit());
+    // int8 [N,K] 2390 x 640 x 5184 20.4 / 21.0, f16 710 x 7104 x 15856 183 / 197, bf16 with few steps 6345 x 448 x 5164 43.0 / 54.2, 3822 x 704 x 9200
+    // 59.4 / 70.9, with GELU behind it 6660 x 128 x 3088 19.7 / 29.5, [K,N] 7633 x 832 x 2704 54.1 / 61.7.
+    const bool transposing8 = elemBytes() == 1 && !transB_, moved = !transposing8 && m_ > 256 && n_ % 256 != 0 && steps > 16 && !outgrowsLaunch(largeTileSplit());
     const double traffic = moved ? (0.09 * static_cast<double>(elements * elemBytes()) + 0.19 * static_cast<double>(m_ * k_ * elemBytes()) + 0.18 * static_cast<double>(m_ * n_)) * 1e-6 : 0;
-    double best = narrow ? 1e30 : (n_ % 256 == 0 ? 0.75 : transposing8 && !outgrowsLaunch(largeTileSplit()) ? 1.1 : 1.0) * largeTileTime(largeTileSplit()) - traffic;
+    double best = narrow ? 1e30 : (n_ % 256 == 0 ? 0.75 : elements >= (1LL << 26) && m_ <= 256 ? 0.8 : transposing8 && !outgrowsLaunch(largeTileSplit()) ? 1.1 : 1.0) * largeTileTime(largeTileSplit()) - traffic;
     for (const SmallShape &w : smallShapes()) {
       if ((narrow && w.m > 64) || k_ * elemBytes() * std::max(w.m, w.n) >= (1LL << 31)) continue;
       // (several tiles a workgroup from 17 steps on: for fewer, what comes behind the loop is a third of their time;

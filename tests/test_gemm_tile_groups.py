@@ -103,3 +103,18 @@ def test_products_of_small_tiles_fit_a_launch_without_allocations_still(m, k, n,
     """The 256 x 256 kernel would ask for 40 to 67 MB of partials here."""
     kernel = driver.HipKernel(op_desc.gemm_bias_act(m, k, n, dtype, act, transpose_b=tb), out_dir=None)
     assert kernel.workspace_bytes <= 16 << 20
+
+
+@pytest.mark.parametrize("m,k,n,dtype,act,tb,small", [
+    # few steps of K, and GELU behind the sums: us on small tiles / 256 x 256
+    (6345, 448, 5164, "bfloat16", "none", True, True), (3822, 704, 9200, "bfloat16", "relu", True, True),      # 43 / 54, 59 / 71
+    (5859, 320, 11392, "float16", "none", False, True), (6660, 128, 3088, "bfloat16", "gelu", True, True),     # 63 / 76, 20 / 30
+    (7633, 832, 2704, "float16", "gelu", False, True), (4524, 312, 5368, "bfloat16", "gelu", False, True),     # 54 / 62, 30 / 40
+    (618, 384, 15488, "float16", "relu", False, True),                                                        # 15.3 / 17.4
+    (216, 16128, 8872, "float16", "none", False, False),                                                      # 151 / 141
+    (3520, 4096, 7892, "int8", "none", True, False), (5072, 1984, 5568, "float16", "relu", False, False),     # 126 / 121, 120 / 112
+    (216, 12544, 9016, "int8", "gelu", True, True),
+])
+def test_the_faster_tiles_are_chosen(m, k, n, dtype, act, tb, small):
+    text = op_desc.gemm_int8_dequant_bias_gelu(m, k, n, transpose_b=tb) if dtype == "int8" else op_desc.gemm_bias_act(m, k, n, dtype, act, transpose_b=tb)
+    assert ("gemm_small_tile<" in driver.HipKernel(text, out_dir=None).source) == small
