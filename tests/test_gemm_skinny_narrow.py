@@ -4,6 +4,7 @@ import re
 import pytest
 
 from akg_amd import driver, op_desc
+from gemm_checks import compiled_notes
 
 
 def _columns(text):
@@ -35,6 +36,7 @@ def test_products_that_take_narrow_strips():
     (64, 704, 1060, "float16", True), (3, 1696, 12064, "bfloat16", False),
     (1, 704, 4808, "int8", False), (17, 1984, 4164, "int8", False), (49, 1856, 11256, "int8", False),
     (5, 1344, 764, "int8", True), (32, 832, 4580, "int8", True), (60, 1216, 736, "int8", True),   # columns that begin inside a line
+    (16, 1152, 11204, "bfloat16", True), (29, 1376, 11988, "float16", True), (25, 1600, 8740, "int8", True),   # eight wavefronts, strips of 64 of [N,K]
 ])
 def test_narrow_strips_against_float64(m, k, n, dtype, tb):
     """float32 sums of k products differ from the exact sum by at most k * 2^-24 of the sum of the products' magnitudes, in
@@ -70,3 +72,13 @@ def test_narrow_strips_against_float64(m, k, n, dtype, tb):
     torch.cuda.synchronize()
     gap = (out.double() - y).abs()
     assert bool((gap <= bound).all()), float((gap / bound).max())
+
+
+@pytest.mark.parametrize("m,k,n,dtype", [
+    (4, 960, 15104, "float16"), (9, 768, 12096, "float16"), (16, 1152, 11200, "bfloat16"), (16, 3072, 10708, "int8"), (20, 1472, 9192, "bfloat16"),
+    (25, 1600, 8736, "int8"), (30, 2048, 11000, "int8"), (32, 1024, 12288, "bfloat16"), (32, 2048, 12288, "bfloat16"), (29, 1344, 11984, "float16"),
+])
+def test_eight_wavefronts_of_64_columns_stay_in_registers(m, k, n, dtype, tmp_path):
+    text = op_desc.gemm_int8_dequant_bias_gelu(m, k, n, transpose_b=True) if dtype == "int8" else op_desc.gemm_bias_act(m, k, n, dtype, "relu", transpose_b=True)
+    kernel, scratch, _ = compiled_notes(text, tmp_path)
+    assert "akg::NarrowStrips<64>()" in kernel.source and kernel.block[0] == 512 and scratch == 0
