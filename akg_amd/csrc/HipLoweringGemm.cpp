@@ -380,7 +380,8 @@ class GemmEmitter {
     if (serial_) return;
     dyn_ = opt_.extentAsArgument && batch_ == 1;
     if (pickSmallTile()) {
-      if (m_ > skinnyRows() || !pickNarrow(0.8 * smallTileRowsTime(kSplit_))) return;
+      // (0.8: 32 products of a split K 0.57 .. 0.71 of the time, without a split 0.94 between 0.72 and 0.8, six of 34 slower by up to 9 %)
+      if (m_ > skinnyRows() || !pickNarrow((kSplit_ > 1 ? 0.8 : 0.72) * smallTileRowsTime(kSplit_))) return;
       tileM_ = tileN_ = 0;
     }
     kSplit_ = 1;
@@ -424,8 +425,8 @@ class GemmEmitter {
   // which every strip reads, weigh more than its columns. us, strips of 128 columns / narrow ones: bf16 [N,K] 8 x 640 x 1336 6.0 / 3.2,
   // 4 x 5056 x 2176 10.0 / 6.2, 32 x 7040 x 1832 13.7 / 11.0, 16 x 7360 x 3536 15.5 / 13.5; [K,N] 2 x 512 x 2912 5.3 / 3.4, 25 x 896 x 5656 9.2 / 5.2,
   // 16 x 2880 x 5408 11.3 / 7.7, 5 x 6592 x 560 8.1 / 12.7, 26 x 5248 x 8632 27 / 32; int8 [N,K] 9 x 2688 x 3760 7.7 / 4.4, [K,N] 1 x 1920 x
-  // 4808 8.2 / 6.3; small tiles / narrow strips: int8 [K,N] 49 x 1856 x 11256 16.6 / 10.0, bf16 [N,K] 62 x 1536 x 5880 7.7 / 8.1. Of the 122
-  // products 0.80 of the time in the geometric mean, the worst 1.1 of it.
+  // 4808 8.2 / 6.3; small tiles / narrow strips: int8 [K,N] 49 x 1856 x 11256 16.6 / 10.0, bf16 [N,K] 62 x 1536 x 5880 7.7 / 8.1. 390
+  // other products that take them need 0.68 of the time in the geometric mean, int8 32 x 7616 x 6172 15.2 / 16.3 the slowest of them.
   // More than 32 rows only with the weights that were measured, up to 24 MiB. A weight that is read past the caches keeps its kernel, as does one of a description with an open
   // row count or of several batches. (AKG_HIP_VARIANT bit 8 keeps the strips of 128 columns.)
   bool pickNarrow(double other) {
@@ -433,6 +434,12 @@ class GemmEmitter {
     if (dyn_ || batch_ != 1 || !skinnyTakes() || opt_.split > 0 || opt_.block > 0 || opt_.chunks > 0 || (opt_.variant & 256)) return false;
     const int64_t kBytes = k_ * elemBytes();
     if (kBytes % 64 != 0 || kBytes < 640 || weightBytes() >= ((m_ <= 32 ? 96LL : 24LL) << 20)) return false;
+    // Rows of a [K,N] weight that lie a multiple of 256 bytes apart: the half lines that a strip asks for meet in few channels. us, strips
+    // of 128 columns / narrow ones: int8 2 x 3584 x 5120 8.3 / 13.1, 8 x 2240 x 23552 15.0 / 20.6, f16 8 x 4096 x 8192 14.9 / 19.5, bf16 3 x 3584 x 3072
+    // 8.9 / 10.9, int8 16 x 3584 x 4608 8.5 / 9.7, 4 x 2048 x 5120 7.0 / 8.5; within these limits 390 products 0.67 of the time, three slower by 2 % and more (1.03). Long
+    // columns of a [N,K] weight that begin inside lines: bf16 4 x 5216 x 256 6.0 / 6.9, 2 x 6880 x 936 7.8 / 9.1, int8 2 x 13888 x 1008 8.0 / 8.9.
+    if (!transB_ && n_ * elemBytes() % 256 == 0 && (kBytes > (n_ * elemBytes() % 1024 != 0 ? 3200 : elemBytes() == 1 ? 1600 : 2560) || weightBytes() >= (32LL << 20))) return false;
+    if (transB_ && kBytes % 128 != 0 && kBytes > 8192 && m_ <= 32) return false;
     int64_t cols = 0;
     double best = other;
     for (const int64_t width : {16, 32, 64}) {

@@ -82,3 +82,20 @@ def test_eight_wavefronts_of_64_columns_stay_in_registers(m, k, n, dtype, tmp_pa
     text = op_desc.gemm_int8_dequant_bias_gelu(m, k, n, transpose_b=True) if dtype == "int8" else op_desc.gemm_bias_act(m, k, n, dtype, "relu", transpose_b=True)
     kernel, scratch, _ = compiled_notes(text, tmp_path)
     assert "akg::NarrowStrips<64>()" in kernel.source and kernel.block[0] == 512 and scratch == 0
+
+
+@pytest.mark.parametrize("m,k,n,dtype,tb", [
+    # rows of a [K,N] weight that lie a multiple of 256 bytes apart: us on strips of 128 columns / narrow ones
+    (2, 3584, 5120, "int8", False), (8, 2240, 23552, "int8", False),             # 8.3 / 13.1, 15.0 / 20.6
+    (8, 4096, 8192, "float16", False), (3, 3584, 3072, "bfloat16", False),       # 14.9 / 19.5, 8.9 / 10.9
+    (2, 2080, 5120, "bfloat16", False), (16, 3584, 4608, "int8", False),         # 8.3 / 9.4, 8.5 / 9.7
+    (4, 2048, 5120, "int8", False), (2, 2560, 6144, "int8", False),              # 7.0 / 8.5, 7.6 / 8.4
+    (29, 3616, 7424, "bfloat16", False), (16, 5824, 8960, "int8", False),        # 15.1 / 18.3, 15.3 / 19.9
+    # long columns of a [N,K] weight that begin inside lines
+    (4, 5216, 256, "bfloat16", True), (2, 6880, 936, "bfloat16", True), (2, 13888, 1008, "int8", True),   # 6.0 / 6.9, 7.8 / 9.1, 8.0 / 8.9
+    # small tiles without a split
+    (43, 1184, 4416, "bfloat16", True), (46, 1088, 4208, "float16", True), (45, 2176, 7720, "int8", True),   # 6.8 / 7.4, 6.1 / 6.6, 7.2 / 7.7
+])
+def test_products_that_narrow_strips_would_slow_down(m, k, n, dtype, tb):
+    text = op_desc.gemm_int8_dequant_bias_gelu(m, k, n, transpose_b=tb) if dtype == "int8" else op_desc.gemm_bias_act(m, k, n, dtype, "none", transpose_b=tb)
+    assert _columns(text) is None
