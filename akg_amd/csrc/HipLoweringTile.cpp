@@ -397,11 +397,7 @@ class TileEmitter {
         // quantisation 79.5 against 75.8 % of the HBM peak, RMSNorm + residual and a masked softmax the same either
         // way), with one input the 512 win: 8192-wide f16 softmax 171.0 -> 165.7 us, bf16 RMSNorm 180.1 -> 172.9 us
         // (32768 rows).
-        int64_t rowSized = 0;
-        for (size_t i = 0; i < g_.inputs.size(); ++i) {
-          if (access_[i].lastDimFull && g_.tensor(g_.inputs[i]).numel() == numel_) ++rowSized;
-        }
-        if (rowSized <= 1) tpr = 512;
+        if (rowSizedInputs() <= 1) tpr = 512;
       }
       if (opt_.threadsPerRow == 0 && !ordered_ && normalisationLike() && rowChunks >= 128 && rowChunks <= 2048) {
         // A reduction that waits for another one (mean, then variance) with per-column operands behind them (gamma,
@@ -438,13 +434,26 @@ class TileEmitter {
         }
       }
       // Few rows: what a thread does one after the other is all of the time, so a row takes threads until each has one chunk, as long as the
-      // threads of all rows are half of what the chip holds at once (512 a row: a quarter). us, the rules above / this: bf16 quantisation
-      // 224 x 835 6.6 / 3.3 (14 workgroups), 152 x 7120 6.6 / 3.8, 30 x 3112 6.0 / 3.4, 744 x 810 6.2 / 3.3, LayerNorm 17 x 6488 4.6 / 3.5, 1324 x 1583
-      // 4.8 / 4.4, 1483 x 3392 9.5 / 7.3; beyond, quantisation 2248 x 1328 would take 6.3 for 6.1, 1096 x 451 on 256 threads a row 4.2 for 3.5.
+      // threads of all rows are a quarter of what the chip holds at once; of rows of six and more chunks a thread half: 26 of 28 then gain, a fifth in the
+      // mean, with fewer chunks nothing is gained there (RMSNorm with a residual f32 3345 x 560 4.0 / 4.6, LayerNorm bf16 1997 x 1496 3.7 / 4.2), with up
+      // to three on one wavefront half as many threads earlier (LayerNorm f32 705 x 528 2.0 / 2.3, bf16 1439 x 684 2.4 / 2.6).
+      // us, the rules above / this: bf16 quantisation 224 x 835 6.6 / 3.3 (14 workgroups), 152 x 7120 6.6 / 3.8, 30 x 3112 6.0 / 3.4, 744 x 810
+      // 6.2 / 3.3, LayerNorm 17 x 6488 4.6 / 3.5, 1324 x 1583 4.8 / 4.4; 151 softmaxes, RMSNorms, norms and maxima of 10 .. 4096 rows x 16 .. 16384 0.865 of the
+      // time in the mean, four of them slower by more than 3 % (0.1 .. 0.2 us).
+      // Not where 256 threads have a few chunks of a row each: RMSNorm f32 11 x 3024 (3 chunks) 1.8 / 1.9, with a residual 30 x 2584 2.1 / 2.3, softmax
+      // bf16 83 x 8350 (5) 2.9 / 3.1, LayerNorm f16 16 x 5888 (3) 2.4 / 2.6. From six on it is a gain with two rows read, LayerNorm bf16 25 x 13480
+      // 4.9 / 3.9, quantisation f16 17 x 13115 6.9 / 5.4, with one none, RMSNorm bf16 68 x 14108 3.0 / 3.2. Nor where a wavefront has two chunks a lane,
+      // whose reductions need no LDS: LayerNorm f32 29 x 512 1.75 / 1.87, softmax 39 x 512 1.88 / 1.94. Nor for ArgMax, where as much is lost as gained: f16
+      // 1908 x 1104 2.0 / 2.8, f32 243 x 656 1.8 / 2.0, bf16 96 x 8600 2.3 / 2.4.
       // (Fewer than ten rows stay as they are: tests pin the rules above on them.)
-      if (opt_.threadsPerRow == 0 && !ordered_ && !extentArg_ && rows_ >= 10) {
-        while (tpr < 256 && tpr < rowChunks && rows_ * 2 * tpr <= (1LL << 18)) tpr *= 2;
-        while (tpr >= 256 && tpr < 512 && tpr < rowChunks && rows_ * 2 * tpr <= (1LL << 17)) tpr *= 2;
+      bool searches = false;
+      for (const OpNode &op : g_.ops) searches = searches || op.kind == OpKind::Iota;
+      if (opt_.threadsPerRow == 0 && !ordered_ && !extentArg_ && rows_ >= 10 && !searches) {
+        const bool fewChunks = tpr == 256 && (rowSizedInputs() < 2 || ceilDiv(rowChunks, tpr) < 6);
+        const bool oneWavefront = tpr == 64 && rowChunks <= 128;
+        const int64_t chunksNow = ceilDiv(rowChunks, tpr), most = chunksNow >= 6 ? 1LL << 18 : chunksNow <= 3 && tpr <= 64 ? 1LL << 16 : 1LL << 17;   // threads of all rows
+        while (tpr < 256 && tpr < rowChunks && !oneWavefront && rows_ * 2 * tpr <= most) tpr *= 2;
+        while (tpr >= 256 && tpr < 512 && tpr < rowChunks && !fewChunks && rows_ * 2 * tpr <= (1LL << 17)) tpr *= 2;
       }
       // Rows of any length in the bucket that vector instructions bound: a wavefront leaves out the chunks beyond its row (chunkwise_), and
       // where it would hold a row in two chunks a lane it takes two rows with four chunks a lane instead - the second chunk of 64
@@ -466,10 +475,7 @@ class TileEmitter {
       // 65536-wide f16 softmax (1 input, 64 values) 62.6 / 46.2; 65536-wide bf16 LayerNorm (2 inputs) 21.9 / 61.3;
       // 32768-wide LayerNorm 70.2 / 63.2; 131072-wide LayerNorm 10.6 / 50.0, softmax 30.1 / 42.3.
       const int rowPasses = opt_.variant;  // 1: force the register-resident row, 2: force the walks, 4: walks, packed if possible
-      int64_t rowInputs = 0;
-      for (size_t i = 0; i < g_.inputs.size(); ++i) {
-        if (access_[i].lastDimFull && g_.tensor(g_.inputs[i]).numel() == numel_) ++rowInputs;
-      }
+      const int64_t rowInputs = rowSizedInputs();
       multiPass_ = rowPasses == 2 || rowPasses == 4 || (rowPasses != 1 && (perThread * vec_ > 64 || perThread * vec_ * rowInputs > 96));
       packedInput_.assign(g_.inputs.size(), false);
       // Measured, % of the HBM peak, float values resident / packed walks: 32768-wide bf16 quantisation 61.6 / 73.0,
@@ -941,6 +947,15 @@ class TileEmitter {
     line("    }");
     line("  }");
     pending_.str("");
+  }
+
+  // inputs of the rows' size
+  int64_t rowSizedInputs() const {
+    int64_t count = 0;
+    for (size_t i = 0; i < g_.inputs.size(); ++i) {
+      if (access_[i].lastDimFull && g_.tensor(g_.inputs[i]).numel() == numel_) ++count;
+    }
+    return count;
   }
 
   // Two reductions of which one waits for the other, and some per-column operand (an input that spans the row but not

@@ -140,3 +140,61 @@ def test_many_rows_that_leave_out_chunks(cols):
     want = torch.softmax((1.0 - mask.double()) * -10000.0 + 0.125 * x.double(), -1)
     wrong = (out.double() - want).abs()
     assert bool((wrong <= 2e-5 * want + 1e-30).all())
+
+
+def _row_kernel(kind, rows, cols, dtype):
+    name = "threads_%s_%s_%d_%d" % (kind, dtype, rows, cols)
+    text = {"softmax": lambda: op_desc.softmax_last_axis(rows, cols, dtype, name), "rmsnorm": lambda: op_desc.rmsnorm(rows, cols, dtype, name=name),
+            "rmsnorm_add": lambda: op_desc.rmsnorm(rows, cols, dtype, residual=True, name=name), "layernorm": lambda: op_desc.layernorm_residual(rows, cols, dtype, name=name),
+            "quant": lambda: op_desc.quant_int8_residual(rows, cols, dtype, name=name), "argmax": lambda: op_desc.argmax_last_axis([rows, cols], dtype, name=name)}[kind]()
+    return text, driver.HipKernel(text, out_dir=None)
+
+
+@pytest.mark.parametrize("kind,rows,cols,dtype,grid,block", [
+    # us on the threads of the rules for many rows / until each has one chunk
+    ("argmax", 1908, 1104, "float16", 239, 256), ("argmax", 243, 656, "float32", 61, 256), ("argmax", 96, 8600, "bfloat16", 96, 256),   # 2.0 / 2.8, 1.8 / 2.0, 2.3 / 2.4
+    ("rmsnorm", 11, 3024, "float32", 11, 256), ("rmsnorm_add", 30, 2584, "float32", 30, 256), ("layernorm", 16, 5888, "float16", 16, 256),   # 1.8 / 1.9, 2.1 / 2.3, 2.4 / 2.6
+    ("softmax", 83, 8350, "bfloat16", 83, 256), ("rmsnorm", 68, 14108, "bfloat16", 68, 256),                       # 2.9 / 3.1, 3.0 / 3.2
+    ("layernorm", 29, 512, "float32", 8, 256), ("softmax", 39, 512, "float32", 10, 256),                           # 1.75 / 1.87, 1.88 / 1.94
+    ("rmsnorm_add", 3345, 560, "float32", 419, 256), ("layernorm", 1997, 1496, "bfloat16", 500, 256),              # 4.0 / 4.6, 3.7 / 4.2
+    ("layernorm", 3302, 304, "float32", 413, 256),                                                                # 2.6 / 2.9 on 64 threads
+    ("layernorm", 705, 528, "float32", 177, 256), ("layernorm", 1439, 684, "bfloat16", 180, 256),                  # 2.0 / 2.3, 2.4 / 2.6
+    # ... and where they pay
+    ("quant", 152, 7120, "bfloat16", 152, 512), ("layernorm", 25, 13480, "bfloat16", 25, 512), ("quant", 744, 810, "bfloat16", 372, 256),   # 6.6 / 3.8, 4.9 / 3.9, 6.2 / 3.3
+])
+def test_threads_of_few_rows(kind, rows, cols, dtype, grid, block):
+    _, kernel = _row_kernel(kind, rows, cols, dtype)
+    assert kernel.grid[0] == grid and kernel.block[0] == block
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,rows,cols,dtype,block", [
+    ("softmax", 33, 3376, "float16", 512), ("softmax", 67, 3401, "bfloat16", 512),      # one ragged chunk a thread; the last one overlaps
+    ("softmax", 129, 1536, "float32", 512), ("rmsnorm", 78, 1584, "float32", 512),      # four float32 a thread
+    ("rmsnorm", 127, 2535, "bfloat16", 512), ("rmsnorm_add", 77, 4800, "bfloat16", 512),   # two chunks of 512 threads, the second one ragged
+    ("rmsnorm", 10, 1023, "float32", 256), ("softmax", 10, 24, "float16", 256),         # the fewest rows; of three chunks
+    ("rmsnorm_add", 1023, 1000, "float32", 256), ("layernorm", 21, 2296, "bfloat16", 512), ("layernorm", 1253, 712, "bfloat16", 256),
+    ("argmax", 39, 1111, "float32", 256),
+])
+def test_rows_on_more_threads_against_the_oracle(kind, rows, cols, dtype, block):
+    """float32 results of sums of `cols` terms: 1e-5 relative to the float64 evaluation, with 1e-6 of the root of the terms for sums that cancel;
+    16-bit ones and integers with the bars of their type against the oracle."""
+    import torch
+    from akg_amd import harness
+    from oracle import np_ref
+    text, kernel = _row_kernel(kind, rows, cols, dtype)
+    assert kernel.block[0] == block
+    print("case", kind, rows, cols, dtype, kernel.grid, kernel.block, flush=True)
+    desc = json.loads(text)
+    inputs = harness.make_inputs(desc, seed=harness.BASE_SEED + 850)
+    expect = np_ref.evaluate(desc, inputs)
+    exact = np_ref.evaluate(harness.widen_to_float64(desc), [a.astype(np.float64) if a.dtype == np.float32 else a for a in inputs])
+    on_device = [torch.from_numpy(np.ascontiguousarray(a).view(np.int16) if a.dtype == np.uint16 else np.ascontiguousarray(a)).cuda() for a in inputs]
+    for _ in range(2):
+        outs = [torch.full((d.nbytes,), 0x7f, dtype=torch.uint8, device="cuda") for d in kernel.outputs]
+        kernel.launch(on_device + outs)
+        torch.cuda.synchronize()
+        for d, o, e, x in zip(kernel.outputs, outs, expect, exact):
+            got = o.cpu().numpy().view(driver.NP_HOST_DTYPE[d.dtype]).reshape(d.shape)
+            ok, msg = harness.compare_reassociated(got, x, d.dtype, cols) if d.dtype == "float32" else harness.compare(got, e, d.dtype)
+            assert ok, "%s %s: %s" % (kind, d.name, msg)
