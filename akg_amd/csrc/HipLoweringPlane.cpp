@@ -277,7 +277,8 @@ class PlaneEmitter {
       parts_ = 0;
       // Half of the registers may hold the elements as they are computed with: the walks behind the first then neither unpack them nor
       // compute what the walk before did (a batch norm's instructions are 4 of the 8 us of bf16 [64,128,28,28]: 809 -> 641, 8.0 -> 7.5 us).
-      keepsUnpacked_ = resident * vec_ * fullInputs <= 65536 / block_;
+      // A single input of 32-bit elements has nothing to unpack, and kept it is only longer alive (range of f32 [79,803,8,8] 4.4 -> 5.0).
+      keepsUnpacked_ = resident * vec_ * fullInputs <= 65536 / block_ && !(fullInputs == 1 && fullBytes >= 4);
       return;
     }
     // One launch per level: 128 bytes of loads in flight per thread, less where that leaves less than four workgroups per

@@ -178,3 +178,22 @@ def test_mean_and_variance_are_as_exact_as_by_one_kernel_per_level(shape, dtype,
     several = driver.HipKernel(text, out_dir=None)
     assert one.family == "plane_reduce" and several.family == "staged"
     assert (errors(one) <= 1.1 * errors(several)).all()
+
+
+def test_elements_that_stay_unpacked_from_walk_to_walk():
+    """Where they fit half of the registers, and where there is something to unpack or to compute: of a single float32 input there is not."""
+    def kept(text):
+        kernel = driver.HipKernel(text, out_dir=None)
+        assert kernel.family == "plane_reduce" and "_level0" not in kernel.source
+        return "akg::forget_unpacked" not in kernel.source
+    assert kept(_bn(64, 128, 28, 28, "bfloat16")) and kept(_backward(12, 20, 14, 14)) and kept(_range([41, 20, 7, 7], [0, 2, 3], "float16"))
+    assert not kept(_range([79, 803, 8, 8], [0, 2, 3], "float32")) and not kept(_bn(64, 128, 28, 28, "float32"))
+    assert kept(_bn(127, 49, 21, 24, "float16")) and not kept(_bn(128, 49, 24, 24, "float16"))     # 64 elements a thread of 1024, 72
+
+
+def test_channels_on_either_side_of_a_launch_per_level():
+    def by_level(text):
+        return "_level0" in driver.HipKernel(text, out_dir=None).source
+    assert not by_level(_bn(100, 16, 28, 32, "bfloat16")) and by_level(_bn(101, 16, 28, 32, "bfloat16"))    # 88 and 96 elements a thread
+    assert not by_level(_bn(112, 48, 28, 36, "bfloat16")) and by_level(_bn(116, 48, 28, 36, "bfloat16"))    # 112 and 120
+    assert not by_level(_bn(116, 56, 28, 36, "bfloat16"))
