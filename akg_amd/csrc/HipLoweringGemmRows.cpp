@@ -181,7 +181,10 @@ class GemmRowsEmitter {
   // tiles so is B. us, half lines of sixteen rows / the tensors / both: [60,640,64] x 640 48.5 / 45.7 / 44.9, [24,896,64] x 896 40.6 / 39.7 / 37.3,
   // [20,2048,64] x 1024 68.6 / 67.2 / 63.5, [13,664,64] x 664 (one row tile) 16.3 / 15.9 / 16.4; four wavefronts [192,512,64] x 512 72.7 / 72.9 / 76.5,
   // sixteen [26,1160,64] x 1160 73.0 / 74.2 / 74.0, two [300,256,64] x 256 33.9 / 34.6 / 34.7.
-  bool byLines() const { return wavesC_ == 8; }
+  // With more than 64 of K the products are more of the time and the lines are waited for in front of them: [78,648,192] x 648 103 / 107, [63,712,128] x 712
+  // 59.1 / 61.3, [109,142,96] x 712 21.1 / 21.8, 28 shapes 1.014 in the mean; only from ten workgroups a CU on and up to 128 they are a gain, [115,864,128] x 864 223 / 218,
+  // [259,560,128] x 560 191 / 185, [139,592,128] x 592 115 / 111. Up to 64 the mean of 24 is 0.965, the worst 1.03.
+  bool byLines() const { return wavesC_ == 8 && (k_ <= 64 || (k_ <= 128 && batch_ * rowGroups() >= 2560)); }
 
   // Tensors of the scores' columns besides the scores, in 32-bit values per element: what is read and what is written (a
   // float32 result is computed by the longer forms of the functions in front of it: one more).

@@ -301,3 +301,13 @@ def test_types_masks_and_values_at_the_ends_against_two_kernels(mask_type, n, mo
         else:
             bound = b.abs() * (2.0 ** -9 + 2.0 ** -13 + unit[d.dtype]) + (2.0 ** -9 if a.numel() <= 48 * 250 else 2.0 ** -24)
             assert bool(((a - b).abs() <= bound).all()), (d.dtype, float(((a - b).abs() / bound).max()))
+
+
+@pytest.mark.parametrize("batch,m,k,n,lines", [
+    (60, 640, 64, 640, True), (108, 568, 32, 568, True), (115, 864, 128, 864, True),             # us by half lines / by whole ones: 48.5 / 44.9, 39.5 / 38.4, 223 / 218
+    (63, 712, 128, 712, False), (78, 648, 192, 648, False), (109, 142, 96, 712, False),          # 59.1 / 61.3, 103 / 107, 21.1 / 21.8
+    (192, 512, 64, 512, False),
+])
+def test_masks_by_whole_lines_with_a_short_k(batch, m, k, n, lines):
+    kernel = driver.HipKernel(op_desc.attention_probabilities(batch, m, k, n, "bfloat16", "lines_%d_%d_%d_%d" % (batch, m, k, n)), out_dir=None)
+    assert kernel.family == "gemm_rows" and ("akg::load_own_row_if<" in kernel.source) == lines
