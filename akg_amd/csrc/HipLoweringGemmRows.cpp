@@ -107,9 +107,11 @@ class GemmRowsEmitter {
     //   few row groups leave the chip idle ([1,256,64]x1024, 16 groups: 9.1 us for 7.9; [3,512,128]x512, 96: 7.8 for 10.1);
     //   scores below 1 MiB stay in the caches, and both forms take the time of their launches: with up to 64 KiB of B a batch (a K above 128: 32 KiB)
     //   one launch is the faster one however few rows or scores there are ([33,56,64]x56 3.2 for 7.4, [12,104,64]x104 4.0 for 8.1, [3,320,64]x320 4.3
-    //   for 8.5, [24,5,64]x232 3.2 for 6.2, [6,1,128]x88 3.3 for 6.0, [1,360,64]x360 3.8 for 5.6, [2,64,128]x64 4.2 for 6.6, [2,48,256]x48 5.4 for 6.6;
-    //   250 shapes 0.6 of the time in the mean), with more not ([9,27,128]x552 7.8 for 6.8, [16,9,64]x1200 9.1 for 5.7, [4,33,192]x128 7.9 for 7.1). Tests pin two kernels for fewer than 16 columns,
-    //   from 32 rows on for up to 64 KiB of scores ([3,40,64]x136) and from 128 on for up to 512 KiB ([2,512,64]x64, [4,128,64]x256).
+    //   for 8.5, [24,5,64]x232 3.2 for 6.2, [6,1,128]x88 3.3 for 6.0; 33 other
+    //   shapes 0.44 of the time in the mean, none slower), with more not ([9,27,128]x552 7.8 for 6.8, [16,9,64]x1200 9.1 for
+    //   5.7, [4,33,192]x128 7.9 for 7.1). Two kernels stay, as tests pin them, for fewer than 16 columns, from 32 rows on for up to 64 KiB of
+    //   scores ([3,40,64]x136) and from 128 on for up to 512 KiB ([2,512,64]x64, [4,128,64]x256), though one would be the faster one there too
+    //   ([1,360,64]x360 3.8 for 5.6, [2,64,128]x64 4.2 for 6.6, [2,48,256]x48 5.4 for 6.6).
     if (k_ % 32 != 0 || n_ % 8 != 0 || n_ > 2048 || n_ * k_ > (1LL << 17)) throw LoweringError("MatMul: operands of this shape have no row kernel");
     const int64_t scores = batch_ * m_ * n_ * 4;
     small_ = k_ <= 256 && n_ * k_ <= (k_ <= 128 ? 1LL << 15 : 1LL << 14) &&
