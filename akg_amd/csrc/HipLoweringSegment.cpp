@@ -499,14 +499,18 @@ __device__ inline void chunk_sort(const int (&key)[TILES], unsigned (&slot)[TILE
 }
 )AKG";
 
+// Values of a list that are in flight (add_list). Integers: with 48 the compiler, free to add them in any order, moves the requests together
+// and spills nine registers and more (us, int32 956289 x 1 into 14006 17.0 before there was add_list / 18.0 with 48 / 16.2 with 16).
+int addBlock(const std::string &computeType) { return computeType == "float" ? 48 : 16; }
+
 // Device code of the launches that add lists out of LDS.
 const char *const kAddList = R"AKG(
-// acc, then list[0] .. list[n - 1] added to it one after the other. `list` begins at a multiple of 16 bytes; up to 384 bytes behind its
-// end are read and not added. An addition takes 4.4 cycles and LDS up to 230, so every value is requested 44 additions ahead and the
+// acc, then list[0] .. list[n - 1] added to it one after the other. `list` begins at a multiple of 16 bytes; up to ADD_BLOCK values behind
+// its end are read and not added. A float addition takes 4.4 cycles and LDS up to 230, so every value is requested 44 additions ahead and the
 // order is given: left to itself the compiler requests values in front of the last two additions before them (13.7 cycles an addition).
-constexpr int ADD_BLOCK = 48;
 template <typename T, typename Add>
 __device__ inline T add_list(const T *list, int n, T acc, Add add) {
+  static_assert(sizeof(T) == 4, "four values a request");
   typedef T quad_t __attribute__((ext_vector_type(4)));
   constexpr int BLOCK = ADD_BLOCK, QUADS = BLOCK / 4;
   const quad_t *quads = reinterpret_cast<const quad_t *>(list);
@@ -911,7 +915,7 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
   }
   s << "struct __attribute__((aligned(4))) row_t { unsigned w[ROW_WORDS]; };\n";
   s << "typedef unsigned quad_words __attribute__((ext_vector_type(4)));\n";
-  s << kChunkSort << kAddList << kChunkRank;
+  s << "constexpr int ADD_BLOCK = " << addBlock(ct) << ";\n" << kChunkSort << kAddList << kChunkRank;
   s << "}  // namespace\n\n";
   std::ostringstream params;
   for (size_t i = 0; i < g.inputs.size(); ++i) {
@@ -986,7 +990,7 @@ LoweredKernel lowerSegmentChunked(const OpGraph &g, const LoweringOptions &optio
   s << "  // a round's entries: whose run each is, and where entry k of the round is less k for every run\n";
   s << "  __shared__ unsigned short akg_run[CAP];\n  __shared__ unsigned akg_base[W * 64];\n";
   s << "  // column c of a round's rows from c * PLANE on, lists per segment; what add_list reads behind the last one\n";
-  s << "  __shared__ __attribute__((aligned(16))) " << ct << " akg_plane[ROW * PLANE + 2 * ADD_BLOCK];\n";
+  s << "  __shared__ __attribute__((aligned(16))) " << ct << " akg_plane[ROW * PLANE + ADD_BLOCK];\n";
   s << "  __shared__ unsigned short akg_cnt[W * S];\n";
   s << "  __shared__ unsigned akg_start[S], akg_len[S], akg_scan[W], akg_sums[W], akg_taken[W], akg_total[W];\n";
   s << "  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, w = tid >> 6;\n";
@@ -1271,7 +1275,7 @@ __device__ inline void sum_records(const unsigned *__restrict__ ws, store_t *__r
   __shared__ unsigned short akg_run[CAP];             // whose run each entry of the round is
   __shared__ run_t akg_base[W * 64];
   // column c of a round's rows from c * PLANE on, lists per segment; what add_list reads behind the last one
-  __shared__ __attribute__((aligned(16))) compute_t akg_plane[ROW * PLANE + 2 * ADD_BLOCK];
+  __shared__ __attribute__((aligned(16))) compute_t akg_plane[ROW * PLANE + ADD_BLOCK];
   __shared__ unsigned short akg_cnt[W * S];
   __shared__ unsigned akg_start[S], akg_len[S], akg_scan[W], akg_sums[W], akg_taken[W], akg_cut;
   const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, w = tid >> 6;
@@ -1433,7 +1437,7 @@ LoweredKernel lowerSegmentRecords(const OpGraph &g, const LoweringOptions &optio
   s << "struct __attribute__((aligned(4))) row_t { unsigned w[ROW_WORDS]; };\n";
   s << "union cell_t { row_t r; store_t v[ROW_WORDS * 4 / sizeof(store_t)]; };\n";
   s << "typedef unsigned quad_words __attribute__((ext_vector_type(4)));\n";
-  s << kChunkSort << kAddList << kRecordCode;
+  s << "constexpr int ADD_BLOCK = " << addBlock(ct) << ";\n" << kChunkSort << kAddList << kRecordCode;
   s << "}  // namespace\n\n";
   std::ostringstream params;
   for (size_t i = 0; i < g.inputs.size(); ++i) {

@@ -105,3 +105,11 @@ def test_bit_for_bit_the_serial_loop(positions, width, segments, dtype, ids, pat
     if chunks:
         monkeypatch.setenv("AKG_HIP_CHUNKS", str(chunks))
     _check_bits(positions, width, segments, dtype, ids, pattern, tmp_path)
+
+
+@pytest.mark.parametrize("positions,width,segments", [(956289, 1, 14006), (365857, 3, 609), (2180885, 3, 1444), (784959, 1, 590)])
+def test_integer_sums_stay_in_registers(positions, width, segments, tmp_path):
+    from gemm_checks import compiled_notes
+    text = op_desc.unsorted_segment_sum([positions], [width], segments, "int32", "int32", "ints_%d_%d_%d" % (positions, width, segments))
+    kernel, scratch, _ = compiled_notes(text, tmp_path)
+    assert "grouped by bucket of segments" in kernel.source and scratch == 0
