@@ -99,7 +99,7 @@ class GemmEmitter {
       note << " serial: the reference's k-ordered sum in the declared type on the vector ALUs, tile=64x" << 16 * epiWidth()
            << " grid=" << k.grid[0];
     } else if (skinny_) {
-      note << " skinny: strips of " << stripCols() << " columns, B " << (narrowCols_ > 0 ? "straight into MFMA operands, all of K" : skinnyLines() ? (streamsLines() ? "by whole lines past the caches" : "by whole lines") : "straight into MFMA operands")
+      note << " skinny: strips of " << stripCols() << " columns, B " << (narrowCols_ > 0 ? (transB_ ? "by whole lines, all of K" : "transposed in registers, all of K") : skinnyLines() ? (streamsLines() ? "by whole lines past the caches" : "by whole lines") : "straight into MFMA operands")
            << ", mfma=" << mfmaName(narrowCols_ > 0) << " waves=" << skinnyWaves() << " grid=" << k.grid[0];
     } else if (tileM_ > 0) {
       const int unitM = tileM_ % 128 == 0 ? 128 : 64, unitN = tileN_ % 128 == 0 ? 128 : 64;
