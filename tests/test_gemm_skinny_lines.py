@@ -97,3 +97,32 @@ def test_lines_of_columns_that_end_inside_one_are_whole_from_4_mib_of_all_batche
     assert not whole(op_desc.gemm_bias_act(16, 240, 16384, "bfloat16", "none", transpose_b=True))  # not a line per wavefront
     assert whole(op_desc.batch_matmul_scale_mask(8, 16, 528, 512, "bfloat16", True, "lines_seam"))
     assert not whole(op_desc.batch_matmul_scale_mask(7, 16, 528, 512, "bfloat16", True, "lines_seam"))
+
+
+def _takes_wide_strips(text):
+    source = driver.HipKernel(text, out_dir=None)
+    assert "gemm_skinny<" in source.source and "NarrowStrips" not in source.source and source.workspace_bytes > 0
+    return source
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,n,dtype", [(1, 1024, 1000, "bfloat16"), (33, 2048, 516, "float16"), (32, 8256, 272, "int8"), (5, 8256, 520, "int8"), (64, 1088, 904, "int8")])
+def test_lines_of_strips_of_128_columns_where_narrow_ones_are_the_default(m, k, n, dtype, monkeypatch):
+    """Split ranges, tails and ragged strips of a [N,K] weight, with the bounds of the test above."""
+    monkeypatch.setenv("AKG_HIP_VARIANT", "256")
+    _takes_wide_strips(op_desc.gemm_int8_dequant_bias_gelu(m, k, n, transpose_b=True) if dtype == "int8" else op_desc.gemm_bias_act(m, k, n, dtype, "none", transpose_b=True))
+    test_lines_of_a_transposed_weight_against_float64(m, k, n, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,m,k,n,tb", [
+    ("bf16", 1, 1024, 520, False), ("bf16", 16, 4096, 1024, False), ("bf16", 33, 2048, 264, False), ("i8", 32, 4096, 260, False), ("i8", 64, 4096, 520, False),
+    ("f16", 16, 2048, 264, True), ("f16", 48, 1024, 136, True), ("bf16", 32, 8192, 136, True), ("i8", 50, 8192, 128, True),
+])
+def test_strips_of_128_columns_with_a_split_against_the_oracle(kind, m, k, n, tb, monkeypatch, tmp_path):
+    """One row to 64, both layouts, three element types, ranges of K that workgroups share."""
+    from test_gpu_parity import test_skinny_matmul_streams_b_into_mfma_operands as against_the_oracle
+    monkeypatch.setenv("AKG_HIP_VARIANT", "256")
+    _takes_wide_strips(op_desc.gemm_int8_dequant_bias_gelu(m, k, n, "bfloat16", tb) if kind == "i8" else
+                       op_desc.gemm_bias_act(m, k, n, "bfloat16" if kind == "bf16" else "float16", "gelu", tb))
+    against_the_oracle((kind, m, k, n, tb), tmp_path)
