@@ -277,8 +277,10 @@ class PlaneEmitter {
       parts_ = 0;
       // Half of the registers may hold the elements as they are computed with: the walks behind the first then neither unpack them nor
       // compute what the walk before did (a batch norm's instructions are 4 of the 8 us of bf16 [64,128,28,28]: 809 -> 641, 8.0 -> 7.5 us).
-      // A single input of 32-bit elements has nothing to unpack, and kept it is only longer alive (range of f32 [79,803,8,8] 4.4 -> 5.0).
-      keepsUnpacked_ = resident * vec_ * fullInputs <= 65536 / block_ && !(fullInputs == 1 && fullBytes >= 4);
+      // A single input of 32-bit elements has nothing to unpack, and kept it is only longer alive (range of f32 [79,803,8,8] 4.4 -> 5.0). And with more
+      // channels than CUs two workgroups of 1024 threads share one only with half of the registers: bf16 [19,766,51,51] 29.1 -> 32.0, f16 [24,989,44,44]
+      // 31.0 -> 33.1.
+      keepsUnpacked_ = resident * vec_ * fullInputs <= 65536 / block_ && !(fullInputs == 1 && fullBytes >= 4) && (block_ < 1024 || kept_ <= opt_.computeUnits);
       return;
     }
     // One launch per level: 128 bytes of loads in flight per thread, less where that leaves less than four workgroups per

@@ -188,6 +188,7 @@ def test_elements_that_stay_unpacked_from_walk_to_walk():
         return "akg::forget_unpacked" not in kernel.source
     assert kept(_bn(64, 128, 28, 28, "bfloat16")) and kept(_backward(12, 20, 14, 14)) and kept(_range([41, 20, 7, 7], [0, 2, 3], "float16"))
     assert not kept(_range([79, 803, 8, 8], [0, 2, 3], "float32")) and not kept(_bn(64, 128, 28, 28, "float32"))
+    assert not kept(_bn(19, 766, 51, 51, "bfloat16")) and kept(_bn(19, 236, 51, 51, "bfloat16"))    # 1024 threads: two workgroups a CU with half of the registers
     assert kept(_bn(127, 49, 21, 24, "float16")) and not kept(_bn(128, 49, 24, 24, "float16"))     # 64 elements a thread of 1024, 72
 
 
