@@ -262,15 +262,17 @@ class PlaneEmitter {
     // spill; with 256 channels and more that is still the faster form: range of int8 [32000,700,6] 352 us, 491 by level, 390 by one kernel
     // per level and value as before. It is the slower one for f32 results of int8 runs of six: [12288,700,6] 174, by such kernels 161.)
     // Few channels leave CUs idle in the resident form, and many elements a thread make that the longer way. us, resident / by level,
-    // batch norms: bf16, 16 channels of 72 elements a thread 6.8 / 8.4, of 96 8.5 / 8.3, of 128 10.9 / 8.4; 32 channels 7.3 / 8.5, 9.3 / 8.6,
-    // 11.7 / 9.5; 48 channels of 96 9.9 / 10.0, of 128 12.3 / 11.5; 64 channels of 128 12.6 / 12.8; f32, 24 channels of 36 6.1 / 8.6, of 52 8.4 / 8.6.
+    // batch norms: 16 bits, [201,16,21,21] (88 elements a thread) 13.1 / 7.4, [931,24,9,9] 14.3 / 7.9, [73,21,32,36] 9.0 / 7.2, [38,28,19,105] 11.9 / 7.8, 27 of 29
+    // with 9 .. 11 chunks a thread slower resident, by a quarter in the mean; 48 channels of 96 9.9 / 10.0, of 128 12.3 / 11.5, 38 of ragged runs [105,38,35,35]
+    // 19.0 / 10.1; 64 channels of 128 12.6 / 12.8; f32, 9 .. 15 chunks, 13 norms a fifth faster resident, [61,31,33,17] 5.1 / 7.3, [57,29,23,47] 7.4 / 8.2.
     // With one level of reductions, resident / by level / one kernel per level and value: int8 range of [64,32,64,64] 17.2 / 7.0 / 11.5,
     // [30000,32,2,3] 91.7 / 24 / 25.4. Short runs, which share their lines, earlier: i32 range of [3072,16,6] 11.9 / 5.2 / 9.1,
     // with 128 channels and one level range of f16 [12288,128,6] 62 / 33 / 46, of i32 [6144,128,6] 33.5 / 20.6 / 30.5 (batch norms, of two
     // levels, stay: bf16 [16384,128,6] 54.6 / 61).
     const int64_t runBytes = inner_ * widest;
     const bool fewChannels = runBytes < 64 ? (kept_ <= 32 && perChannel > 4096) || (kept_ < 256 && resident > 8 && lastWalk_ == 1)
-                             : lastWalk_ == 1 ? kept_ <= 32 && resident > 8 : kept_ <= 48 && resident * vec_ >= (kept_ <= 32 ? 96 : 120);
+                             : kept_ <= 32 ? resident > 8 && (lastWalk_ == 1 || fullBytes < 4 * fullInputs || resident * vec_ >= 96)
+                                           : kept_ <= 48 && lastWalk_ > 1 && resident * vec_ >= 120;
     if (resident * regsPerChunk <= 64 && opt_.split <= 1 && (!fewChannels || opt_.split == 1)) {
       block_ = block;
       chunks_ = static_cast<int>(resident);

@@ -195,6 +195,10 @@ def test_elements_that_stay_unpacked_from_walk_to_walk():
 def test_channels_on_either_side_of_a_launch_per_level():
     def by_level(text):
         return "_level0" in driver.HipKernel(text, out_dir=None).source
-    assert not by_level(_bn(100, 16, 28, 32, "bfloat16")) and by_level(_bn(101, 16, 28, 32, "bfloat16"))    # 88 and 96 elements a thread
+    assert not by_level(_bn(73, 16, 28, 32, "bfloat16")) and by_level(_bn(74, 16, 28, 32, "bfloat16"))      # eight and nine chunks a thread
+    # us, resident / by level: 13.1 / 7.4, 14.3 / 7.9, 11.9 / 7.8, 9.0 / 7.2
+    assert by_level(_bn(201, 16, 21, 21, "float16")) and by_level(_bn(931, 24, 9, 9, "bfloat16")) and by_level(_bn(38, 28, 19, 105, "bfloat16"))
+    assert by_level(_bn(73, 21, 32, 36, "float16"))
+    assert not by_level(_bn(61, 31, 33, 17, "float32")) and not by_level(_bn(57, 29, 23, 47, "float32"))    # 5.1 / 7.3, 7.4 / 8.2
     assert not by_level(_bn(112, 48, 28, 36, "bfloat16")) and by_level(_bn(116, 48, 28, 36, "bfloat16"))    # 112 and 120
     assert not by_level(_bn(116, 56, 28, 36, "bfloat16"))
