@@ -99,3 +99,10 @@ def test_eight_wavefronts_of_64_columns_stay_in_registers(m, k, n, dtype, tmp_pa
 def test_products_that_narrow_strips_would_slow_down(m, k, n, dtype, tb):
     text = op_desc.gemm_int8_dequant_bias_gelu(m, k, n, transpose_b=tb) if dtype == "int8" else op_desc.gemm_bias_act(m, k, n, dtype, "none", transpose_b=tb)
     assert _columns(text) is None
+
+
+@pytest.mark.parametrize("tb,way", [(True, "by whole lines, all of K"), (False, "transposed in registers, all of K")])
+def test_the_schedule_note_says_how_the_weight_is_read(tb, way, tmp_path):
+    kernel = driver.HipKernel(op_desc.gemm_bias_act(8, 640, 1336, "bfloat16", "none", transpose_b=tb), out_dir=str(tmp_path))
+    assert "akg::NarrowStrips<" in kernel.source
+    assert any("B " + way in f.read_text() for f in tmp_path.glob("*.json"))
