@@ -113,3 +113,19 @@ def test_integer_sums_stay_in_registers(positions, width, segments, tmp_path):
     text = op_desc.unsorted_segment_sum([positions], [width], segments, "int32", "int32", "ints_%d_%d_%d" % (positions, width, segments))
     kernel, scratch, _ = compiled_notes(text, tmp_path)
     assert "grouped by bucket of segments" in kernel.source and scratch == 0
+
+
+@pytest.mark.parametrize("positions,width,segments,dtype,values", [
+    (65101, 4, 1536, "bfloat16", 16), (579545, 2, 16024, "float16", 16), (100000, 2, 196, "float16", 16), (100000, 2, 195, "float16", 48),   # 510 and 514 positions a segment
+    (4405314, 4, 901, "bfloat16", 48), (65101, 4, 1536, "float32", 48), (365857, 3, 609, "int32", 16),
+])
+def test_values_of_a_list_in_flight(positions, width, segments, dtype, values):
+    kernel = driver.HipKernel(op_desc.unsorted_segment_sum([positions], [width], segments, dtype, "int32", "flight_%s_%d_%d_%d" % (dtype, positions, width, segments)), out_dir=None)
+    assert "constexpr int ADD_BLOCK = %d;" % values in kernel.source
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("positions,width,segments,dtype", [(65101, 4, 1536, "bfloat16"), (100000, 2, 196, "float16"), (100000, 2, 195, "float16"), (70001, 4, 2000, "int32")])
+def test_lists_with_fewer_and_more_values_in_flight(positions, width, segments, dtype, tmp_path):
+    for pattern in ("uniform", "one_segment"):
+        _check_bits(positions, width, segments, dtype, "int32", pattern, tmp_path)
